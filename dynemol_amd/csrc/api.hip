@@ -1531,7 +1531,13 @@ static int multi_coefficients(dh_system* s, double dt, int m, int* Kq) {
             for (int k = Kq[q] + 1; k <= Kq[q - 1] + 1; ++k) row[k] = cplx{0.0, 0.0};
             Kq[q] = Kq[q - 1];
         }
-    for (int q = 0; q < m; ++q) s->kq_h[q] = Kq[q];
+    // a panel pass reads a row up to PANEL terms past its last one: zeros there,
+    // not what an earlier series left in the staging row
+    for (int q = 0; q < m; ++q) {
+        cplx* row = s->coefm_h + (size_t)q * CS;
+        for (int k = Kq[q] + 1; k <= std::min(Kq[q] + PANEL, CS - 1); ++k) row[k] = cplx{0.0, 0.0};
+        s->kq_h[q] = Kq[q];
+    }
     DH_HIP(hipMemcpyAsync(s->coefm, s->coefm_h, sizeof(cplx) * (size_t)m * CS, hipMemcpyHostToDevice, st));
     DH_HIP(hipMemcpyAsync(s->kq_d, s->kq_h, sizeof(int) * m, hipMemcpyHostToDevice, st));
     DH_HIP(hipEventRecord(s->coefm_ev, st));
