@@ -68,6 +68,7 @@ static int scratch_setup(int device) {
 
 struct dh_context {
     int device = 0;
+    int cus = 0;  // compute units that a cooperative launch can fill (0: no cooperative launches)
     hipStream_t stream = nullptr;
     // shared workspace for operator builds (one build at a time per context)
     int ws_ld = 0;
@@ -225,8 +226,12 @@ extern "C" int dh_init(int device, dh_context** out) {
     DH_HIP(hipSetDevice(device));
     const int src = scratch_setup(device);
     if (src) return src;
+    int cus = 0, coop = 0;
+    DH_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    DH_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device));
     dh_context* c = new dh_context();
     c->device = device;
+    c->cus = coop ? cus : 0;
     DH_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     if (dalloc(&c->d_info, 1)) {
         delete c;
@@ -1030,12 +1035,39 @@ struct SeriesOps {
     const int* Kq = nullptr;  // the same table on the host
     cplx* ring = nullptr;
     long ring_stride = 0;
+    // > 0: the series may run in one launch with H resident on that many compute
+    // units (series.hip), its exchange ring in `partial` (partial_cplx elements)
+    int cus = 0;
+    long partial_cplx = 0;
 };
 
+// whether a series of these operands runs in one launch (else one per term):
+// FP64, the operator fits the chip, and no term kernel is forced
+static bool series_resident(const dh_context* c, int prec, int ld, int R) {
+    return prec == 0 && !matvec_forced() && resident_series_fits(ld, R, c->cus);
+}
 
 static int series_core(const SeriesOps& o, hipStream_t st) {
     const int R = o.R;
     const double c = o.c, r = o.r;
+    if (o.cus > 0) {
+        ResidentArgs ra{};
+        ra.H = o.H;
+        ra.ld = o.ld;
+        ra.N = o.N;
+        ra.R = R;
+        ra.m = o.m > 0 ? o.m : 1;
+        ra.K = o.K;
+        ra.c = c;
+        ra.r = r;
+        ra.phi = o.phi;
+        ra.acc = o.m > 0 ? o.accm : o.acc;
+        ra.acc_stride = o.accm_stride;
+        ra.coef = o.m > 0 ? o.coefm : o.coef;
+        ra.coef_stride = o.coefm_stride;
+        ra.kq = o.m > 0 ? o.kq : nullptr;
+        if (launch_resident_series(ra, o.partial, o.partial_cplx * (long)sizeof(cplx), o.cus, st)) return DH_OK;
+    }
     MatvecArgs a{};
     a.M = o.H;
     a.ld = o.ld;
@@ -1151,8 +1183,10 @@ static int series_core(const SeriesOps& o, hipStream_t st) {
 }
 
 // One Chebyshev evaluation phi <- sum_k a_k T_k(Hh) phi, result in s->acc.
-static int series_launches(dh_system* s) {
+static int series_launches(dh_system* s, bool one_launch = true) {
     SeriesOps o{};
+    o.partial_cplx = partial_cplx_for(s->N, s->W);
+    if (one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) o.cus = s->ctx->cus;
     o.H = s->Hth;
     o.H32 = s->H32;
     o.Hlo = s->Hlo;
@@ -1183,9 +1217,11 @@ static int series_launches(dh_system* s) {
 // The term series as one hipGraph launch: captured once per (K, bounds, buffer
 // assignment, precision, term kernel) and replayed on later steps.  The series
 // is kernels only (no memset nodes, no host synchronisation).
-static int chebyshev_series(dh_system* s) {
-    // the FP32-product modes call rocBLAS, which stays out of stream capture
-    if (!s->use_graph || fp32_products(s)) return series_launches(s);
+static int chebyshev_series(dh_system* s, bool one_launch = true) {
+    // the FP32-product modes call rocBLAS, which stays out of stream capture; a
+    // series in one launch has nothing to capture
+    if (!s->use_graph || fp32_products(s)) return series_launches(s, one_launch);
+    if (one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) return series_launches(s);
     hipStream_t st = s->ctx->stream;
     const int variant = matvec_variant_for(s->N, 2 * s->W, TRI_FULL);
     for (auto& g : s->graphs)
@@ -1201,7 +1237,7 @@ static int chebyshev_series(dh_system* s) {
         g.exec = nullptr;
     }
     DH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    const int rc = series_launches(s);
+    const int rc = series_launches(s, false);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(st, &graph);
     if (rc) {
@@ -1260,7 +1296,7 @@ static void launch_outputs(dh_system* s) {
 // One step of dt (eV^-1) with the norm check: the term series, the new state's
 // norms and the outputs, then one host wait; a step whose norm drifts is
 // redone with wider bounds (at most 4 attempts).  phi holds the current state.
-static int propagate_checked(dh_system* s, double dt, int* n_terms) {
+static int propagate_checked(dh_system* s, double dt, int* n_terms, bool one_launch = true) {
     hipStream_t st = s->ctx->stream;
     const int R = 2 * s->W;
     launch_column_norms(s->N, R, s->phi, s->norms0, st);
@@ -1273,7 +1309,9 @@ static int propagate_checked(dh_system* s, double dt, int* n_terms) {
         int rc = ensure_coefficients(s, dt);
         if (rc) return rc;
         if (s->timing) DH_HIP(hipEventRecord(s->ev0, st));
-        rc = chebyshev_series(s);
+        // a repeat runs one launch per term: it also covers a series in one launch
+        // that gave up waiting (NaN norms)
+        rc = chebyshev_series(s, one_launch && attempt == 0);
         if (rc) return rc;
         if (s->timing) DH_HIP(hipEventRecord(s->ev1, st));
         std::swap(s->phi, s->acc);  // phi <- new state; acc keeps the old one
@@ -1304,9 +1342,10 @@ static int propagate_checked(dh_system* s, double dt, int* n_terms) {
             if (n_terms) *n_terms = s->K + 1;
             return DH_OK;
         }
-        // the bounds did not enclose the spectrum: restore and widen
+        // the bounds did not enclose the spectrum: restore and widen (NaN norms
+        // after a series in one launch say nothing about the bounds)
         std::swap(s->phi, s->acc);
-        s->widen *= 1.25;
+        if (attempt > 0 || std::isfinite(drift)) s->widen *= 1.25;
         s->stats[3] += 1;
     }
     // outputs of the restored (pre-step) state, as before the call
@@ -1591,6 +1630,8 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     o.ring = s->ring;
     o.ring_stride = acc_n;
     o.K = Kq[m - 1];
+    o.partial_cplx = partial_cplx_for(s->N, s->W);
+    if (series_resident(s->ctx, s->precision, s->ld, R)) o.cus = s->ctx->cus;
     if (int rc = series_core(o, st)) return rc;
     DH_HIP(hipGetLastError());
     *kmax = Kq[m - 1];
@@ -1771,7 +1812,7 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
             DH_HIP(hipMemcpyAsync(s->phi, d.ck_phi, sizeof(cplx) * s->ld * R, hipMemcpyDeviceToDevice, st));
             DH_HIP(hipMemcpyAsync(s->out, d.ck_out, sizeof(cplx) * s->ld * 3 * W, hipMemcpyDeviceToDevice, st));
             for (int i = j; i < jend; ++i) {
-                if ((rc = propagate_checked(s, dt, &last_terms))) return rc;
+                if ((rc = propagate_checked(s, dt, &last_terms, false))) return rc;
                 DH_HIP(hipMemcpyAsync(d.pops + (size_t)i * W * NP, s->pops, sizeof(double) * W * NP,
                                       hipMemcpyDeviceToDevice, st));
                 DH_HIP(hipMemcpyAsync(d.erg + (size_t)i * W * 2, s->erg, sizeof(double) * W * 2,
@@ -1866,6 +1907,7 @@ extern "C" int dh_propagation_elhl(dh_context* ctx, const int* Np, const double*
 // counters, Bessel table and coefficients, norms; 256-byte aligned pieces.
 struct ApplyWork {
     cplx *x0, *x1, *acc, *partial;
+    long partial_cplx;
     unsigned* counters;
     double *J, *norms0, *norms1;
     cplx* coef;
@@ -1888,6 +1930,7 @@ static size_t apply_layout(int N, int R, char* base, ApplyWork* w) {
     t.x1 = (cplx*)take(sizeof(cplx) * ld * R);
     t.acc = (cplx*)take(sizeof(cplx) * ld * R);
     t.partial = (cplx*)take(sizeof(cplx) * part);
+    t.partial_cplx = part;
     t.counters = (unsigned*)take(sizeof(unsigned) * ld);
     t.J = (double*)take(sizeof(double) * (KMAX_ALLOC + 2));
     t.coef = (cplx*)take(sizeof(cplx) * (KMAX_ALLOC + 2));
@@ -1936,6 +1979,8 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
     o.counters = w.counters;
     o.coef = w.coef;
     o.prec = 0;
+    o.partial_cplx = w.partial_cplx;
+    const bool one_launch = series_resident(ctx, 0, ldh, R);
     double widen = 1.0, drift = 0.0;
     double n0[8], n1[8];  // R <= 8 (check_apply_args); no host allocation on this path
     for (int attempt = 0; attempt < 4; ++attempt) {
@@ -1953,6 +1998,7 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
         o.K = K;
         o.c = c;
         o.r = r;
+        o.cus = one_launch && attempt == 0 ? ctx->cus : 0;
         if (int rc = series_core(o, st)) return rc;
         launch_column_norms(N, R, w.acc, w.norms1, st);
         DH_HIP(hipGetLastError());
@@ -1970,7 +2016,9 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
             if (n_terms) *n_terms = K + 1;
             return DH_OK;
         }
-        widen *= 1.25;  // the bounds did not enclose the spectrum; phi is untouched
+        // the bounds did not enclose the spectrum (NaN norms after a series in one
+        // launch: it gave up waiting, and runs again term by term); phi is untouched
+        if (attempt > 0 || std::isfinite(drift)) widen *= 1.25;
     }
     dh::set_error("dh_chebyshev_apply: Chebyshev series lost the norm (drift %g) after widening the bounds", drift);
     return DH_ERR_DIVERGED;

@@ -2267,6 +2267,7 @@ void matvec_set_tuned(int N, int R, int tri, int variant) {
     g_tuned.push_back({TuneKey{N, R, tri}, variant});
 }
 void matvec_force_variant(int v) { g_variant_override = v; }
+bool matvec_forced() { return g_variant_override >= 0; }
 int matvec_variant_count() { return MV_VARIANTS; }
 
 void launch_matvec_variant(const MatvecArgs& a, int variant, hipStream_t st) {

@@ -202,6 +202,7 @@ int matvec_variant_for(int N, int R, int tri);
 void matvec_set_tuned(int N, int R, int tri, int variant);
 bool matvec_is_tuned(int N, int R, int tri);
 void matvec_force_variant(int v);
+bool matvec_forced();
 int matvec_variant_count();
 void launch_cheb_gemm(const MatvecArgs& a, int prec, hipStream_t st);
 // split-K matrix-core term GEMM (prec 0: FP64, 1: FP32 products on M32, 2: FP64
@@ -249,6 +250,30 @@ void launch_to_bf16(const float* a, unsigned short* b, long n, hipStream_t st);
 void launch_lib_reduce(const MatvecArgs& a, const float* Phi, const float* Plo, int S, hipStream_t st);
 void launch_identity_pad(double* S, double* h, int N, int ld, hipStream_t st);
 
+
+// ---------------------------------------------------------------- resident series (series.hip)
+// A whole Chebyshev series (one launch, H resident on the chip): accumulator q
+// < m at acc + q * acc_stride takes sum_k coef[q * coef_stride + k] T_k over
+// k <= kq[q] (device table; null: k <= K for the one accumulator), Hh = (H - c)
+// / r, T_0 = phi (N x R row-major).  H: ld x ld, symmetric, rows and columns >=
+// N zero off the diagonal.  The last four fields are the launcher's.
+struct ResidentArgs {
+    const double* H;
+    int ld, N, R, m, K;
+    double c, r;
+    const cplx* phi;
+    cplx* acc;
+    long acc_stride;
+    const cplx* coef;
+    int coef_stride;
+    const int* kq;
+    char* ring;
+    int slots, slot_bytes;
+    unsigned* flags;
+};
+bool resident_series_fits(int ld, int R, int cus);
+// false: not launched (shape, scratch or device do not allow it)
+bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, int cus, hipStream_t st);
 
 // Small grouped helpers for multi-system batches.
 struct NormTask {

@@ -1,4 +1,11 @@
-"""Multi-step Chebyshev series (dh_propagate_steps): coefficients and accumulators."""
+"""A Chebyshev series in one launch with the operator resident on the chip (series.hip).
+
+The same propagation term by term (a forced matvec variant) is the comparison:
+both evaluate the same FP64 series of about 63 terms on an operator of half
+width 34 eV, and the recurrence carries each term's rounding (a dot product of
+N terms, below 1e-15 of the state's norm) at most K times, so the two differ by
+less than 63^2 * 1e-15 = 4e-12 of the norm; 1e-11 is asserted.
+"""
 import numpy as np
 import pytest
 
@@ -14,6 +21,53 @@ def ctx():
     c = hip.Context(0)
     yield c
     c.close()
+
+
+@pytest.fixture(scope="module")
+def operator():
+    """One 4160 x 4160 symmetric matrix; its leading blocks are the operators."""
+    rng = np.random.default_rng(5)
+    x = rng.normal(size=(4160, 4160))
+    return x + x.T
+
+
+def _apply(ctx, operator, N, R, variant):
+    ld = (N + 63) // 64 * 64
+    H = np.eye(ld)
+    H[:N, :N] = operator[:N, :N] * (34.0 / np.sqrt(8.0 * N))
+    H[np.arange(N), np.arange(N)] -= 6.0
+    rng = np.random.default_rng(N + R)
+    phi = np.full((ld, R), 7.0 + 3.0j)  # rows past N: the call clears them
+    phi[:N] = (rng.normal(size=(N, R)) + 1j * rng.normal(size=(N, R))) / np.sqrt(2.0 * N)
+    bufs = [hip.DeviceBuffer(H.nbytes), hip.DeviceBuffer(phi.nbytes), hip.DeviceBuffer(hip.chebyshev_work_bytes(N, R))]
+    try:
+        bufs[0].upload(H)
+        bufs[1].upload(phi)
+        # a dirty work buffer: nothing in it may be taken for data
+        bufs[2].upload(np.full(bufs[2].nbytes // 8, np.nan))
+        hip.force_matvec_variant(variant)
+        k = hip.chebyshev_apply(ctx, N, bufs[0].ptr, ld, [-42.0, 30.0], DT, R, bufs[1].ptr, bufs[2].ptr,
+                                bufs[2].nbytes)
+        return bufs[1].download((ld, R), np.complex128), k
+    finally:
+        hip.force_matvec_variant(-1)
+        for b in bufs:
+            b.close()
+
+
+# edges of the tiles (16 rows and 128 columns per group of the 8 waves), of the register and LDS parts of
+# the operator (N = 2944: the last of it in registers at R = 4), of the rows per workgroup at R = 8
+# (2048) and of the sizes that stay resident (3584 at R = 8, 4096); 3585 and 4097 run term by term
+@pytest.mark.parametrize("N,R", [(1, 2), (16, 4), (63, 1), (64, 8), (65, 4), (129, 2), (130, 8), (960, 4), (1025, 8),
+                                 (1100, 4), (2048, 8), (2049, 8), (2944, 4), (3000, 4), (3009, 1), (3584, 8),
+                                 (3585, 8), (4096, 4), (4096, 2), (4097, 2)])
+def test_series_matches_terms(ctx, operator, N, R):
+    print(f"[gpu] series in one launch, N={N}, R={R}", flush=True)
+    a, ka = _apply(ctx, operator, N, R, -1)
+    b, kb = _apply(ctx, operator, N, R, 1)
+    assert ka == kb
+    assert np.linalg.norm(a - b) <= 1e-11 * np.linalg.norm(b)
+    assert np.abs(a[N:]).max(initial=0.0) == 0.0
 
 
 @pytest.mark.parametrize("variant", [15, 18, -1])
@@ -38,3 +92,28 @@ def test_short_series_after_a_long_one(ctx, variant):
     finally:
         hip.force_matvec_variant(-1)
     assert np.abs(out[0] - out[1]).max() < 1e-12 * np.abs(out[0]).max()
+
+
+@pytest.mark.parametrize("n_wp,n_steps", [(1, 1), (2, 23), (3, 12), (4, 11)])
+def test_multi_step_series(ctx, n_wp, n_steps):
+    """Several accumulators per series (up to 10 steps), 2 to 8 columns."""
+    st = ch_cluster(seed=1)
+    b = st.basis()
+    rng = np.random.default_rng(n_wp)
+    c = (rng.normal(size=(n_wp, b.N)) + 1j * rng.normal(size=(n_wp, b.N))) / np.sqrt(2.0 * b.N)
+    out = []
+    for variant in (-1, 1):
+        hip.force_matvec_variant(variant)
+        try:
+            s = hip.System(ctx, b, n_wp=n_wp, n_frag=2)
+            s.build(st.coords)
+            for w in range(n_wp):
+                s.set_initial_state(w, c[w], c[w])
+            pops, erg, _ = s.propagate_steps(n_steps, DT)
+            out.append((pops, erg, np.stack([s.wavepacket(w)[1] for w in range(n_wp)])))
+            s.close()
+        finally:
+            hip.force_matvec_variant(-1)
+    assert np.abs(out[0][0] - out[1][0]).max() < 1e-11 * np.abs(out[1][0]).max()
+    assert np.abs(out[0][1] - out[1][1]).max() < 1e-11 * np.abs(out[1][1]).max()
+    assert np.linalg.norm(out[0][2] - out[1][2]) <= 1e-11 * np.linalg.norm(out[1][2])
