@@ -10,6 +10,8 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace dh {
 
 constexpr int GK = 16;  // k-depth of one LDS stage
@@ -588,6 +590,20 @@ __global__ void identity_pad_kernel(double* S, double* h, int ld) {
 void launch_identity_pad(double* S, double* h, int N, int ld, hipStream_t st) {
     (void)N;
     hipLaunchKernelGGL(identity_pad_kernel, dim3(4096), dim3(256), 0, st, S, h, ld);
+}
+
+// rows x cols column-major block between two pitches (rows as lanes: coalesced
+// both ways; HBM-bound)
+__global__ __launch_bounds__(256) void repitch_kernel(double* __restrict__ dst, long ldd,
+                                                      const double* __restrict__ src, long lds, int rows) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < rows) dst[ldd * blockIdx.y + i] = src[lds * blockIdx.y + i];
+}
+void launch_repitch(double* dst, long ldd, const double* src, long lds, int rows, int cols, hipStream_t st) {
+    constexpr int MAX_Y = 32768;  // columns per launch (grid limit)
+    for (int c = 0; c < cols; c += MAX_Y)
+        hipLaunchKernelGGL(repitch_kernel, dim3((rows + 255) / 256, std::min(cols - c, MAX_Y)), dim3(256), 0, st,
+                           dst + ldd * c, ldd, src + lds * c, lds, rows);
 }
 
 }  // namespace dh

@@ -116,6 +116,7 @@ void launch_cholesky(double* A, int ld, double* Dinv, int* info, hipStream_t st)
 // work: ld * ld / 2 doubles
 void launch_trtri_lower(const double* L, double* Linv, const double* Dinv, int ld, double* work, hipStream_t st);
 void launch_symmetrize_from_lower(double* A, int ld, hipStream_t st);
+void launch_repitch(double* dst, long ldd, const double* src, long lds, int rows, int cols, hipStream_t st);
 void launch_copy_matrix(const double* src, double* dst, long n, hipStream_t st);
 
 // ---------------------------------------------------------------- propagation
