@@ -121,6 +121,9 @@ struct dh_system {
     int *kq_d = nullptr, *kq_h = nullptr;  // the accumulators' last terms (device; pinned staging)
     hipEvent_t coefm_ev = nullptr;
     bool coefm_pending = false;
+    int coefm_stride = 0;                  // row pitch of coefm
+    int coefm_m = 0, coefm_Kq[MULTI_MAX];  // what coefm holds: m rows for (dt, c, r)
+    double coefm_dt = 0.0, coefm_c = 0.0, coefm_r = 0.0;
     // observables
     double *pops = nullptr, *erg = nullptr, *norms = nullptr, *norms0 = nullptr, *norms1 = nullptr;
     // host state
@@ -1599,10 +1602,19 @@ static int multi_coefficients(dh_system* s, double dt, int m, int* Kq) {
         DH_HIP(hipHostMalloc((void**)&s->kq_h, sizeof(int) * MULTI_MAX, hipHostMallocDefault));
         DH_HIP(hipEventCreateWithFlags(&s->coefm_ev, hipEventDisableTiming));
     }
-    if (s->coefm_pending) DH_HIP(hipEventSynchronize(s->coefm_ev));  // the staging buffers are free again
     const double c = 0.5 * (s->emax + s->emin);
     const double r = 0.5 * (s->emax - s->emin) * s->widen;
-    for (int q = 0; q < m; ++q) {
+    if (m == s->coefm_m && dt == s->coefm_dt && c == s->coefm_c && r == s->coefm_r) {
+        for (int q = 0; q < m; ++q) Kq[q] = s->coefm_Kq[q];
+        return DH_OK;
+    }
+    if (s->coefm_pending) DH_HIP(hipEventSynchronize(s->coefm_ev));  // the staging buffers are free again
+    s->coefm_m = 0;
+    // the last row is the longest: its length sets the pitch, so that only the
+    // terms of this series are copied (a panel pass reads a row up to PANEL
+    // terms past its last one: zeros there)
+    int pitch = 0;
+    for (int q = m - 1; q >= 0; --q) {
         cplx* row = s->coefm_h + (size_t)q * CS;
         const int k = bessel_coef_host(r * (q + 1) * dt, c * (q + 1) * dt, KMAX_ALLOC, BESSEL_TOL, row);
         if (k <= 0 && r * dt > 1e-12) {
@@ -1610,23 +1622,24 @@ static int multi_coefficients(dh_system* s, double dt, int m, int* Kq) {
             return DH_ERR_STATE;
         }
         Kq[q] = k;
+        pitch = std::max(pitch, std::min(k + PANEL + 2, CS));
     }
-    for (int q = 1; q < m; ++q)
-        if (Kq[q] < Kq[q - 1]) {
-            cplx* row = s->coefm_h + (size_t)q * CS;
-            for (int k = Kq[q] + 1; k <= Kq[q - 1] + 1; ++k) row[k] = cplx{0.0, 0.0};
-            Kq[q] = Kq[q - 1];
-        }
-    // a panel pass reads a row up to PANEL terms past its last one: zeros there,
-    // not what an earlier series left in the staging row
     for (int q = 0; q < m; ++q) {
-        cplx* row = s->coefm_h + (size_t)q * CS;
-        for (int k = Kq[q] + 1; k <= std::min(Kq[q] + PANEL, CS - 1); ++k) row[k] = cplx{0.0, 0.0};
-        s->kq_h[q] = Kq[q];
+        const cplx* row = s->coefm_h + (size_t)q * CS;
+        cplx* to = s->coefm_h + (size_t)q * pitch;  // at or below row: moved in order
+        for (int k = 0; k <= Kq[q]; ++k) to[k] = row[k];
+        for (int k = Kq[q] + 1; k < pitch; ++k) to[k] = cplx{0.0, 0.0};
+        if (q > 0) Kq[q] = std::max(Kq[q], Kq[q - 1]);
+        s->kq_h[q] = s->coefm_Kq[q] = Kq[q];
     }
-    DH_HIP(hipMemcpyAsync(s->coefm, s->coefm_h, sizeof(cplx) * (size_t)m * CS, hipMemcpyHostToDevice, st));
+    s->coefm_stride = pitch;
+    DH_HIP(hipMemcpyAsync(s->coefm, s->coefm_h, sizeof(cplx) * (size_t)m * pitch, hipMemcpyHostToDevice, st));
     DH_HIP(hipMemcpyAsync(s->kq_d, s->kq_h, sizeof(int) * m, hipMemcpyHostToDevice, st));
     DH_HIP(hipEventRecord(s->coefm_ev, st));
+    s->coefm_m = m;
+    s->coefm_dt = dt;
+    s->coefm_c = c;
+    s->coefm_r = r;
     s->coefm_pending = true;
     return DH_OK;
 }
@@ -1642,7 +1655,6 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     hipStream_t st = s->ctx->stream;
     const int R = 2 * s->W;
     const long acc_n = (long)s->ld * R;
-    constexpr int CS = KMAX_ALLOC + 2;
     int Kq[MULTI_MAX];
     if (int rc = multi_coefficients(s, dt, m, Kq)) return rc;
     const double c = 0.5 * (s->emax + s->emin);
@@ -1671,7 +1683,7 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     o.accm = s->accm;
     o.accm_stride = acc_n;
     o.coefm = s->coefm;
-    o.coefm_stride = CS;
+    o.coefm_stride = s->coefm_stride;
     o.kq = s->kq_d;
     o.Kq = Kq;
     o.ring = s->ring;
@@ -2431,6 +2443,14 @@ struct dh_batch {
     // members in a precision mode other than FP64 run their own term series
     // (FP32 matrix-core GEMM or FP32-stored operator) inside the batch step
     std::vector<char> solo;
+    // solo[i] = 2: FP64 members whose series runs in launches of its own with the
+    // operators resident on the chip (series.hip), several members per launch
+    ResidentArgs* d_res = nullptr;  // [n]
+    int2* d_map = nullptr;  // map_cap entries (grown on demand)
+    size_t map_cap = 0;
+    std::vector<ResidentArgs> h_res;
+    std::vector<int2> h_map;
+    std::vector<ResidentRound> rounds;
     // host copies of the last uploaded tables: uploaded again only on change
     std::vector<MatvecArgs> h_args;
     std::vector<NormTask> h_norms;
@@ -2444,6 +2464,7 @@ struct dh_batch {
 // blocks, 1: symmetric half storage); every later batch of that R runs the
 // same kernels, so a system's arithmetic does not depend on its batch.
 static int g_batch_family[6] = {-1, -1, -1, -1, -1, -1};
+static bool g_batch_forced[6] = {};  // dh_test_force_batch_family: grouped term launches for every member
 static std::mutex g_batch_family_mu;
 static int batch_family_slot(int R) { return R == 2 ? 1 : R == 4 ? 2 : R == 8 ? 3 : R == 16 ? 4 : R == 32 ? 5 : 0; }
 
@@ -2494,8 +2515,9 @@ static std::vector<double> batch_graph_key(const dh_batch* b, bool multi) {
 // terms, outside the capture (the FP32-product modes call rocBLAS)
 static int batch_solo_series(dh_batch* b) {
     for (int i = 0; i < b->n; ++i)
-        if (b->solo[i])
+        if (b->solo[i] == 1)
             if (int rc = series_launches(b->sys[i])) return rc;
+    if (launch_resident_rounds(b->d_res, (int)b->h_res.size(), b->d_map, b->rounds, b->ctx->stream)) return DH_ERR_HIP;
     return DH_OK;
 }
 
@@ -2545,7 +2567,7 @@ extern "C" int dh_batch_destroy(dh_batch* b) {
     if (b->gexec) hipGraphExecDestroy(b->gexec);
     if (b->ev0) hipEventDestroy(b->ev0);
     if (b->ev1) hipEventDestroy(b->ev1);
-    void* ptrs[] = {b->d_args,  b->d_task_desc, b->d_task_blk, b->d_norms,  b->d_copy,  b->d_obs,  b->d_nval,
+    void* ptrs[] = {b->d_res, b->d_map, b->d_args,  b->d_task_desc, b->d_task_blk, b->d_norms,  b->d_copy,  b->d_obs,  b->d_nval,
                     b->d_t1_desc, b->d_t1_idx,  b->d_t2_desc,  b->d_t2_idx, b->d_sysS, b->d_panel, b->d_p_desc,
                     b->d_p_blk};
     for (void* p : ptrs)
@@ -2593,6 +2615,7 @@ extern "C" int dh_batch_create(dh_context* ctx, int n, dh_system* const* systems
     BALLOC(b->d_nval, (size_t)2 * n * R);
     long ptasks = 0;
     for (auto* s : b->sys) ptasks += ((long)s->N * R + 255) / 256;
+    BALLOC(b->d_res, (size_t)n);
     BALLOC(b->d_panel, (size_t)n);
     BALLOC(b->d_p_desc, (size_t)ptasks);
     BALLOC(b->d_p_blk, (size_t)ptasks);
@@ -2707,6 +2730,27 @@ static MatvecArgs batch_ring_desc(dh_system* s, int kind) {
     return a;
 }
 
+// Members whose series runs in resident launches: every FP64 member that fits,
+// unless a test asks for the grouped term kernels.
+static bool batch_member_resident(const dh_batch* b, dh_system* s, ResidentArgs* out = nullptr) {
+    {
+        std::lock_guard<std::mutex> lk(g_batch_family_mu);
+        if (g_batch_forced[batch_family_slot(b->R)]) return false;
+    }
+    if (s->precision != 0 || matvec_forced()) return false;
+    ResidentArgs a{};
+    a.H = s->Hth;
+    a.ld = s->ld;
+    a.N = s->N;
+    a.R = b->R;
+    a.m = 1;
+    a.phi = s->phi;
+    if (!resident_batch_member(&a, s->partial, partial_cplx_for(s->N, s->W) * (long)sizeof(cplx), b->ctx->cus))
+        return false;
+    if (out) *out = a;
+    return true;
+}
+
 // host -> device table copy, only when the content changed since the last copy
 // (from the batch's own copy, which outlives the asynchronous transfer)
 template <class T>
@@ -2717,6 +2761,54 @@ static int upload_if_changed(std::vector<T>& cache, const std::vector<T>& v, T* 
     cache = v;
     if (!cache.empty()) DH_HIP(hipMemcpyAsync(dst, cache.data(), sizeof(T) * cache.size(), hipMemcpyHostToDevice, st));
     return DH_OK;
+}
+
+// The resident members' tables for a series of m steps (1: the system's one-step
+// coefficients into acc, else its rows into accm).  A member that turns out not
+// to fit a launch sends every resident member back to the grouped kernels.
+static int batch_resident_tables(dh_batch* b, std::vector<char>& solo, int m, hipStream_t st) {
+    std::vector<ResidentArgs> res;
+    for (int i = 0; i < b->n; ++i) {
+        if (solo[i] != 2) continue;
+        dh_system* s = b->sys[i];
+        ResidentArgs a{};
+        if (!batch_member_resident(b, s, &a)) continue;
+        a.m = m;
+        a.c = 0.5 * (s->emax + s->emin);
+        a.r = 0.5 * (s->emax - s->emin) * s->widen;
+        if (m == 1) {
+            a.K = s->K;
+            a.acc = s->acc;
+            a.coef = s->coef;
+        } else {
+            a.K = s->coefm_Kq[m - 1];
+            a.acc = s->accm;
+            a.acc_stride = (long)s->ld * b->R;
+            a.coef = s->coefm;
+            a.coef_stride = s->coefm_stride;
+            a.kq = s->kq_d;
+        }
+        res.push_back(a);
+    }
+    std::vector<int2> map;
+    if (!resident_batch_rounds(res, b->ctx->cus, &map, &b->rounds)) {
+        for (char& c : solo)
+            if (c == 2) c = 0;
+        res.clear();
+        map.clear();
+        b->rounds.clear();
+    }
+    if (map.size() > b->map_cap) {
+        DH_HIP(hipStreamSynchronize(st));
+        if (b->d_map) hipFree(b->d_map);
+        b->d_map = nullptr;
+        b->map_cap = 0;
+        b->h_map.clear();
+        DALLOC(b->d_map, map.size());
+        b->map_cap = map.size();
+    }
+    if (int rc = upload_if_changed(b->h_res, res, b->d_res, st)) return rc;
+    return upload_if_changed(b->h_map, map, b->d_map, st);
 }
 
 // Times the first grouped term (k = 1: reads phi, writes x1 and acc, which the
@@ -2758,6 +2850,7 @@ extern "C" int dh_test_force_batch_family(int R, int family) {
               "dh_test_force_batch_family: bad argument");
     std::lock_guard<std::mutex> lk(g_batch_family_mu);
     g_batch_family[batch_family_slot(R)] = family;
+    g_batch_forced[batch_family_slot(R)] = family >= 0;
     return DH_OK;
 }
 
@@ -2866,7 +2959,7 @@ extern "C" int dh_batch_propagate(dh_batch* b, double t_init, double t_max, int*
     std::vector<char> solo(n);
     for (int i = 0; i < n; ++i) {
         dh_system* s = b->sys[i];
-        solo[i] = s->precision != 0;
+        solo[i] = s->precision != 0 ? 1 : batch_member_resident(b, s) ? 2 : 0;
         if (s->phi_dirty) {
             convert_ao_to_phi(s);
             s->phi_dirty = false;
@@ -2875,9 +2968,10 @@ extern "C" int dh_batch_propagate(dh_batch* b, double t_init, double t_max, int*
         if (rc) return rc;
     }
     // task tables by term count (descending); members in other precision modes
-    // add no grouped term tasks
+    // and resident ones add no grouped term tasks
     std::vector<int> Ks(n);
     for (int i = 0; i < n; ++i) Ks[i] = b->sys[i]->K;
+    if (int rc = batch_resident_tables(b, solo, 1, st)) return rc;
     const bool retable = Ks != b->Ks || solo != b->solo || b->prefix.empty();
     if (retable)
         if (int rc = batch_retable(b, Ks, solo, st)) return rc;
@@ -2911,18 +3005,19 @@ extern "C" int dh_batch_propagate(dh_batch* b, double t_init, double t_max, int*
             const double n0 = nv[(size_t)i * R + c], n1 = nv[(size_t)n * R + (size_t)i * R + c];
             const double d = n0 > 0 ? std::fabs(n1 - n0) / n0 : 0.0;
             if (!(d < tol)) ok[i] = 0;
+            if (!std::isfinite(n1)) ok[i] = -1;
             if (std::isfinite(d)) maxdrift = std::max(maxdrift, d);
         }
     }
     // commit acc -> phi for systems whose norm held
     std::vector<CopyTask> ct;
     for (int i = 0; i < n; ++i)
-        if (ok[i]) ct.push_back(CopyTask{b->sys[i]->acc, b->sys[i]->phi, (long)b->sys[i]->N * R});
+        if (ok[i] > 0) ct.push_back(CopyTask{b->sys[i]->acc, b->sys[i]->phi, (long)b->sys[i]->N * R});
     if (int rc = upload_if_changed(b->h_copy, ct, b->d_copy, st)) return rc;
     launch_grouped_copy(b->d_copy, (int)ct.size(), st);
     // the mixed mode's per-step FP64 norm restoration, as in its single step
     for (int i = 0; i < n; ++i)
-        if (ok[i] && fp32_products(b->sys[i]))
+        if (ok[i] > 0 && fp32_products(b->sys[i]))
             launch_renorm_columns(b->sys[i]->phi, b->sys[i]->N, R, b->d_nval + (size_t)i * R,
                                   b->d_nval + (size_t)n * R + (size_t)i * R, st);
     // outputs of every member
@@ -2945,14 +3040,15 @@ extern "C" int dh_batch_propagate(dh_batch* b, double t_init, double t_max, int*
     DH_HIP(hipStreamSynchronize(st));
     for (int i = 0; i < n; ++i) {
         dh_system* s = b->sys[i];
-        if (ok[i]) {
+        if (ok[i] > 0) {
             s->stats[0] = s->K + 1;
             s->stats[1] += 1;
             s->stats[2] += s->K + 3;
             continue;
         }
         // bounds did not enclose this system's spectrum: redo it alone with widening
-        s->widen *= 1.25;
+        // (NaN norms say nothing about the bounds)
+        if (ok[i] == 0 || solo[i] != 2) s->widen *= 1.25;
         s->stats[3] += 1;
         b->stats[3] += 1;
         int rc = dh_propagate(s, t_init, t_max, nullptr);
@@ -2979,10 +3075,14 @@ extern "C" int dh_batch_propagate_steps(dh_batch* b, int n_steps, double dt_ps, 
     const double dt = dt_ps / H_BAR;
     const int n = b->n, R = b->R;
     int done = 0, kmax_seen = 0;
-    bool all_fp64 = true;
-    for (auto* s : b->sys) all_fp64 = all_fp64 && s->precision == 0;
+    bool all_fp64 = true, all_resident = true;
+    for (auto* s : b->sys) {
+        all_fp64 = all_fp64 && s->precision == 0;
+        all_resident = all_resident && batch_member_resident(b, s);
+        if (int rc = check_ready(s, "dh_batch_propagate_steps")) return rc;
+    }
     // the first step tunes the batch (kernel family, task tables) as usual
-    if (b->prefix.empty() || !all_fp64 || !b->sym_ok) {
+    if ((b->prefix.empty() && !all_resident) || !all_fp64 || !b->sym_ok) {
         int k = 0;
         if (int rc = dh_batch_propagate(b, 0.0, dt_ps, &k)) return rc;
         kmax_seen = k;
@@ -2997,7 +3097,6 @@ extern "C" int dh_batch_propagate_steps(dh_batch* b, int n_steps, double dt_ps, 
         if (max_terms) *max_terms = kmax_seen;
         return DH_OK;
     }
-    const long cs = KMAX_ALLOC + 2;
     while (done < n_steps) {
         int m = std::min(MULTI_MAX, n_steps - done);
         for (auto* s : b->sys) {
@@ -3021,6 +3120,8 @@ extern "C" int dh_batch_propagate_steps(dh_batch* b, int n_steps, double dt_ps, 
             Ks[i] = Kq[m - 1];
         }
         std::vector<char> solo(n, 0);
+        for (int i = 0; i < n; ++i) solo[i] = batch_member_resident(b, b->sys[i]) ? 2 : 0;
+        if (int rc = batch_resident_tables(b, solo, m, st)) return rc;
         if (Ks != b->Ks || solo != b->solo || b->prefix.empty())
             if (int rc = batch_retable(b, Ks, solo, st)) return rc;
         // term descriptors over the members' rings; the output descriptors
@@ -3039,7 +3140,7 @@ extern "C" int dh_batch_propagate_steps(dh_batch* b, int n_steps, double dt_ps, 
             p.accm = s->accm;
             p.accm_stride = (long)s->ld * R;
             p.coefm = s->coefm;
-            p.coefm_stride = (int)cs;
+            p.coefm_stride = s->coefm_stride;
             p.ring = s->ring;
             p.ring_stride = (long)s->ld * R;
             p.phi = s->phi;
@@ -3120,7 +3221,7 @@ extern "C" int dh_batch_propagate_steps(dh_batch* b, int n_steps, double dt_ps, 
         b->stats[0] += m;
         b->stats[1] += b->Kmax;
         b->stats[2] = maxdrift;
-        kmax_seen = std::max(kmax_seen, b->Kmax + 1);
+        kmax_seen = std::max(kmax_seen, *std::max_element(Ks.begin(), Ks.end()) + 1);
         done += m;
     }
     if (max_terms) *max_terms = kmax_seen;

@@ -1,5 +1,7 @@
 // Kernel launchers shared between the translation units of the library.
 #pragma once
+#include <vector>
+
 #include "common.hpp"
 
 namespace dh {
@@ -257,7 +259,7 @@ void launch_identity_pad(double* S, double* h, int N, int ld, hipStream_t st);
 // < m at acc + q * acc_stride takes sum_k coef[q * coef_stride + k] T_k over
 // k <= kq[q] (device table; null: k <= K for the one accumulator), Hh = (H - c)
 // / r, T_0 = phi (N x R row-major).  H: ld x ld, symmetric, rows and columns >=
-// N zero off the diagonal.  The last four fields are the launcher's.
+// N zero off the diagonal.  The last five fields are the launcher's.
 struct ResidentArgs {
     const double* H;
     int ld, N, R, m, K;
@@ -269,12 +271,24 @@ struct ResidentArgs {
     int coef_stride;
     const int* kq;
     char* ring;
-    int slots, slot_bytes;
+    int slots, slot_bytes, groups;
     unsigned* flags;
 };
 bool resident_series_fits(int ld, int R, int cus);
 // false: not launched (shape, scratch or device do not allow it)
 bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, int cus, hipStream_t st);
+// Batches: whether a member can run so (fills in the launcher's fields), the
+// launches that cover the members (map: workgroup -> member, its workgroup
+// there), and the launches themselves with both tables on the device.
+struct ResidentRound {
+    const void* f;
+    int threads, lds, first, wgs;
+};
+bool resident_batch_member(ResidentArgs* a, void* scratch, long scratch_bytes, int cus);
+bool resident_batch_rounds(const std::vector<ResidentArgs>& members, int cus, std::vector<int2>* map,
+                           std::vector<ResidentRound>* rounds);
+int launch_resident_rounds(const ResidentArgs* d_members, int n, const int2* d_map,
+                           const std::vector<ResidentRound>& rounds, hipStream_t st);
 
 // Small grouped helpers for multi-system batches.
 struct NormTask {

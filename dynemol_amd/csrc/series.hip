@@ -21,13 +21,16 @@
 
 namespace dh {
 
-// Work split: workgroup b owns RB = 4 RG consecutive rows; its 8 waves split
-// the columns (the reduction index) into 8 ranges of `groups` 16-column groups.
+// Work split: workgroup b owns RB = 4 RG consecutive rows; its NW waves split
+// the columns (the reduction index) into NW ranges of `groups` 16-column groups.
 // A group's products are FP64 MFMA 4x4x4 in 4 blocks (lanes A: 16k + 4b + i,
-// B: 16k + 4b + j, D: 16i + 4b + j) with block b taking columns 4b..4b+3 of the
-// group, so a B operand (x) feeds every row group without replication: lane
-// 16k + 4b + j loads x[16g + 4b + k][j], 16 bytes (re, im) per lane, 1 KB
-// contiguous per wave.  A operands (H) stay in the lane's registers, up to what
+// B: 16k + 4b + j, D: 16i + 4b + j) with block b taking columns b, 4 + b, 8 + b,
+// 12 + b of the group, so a B operand (x) feeds every row group without
+// replication: lane 16k + 4b + j takes x[16g + 4k + b][j], 16 bytes (re, im).
+// The ring keeps the vectors in this order (per group of 16 rows and pass of 4
+// columns, the 64 lanes' values), so a load is 1 KB contiguous: in row-major
+// order its quarter-waves touched 4 half-used lines each, and a CU got 22 bytes
+// per clock.  A operands (H) stay in the lane's registers, up to what
 // 256 registers hold beside the products (23 groups at R = 4), and in LDS from
 // there on.  At R = 4 a group is 8 MFMAs of 16 cycles on one load; N = 4096: 32
 // groups per wave, 3.4 us of matrix-core time per term.
@@ -47,15 +50,12 @@ namespace dh {
 // waiting for good, the kernel drains, and its workgroup's accumulators are
 // written as NaN, which the caller's norm check turns into a repeat of the
 // step with one launch per term.
-constexpr int RS_WAVES = 8;
-constexpr int RS_THREADS = RS_WAVES * 64;
 // Copies of the flags, each polled by every RS_COPIES-th workgroup: with one
 // copy the 2048 waves' polls of the same few lines queue up at one memory
 // channel (a term at N = 4096, R = 4: 8.9 us with one copy, 7.6 with 8).
 constexpr int RS_COPIES = 16;
-constexpr int RS_NQ = (MULTI_MAX + RS_WAVES - 1) / RS_WAVES;  // accumulators per wave
-constexpr unsigned long long RS_WAIT_TICKS = 200000000ull;    // 2 s of the 100 MHz wall clock
-constexpr int AUX_DEVICE_SCOPE = 16;                          // buffer store: sc1
+constexpr unsigned long long RS_WAIT_TICKS = 200000000ull;  // 2 s of the 100 MHz wall clock
+constexpr int AUX_DEVICE_SCOPE = 16;                        // buffer store: sc1
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 // the coefficient table does not change during the launch: constant address
@@ -82,40 +82,62 @@ __device__ __forceinline__ double rs_block_sum(double v) {
 // (global stores may still be in flight, unlike with __syncthreads)
 __device__ __forceinline__ void rs_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// RC: passes of 4 complex columns over H per term (1: R <= 4, 2: R <= 8), a lane's
-// x being one complex column; 0: one pass of up to 4 real columns (R <= 2).
-// NT: groups per wave, a compile-time count so that the loads of x run ahead of
-// the products through the whole unrolled sequence.
-constexpr int rs_most(int rc) { return rc == 0 ? 24 : rc == 1 ? 23 : 20; }
-template <int RG, int NT, int RC>
-__global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const ResidentArgs a) {
+// RC: column class.  1 (R <= 4): a lane's x is one complex column; 0 (R <= 2): one
+// of up to 4 real columns; 2 (R <= 8): 16 real columns fill a 16x16x4 MFMA (WIDE,
+// 16 rows per workgroup: A is H as loaded with lanes (k, row), B one real column
+// per lane, no block sums; measured 64 cycles per 1024 products where the 4x4x4
+// form takes 80 to 88), or with 8 rows (RG = 2) two sets of 4 complex columns.
+// NT: the most groups per wave, a compile-time count so that the loads of x run
+// ahead of the products through the whole unrolled sequence (groups past the
+// system's own count are zero, so the sums do not depend on NT).  blk of nblk:
+// this workgroup's place in its system.
+constexpr int rs_most(int rc) { return rc == 0 ? 24 : rc == 1 ? 23 : 22; }
+// Groups of x in flight per wave: the loads of a term are bound by their
+// latency, so as many as the registers beside H hold.  Up to 8 groups of a
+// WIDE kernel this leaves room for three waves per SIMD.
+constexpr int rs_depth(int rg, int nt, int nreg, int rc) {
+    const int d = rg == 2    ? 6
+                  : rc == 2  ? (nt > 8 ? (180 - 8 * nreg) / 8 : (88 - 8 * nreg) / 8)
+                  : nreg > 20 ? 4
+                             : (184 - 8 * nreg) / 4;
+    return d < 2 ? std::min(2, nt) : std::min(d, nt);
+}
+template <int NW, int RG, int NT, int RC>
+__device__ __forceinline__ void resident_body(const ResidentArgs& a, const int blk, const int nblk) {
     constexpr int NREG = RG == 4 && NT > rs_most(RC) ? rs_most(RC) : NT, NL = NT - NREG;
-    constexpr bool PAIR = RC > 0;
-    constexpr int RB = 4 * RG, np = PAIR ? RC : 1;
-    // x loads in flight per wave: what the registers beside H allow
-    constexpr int DEPTH = std::min(NT, RG == 2 ? 6 : NREG > 20 ? 4 : NREG > 12 ? 6 : 8);
+    constexpr int NQ = (MULTI_MAX + NW - 1) / NW;  // accumulators per wave
+    constexpr bool PAIR = RC > 0, WIDE = RC == 2 && RG == 4;
+    constexpr int RB = 4 * RG;
+    constexpr int PT = RC == 2 && !WIDE ? 2 : 1;  // column sets
+    constexpr int XL = WIDE ? 2 : PT;             // loads of x per group
+    constexpr int PC = WIDE ? 8 : 4;              // columns per row of a wave's partial sums
+    constexpr int DEPTH = rs_depth(RG, NT, NREG, RC);
     using xv_t = typename std::conditional<PAIR, double2, double>::type;
     extern __shared__ double smem[];
     const int R = a.R;
-    constexpr int n = NT;
-    double* const hs = smem;                                       // [NL][8][RG][64]
-    cplx* const part = reinterpret_cast<cplx*>(hs + NL * RS_WAVES * RG * 64);  // [np][8][RB * 4]
-    cplx* const ts = part + np * RS_WAVES * RB * 4;                // [3][RB * R]: the last three terms' own rows
+    const int n = a.groups;
+    double* const hs = smem;                                       // [NL][NW][RG][64]
+    cplx* const part = reinterpret_cast<cplx*>(hs + NL * NW * RG * 64);  // [PT][NW][RB * PC]
+    cplx* const ts = part + PT * NW * RB * PC;                           // [3][RB * R]: the last three terms' own rows
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int lk = lane >> 4, lb = (lane >> 2) & 3, lj = lane & 3;
     const int N = a.N, ld = a.ld;
-    const int r0 = blockIdx.x * RB, k0 = w * n * 16;
+    const int r0 = blk * RB, k0 = w * n * 16;
     const bool active = k0 < ld;      // this wave has columns
     const int E = RB * R;             // own elements
 
-    // H: rows r0 + 4 rg + lj, columns k0 + 16 g + 4 lb + lk; ld is a multiple of
-    // 64, so a group lies inside the matrix or past it (zero) as a whole
+    // H: rows r0 + 4 rg + lj, columns k0 + 16 g + 4 lk + lb (WIDE: row r0 + (lane &
+    // 15), columns k0 + 16 g + 4 rg + lk, read as the transposed element: 16 lanes
+    // contiguous either way); ld is a multiple of 64, so a group lies inside the
+    // matrix or past it (zero) as a whole
     const int ng = active ? min(n, (ld - k0) / 16) : 0;
     double h[NREG][RG];
-    const double* const hcol = a.H + (long)ld * (r0 + lj) + 4 * lb + lk;
+    const double* const hcol =
+        a.H + (WIDE ? r0 + (lane & 15) + (long)ld * lk : (long)ld * (r0 + lj) + 4 * lk + lb);
     auto hval = [&](int g, int rg) {
-        const double v = hcol[(long)ld * (4 * rg) + (g < ng ? k0 + 16 * g : 0)];
+        const long col = g < ng ? k0 + 16 * g : 0;
+        const double v = hcol[WIDE ? (long)ld * (col + 4 * rg) : (long)ld * (4 * rg) + col];
         return g < ng ? v : 0.0;
     };
 #pragma unroll
@@ -125,38 +147,51 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
 #pragma unroll 1
     for (int g = 0; g < NL; ++g)
 #pragma unroll
-        for (int rg = 0; rg < RG; ++rg) hs[((g * RS_WAVES + w) * RG + rg) * 64 + lane] = hval(NREG + g, rg);
+        for (int rg = 0; rg < RG; ++rg) hs[((g * NW + w) * RG + rg) * 64 + lane] = hval(NREG + g, rg);
 
-    // the wave's accumulators: q = w + 8 v, elements lane + 64 u of the workgroup's rows
+    // the wave's accumulators: q = w + NW v, elements lane + 64 u of the workgroup's rows
     constexpr int NE = (RB * (PAIR ? 4 * RC : 2) + 63) / 64;
-    cplx acc[RS_NQ][NE];
-    int kq[RS_NQ];
+    cplx acc[NQ][NE];
+    int kq[NQ];
 #pragma unroll
-    for (int v = 0; v < RS_NQ; ++v) {
-        const int q = w + RS_WAVES * v;
+    for (int v = 0; v < NQ; ++v) {
+        const int q = w + NW * v;
         kq[v] = q < a.m ? (a.kq ? __builtin_amdgcn_readfirstlane(a.kq[q]) : a.K) : -1;
     }
     const __amdgpu_buffer_rsrc_t ring =
         __builtin_amdgcn_make_buffer_rsrc(a.ring, 0, (int)(a.slots * a.slot_bytes), 0x00020000);
-    // element e's place in a slot: its row-major position
+    constexpr int gbytes = XL * 64 * (int)sizeof(xv_t);  // a group's part of a slot
+    // element e of the workgroup's rows goes to its lane's place (WIDE: load q
+    // holds rows 8 q + k and 8 q + 4 + k of lane 16k + real column side by side)
     auto publish = [&](int e, cplx T, int slot) {
+        const int row = r0 + e / R, col = e % R;
+        const int to = (row >> 4) * gbytes, so = slot * a.slot_bytes;
         v4i bits;
         bits[0] = __double2loint(T.re);
         bits[1] = __double2hiint(T.re);
         bits[2] = __double2loint(T.im);
         bits[3] = __double2hiint(T.im);
-        __builtin_amdgcn_raw_buffer_store_b128(bits, ring, (r0 * R + e) * 16, slot * a.slot_bytes, AUX_DEVICE_SCOPE);
+        if constexpr (WIDE) {
+            const int at = to + (row >> 3 & 1) * 1024 + (16 * (row & 3) + 2 * col) * 16 + (row >> 2 & 1) * 8;
+            __builtin_amdgcn_raw_buffer_store_b64(bits.xy, ring, at, so, AUX_DEVICE_SCOPE);
+            __builtin_amdgcn_raw_buffer_store_b64(bits.zw, ring, at + 16, so, AUX_DEVICE_SCOPE);
+        } else {
+            const int at = 16 * (row >> 2 & 3) + 4 * (row & 3) + (PAIR ? (col & 3) + 64 * (col >> 2) : 2 * col);
+            __builtin_amdgcn_raw_buffer_store_b128(bits, ring, to + at * (int)sizeof(xv_t), so, AUX_DEVICE_SCOPE);
+        }
     };
+    // waves 0..SW-1 add up the waves' sums and publish 64 elements each; a flag per
+    // publishing wave
+    constexpr int SW = RB * (PAIR ? 4 * RC : 2) > 64 ? 2 : 1;
     auto raise = [&](unsigned v) {  // after this wave's stores have arrived
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (lane < RS_COPIES)
-            __hip_atomic_store(a.flags + lane * (int)gridDim.x + blockIdx.x, v, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(a.flags + (lane * nblk + blk) * SW + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
 
     // T_0 = phi (rows >= N as zero)
-    if (w == 0) {
-        for (int e = lane; e < E; e += 64) {
+    if (w < SW) {
+        for (int e = lane + 64 * w; e < min(E, 64 * (w + 1)); e += 64) {
             const int row = r0 + e / R;
             const cplx T = row < N ? a.phi[(long)r0 * R + e] : cplx{0.0, 0.0};
             publish(e, T, 0);
@@ -166,31 +201,25 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
     }
     rs_lds_barrier();
 #pragma unroll
-    for (int v = 0; v < RS_NQ; ++v)
+    for (int v = 0; v < NQ; ++v)
         if (kq[v] >= 0) {
-            const cplx c0 = rs_coef(a.coef + (long)(w + RS_WAVES * v) * a.coef_stride);
+            const cplx c0 = rs_coef(a.coef + (long)(w + NW * v) * a.coef_stride);
 #pragma unroll
             for (int u = 0; u < NE; ++u)
                 if (lane + 64 * u < E) acc[v][u] = cmul(c0, ts[lane + 64 * u]);
         }
 
-    // this lane's x of the wave's group g: row k0 + 16 g + 4 lb + lk, column
-    // 4 p + lj (columns past the last read it again; their sums are not kept).
-    // Groups past ld read the last one (their H is zero).
-    const int C2 = PAIR ? R : 2 * R;  // x values per row
-    const int xbytes = (int)sizeof(xv_t);
-    const int gstride = 16 * R * 16;
     // flags of the rows this wave reads
-    const int f0 = k0 / RB, nf = active ? (min(k0 + 16 * n, ld) + RB - 1) / RB - f0 : 0;
-    const unsigned* const myflag = a.flags + (int)(blockIdx.x % RS_COPIES) * (int)gridDim.x + f0 + min(lane, max(nf - 1, 0));
+    const int f0 = k0 / RB, nf = active ? ((min(k0 + 16 * n, ld) + RB - 1) / RB - f0) * SW : 0;
+    const unsigned* const myflag = a.flags + ((blk % RS_COPIES) * nblk + f0) * SW + min(lane, max(nf - 1, 0));
     bool dead = false;
     const double a1 = 1.0 / a.r, b1 = -a.c / a.r;
     const int K = max(a.K, 1);
     for (int k = 1; k <= K; ++k) {
-        cplx ck[RS_NQ];
+        cplx ck[NQ];
 #pragma unroll
-        for (int v = 0; v < RS_NQ; ++v)
-            if (k <= kq[v]) ck[v] = rs_coef(a.coef + (long)(w + RS_WAVES * v) * a.coef_stride + k);
+        for (int v = 0; v < NQ; ++v)
+            if (k <= kq[v]) ck[v] = rs_coef(a.coef + (long)(w + NW * v) * a.coef_stride + k);
         if (active) {
             if (!dead) {
                 unsigned long long t0 = 0;
@@ -210,65 +239,75 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
             asm volatile("" ::: "memory");
             const int slot = (k - 1) % a.slots;
             if (slot == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            // PT passes together (their loads and products interleave), where the
-            // registers allow
-            constexpr int PT = RG == 4 ? 1 : np;
-#pragma unroll 1
-            for (int p0 = 0; p0 < np; p0 += PT) {
-                int xoff[PT];
+            // (columns past the last are not written: their sums are not kept;
+            // groups past ld read the last one: their H is zero)
+            const int xoff = lane * (int)sizeof(xv_t);
+            const int soff = slot * a.slot_bytes + (k0 >> 4) * gbytes;
+            auto xload = [&](int g, int p) -> xv_t {
+                const int so = soff + min(g, max(ng, 1) - 1) * gbytes;
+                if constexpr (PAIR)
+                    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(ring, xoff + p * 1024, so, 0));
+                else
+                    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ring, xoff, so, 0));
+            };
+            double yr[PT][RG], yi[PT][RG];
+            v4d yw[2];  // WIDE: even and odd steps of 4 columns
 #pragma unroll
-                for (int p = 0; p < PT; ++p)
-                    xoff[p] = ((k0 + 4 * lb + lk) * C2 + min(4 * (p0 + p) + lj, C2 - 1)) * xbytes;
-                const int soff = slot * a.slot_bytes;
-                auto xload = [&](int g, int p) -> xv_t {
-                    const int so = soff + min(g, max(ng, 1) - 1) * gstride;
-                    if constexpr (PAIR)
-                        return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(ring, xoff[p], so, 0));
-                    else
-                        return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ring, xoff[p], so, 0));
-                };
-                double yr[PT][RG], yi[PT][RG];
+            for (int p = 0; p < PT; ++p)
 #pragma unroll
-                for (int p = 0; p < PT; ++p)
+                for (int rg = 0; rg < RG; ++rg) yr[p][rg] = yi[p][rg] = 0.0;
+            yw[0] = yw[1] = (v4d){0.0, 0.0, 0.0, 0.0};
+            // the products of load p of a group with its operator values
+            auto mma = [&](const double (&hv)[RG], xv_t x, int p) {
+                if constexpr (WIDE) {
+                    yw[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(hv[2 * p], x.x, yw[0], 0, 0, 0);
+                    yw[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(hv[2 * p + 1], x.y, yw[1], 0, 0, 0);
+                } else {
 #pragma unroll
-                    for (int rg = 0; rg < RG; ++rg) yr[p][rg] = yi[p][rg] = 0.0;
-                auto mma = [&](double hv, xv_t x, int p, int rg) {
-                    if constexpr (PAIR) {
-                        yr[p][rg] = __builtin_amdgcn_mfma_f64_4x4x4f64(hv, x.x, yr[p][rg], 0, 0, 0);
-                        yi[p][rg] = __builtin_amdgcn_mfma_f64_4x4x4f64(hv, x.y, yi[p][rg], 0, 0, 0);
-                    } else {
-                        yr[p][rg] = __builtin_amdgcn_mfma_f64_4x4x4f64(hv, x, yr[p][rg], 0, 0, 0);
+                    for (int rg = 0; rg < RG; ++rg) {
+                        if constexpr (PAIR) {
+                            yr[p][rg] = __builtin_amdgcn_mfma_f64_4x4x4f64(hv[rg], x.x, yr[p][rg], 0, 0, 0);
+                            yi[p][rg] = __builtin_amdgcn_mfma_f64_4x4x4f64(hv[rg], x.y, yi[p][rg], 0, 0, 0);
+                        } else {
+                            yr[p][rg] = __builtin_amdgcn_mfma_f64_4x4x4f64(hv[rg], x, yr[p][rg], 0, 0, 0);
+                        }
                     }
-                };
-                // step s takes register group s, and LDS group NREG + l after
-                // register group NREG - NL + l, whose products cover its LDS reads
-                constexpr int RONLY = NREG - NL;
-                auto group = [](int st) {
-                    return st < RONLY ? st : (st - RONLY) % 2 == 0 ? RONLY + (st - RONLY) / 2 : NREG + (st - RONLY) / 2;
-                };
-                xv_t xb[DEPTH][PT];
-#pragma unroll
-                for (int d = 0; d < DEPTH; ++d)
-#pragma unroll
-                    for (int p = 0; p < PT; ++p) xb[d][p] = xload(group(d), p);
-                double hl[RG];
-#pragma unroll
-                for (int st = 0; st < NT; ++st) {
-                    const int g = group(st);
-                    if (g < NREG && st >= RONLY && NL > 0) {
-#pragma unroll
-                        for (int rg = 0; rg < RG; ++rg)
-                            hl[rg] = hs[(((st - RONLY) / 2 * RS_WAVES + w) * RG + rg) * 64 + lane];
-                    }
-#pragma unroll
-                    for (int p = 0; p < PT; ++p) {
-                        const xv_t x = xb[st % DEPTH][p];
-                        if (st + DEPTH < NT) xb[st % DEPTH][p] = xload(group(st + DEPTH), p);
-#pragma unroll
-                        for (int rg = 0; rg < RG; ++rg) mma(g < NREG ? h[g < NREG ? g : 0][rg] : hl[rg], x, p, rg);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
                 }
+            };
+            // step s takes register group s, and LDS group NREG + l after register
+            // group NREG - NL + l, whose products cover its LDS reads
+            constexpr int RONLY = NREG - NL;
+            auto group = [](int st) {
+                return st < RONLY ? st : (st - RONLY) % 2 == 0 ? RONLY + (st - RONLY) / 2 : NREG + (st - RONLY) / 2;
+            };
+            xv_t xb[DEPTH][XL];
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d)
+#pragma unroll
+                for (int p = 0; p < XL; ++p) xb[d][p] = xload(group(d), p);
+            double hl[RG];
+#pragma unroll
+            for (int st = 0; st < NT; ++st) {
+                const int g = group(st);
+                if (g < NREG && st >= RONLY && NL > 0) {
+#pragma unroll
+                    for (int rg = 0; rg < RG; ++rg) hl[rg] = hs[(((st - RONLY) / 2 * NW + w) * RG + rg) * 64 + lane];
+                }
+#pragma unroll
+                for (int p = 0; p < XL; ++p) {
+                    const xv_t x = xb[st % DEPTH][p];
+                    if (st + DEPTH < NT) xb[st % DEPTH][p] = xload(group(st + DEPTH), p);
+                    if (g < NREG) mma(h[g < NREG ? g : 0], x, p);
+                    else mma(hl, x, p);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (WIDE) {
+                // value v of lane (k, n): row k + 4 v, real column n
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    reinterpret_cast<double*>(part)[(w * RB + lk + 4 * v) * 16 + (lane & 15)] = yw[0][v] + yw[1][v];
+            } else {
                 // lane (i, b, j) keeps row group b (b < RG): row 4 b + i, column j
 #pragma unroll
                 for (int p = 0; p < PT; ++p) {
@@ -286,7 +325,7 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
                     }
                     if (lb < RG) {
                         if constexpr (PAIR) {
-                            part[((p0 + p) * RS_WAVES + w) * RB * 4 + (4 * lb + lk) * 4 + lj] = cplx{vr, vi};
+                            part[(p * NW + w) * RB * 4 + (4 * lb + lk) * 4 + lj] = cplx{vr, vi};
                         } else if (lj < 2 * R) {  // real columns: packed as R complex ones
                             reinterpret_cast<double*>(part)[w * RB * 8 + (4 * lb + lk) * 2 * R + lj] = vr;
                         }
@@ -294,45 +333,42 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
                 }
             }
         } else {
-            for (int e = lane; e < np * RB * 4; e += 64) {
-                const int p = e / (RB * 4), f = e % (RB * 4);
-                part[(p * RS_WAVES + w) * RB * 4 + f] = cplx{0.0, 0.0};
+            for (int e = lane; e < PT * RB * PC; e += 64) {
+                const int p = e / (RB * PC), f = e % (RB * PC);
+                part[(p * NW + w) * RB * PC + f] = cplx{0.0, 0.0};
             }
         }
         rs_lds_barrier();
         cplx* const tk = ts + (k % 3) * E;
-        if (w == 0) {
+        if (w < SW) {
             const cplx* const t1 = ts + ((k + 2) % 3) * E;
             const cplx* const t2 = ts + ((k + 1) % 3) * E;
             const double alpha = k == 1 ? a1 : 2.0 * a1, beta = k == 1 ? b1 : 2.0 * b1;
-#pragma unroll
-            for (int u = 0; u < NE; ++u) {
-                const int e = lane + 64 * u;
-                if (e < E) {
-                    cplx y{0.0, 0.0};
-                    const int row = e / R, col = e % R;
-                    const cplx* pp = PAIR ? part + (col / 4) * RS_WAVES * RB * 4 + row * 4 + col % 4 : part + e;
-#pragma unroll(RG == 4 && NREG > 16 ? 4 : RS_WAVES)
-                    for (int ww = 0; ww < RS_WAVES; ++ww) {
-                        y.re += pp[ww * RB * 4].re;
-                        y.im += pp[ww * RB * 4].im;
-                    }
-                    const cplx xv = t1[e];
-                    cplx T{alpha * y.re + beta * xv.re, alpha * y.im + beta * xv.im};
-                    if (k > 1) {
-                        const cplx x2 = t2[e];
-                        T.re -= x2.re;
-                        T.im -= x2.im;
-                    }
-                    if (k < K) publish(e, T, k % a.slots);
-                    tk[e] = T;
+            const int e = lane + 64 * w;
+            if (e < E) {
+                cplx y{0.0, 0.0};
+                const int row = e / R, col = e % R;
+                const cplx* pp = !PAIR ? part + e : part + (WIDE ? row * 8 + col : (col / 4) * NW * RB * 4 + row * 4 + col % 4);
+#pragma unroll(RG == 4 && NREG > 16 ? 4 : NW)
+                for (int ww = 0; ww < NW; ++ww) {
+                    y.re += pp[ww * RB * PC].re;
+                    y.im += pp[ww * RB * PC].im;
                 }
+                const cplx xv = t1[e];
+                cplx T{alpha * y.re + beta * xv.re, alpha * y.im + beta * xv.im};
+                if (k > 1) {
+                    const cplx x2 = t2[e];
+                    T.re -= x2.re;
+                    T.im -= x2.im;
+                }
+                if (k < K) publish(e, T, k % a.slots);
+                tk[e] = T;
             }
             if (k < K) raise((unsigned)k + 1u);
         }
         rs_lds_barrier();
 #pragma unroll
-        for (int v = 0; v < RS_NQ; ++v)
+        for (int v = 0; v < NQ; ++v)
             if (k <= kq[v]) {
 #pragma unroll
                 for (int u = 0; u < NE; ++u)
@@ -351,8 +387,8 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
     rs_lds_barrier();
     const bool bad = *gave_up != 0u;
 #pragma unroll
-    for (int v = 0; v < RS_NQ; ++v) {
-        const int q = w + RS_WAVES * v;
+    for (int v = 0; v < NQ; ++v) {
+        const int q = w + NW * v;
         if (kq[v] >= 0) {
 #pragma unroll
             for (int u = 0; u < NE; ++u) {
@@ -366,14 +402,41 @@ __global__ __launch_bounds__(RS_THREADS, 2) void resident_series_kernel(const Re
     }
 }
 
+template <int NW, int RG, int NT, int RC>
+__global__ __launch_bounds__(NW * 64, 2) void resident_series_kernel(const ResidentArgs a) {
+    resident_body<NW, RG, NT, RC>(a, blockIdx.x, gridDim.x);
+}
+
+// Several systems in one launch: workgroup i is workgroup map[i].y of member
+// map[i].x (all read through the constant address space: scalar registers).
+template <int NW, int NT, int RC>
+__global__ __launch_bounds__(NW * 64, 2) void resident_grouped_kernel(const ResidentArgs* members, const int2* map) {
+    typedef const __attribute__((address_space(4))) ResidentArgs* args_const;
+    typedef const __attribute__((address_space(4))) int* int_const;
+    const int_const mp = (int_const)(reinterpret_cast<const int*>(map) + 2 * blockIdx.x);
+    const args_const m = (args_const)(members) + mp[0];
+    ResidentArgs a;
+    a.H = m->H; a.ld = m->ld; a.N = m->N; a.R = m->R; a.m = m->m; a.K = m->K; a.c = m->c; a.r = m->r;
+    a.phi = m->phi; a.acc = m->acc; a.acc_stride = m->acc_stride; a.coef = m->coef; a.coef_stride = m->coef_stride;
+    a.kq = m->kq; a.ring = m->ring; a.slots = m->slots; a.slot_bytes = m->slot_bytes; a.groups = m->groups;
+    a.flags = m->flags;
+    resident_body<NW, 4, NT, RC>(a, mp[1], a.ld / 16);
+}
+
+__global__ __launch_bounds__(256) void resident_clear_kernel(const ResidentArgs* members) {
+    const ResidentArgs a = members[blockIdx.x];
+    const int n = (int)(a.ring - reinterpret_cast<char*>(a.flags)) / 4;
+    for (int i = threadIdx.x; i < n; i += 256) a.flags[i] = 0u;
+}
+
 // ------------------------------------------------------------------ plan
 // Rows per workgroup: 16 (RG = 4), which reads x least often per product; 8 for
-// R > 4 while that leaves at most 256 workgroups, since both passes over H then
-// run together (N = 2048, R = 8: 5.5 against 7.6 us per term; at R = 4 8 rows
-// measured the same as 16).  NT: the groups a
-// wave needs, rounded up to even above 8 (the surplus is zero).
+// R > 4 while that leaves at most 256 workgroups, twice as many CUs at work (N =
+// 2048, R = 8: 5.4 against 6.6 us per term; at R = 4 8 rows measured the same as
+// 16).  NT: the groups a wave needs, rounded up to even above 8 (the surplus is
+// zero); for R > 4 at most 30, the rest of H no longer fits the LDS.
 struct ResidentPlan {
-    int RG = 0, RC = 0, NT = 0, wgs = 0, lds = 0;
+    int RG = 0, RC = 0, NT = 0, groups = 0, wgs = 0, lds = 0;
     bool ok = false;
 };
 
@@ -383,28 +446,29 @@ static ResidentPlan resident_plan(int ld, int R, int cus) {
     p.RC = R <= 2 ? 0 : R <= 4 ? 1 : 2;
     p.RG = p.RC == 2 && ld <= 2048 ? 2 : 4;
     p.wgs = ld / (4 * p.RG);
-    const int n = (ld / 16 + RS_WAVES - 1) / RS_WAVES;
+    constexpr int NW = 8;
+    const int n = p.groups = (ld / 16 + NW - 1) / NW;
     p.NT = n <= 8 ? n : (n + 1) / 2 * 2;
     const int np = p.RC == 2 ? 2 : 1, nl = p.RG == 4 ? std::max(0, p.NT - rs_most(p.RC)) : 0;
-    p.lds = nl * RS_WAVES * p.RG * 64 * 8 + np * RS_WAVES * 4 * p.RG * 4 * 16 + 3 * 4 * p.RG * R * 16;
-    p.ok = p.wgs <= cus && p.lds <= 160 * 1024 && (p.RC < 2 || p.NT <= 28);
+    p.lds = nl * NW * p.RG * 64 * 8 + np * NW * 4 * p.RG * 4 * 16 + 3 * 4 * p.RG * R * 16;
+    p.ok = p.wgs <= cus && p.lds <= 160 * 1024 && (p.RC < 2 || p.NT <= 30);
     return p;
 }
 
 bool resident_series_fits(int ld, int R, int cus) { return resident_plan(ld, R, cus).ok; }
 
 // bytes of one ring slot, and of the flags in front of the ring
-static long resident_slot_bytes(int ld, int R) { return (long)ld * R * 16; }
+static long resident_slot_bytes(int ld, int R) { return (long)ld * (R <= 2 ? 32 : R <= 4 ? 64 : 128); }
 static long resident_flag_bytes(int ld) { return (long)RS_COPIES * (ld / 4) * 4; }
 
 template <int RG, int NT, int RC>
 static hipError_t resident_go(const ResidentArgs& a, const ResidentPlan& p, hipStream_t st) {
-    const void* f = reinterpret_cast<const void*>(&resident_series_kernel<RG, NT, RC>);
+    const void* f = reinterpret_cast<const void*>(&resident_series_kernel<8, RG, NT, RC>);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, p.lds);
     if (e != hipSuccess) return e;
     ResidentArgs arg = a;
     void* params[] = {&arg};
-    return hipLaunchCooperativeKernel(f, dim3(p.wgs), dim3(RS_THREADS), params, (unsigned)p.lds, st);
+    return hipLaunchCooperativeKernel(f, dim3(p.wgs), dim3(512), params, (unsigned)p.lds, st);
 }
 
 // the kernel of p.NT among LO, LO + STEP, ..., HI
@@ -420,24 +484,136 @@ static hipError_t resident_launch(const ResidentArgs& a, const ResidentPlan& p, 
     if (p.RC == 0) return few ? resident_pick<4, 0, 1, 8, 1>(a, p, st) : resident_pick<4, 0, 10, 32, 2>(a, p, st);
     if (p.RC == 1) return few ? resident_pick<4, 1, 1, 8, 1>(a, p, st) : resident_pick<4, 1, 10, 32, 2>(a, p, st);
     if (p.RG == 2) return few ? resident_pick<2, 2, 1, 8, 1>(a, p, st) : resident_pick<2, 2, 10, 16, 2>(a, p, st);
-    return resident_pick<4, 2, 18, 28, 2>(a, p, st);
+    return resident_pick<4, 2, 18, 30, 2>(a, p, st);
 }
 
 // scratch: flags, then as many ring slots as fit (at least 4)
+static bool resident_scratch(ResidentArgs* a, void* scratch, long scratch_bytes) {
+    const long fb = resident_flag_bytes(a->ld), sb = resident_slot_bytes(a->ld, a->R);
+    const long slots = std::min(64L, (scratch_bytes - fb) / sb);
+    if (slots < 4 || a->m < 1 || a->m > MULTI_MAX) return false;
+    a->flags = static_cast<unsigned*>(scratch);
+    a->ring = static_cast<char*>(scratch) + fb;
+    a->slots = (int)slots;
+    a->slot_bytes = (int)sb;
+    return true;
+}
+
 bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, int cus, hipStream_t st) {
     const ResidentPlan p = resident_plan(a.ld, a.R, cus);
-    const long fb = resident_flag_bytes(a.ld), sb = resident_slot_bytes(a.ld, a.R);
-    const long slots = std::min(64L, (scratch_bytes - fb) / sb);
-    if (!p.ok || slots < 4 || a.m < 1 || a.m > MULTI_MAX) return false;
-    a.flags = static_cast<unsigned*>(scratch);
-    a.ring = static_cast<char*>(scratch) + fb;
-    a.slots = (int)slots;
-    a.slot_bytes = (int)sb;
-    launch_zero_u32(a.flags, (int)(fb / 4), st);
+    if (!p.ok || !resident_scratch(&a, scratch, scratch_bytes)) return false;
+    a.groups = p.groups;
+    launch_zero_u32(a.flags, (int)(resident_flag_bytes(a.ld) / 4), st);
     const hipError_t e = resident_launch(a, p, st);
     if (e == hipSuccess) return true;
     (void)hipGetLastError();  // not launched: the caller runs the series term by term
     return false;
+}
+
+// ------------------------------------------------------------------ batches
+// A batch fills the chip with many systems, so its kernels are chosen for
+// throughput: 16 rows per workgroup, both passes of R > 4 together, and 4 waves
+// per workgroup up to ld = 1024, so that two or more workgroups share a CU and
+// cover each other's exchange.  The split of a system's sums depends on its ld
+// and R alone: its bits are the same in every batch.  64 systems of N 256-2048
+// with 4 wavepackets, 40 steps: 214 ms with one grouped launch per term, 152 ms
+// here; a launch of 8 systems of N = 1000 takes 7.7 us per term, 3.4 of them
+// matrix-core time (both workgroups of a CU wait at the same time).
+static int batch_waves(int ld) { return ld <= 1024 ? 4 : 8; }
+static int batch_lds(int nw, int R) {
+    return (R > 4 ? 2 : 1) * nw * 16 * 4 * 16 + 3 * 16 * R * 16;
+}
+
+// the grouped kernel for (waves, most groups per wave, columns), its workgroups
+// per CU, and the NT it was built for
+struct GroupedKernel {
+    const void* f = nullptr;
+    int nt = 0;
+};
+template <int NW, int RC>
+static GroupedKernel grouped_pick(int n) {
+#define DH_GROUPED(NT) \
+    if (n <= NT) return GroupedKernel{reinterpret_cast<const void*>(&resident_grouped_kernel<NW, NT, RC>), NT}
+    if constexpr (NW == 4) {
+        DH_GROUPED(2);
+        DH_GROUPED(4);
+        DH_GROUPED(6);
+        DH_GROUPED(8);
+    }
+    DH_GROUPED(10);
+    DH_GROUPED(12);
+    DH_GROUPED(14);
+    DH_GROUPED(16);
+#undef DH_GROUPED
+    return GroupedKernel{};
+}
+static GroupedKernel grouped_kernel(int nw, int n, int R) {
+    const int rc = R <= 2 ? 0 : R <= 4 ? 1 : 2;
+    if (nw == 4) return rc == 0 ? grouped_pick<4, 0>(n) : rc == 1 ? grouped_pick<4, 1>(n) : grouped_pick<4, 2>(n);
+    return rc == 0 ? grouped_pick<8, 0>(n) : rc == 1 ? grouped_pick<8, 1>(n) : grouped_pick<8, 2>(n);
+}
+
+bool resident_batch_member(ResidentArgs* a, void* scratch, long scratch_bytes, int cus) {
+    if (cus <= 0 || a->ld > 2048 || a->R > 8 || a->ld / 16 > cus) return false;
+    if (!resident_scratch(a, scratch, scratch_bytes)) return false;
+    const int nw = batch_waves(a->ld);
+    a->groups = (a->ld / 16 + nw - 1) / nw;
+    return true;
+}
+
+// Launches: members of one wave count and about one size, as many as fit the
+// chip together (largest first, so that a launch's members need about the same
+// NT and take about as long).  Tried, with no gain: a member's workgroups on as
+// few XCDs as hold them, different priorities or a delayed start for the
+// workgroups that share a CU.
+bool resident_batch_rounds(const std::vector<ResidentArgs>& members, int cus, std::vector<int2>* map,
+                           std::vector<ResidentRound>* rounds) {
+    map->clear();
+    rounds->clear();
+    std::vector<int> order(members.size());
+    for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
+        return members[x].ld != members[y].ld ? members[x].ld > members[y].ld : members[x].K > members[y].K;
+    });
+    int room = 0, nw = 0;
+    for (int i : order) {
+        const ResidentArgs& a = members[i];
+        const int wgs = a.ld / 16, w = batch_waves(a.ld);
+        if (w != nw || wgs > room) {
+            const GroupedKernel k = grouped_kernel(w, a.groups, a.R);
+            const int lds = batch_lds(w, a.R);
+            int per_cu = 0;
+            if (!k.f || hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.f, w * 64, (size_t)lds) != hipSuccess ||
+                per_cu * cus < wgs) {
+                (void)hipGetLastError();
+                return false;
+            }
+            rounds->push_back(ResidentRound{k.f, w * 64, lds, (int)map->size(), 0});
+            room = per_cu * cus;
+            nw = w;
+        }
+        for (int g = 0; g < wgs; ++g) map->push_back(make_int2(i, g));
+        rounds->back().wgs += wgs;
+        room -= wgs;
+    }
+    return true;
+}
+
+int launch_resident_rounds(const ResidentArgs* d_members, int n, const int2* d_map,
+                           const std::vector<ResidentRound>& rounds, hipStream_t st) {
+    if (n <= 0) return 0;
+    hipLaunchKernelGGL(resident_clear_kernel, dim3(n), dim3(256), 0, st, d_members);
+    for (const ResidentRound& r : rounds) {
+        const int2* map = d_map + r.first;
+        void* params[] = {&d_members, &map};
+        const hipError_t e = hipLaunchCooperativeKernel(r.f, dim3(r.wgs), dim3(r.threads), params, (unsigned)r.lds, st);
+        if (e != hipSuccess) {
+            set_error("resident batch series: %s", hipGetErrorString(e));
+            return -1;
+        }
+    }
+    return 0;
 }
 
 }  // namespace dh

@@ -117,3 +117,36 @@ def test_multi_step_series(ctx, n_wp, n_steps):
     assert np.abs(out[0][0] - out[1][0]).max() < 1e-11 * np.abs(out[1][0]).max()
     assert np.abs(out[0][1] - out[1][1]).max() < 1e-11 * np.abs(out[1][1]).max()
     assert np.linalg.norm(out[0][2] - out[1][2]) <= 1e-11 * np.linalg.norm(out[1][2])
+
+
+# members at the edges of the batch kernels (4 waves up to ld = 1024, 8 up to 2048; 2050 runs in grouped
+# launches), of different sizes, against the grouped dense kernel
+@pytest.mark.parametrize("n_wp", [1, 2, 4])
+def test_batch_series_matches_terms(ctx, n_wp):
+    sizes = [5, 64, 130, 960, 1024, 1025, 1100, 2048, 2050]
+    out = []
+    for family in (-1, 0):
+        hip.force_batch_family(2 * n_wp, family)
+        try:
+            systems = []
+            for N in sizes:
+                rng = np.random.default_rng(N)
+                a, b = rng.normal(size=(2, N, N)) / np.sqrt(N)
+                s = hip.System(ctx, n_orb=N, n_wp=n_wp)
+                s.load_operators(np.eye(N) + 0.02 * (a + a.T), 8.0 * (b + b.T) - 10.0 * np.eye(N))
+                for w in range(n_wp):
+                    c = (rng.normal(size=N) + 1j * rng.normal(size=N)) / np.sqrt(2.0 * N)
+                    s.set_initial_state(w, c, c)
+                systems.append(s)
+            batch = hip.Batch(ctx, systems)
+            batch.propagate(0.0, DT)
+            batch.propagate_steps(12, DT)
+            out.append([[s.wavepacket(w)[1] for w in range(n_wp)] for s in systems])
+            batch.close()
+            for s in systems:
+                s.close()
+        finally:
+            hip.force_batch_family(2 * n_wp, -1)
+    for N, x, y in zip(sizes, *out):
+        for w in range(n_wp):
+            assert np.linalg.norm(x[w] - y[w]) <= 1e-11 * np.linalg.norm(y[w]), N
