@@ -841,7 +841,7 @@ extern "C" int dh_build_operators(dh_system* s, double cutoff, double s_drop) {
     int rc = ensure_ws(s->ctx, s->ld);
     if (rc) return rc;
     s->ctx->ws_owner = s;
-    if (launch_build_SH(s->bd, s->N, s->ld, s->ctx->S, s->ctx->h, cutoff, s_drop, s->ctx->stream)) {
+    if (launch_build_SH(s->bd, s->N, s->ld, s->ctx->S, s->ctx->h, cutoff, s_drop, s->ctx->W, s->ctx->stream)) {
         dh::set_error("dh_build_operators: kernel launch failed: %s", hipGetErrorString(hipGetLastError()));
         return DH_ERR_HIP;
     }
@@ -1503,7 +1503,7 @@ static int side_launch(dh_system* s, const double* d_geo, double cutoff, double 
     DH_HIP(hipMemcpyAsync(h.coords, d_geo, sizeof(double) * 3 * s->n_atoms, hipMemcpyDeviceToDevice, c->side));
     BasisDev b2 = s->bd;
     b2.coords = h.coords;
-    if (launch_build_SH(b2, s->N, s->ld, c->S2, c->h2, cutoff, s_drop, c->side)) {
+    if (launch_build_SH(b2, s->N, s->ld, c->S2, c->h2, cutoff, s_drop, c->W2, c->side)) {
         dh::set_error("dh_propagate_steps: kernel launch failed: %s", hipGetErrorString(hipGetLastError()));
         return DH_ERR_HIP;
     }

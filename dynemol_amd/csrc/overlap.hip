@@ -1,333 +1,196 @@
 // STO overlap S and Wolfsberg-Helmholz Hueckel h, built on the device.
 //
-// Follows the reference's two-centre scheme (overlap_D.f:144-311): for every
-// atom pair (ia > ib) within the cutoff, lined-up-frame overlaps
-// <n l m | n' l' m> from the Fernandez-Rico basic integrals and the L, L', M
-// recursions (SOLAP, overlap_D.f:658-962), STO normalisation (GET_ANOR,
-// :466-517), then rotation to the molecular frame with real-harmonic rotation
-// matrices (ROTAR/DLMN, :983-1191).  h_ij = X_ij * S_ij (hamiltonians.f:33-63).
+// The reference's two-centre scheme (overlap_D.f:144-311): for every atom pair
+// (ia > ib) within the cutoff, lined-up-frame overlaps <n l m | n' l' m> (SOLAP,
+// overlap_D.f:658-962) of normalised STOs (GET_ANOR, :466-517), then rotation to
+// the molecular frame (ROTAR/DLMN, :983-1191).  h_ij = X_ij * S_ij
+// (hamiltonians.f:33-63).
 //
-// Work decomposition: one thread per (atom pair, shell pair).  A shell is the
-// set of 2l+1 orbitals sharing (n, l, zeta, coef) on one atom; the lined-up
-// integrals depend only on the shell pair, so each thread evaluates them once
-// and writes the (2la+1) x (2lb+1) block of S and h (and the mirrored block).
-// The reference evaluates SOLAP once per orbital pair instead.
+// The lined-up overlaps are integrated in prolate spheroidal coordinates: with
+// xi in [1, inf) and eta in [-1, 1] the integrand is exp(-p xi - t eta) (p, t =
+// (za +- zb) R / 2) times a polynomial of degree <= na + nb <= 10 in each, so
+// 8-point Gauss-Laguerre in xi is exact and Gauss-Legendre in eta converges to
+// rounding: 16 points for |t| < 4, 24 for |t| < 16, else 32 on the part of
+// [-1, 1] where exp(-|t| ...) > e^-80.  The polynomial is evaluated in factored
+// form (radii and heights over both centres), so nothing cancels, and a
+// thread needs no tables: the recursions of the published scheme kept 7 KB of
+// them per lane in scratch memory, whose traffic bound the kernel (N = 4096: 3.9
+// ms; N = 514: 1.4 ms).
+//
+// Work decomposition: the atom pairs within the cutoff are collected into a
+// list, and one thread takes one (pair, shell pair).  A shell is the set of
+// 2l+1 orbitals sharing (n, l, zeta, coef) on one atom; a thread evaluates the
+// min(la, lb) + 1 lined-up overlaps together and writes the (2la+1) x (2lb+1)
+// block of S and h (and the mirrored block).
 #include "common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
+
 namespace dh {
 
-// Bounds for the compact device tables: n <= 5, l <= 2 (s, p, d shells).
-constexpr int SQ_NMAX = 5;
-constexpr int SQ_LMAX = 2;
-constexpr int SQ_D = SQ_NMAX + 3 * SQ_LMAX + 1;  // smat index range 0..SQ_D-1 (nmax <= n+l+2l' = 11)
-constexpr int SQ_HA = SQ_D + 2;                   // 1F1 'a' index range
-constexpr int SQ_HG = 2 * SQ_D + 3;               // 1F1 'g' index range (ngmax <= 24)
+// Gauss-Legendre nodes and weights, positive half: 16, 24 and 32 points
+__constant__ double GL_X[36] = {
+    0.09501250983763744, 0.2816035507792589, 0.45801677765722737, 0.6178762444026438, 0.755404408355003,
+    0.8656312023878318, 0.9445750230732326, 0.9894009349916499,
+    0.06405689286260563, 0.1911188674736163, 0.3150426796961634, 0.4337935076260451, 0.5454214713888396,
+    0.6480936519369755, 0.7401241915785544, 0.820001985973903, 0.8864155270044011, 0.9382745520027328,
+    0.9747285559713095, 0.9951872199970213,
+    0.04830766568773832, 0.1444719615827965, 0.23928736225213706, 0.33186860228212767, 0.42135127613063533,
+    0.5068999089322294, 0.5877157572407623, 0.6630442669302152, 0.7321821187402897, 0.7944837959679424,
+    0.84936761373257, 0.8963211557660521, 0.9349060759377397, 0.9647622555875064, 0.9856115115452684,
+    0.9972638618494816};
+__constant__ double GL_W[36] = {
+    0.1894506104550685, 0.18260341504492358, 0.16915651939500254, 0.14959598881657674, 0.12462897125553388,
+    0.09515851168249279, 0.062253523938647894, 0.027152459411754096,
+    0.12793819534675216, 0.1258374563468283, 0.12167047292780339, 0.1155056680537256, 0.10744427011596563,
+    0.09761865210411388, 0.08619016153195327, 0.0733464814110803, 0.05929858491543678, 0.04427743881741981,
+    0.028531388628933663, 0.0123412297999872,
+    0.0965400885147278, 0.09563872007927486, 0.09384439908080457, 0.09117387869576389, 0.08765209300440381,
+    0.08331192422694675, 0.07819389578707031, 0.0723457941088485, 0.06582222277636185, 0.058684093478535544,
+    0.050998059262376175, 0.04283589802222668, 0.03427386291302143, 0.02539206530926206, 0.01627439473090567,
+    0.007018610009470096};
+// Gauss-Laguerre, 8 points
+__constant__ double LAG_X[8] = {
+    0.170279632305101, 0.9037017767993799, 2.2510866298661307, 4.266700170287659, 7.0459054023934655,
+    10.758516010180996, 15.740678641278004, 22.863131736889265};
+__constant__ double LAG_W[8] = {
+    0.3691885893416375, 0.41878678081434295, 0.1757949866371718, 0.03334349226121565, 0.0027945362352256725,
+    9.076508773358213e-05, 8.485746716272531e-07, 1.0480011748715104e-09};
 
-__device__ __forceinline__ double rre(int i) { return (double)i; }
-__device__ __forceinline__ double rreali(int i) { return i == 0 ? 0.0 : 1.0 / (double)i; }
-
-__device__ double dfact(int n) {
-    double f = 1.0;
-    for (int i = 2; i <= n; ++i) f *= (double)i;
-    return f;
-}
-
-// Lined-up overlaps of unnormalised STOs, sol[0..min(la,lb)].
-__device__ void solap_dev(int na, int la, double za, int nb, int lb, double zb, double R, double* sol) {
-    const double pi4 = 12.566370614359172953850573533118012;
-    double h1f1[SQ_HA * SQ_HG];
-    double smat[SQ_D * SQ_D], smataux[SQ_D * SQ_D], smatm[SQ_D * SQ_D];
-#define H1(a, g) h1f1[(a) * SQ_HG + (g)]
-#define SM(n, np) smat[(n) * SQ_D + (np)]
-#define SA(n, np) smataux[(n) * SQ_D + (np)]
-#define SMM(n, np) smatm[(n) * SQ_D + (np)]
-    // h1f1 needs no clearing: level ngmax is filled for a = 1..namax, level j
-    // for a = 1..min(namax, j - 1) from level j + 1, and every later read
-    // (j + 1, k + 2) has j + 1 <= min(namax, k + 1).  Nor do smat, smataux and
-    // smatm: the basic integrals fill n = nmin..nmax, n' = n'min..n'max - (n -
-    // nmin), and every read of the L, L' and M recursions that follow lands on
-    // an entry written before it (checked over every n <= 5, l <= 2 shell
-    // pair in both zeta orders, all indices within the 12 x 12 tables).
-    int nmin, nmax, npmin, npmax;
-    double z, zp;
-    const bool a_first = za >= zb;
-    if (a_first) {
-        nmin = na - la; nmax = na + la + 2 * lb;
-        npmin = nb - lb; npmax = nb + lb + 2 * la;
-        z = za; zp = zb;
-    } else {
-        nmin = nb - lb; nmax = nb + lb + 2 * la;
-        npmin = na - la; npmax = na + la + 2 * lb;
-        z = zb; zp = za;
-    }
-    const double expzR = exp(-z * R);
-    const int ngmax = nmax + npmax + 2;
-    const int namax = npmax + 1;
-    const double arg = (z - zp) * R;
-    const int iz = (int)z;
-    int ia = (ngmax - iz) / 2;
-    if (ia < 1) ia = 1;
-    if (ia >= namax) ia = namax - 1;
-
-    // 1F1[ia, ngmax, arg] and 1F1[ia+1, ngmax, arg] by their series
-    double auxa = arg * rre(ia) * rreali(ngmax), f11a = 1.0;
-    double auxb = arg * rre(ia + 1) * rreali(ngmax), f11b = 1.0;
-    for (int i = 1; i <= 1000; ++i) {
-        f11a += auxa;
-        f11b += auxb;
-        auxa = auxa * rre(ia + i) * arg * rreali(ngmax + i) * rreali(i + 1);
-        auxb = auxb * rre(ia + i + 1) * arg * rreali(ngmax + i) * rreali(i + 1);
-        if (auxb < 1.0e-35 * f11b) break;
-    }
-    H1(ia, ngmax) = f11a;
-    H1(ia + 1, ngmax) = f11b;
-    double aux = arg - rre(ngmax);
-    for (int i = ia + 1; i <= namax - 1; ++i)
-        H1(i + 1, ngmax) = ((aux + rre(2 * i)) * H1(i, ngmax) + rre(ngmax - i) * H1(i - 1, ngmax)) * rreali(i);
-    for (int i = ia; i >= 2; --i)
-        H1(i - 1, ngmax) = (rre(i) * H1(i + 1, ngmax) - (aux + rre(2 * i)) * H1(i, ngmax)) * rreali(ngmax - i);
-    for (int j = ngmax - 1; j >= 2; --j) {
-        H1(1, j) = (H1(2, j + 1) + rre(j - 1) * H1(1, j + 1)) * rreali(j);
-        aux = arg * rreali(j);
-        const int top = min(namax - 1, j - 2);
-        for (int i = 1; i <= top; ++i) H1(i + 1, j) = aux * H1(i + 1, j + 1) + H1(i, j);
-    }
-
-    // basic integrals <N00|N'00>
-    {
-        const bool mcopy = min(la, lb) > 0;
-        const double zzpR = (z + zp) * R;
-        const double zzpi = 1.0 / (z + zp);
-        double zzpin = 1.0;
-        for (int e = 0; e < nmin + npmin + 1; ++e) zzpin *= zzpi;
-        for (int n = nmin; n <= nmax; ++n) {
-            double zzpinp = zzpin;
-            for (int np = npmin; np <= npmax - n + nmin; ++np) {
-                double auxk = dfact(n + np) * zzpinp;
-                double sumk = 0.0;
-                for (int k = 0; k <= n + np; ++k) {
-                    double sumj = 0.0;
-                    for (int j = max(0, k - n); j <= min(k, np); ++j)
-                        sumj += H1(j + 1, k + 2) / (dfact(n + j - k) * dfact(np - j));
-                    sumk += sumj * auxk;
-                    auxk = auxk * zzpR * rreali(n + np - k) * rreali(k + 2);
-                }
-                const double v = pi4 * expzR * dfact(n) * dfact(np) * sumk;
-                // smataux needs no copy (every read of it sees a recursion
-                // write), smatm only when an M step follows (min(la, lb) > 0)
-                if (a_first) {
-                    SM(n, np) = v;
-                    if (mcopy) SMM(n, np) = v;
+// Lined-up overlaps of two normalised STOs (A at the origin, B at R on z, both
+// along the same axes), acc[m] += cc <n l m | n' l' m>, m = 0..min(LA, LB).
+template <int LA, int LB>
+__device__ __forceinline__ void lined_up(int na, double za, int nb, double zb, double R, double cc, double* acc) {
+    constexpr int MS = LA < LB ? LA : LB;
+    const double hr = 0.5 * R, p = (za + zb) * hr, t = (za - zb) * hr, at = fabs(t);
+    const double sg = t < 0.0 ? -1.0 : 1.0;  // exp(-t eta) is largest at eta = -sg
+    const double pinv = 1.0 / p, low = fmin(za, zb) * R;  // p - |t|
+    const double len = at > 40.0 ? 40.0 / at : 1.0;       // half length of the eta interval
+    const int tier = at < 4.0 ? 0 : at < 16.0 ? 1 : 2;
+    double sum[MS + 1];
+#pragma unroll
+    for (int m = 0; m <= MS; ++m) sum[m] = 0.0;
+    // one pass per point count that any lane of the wave needs: the nodes are then
+    // the same for the whole wave (scalar loads); a lane adds its own pass only
+    for (int tr = 0; tr < 3; ++tr) {
+        if (__ballot(tier == tr) == 0) continue;
+        const int o = tr == 0 ? 0 : tr == 1 ? 8 : 20, half = tr == 0 ? 8 : tr == 1 ? 12 : 16;
+        double part[MS + 1];
+#pragma unroll
+        for (int m = 0; m <= MS; ++m) part[m] = 0.0;
+        for (int j = 0; j < 2 * half; ++j) {
+            const double x = j < half ? GL_X[o + j] : -GL_X[o + j - half];
+            const double u = len * (1.0 + x);             // distance from the heavy end
+            const double eta = sg * (u - 1.0);
+            const double we = GL_W[o + (j < half ? j : j - half)] * exp(-low - at * u);
+            const double e1 = 1.0 - eta * eta;
+            double in[MS + 1];
+#pragma unroll
+            for (int m = 0; m <= MS; ++m) in[m] = 0.0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const double xi = 1.0 + LAG_X[i] * pinv;
+                const double ra = xi + eta, rb = xi - eta;          // radii, in R / 2
+                const double ha = 1.0 + xi * eta, hb = xi * eta - 1.0;  // heights z_A, z_B
+                const double q2 = (xi * xi - 1.0) * e1;             // distance from the axis, squared
+                double f = LAG_W[i];
+                for (int e = LA; e < na; ++e) f *= ra;  // r^(n-1-l) and the volume factor
+                for (int e = LB; e < nb; ++e) f *= rb;
+                // r^l P_l^m over rho^m of either centre
+                if constexpr (LA == 1 && LB == 0) f *= ha;
+                if constexpr (LA == 0 && LB == 1) f *= hb;
+                if constexpr (LA == 2 && LB == 0) f *= 1.5 * ha * ha - 0.5 * ra * ra;
+                if constexpr (LA == 0 && LB == 2) f *= 1.5 * hb * hb - 0.5 * rb * rb;
+                if constexpr (MS == 0) {
+                    in[0] += f;
                 } else {
-                    SM(np, n) = v;
-                    if (mcopy) SMM(np, n) = v;
+                    const double a0 = LA == 1 ? ha : 1.5 * ha * ha - 0.5 * ra * ra;
+                    const double b0 = LB == 1 ? hb : 1.5 * hb * hb - 0.5 * rb * rb;
+                    const double a1 = LA == 1 ? 1.0 : 3.0 * ha, b1 = LB == 1 ? 1.0 : 3.0 * hb;
+                    in[0] += f * a0 * b0;
+                    in[1] += f * a1 * b1 * q2;
+                    if constexpr (MS == 2) in[2] += 9.0 * f * q2 * q2;
                 }
-                zzpinp *= zzpi;
             }
-            zzpin *= zzpi;
+#pragma unroll
+            for (int m = 0; m <= MS; ++m) part[m] += we * in[m];
         }
+#pragma unroll
+        for (int m = 0; m <= MS; ++m)
+            if (tier == tr) sum[m] = part[m];
     }
-
-    nmin = na - la; nmax = na + la + 2 * lb;
-    npmin = nb - lb; npmax = nb + lb + 2 * la;
-    const double Rinv = 1.0 / R, R2 = R * R, R4 = R2 * R2;
-    double updltm0i = 0.5;
-    const int mtop = min(la, lb);
-    for (int m = 0; m <= mtop; ++m) {
-        if (la > m) {
-            for (int np = npmin; np <= npmax - 2; ++np) {
-                double saux = SM(nmin, np);
-                for (int n = nmin + 1; n <= nmax - 1 - np + npmin; ++n) {
-                    const double sbux = rre(2 * m + 1) * 0.5 * Rinv * (SM(n + 1, np) + R2 * saux - SM(n - 1, np + 2));
-                    saux = SM(n, np);
-                    SA(n, np) = saux;
-                    SM(n, np) = sbux;
-                }
-            }
-            for (int ll = m + 1; ll <= la - 1; ++ll)
-                for (int np = npmin; np <= npmax - 2 * (ll + 1 - m); ++np) {
-                    double saux = SM(nmin + ll - m, np);
-                    for (int n = nmin + 1 + ll - m; n <= nmax - 1 - np + npmin - ll + m; ++n) {
-                        const double sbux =
-                            rre(2 * ll + 1) * 0.5 * rreali(ll - m + 1) * Rinv * (SM(n + 1, np) + R2 * saux - SM(n - 1, np + 2)) -
-                            rre(ll + m) * rreali(ll - m + 1) * SA(n, np);
-                        saux = SM(n, np);
-                        SA(n, np) = saux;
-                        SM(n, np) = sbux;
-                    }
-                }
-        }
-        if (lb > m) {
-            for (int n = nmin + la - m; n <= nmax - la + m - 2; ++n) {
-                double saux = SM(n, npmin);
-                for (int np = npmin + 1; np <= npmax - 2 * (la - m) - n + nmin + la - m - 1; ++np) {
-                    const double sbux = -rre(2 * m + 1) * 0.5 * Rinv * (SM(n, np + 1) + R2 * saux - SM(n + 2, np - 1));
-                    saux = SM(n, np);
-                    SA(n, np) = saux;
-                    SM(n, np) = sbux;
-                }
-            }
-            for (int ll = m + 1; ll <= lb - 1; ++ll)
-                for (int n = nmin + la - m; n <= nmax - la + m - 2 * (ll + 1 - m); ++n) {
-                    double saux = SM(n, npmin + ll - m);
-                    for (int np = npmin + 1 + ll - m; np <= npmax - 2 * (la - m) - n + nmin + la - m - ll + m - 1; ++np) {
-                        const double sbux =
-                            -rre(2 * ll + 1) * 0.5 * rreali(ll - m + 1) * Rinv * (SM(n, np + 1) + R2 * saux - SM(n + 2, np - 1)) -
-                            rre(ll + m) * rreali(ll - m + 1) * SA(n, np);
-                        saux = SM(n, np);
-                        SA(n, np) = saux;
-                        SM(n, np) = sbux;
-                    }
-                }
-        }
-        sol[m] = SM(na, nb);
-        if (m == mtop) break;
-        nmin += 1; nmax -= 3; npmin += 1; npmax -= 3;
-        aux = updltm0i * 0.25 * rre(2 * m + 1) * rre(2 * m + 1) * Rinv * Rinv;
-        for (int n = nmin; n <= nmax; ++n)
-            for (int np = npmin; np <= npmax - n + nmin; ++np)
-                SA(n, np) = aux * (2.0 * (SMM(n + 1, np + 1) + R2 * (SMM(n + 1, np - 1) + SMM(n - 1, np + 1))) -
-                                   SMM(n + 3, np - 1) - SMM(n - 1, np + 3) - R4 * SMM(n - 1, np - 1));
-        for (int n = nmin; n <= nmax; ++n)
-            for (int np = npmin; np <= npmax - n + nmin; ++np) {
-                SM(n, np) = SA(n, np);
-                SMM(n, np) = SA(n, np);
-            }
-        updltm0i = 1.0;
+    // (R/2)^(na + nb + 1) / p, the radial norms and the norms of the harmonics
+    double fa = 1.0, fb = 1.0;
+    for (int i = 2; i <= 2 * na; ++i) fa *= (double)i;
+    for (int i = 2; i <= 2 * nb; ++i) fb *= (double)i;
+    double c = len * pinv * hr;
+    const double xa = 2.0 * za * hr, xb = 2.0 * zb * hr;
+    for (int i = 0; i < na; ++i) c *= xa;
+    for (int i = 0; i < nb; ++i) c *= xb;
+    c *= cc * 0.5 * sqrt(4.0 * za * zb * (2 * LA + 1) * (2 * LB + 1) / (fa * fb));
+    // (l - m)! / (l + m)! under the root: l = 1: 1, 1/2; l = 2: 1, 1/6, 1/24
+    acc[0] += c * sum[0];
+    if constexpr (MS >= 1) {
+        constexpr double g = LA + LB == 2 ? 0.5 : LA + LB == 3 ? 0.28867513459481288225 : 1.0 / 6.0;
+        acc[1] += c * g * sum[1];
     }
-#undef H1
-#undef SM
-#undef SA
-#undef SMM
+    if constexpr (MS == 2) acc[2] += c * (1.0 / 24.0) * sum[2];
 }
 
-// Real-harmonic rotation matrices up to l = 2 for the A->B axis (gamma = 0).
-// rl[(mp+2) + 5*((m+2) + 5*l)], l = 0..2.
-#define RX(mp, m, l) (((mp) + 2) + 5 * (((m) + 2) + 5 * (l)))
-__device__ void rotation_dev(double xab, double yab, double zab, int lmax, double* rl, double* Rab_out) {
-    const double root2 = 1.414213562373095;
-    double dl[75];
-    for (int i = 0; i < 75; ++i) {
-        dl[i] = 0.0;
-        rl[i] = 0.0;
-    }
-    const double xy = sqrt(xab * xab + yab * yab);
-    double sinal, cosal;
-    if (xy > 1.0e-10) {
-        sinal = yab / xy;
-        cosal = xab / xy;
+// Column m of the rotation of the real harmonics of order l (y, z, x for l = 1;
+// xy, yz, z2, xz, x2-y2 for l = 2): lined-up axes e1, e2, u in the molecular frame.
+// l = 2 from the traceless forms of the axes: column +-1 is (e u^T + u e^T) /
+// sqrt 2, column +-2 (e1 e2^T + e2 e1^T) / sqrt 2 and (e1 e1^T - e2 e2^T) / sqrt 2.
+struct Axes {
+    double e1[3], e2[3], u[3];
+};
+__device__ __forceinline__ void d_mixed(const double* a, const double* b, double* o) {  // a, b perpendicular
+    o[0] = a[0] * b[1] + a[1] * b[0];
+    o[1] = a[1] * b[2] + a[2] * b[1];
+    o[2] = 1.73205080756887729353 * a[2] * b[2];
+    o[3] = a[0] * b[2] + a[2] * b[0];
+    o[4] = a[0] * b[0] - a[1] * b[1];
+}
+template <int L>
+__device__ __forceinline__ void rotation_column(const Axes& x, int m, double* o) {
+    if constexpr (L == 0) {
+        o[0] = 1.0;
+    } else if constexpr (L == 1) {
+        const double* v = m == 0 ? x.u : m == 1 ? x.e1 : x.e2;
+        o[0] = v[1];
+        o[1] = v[2];
+        o[2] = v[0];
+    } else if (m == 0) {
+        const double* u = x.u;
+        constexpr double s3 = 1.73205080756887729353;
+        o[0] = s3 * u[0] * u[1];
+        o[1] = s3 * u[1] * u[2];
+        o[2] = 1.5 * u[2] * u[2] - 0.5;
+        o[3] = s3 * u[0] * u[2];
+        o[4] = 0.5 * s3 * (u[0] * u[0] - u[1] * u[1]);
+    } else if (m == 1) {
+        d_mixed(x.e1, x.u, o);
+    } else if (m == -1) {
+        d_mixed(x.e2, x.u, o);
+    } else if (m == -2) {
+        d_mixed(x.e1, x.e2, o);
     } else {
-        sinal = 0.0;
-        cosal = 1.0;
-    }
-    const double Rab = sqrt(xab * xab + yab * yab + zab * zab);
-    *Rab_out = Rab;
-    double sinbet = xy / Rab, cosbet = zab / Rab;
-    dl[RX(0, 0, 0)] = 1.0;
-    rl[RX(0, 0, 0)] = 1.0;
-    if (lmax == 0) return;
-    dl[RX(1, 1, 1)] = (1.0 + cosbet) * 0.5;
-    dl[RX(1, 0, 1)] = -sinbet / root2;
-    dl[RX(1, -1, 1)] = (1.0 - cosbet) * 0.5;
-    dl[RX(0, 1, 1)] = -dl[RX(1, 0, 1)];
-    dl[RX(0, 0, 1)] = dl[RX(1, 1, 1)] - dl[RX(1, -1, 1)];
-    dl[RX(0, -1, 1)] = dl[RX(1, 0, 1)];
-    dl[RX(-1, 1, 1)] = dl[RX(1, -1, 1)];
-    dl[RX(-1, 0, 1)] = dl[RX(0, 1, 1)];
-    dl[RX(-1, -1, 1)] = dl[RX(1, 1, 1)];
-    // gamma = 0: cos(ga) = 1, sin(ga) = 0
-    rl[RX(0, 0, 1)] = dl[RX(0, 0, 1)];
-    rl[RX(1, 0, 1)] = root2 * dl[RX(0, 1, 1)] * cosal;
-    rl[RX(-1, 0, 1)] = root2 * dl[RX(0, 1, 1)] * sinal;
-    rl[RX(0, 1, 1)] = root2 * dl[RX(1, 0, 1)];
-    rl[RX(0, -1, 1)] = 0.0;
-    rl[RX(1, 1, 1)] = dl[RX(1, 1, 1)] * cosal - dl[RX(1, -1, 1)] * cosal;
-    rl[RX(1, -1, 1)] = -dl[RX(1, 1, 1)] * sinal - dl[RX(1, -1, 1)] * sinal;
-    rl[RX(-1, 1, 1)] = dl[RX(1, 1, 1)] * sinal - dl[RX(1, -1, 1)] * sinal;
-    rl[RX(-1, -1, 1)] = dl[RX(1, 1, 1)] * cosal + dl[RX(1, -1, 1)] * cosal;
-    if (lmax < 2) return;
-    double tgbet2;
-    if (fabs(sinbet) < 1.0e-10) {
-        tgbet2 = 0.0;
-        sinbet = 0.0;
-        cosbet = copysign(1.0, cosbet);
-    } else {
-        tgbet2 = (1.0 - cosbet) / sinbet;
-    }
-    // DLMN for l = 2
-    const int l = 2;
-    int iinf = 1 - l, isup = -iinf;
-    auto root = [](int i) { return sqrt((double)i); };
-    auto rooti = [](int i) { return 1.0 / sqrt((double)i); };
-    dl[RX(l, l, l)] = dl[RX(isup, isup, l - 1)] * (1.0 + cosbet) * 0.5;
-    dl[RX(l, -l, l)] = dl[RX(isup, -isup, l - 1)] * (1.0 - cosbet) * 0.5;
-    for (int m = isup; m >= iinf; --m) dl[RX(l, m, l)] = -tgbet2 * root(l + m + 1) * rooti(l - m) * dl[RX(l, m + 1, l)];
-    const double al = l, al1 = al - 1.0, tal1 = al + al1, ali = 1.0 / al1, cosaux = cosbet * al * al1;
-    for (int mp = l - 1; mp >= 0; --mp) {
-        const int laux = l + mp, lbux = l - mp;
-        const double a2 = rooti(laux) * rooti(lbux) * ali;
-        const double cux = root(laux - 1) * root(lbux - 1) * al;
-        for (int m = isup; m >= iinf; --m) {
-            const int lauz = l + m, lbuz = l - m;
-            const double factor = a2 * rooti(lauz) * rooti(lbuz);
-            double term = tal1 * (cosaux - (double)m * (double)mp) * dl[RX(mp, m, l - 1)];
-            if (lbuz != 1 && lbux != 1) term -= dl[RX(mp, m, l - 2)] * cux * root(lauz - 1) * root(lbuz - 1);
-            dl[RX(mp, m, l)] = factor * term;
-        }
-        iinf += 1;
-        isup -= 1;
-    }
-    double sign = 1.0;
-    iinf = -l;
-    isup = l - 1;
-    for (int m = l; m >= 1; --m) {
-        for (int mp = iinf; mp <= isup; ++mp) {
-            dl[RX(mp, m, l)] = sign * dl[RX(m, mp, l)];
-            sign = -sign;
-        }
-        iinf += 1;
-        isup -= 1;
-    }
-    iinf = -l;
-    isup = iinf;
-    for (int m = l - 1; m >= -l; --m) {
-        sign = -1.0;
-        for (int mp = isup; mp >= iinf; --mp) {
-            dl[RX(mp, m, l)] = sign * dl[RX(-mp, -m, l)];
-            sign = -sign;
-        }
-        isup += 1;
-    }
-    rl[RX(0, 0, l)] = dl[RX(0, 0, l)];
-    double cosmal = cosal, sinmal = sinal;
-    sign = -1.0;
-    for (int mp = 1; mp <= l; ++mp) {
-        const double a0 = root2 * dl[RX(0, mp, l)];
-        rl[RX(mp, 0, l)] = a0 * cosmal;
-        rl[RX(-mp, 0, l)] = a0 * sinmal;
-        for (int m = 1; m <= l; ++m) {
-            const double a1 = root2 * dl[RX(m, 0, l)];
-            rl[RX(0, m, l)] = a1;
-            rl[RX(0, -m, l)] = 0.0;
-            const double d1 = dl[RX(-mp, -m, l)];
-            const double d2 = sign * dl[RX(mp, -m, l)];
-            rl[RX(mp, m, l)] = d1 * cosmal + d2 * cosmal;
-            rl[RX(mp, -m, l)] = -d1 * sinmal + d2 * sinmal;
-            rl[RX(-mp, m, l)] = d1 * sinmal + d2 * sinmal;
-            rl[RX(-mp, -m, l)] = d1 * cosmal - d2 * cosmal;
-        }
-        sign = -sign;
-        const double t = cosmal * cosal - sinmal * sinal;
-        sinmal = sinmal * cosal + cosmal * sinal;
-        cosmal = t;
+        const double *a = x.e1, *b = x.e2;
+        o[0] = a[0] * a[1] - b[0] * b[1];
+        o[1] = a[1] * a[2] - b[1] * b[2];
+        o[2] = 0.86602540378443864676 * (a[2] * a[2] - b[2] * b[2]);
+        o[3] = a[0] * a[2] - b[0] * b[2];
+        o[4] = 0.5 * (a[0] * a[0] - b[0] * b[0] - a[1] * a[1] + b[1] * b[1]);
     }
 }
 
 // S = 0 with unit diagonal; h = 0 with h_ii = IP_i + V_shift_i.  Pad rows/cols
 // in [N, ld) stay zero (the padded diagonal of S is set to one so that the
 // padded Cholesky factor is the identity).
-__global__ void init_SH_kernel(double* S, double* h, int N, int ld, const double* ip, const double* vshift) {
+__global__ void init_SH_kernel(double* S, double* h, int N, int ld, const double* ip, const double* vshift,
+                               int* count) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;
     const long total = (long)ld * ld;
     for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x) {
         const int i = (int)(t % ld), j = (int)(t / ld);
@@ -341,91 +204,144 @@ __global__ void init_SH_kernel(double* S, double* h, int N, int ld, const double
     }
 }
 
-__global__ void build_SH_kernel(const BasisDev b, double* S, double* h, int ld, double cutoff, double s_drop) {
-    // Shell-pair major, then pairs (p > r) of atoms in basis-signature order:
-    // the 64 lanes of a wavefront share one shell pair and mostly one element
-    // pair, so they follow the same SOLAP branches.
-    const long tid = blockIdx.x * (long)blockDim.x + threadIdx.x;
+// Pairs (ia > ib) within the cutoff, in about basis-signature order: the lanes of
+// a wave of the next kernel then share one element pair for the most part, and
+// none is idle for its distance.
+__global__ __launch_bounds__(256) void pair_list_kernel(const BasisDev b, double cutoff, int* count, int2* list) {
     const long npair = (long)b.n_atoms * (b.n_atoms - 1) / 2;
-    const int sp = (int)(tid / npair);
-    const long q = tid - (long)sp * npair;
-    if (sp >= MAX_SHELLS * MAX_SHELLS) return;
-    // q -> (p > r): q = p*(p-1)/2 + r
-    int p = (int)((1.0 + sqrt(1.0 + 8.0 * (double)q)) * 0.5);
-    while ((long)p * (p - 1) / 2 > q) --p;
-    while ((long)(p + 1) * p / 2 <= q) ++p;
-    const int r = (int)(q - (long)p * (p - 1) / 2);
-    const int ap = b.atom_order[p], ar = b.atom_order[r];
-    // the reference's roles: A is the atom of higher index (overlap_D.f:144-311)
-    const bool p_is_a = ap > ar;
-    const int ia = p_is_a ? ap : ar, ib = p_is_a ? ar : ap;
-    const int sa = p_is_a ? sp / MAX_SHELLS : sp % MAX_SHELLS;
-    const int sb = p_is_a ? sp % MAX_SHELLS : sp / MAX_SHELLS;
-    if (sa >= b.atom_nshell[ia] || sb >= b.atom_nshell[ib]) return;
-    const double xab = b.coords[3 * ib + 0] - b.coords[3 * ia + 0];
-    const double yab = b.coords[3 * ib + 1] - b.coords[3 * ia + 1];
-    const double zab = b.coords[3 * ib + 2] - b.coords[3 * ia + 2];
-    const double R = sqrt(xab * xab + yab * yab + zab * zab);
-    if (R > cutoff) return;
-    const int shA = b.atom_shell0[ia] + sa, shB = b.atom_shell0[ib] + sb;
-    const int na = b.sh_n[shA], la = b.sh_l[shA], nb = b.sh_n[shB], lb = b.sh_l[shB];
-    double rl[75];
-    double Rab;
-    rotation_dev(xab, yab, zab, max(la, lb), rl, &Rab);
-    const double aux = 1.0 / (dfact(2 * na) * dfact(2 * nb));
-    const int msup = min(la, lb);
-    double solnorm[3] = {0.0, 0.0, 0.0};
-    double solvec[3];
-    for (int j = 0; j < b.sh_nzeta[shB]; ++j) {
-        for (int i = 0; i < b.sh_nzeta[shA]; ++i) {
-            const double expb = b.sh_zeta[2 * shB + j], expa = b.sh_zeta[2 * shA + i];
-            solap_dev(na, la, expa, nb, lb, expb, Rab, solvec);
-            // GET_ANOR
-            double anor = pow(expa * 2.0, (double)(na * 2 + 1)) * pow(expb * 2.0, (double)(nb * 2 + 1)) *
-                          (la * 2 + 1.0) * (lb * 2 + 1.0) * aux;
-            anor = sqrt(anor) / (4.0 * 3.141592653589793238462643383279502884);
-            double part[3];
-            for (int m = 0; m <= msup - 1; ++m) {
-                part[m] = solvec[m] * anor;
-                anor = anor / sqrt((la + m + 1.0) * (la - m) * (lb + m + 1.0) * (lb - m));
-                if (m == 0) anor = anor + anor;
+    const long q = blockIdx.x * 256L + threadIdx.x;
+    int2 pr = make_int2(0, 0);
+    bool near = false;
+    if (q < npair) {
+        // q -> (p > r): q = p*(p-1)/2 + r
+        int p = (int)((1.0 + sqrt(1.0 + 8.0 * (double)q)) * 0.5);
+        while ((long)p * (p - 1) / 2 > q) --p;
+        while ((long)(p + 1) * p / 2 <= q) ++p;
+        const int r = (int)(q - (long)p * (p - 1) / 2);
+        const int ap = b.atom_order[p], ar = b.atom_order[r];
+        const double x = b.coords[3 * ap] - b.coords[3 * ar], y = b.coords[3 * ap + 1] - b.coords[3 * ar + 1],
+                     z = b.coords[3 * ap + 2] - b.coords[3 * ar + 2];
+        near = !(sqrt(x * x + y * y + z * z) > cutoff);
+        pr = make_int2(ap, ar);
+    }
+    const unsigned long long mask = __ballot(near);
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    if (lane == 0 && mask) base = atomicAdd(count, __popcll(mask));
+    base = __shfl(base, 0);
+    if (near) list[base + __popcll(mask & ((1ull << lane) - 1))] = pr;
+}
+
+template <int LA, int LB>
+__device__ __forceinline__ void shell_block(const BasisDev& b, int shA, int shB, const Axes& ax, double R, double* S,
+                                            double* h, int ld, double s_drop) {
+    constexpr int MS = LA < LB ? LA : LB;
+    double sig[MS + 1];
+#pragma unroll
+    for (int m = 0; m <= MS; ++m) sig[m] = 0.0;
+    for (int j = 0; j < b.sh_nzeta[shB]; ++j)
+        for (int i = 0; i < b.sh_nzeta[shA]; ++i)
+            lined_up<LA, LB>(b.sh_n[shA], b.sh_zeta[2 * shA + i], b.sh_n[shB], b.sh_zeta[2 * shB + j], R,
+                             b.sh_coef[2 * shA + i] * b.sh_coef[2 * shB + j], sig);
+    double blk[2 * LA + 1][2 * LB + 1];
+#pragma unroll
+    for (int m = -MS; m <= MS; ++m) {
+        double ra[2 * LA + 1], rb[2 * LB + 1];
+        rotation_column<LA>(ax, m, ra);
+        rotation_column<LB>(ax, m, rb);
+        const double s = sig[m < 0 ? -m : m];
+#pragma unroll
+        for (int i = 0; i <= 2 * LA; ++i)
+#pragma unroll
+            for (int j = 0; j <= 2 * LB; ++j) {
+                const double v = s * ra[i] * rb[j];
+                blk[i][j] = m == -MS ? v : blk[i][j] + v;
             }
-            part[msup] = solvec[msup] * anor;
-            const double cc = b.sh_coef[2 * shA + i] * b.sh_coef[2 * shB + j];
-            for (int k = 0; k <= msup; ++k) solnorm[k] += cc * part[k];
-        }
     }
     const int a0 = b.sh_orb0[shA], b0 = b.sh_orb0[shB];
-    for (int mb = -lb; mb <= lb; ++mb) {
-        for (int ma = -la; ma <= la; ++ma) {
-            double s = solnorm[0] * rl[RX(ma, 0, la)] * rl[RX(mb, 0, lb)];
-            for (int k = 1; k <= msup; ++k)
-                s += solnorm[k] * (rl[RX(ma, -k, la)] * rl[RX(mb, -k, lb)] + rl[RX(ma, k, la)] * rl[RX(mb, k, lb)]);
+    // X of the block: IP, k_WH and V_shift per orbital
+#pragma unroll
+    for (int j = 0; j <= 2 * LB; ++j)
+#pragma unroll
+        for (int i = 0; i <= 2 * LA; ++i) {
+            double s = blk[i][j];
             if (fabs(s) < s_drop) s = 0.0;
-            const int a = a0 + ma + la, bo = b0 + mb + lb;
+            const int a = a0 + i, bo = b0 + j;
             const double hv = huckel_x(b.ip[a], b.ip[bo], b.kwh[a], b.kwh[bo], b.vshift[a], b.vshift[bo]) * s;
             S[(long)a + (long)ld * bo] = s;
             S[(long)bo + (long)ld * a] = s;
             h[(long)a + (long)ld * bo] = hv;
             h[(long)bo + (long)ld * a] = hv;
         }
+}
+
+__global__ __launch_bounds__(64) void build_SH_kernel(const BasisDev b, const int* count, const int2* list, double* S,
+                                                      double* h, int ld, double s_drop) {
+    const int q = blockIdx.x * 64 + threadIdx.x;
+    if (q >= *count) return;
+    const int2 pr = list[q];
+    const int sp = blockIdx.y;
+    // the reference's roles: A is the atom of higher index (overlap_D.f:144-311)
+    const bool p_is_a = pr.x > pr.y;
+    const int ia = p_is_a ? pr.x : pr.y, ib = p_is_a ? pr.y : pr.x;
+    const int sa = p_is_a ? sp / MAX_SHELLS : sp % MAX_SHELLS;
+    const int sb = p_is_a ? sp % MAX_SHELLS : sp / MAX_SHELLS;
+    if (sa >= b.atom_nshell[ia] || sb >= b.atom_nshell[ib]) return;
+    Axes ax;
+    double R = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        ax.u[d] = b.coords[3 * ib + d] - b.coords[3 * ia + d];
+        R += ax.u[d] * ax.u[d];
+    }
+    R = sqrt(R);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) ax.u[d] /= R;
+    // e1 = axis x u for the coordinate axis farthest from u, e2 = u x e1
+    const double ux = fabs(ax.u[0]), uy = fabs(ax.u[1]), uz = fabs(ax.u[2]);
+    if (ux <= uy && ux <= uz) {
+        ax.e1[0] = 0.0; ax.e1[1] = -ax.u[2]; ax.e1[2] = ax.u[1];
+    } else if (uy <= uz) {
+        ax.e1[0] = ax.u[2]; ax.e1[1] = 0.0; ax.e1[2] = -ax.u[0];
+    } else {
+        ax.e1[0] = -ax.u[1]; ax.e1[1] = ax.u[0]; ax.e1[2] = 0.0;
+    }
+    const double n1 = 1.0 / sqrt(ax.e1[0] * ax.e1[0] + ax.e1[1] * ax.e1[1] + ax.e1[2] * ax.e1[2]);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) ax.e1[d] *= n1;
+    ax.e2[0] = ax.u[1] * ax.e1[2] - ax.u[2] * ax.e1[1];
+    ax.e2[1] = ax.u[2] * ax.e1[0] - ax.u[0] * ax.e1[2];
+    ax.e2[2] = ax.u[0] * ax.e1[1] - ax.u[1] * ax.e1[0];
+    const int shA = b.atom_shell0[ia] + sa, shB = b.atom_shell0[ib] + sb;
+    switch (3 * b.sh_l[shA] + b.sh_l[shB]) {
+        case 0: shell_block<0, 0>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 1: shell_block<0, 1>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 2: shell_block<0, 2>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 3: shell_block<1, 0>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 4: shell_block<1, 1>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 5: shell_block<1, 2>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 6: shell_block<2, 0>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 7: shell_block<2, 1>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        default: shell_block<2, 2>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
     }
 }
-#undef RX
 
-int launch_build_SH(const BasisDev& b, int N, int ld, double* S, double* h, double cutoff, double s_drop,
+// scratch: a counter, then up to n_atoms (n_atoms - 1) / 2 pairs (8 bytes each)
+int launch_build_SH(const BasisDev& b, int N, int ld, double* S, double* h, double cutoff, double s_drop, void* scratch,
                     hipStream_t st) {
+    int* const count = static_cast<int*>(scratch);
+    int2* const list = reinterpret_cast<int2*>(static_cast<char*>(scratch) + 256);
     {
         const long total = (long)ld * ld;
         int blocks = (int)std::min<long>((total + 255) / 256, 8192);
-        hipLaunchKernelGGL(init_SH_kernel, dim3(blocks), dim3(256), 0, st, S, h, N, ld, b.ip, b.vshift);
+        hipLaunchKernelGGL(init_SH_kernel, dim3(blocks), dim3(256), 0, st, S, h, N, ld, b.ip, b.vshift, count);
     }
     const long npair = (long)b.n_atoms * (b.n_atoms - 1) / 2;
     if (npair > 0) {
-        const long threads = npair * MAX_SHELLS * MAX_SHELLS;
-        const int bs = 64;
-        const long blocks = (threads + bs - 1) / bs;
-        hipLaunchKernelGGL(build_SH_kernel, dim3((unsigned)blocks), dim3(bs), 0, st, b, S, h, ld, cutoff, s_drop);
+        hipLaunchKernelGGL(pair_list_kernel, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, b, cutoff, count,
+                           list);
+        hipLaunchKernelGGL(build_SH_kernel, dim3((unsigned)((npair + 63) / 64), MAX_SHELLS * MAX_SHELLS), dim3(64), 0, st,
+                           b, count, list, S, h, ld, s_drop);
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
