@@ -14,234 +14,172 @@
 
 namespace dh {
 
-constexpr int GK = 16;  // k-depth of one LDS stage
-constexpr int PAD = TILE + 1;
-
-// C = alpha * opA(A) opB(B) + beta * C on 64 x 64 tiles; 256 threads = 4 waves
-// in a 2 x 2 arrangement, each wave owning a 32 x 32 quadrant = 2 x 2 MFMA
-// 16 x 16 blocks.  MFMA f64 16x16x4 operand layout: lane l holds A[l%16][l/16]
-// and B[l/16][l%16]; accumulator value v of lane l is D[l/16 + 4*v][l%16]
-// (f64 layout: the four values of a lane are strided by 4 rows).
-// Tile of a workgroup.  Workgroups start in blockIdx order (x fastest); with a
-// k range that grows with the row (column) tile, the rows (columns) are taken
-// in reverse so that the heaviest tiles start first and the last ones to
-// start are short.  Each tile's arithmetic is the same either way.
-__device__ __forceinline__ void gemm_tile_of(const Gemm& g, int& bi, int& bj) {
-    bi = blockIdx.x;
-    bj = blockIdx.y;
-    if (g.kmode == K_BELOW_ROWTILE) bi = gridDim.x - 1 - bi;
-    else if (g.kmode == K_BELOW_COLTILE) bj = gridDim.y - 1 - bj;
+// C = alpha * opA(A) opB(B) + beta * C on T x T tiles, T = 64 or 32: 256 threads
+// = 4 waves in a 2 x 2 arrangement, each wave a T/2 x T/2 quadrant of 16 x 16
+// MFMA blocks (v_mfma_f64_16x16x4f64: lane l holds A[l%16][l/16] and
+// B[l/16][l%16]; result v of lane l is D[l/16 + 4v][l%16]).  The MFMA is issued
+// with the operands swapped (D^T = B^T A^T), so a lane's four results lie in
+// four columns and each column's 16 rows are contiguous in C.
+//
+// Bound: the matrix cores (64 cycles per instruction and SIMD).  A GK-deep k
+// stage is double-buffered in LDS; the stage after next is fetched into
+// registers while the current one is multiplied, and the next one goes from
+// registers to LDS half way through, so that its writes overlap products (one
+// barrier per stage).  The LDS rows are XOR-swizzled (gemm_sw) instead of
+// padded: operand reads (16 rows x 4 k), row-wise stores and k-wise stores
+// (transposed operands) are all free of bank conflicts.  Full products of 4096:
+// 55 TFLOP/s with T = 64 (3 workgroups a CU); 72 without the fetches, 75 for
+// the bare instructions.  A pair of 128 x 128 tiles per workgroup, which this
+// replaces, took 112 us where N = 576 now takes 18, 474 for L^-1 h at 2112
+// (210 now) and 1416 at 4096 (1257 now).
+//
+// Workgroups start in blockIdx order (x fastest).  With a k range that grows
+// with the row (column) tile, columns (rows) run fastest and the longest tiles
+// start first, so that the last ones to start are short; consecutive
+// workgroups go round the XCDs, so an XCD keeps to an eighth of the fast
+// dimension where that divides by 8 and its tiles share operands in its L2.
+template <int GK>
+__device__ __forceinline__ int gemm_sw(int k) {
+    return ((k & 1) << 4) | (k & 14) | (GK > 16 ? (k >> 4) & 1 : 0);
 }
 
+template <int T, int GK, int TA, int TB>
 __global__ __launch_bounds__(256) void gemm_f64_kernel(Gemm g) {
-    __shared__ double As[GK][PAD];
-    __shared__ double Bs[GK][PAD];
-    int bi, bj;
-    gemm_tile_of(g, bi, bj);
-    const int z = blockIdx.z;
-    if (g.lower_only && bi < bj) return;
-    const int i0 = bi * TILE, j0 = bj * TILE;
-    const double* A = g.A + z * g.strideA;
-    const double* B = g.B + z * g.strideB;
-    double* C = g.C + z * g.strideC;
+    __shared__ double As[2][GK * T];  // As[s][k * T + (i ^ gemm_sw(k))]
+    __shared__ double Bs[2][GK * T];
+    constexpr int MB = T / 32;        // 16 x 16 blocks of a wave per direction
+    constexpr int NL = GK * T / 256;  // values a thread fetches per operand and stage
+    const bool rows_fast = g.kmode == K_BELOW_COLTILE || g.kmode == K_FROM_COLTILE || g.kmode == K_FULL;
+    int bi = rows_fast ? blockIdx.x : blockIdx.y, bj = rows_fast ? blockIdx.y : blockIdx.x;
+    if (g.kmode == K_BELOW_ROWTILE) bi = gridDim.y - 1 - bi;
+    else if (g.kmode == K_BELOW_COLTILE) bj = gridDim.y - 1 - bj;
+    const int i0 = bi * T, j0 = bj * T;
+    if (g.lower_only && i0 / TILE < j0 / TILE) return;
+    const double* A = g.A + (long)blockIdx.z * g.strideA;
+    const double* B = g.B + (long)blockIdx.z * g.strideB;
+    double* C = g.C + (long)blockIdx.z * g.strideC;
     int klo = 0, khi = g.K;
-    if (g.kmode == K_BELOW_ROWTILE) khi = min(g.K, i0 + TILE);
-    else if (g.kmode == K_BELOW_COLTILE) khi = min(g.K, j0 + TILE);
+    if (g.kmode == K_BELOW_ROWTILE) khi = min(g.K, i0 + T);
+    else if (g.kmode == K_BELOW_COLTILE) khi = min(g.K, j0 + T);
     else if (g.kmode == K_FROM_ROWTILE) klo = i0;
     else if (g.kmode == K_FROM_COLTILE) klo = j0;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wi = (w >> 1) * 32, wj = (w & 1) * 32;
-    v4d acc[2][2];
+    const int wi = (w >> 1) * (T / 2), wj = (w & 1) * (T / 2);
+    const int lr = lane & 15, lk = lane >> 4;
+    v4d acc[MB][MB];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < MB; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
-
-    for (int k0 = klo; k0 < khi; k0 += GK) {
-        // stage A tile: rows i0..i0+63, k0..k0+15
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            int ii, kk;
-            if (!g.transA) {
-                ii = t & 63;
-                kk = (t >> 6) + 4 * r;
-            } else {
-                kk = t & 15;
-                ii = (t >> 4) + 16 * r;
-            }
-            const int gi = i0 + ii, gk = k0 + kk;
-            double v = 0.0;
-            if (gi < g.M && gk < khi) v = g.transA ? A[gk + g.lda * (long)gi] : A[gi + g.lda * (long)gk];
-            As[kk][ii] = v;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            int jj, kk;
-            if (!g.transB) {
-                kk = t & 15;
-                jj = (t >> 4) + 16 * r;
-            } else {
-                jj = t & 63;
-                kk = (t >> 6) + 4 * r;
-            }
-            const int gj = j0 + jj, gk = k0 + kk;
-            double v = 0.0;
-            if (gj < g.N && gk < khi) v = g.transB ? B[gj + g.ldb * (long)gk] : B[gk + g.ldb * (long)gj];
-            Bs[kk][jj] = v;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ks = 0; ks < GK; ks += 4) {
-            double av[2], bv[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) av[a] = As[ks + (lane >> 4)][wi + a * 16 + (lane & 15)];
-#pragma unroll
-            for (int b = 0; b < 2; ++b) bv[b] = Bs[ks + (lane >> 4)][wj + b * 16 + (lane & 15)];
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int gi = i0 + wi + a * 16 + (lane >> 4) + 4 * v;
-                const int gj = j0 + wj + b * 16 + (lane & 15);
-                if (gi < g.M && gj < g.N) {
-                    const long idx = gi + g.ldc * (long)gj;
-                    const double old = g.beta == 0.0 ? 0.0 : g.beta * C[idx];
-                    C[idx] = g.alpha * acc[a][b][v] + old;
-                }
-            }
-}
-
-// The same product on 128 x 128 tiles for large M and N: 4 waves in a 2 x 2
-// arrangement, each wave a 64 x 64 quadrant = 4 x 4 MFMA blocks; a 16-deep k
-// stage is double-buffered in LDS and the next stage is fetched into registers
-// while the current one feeds the matrix cores (one barrier per stage).  The
-// MFMA is issued with the operands swapped (D^T = B^T A^T), so a lane's four
-// results lie in four columns and each column's 16 rows are contiguous in C.
-// lower_only: tiles with row-tile < col-tile are skipped at the 64 x 64 level,
-// as in the 64 x 64 kernel.
-constexpr int G2_T = 128, G2_BK = 16, G2_PAD = G2_T + 4;
-
-// One 128 x 128 output tile (bi, bj) of batch z; the LDS stages are the caller's.
-template <int TA, int TB>
-__device__ __forceinline__ void gemm128_tile(const Gemm& g, int bi, int bj, int z, double (*As)[G2_BK][G2_PAD],
-                                             double (*Bs)[G2_BK][G2_PAD]) {
-    if (g.lower_only && bi < bj) return;
-    const int i0 = bi * G2_T, j0 = bj * G2_T;
-    const double* A = g.A + z * g.strideA;
-    const double* B = g.B + z * g.strideB;
-    double* C = g.C + z * g.strideC;
-    int klo = 0, khi = g.K;
-    if (g.kmode == K_BELOW_ROWTILE) khi = min(g.K, i0 + G2_T);
-    else if (g.kmode == K_BELOW_COLTILE) khi = min(g.K, j0 + G2_T);
-    else if (g.kmode == K_FROM_ROWTILE) klo = i0;
-    else if (g.kmode == K_FROM_COLTILE) klo = j0;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wi = (w >> 1) * 64, wj = (w & 1) * 64;
-    v4d acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
-    // C <- C - A B (alpha = -1, beta = 1): C is read into the accumulators
-    // before the k loop, where its latency overlaps the operand loads, and the
-    // products are subtracted (A negated on its way out of LDS, exactly)
+        for (int b = 0; b < MB; ++b) acc[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
+    // C <- C - A B: C is read into the accumulators before the k loop, where its
+    // latency overlaps the operand loads, and the products are subtracted (A
+    // negated on its way out of LDS, exactly)
     const bool cacc = g.c_acc != 0;
     if (cacc) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < MB; ++a)
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
+            for (int b = 0; b < MB; ++b)
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const int gi = i0 + wi + a * 16 + (lane & 15);
-                    const int gj = j0 + wj + b * 16 + (lane >> 4) + 4 * v;
-                    acc[a][b][v] = (gi < g.M && gj < g.N) ? C[gi + g.ldc * (long)gj] : 0.0;
+                    const int gi = min(i0 + wi + a * 16 + lr, g.M - 1), gj = min(j0 + wj + b * 16 + lk + 4 * v, g.N - 1);
+                    acc[a][b][v] = C[gi + g.ldc * (long)gj];
                 }
     }
-
-    double ra[8], rb[8];
-    auto gload = [&](int k0) {
+    // value r of this thread: row (column) ia, depth ka (kb) of the stage; rows
+    // past the edge are read from the last one and their results not stored
+    auto ia = [&](int r) { return TA ? t / GK + (256 / GK) * r : t % T; };
+    auto ka = [&](int r) { return TA ? t % GK : t / T + (256 / T) * r; };
+    auto jb = [&](int r) { return TB ? t % T : t / GK + (256 / GK) * r; };
+    auto kb = [&](int r) { return TB ? t / T + (256 / T) * r : t % GK; };
+    const long sa = TA ? 1 : g.lda, sb = TB ? g.ldb : 1;  // strides of one k
+    unsigned oa[NL], ob[NL];                              // byte offsets from the stage's first k
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int ii = TA ? (t >> 4) + 16 * r : (t & 127);
-            const int kk = TA ? (t & 15) : (t >> 7) + 2 * r;
-            const int gi = i0 + ii, gk = k0 + kk;
-            double v = 0.0;
-            if (gi < g.M && gk < khi) v = TA ? A[gk + g.lda * (long)gi] : A[gi + g.lda * (long)gk];
-            ra[r] = v;
-        }
+    for (int r = 0; r < NL; ++r) {
+        oa[r] = 8u * (unsigned)(min(ia(r), g.M - 1 - i0) * (TA ? (int)g.lda : 1) + ka(r) * (int)sa);
+        ob[r] = 8u * (unsigned)(min(jb(r), g.N - 1 - j0) * (TB ? 1 : (int)g.ldb) + kb(r) * (int)sb);
+    }
+    const double* At = A + (TA ? g.lda * (long)i0 : (long)i0);
+    const double* Bt = B + (TB ? (long)j0 : g.ldb * (long)j0);
+    const int ns = (khi - klo + GK - 1) / GK;  // stages; a last one that is not whole starts earlier,
+    const int skip = ns * GK - (khi - klo);    // its first `skip` depths, done before, count as zero
+    double ra[2][NL], rb[2][NL];
+    auto at = [](const double* base, unsigned o) { return *(const double*)((const char*)base + o); };
+    auto gload = [&](int st, int q) {
+        const int k0 = klo + st * GK - (st == ns - 1 ? skip : 0);
+        const double* Ak = At + sa * k0;
+        const double* Bk = Bt + sb * k0;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int jj = TB ? (t & 127) : (t >> 4) + 16 * r;
-            const int kk = TB ? (t >> 7) + 2 * r : (t & 15);
-            const int gj = j0 + jj, gk = k0 + kk;
-            double v = 0.0;
-            if (gj < g.N && gk < khi) v = TB ? B[gj + g.ldb * (long)gk] : B[gk + g.ldb * (long)gj];
-            rb[r] = v;
-        }
-    };
-    auto swrite = [&](int s) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int ii = TA ? (t >> 4) + 16 * r : (t & 127);
-            const int kk = TA ? (t & 15) : (t >> 7) + 2 * r;
-            As[s][kk][ii] = ra[r];
-        }
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int jj = TB ? (t & 127) : (t >> 4) + 16 * r;
-            const int kk = TB ? (t >> 7) + 2 * r : (t & 15);
-            Bs[s][kk][jj] = rb[r];
+        for (int r = 0; r < NL; ++r) {
+            ra[q][r] = at(Ak, oa[r]);
+            rb[q][r] = at(Bk, ob[r]);
         }
     };
-    int s = 0;
-    if (klo < khi) {
-        gload(klo);
-        swrite(0);
+    auto swrite = [&](int st, int q) {
+        const int z = st == ns - 1 ? skip : 0;
+#pragma unroll
+        for (int r = 0; r < NL; ++r) {
+            As[q][ka(r) * T + (ia(r) ^ gemm_sw<GK>(ka(r)))] = ka(r) < z ? 0.0 : ra[q][r];
+            Bs[q][kb(r) * T + (jb(r) ^ gemm_sw<GK>(kb(r)))] = kb(r) < z ? 0.0 : rb[q][r];
+        }
+    };
+    auto multiply = [&](int q, int st) {  // and, half way, stage st (if there is one) from the registers to the other buffer
+        double av[2][MB], bv[2][MB];
+        auto fetch = [&](int ks) {
+            const int k = ks + lk, x = gemm_sw<GK>(k), p = (ks >> 2) & 1;
+#pragma unroll
+            for (int a = 0; a < MB; ++a) av[p][a] = As[q][k * T + ((wi + a * 16 + lr) ^ x)];
+#pragma unroll
+            for (int b = 0; b < MB; ++b) bv[p][b] = Bs[q][k * T + ((wj + b * 16 + lr) ^ x)];
+        };
+        fetch(0);
+#pragma unroll
+        for (int ks = 0; ks < GK; ks += 4) {
+            if (ks + 4 < GK) fetch(ks + 4);
+            if (ks == GK / 2 && st < ns) swrite(st, 1 - q);
+            __builtin_amdgcn_sched_barrier(0);  // the next operands are on their way before these products start
+            const int p = (ks >> 2) & 1;
+#pragma unroll
+            for (int a = 0; a < MB; ++a)
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+                    acc[a][b] =
+                        __builtin_amdgcn_mfma_f64_16x16x4f64(bv[p][b], cacc ? -av[p][a] : av[p][a], acc[a][b], 0, 0, 0);
+        }
+    };
+    if (khi - klo >= GK) {
+        gload(0, 0);
+        if (ns > 1) gload(1, 1);
+        swrite(0, 0);
+    } else if (khi > klo) {  // one short stage: depths past the end are read from the last one and set to zero
+        const int last = khi - 1 - klo;
+#pragma unroll
+        for (int r = 0; r < NL; ++r) {
+            const int da = max(ka(r) - last, 0), db = max(kb(r) - last, 0);
+            const double va = at(At + sa * klo, oa[r] - 8u * (unsigned)(da * (int)sa));
+            const double vb = at(Bt + sb * klo, ob[r] - 8u * (unsigned)(db * (int)sb));
+            As[0][ka(r) * T + (ia(r) ^ gemm_sw<GK>(ka(r)))] = da ? 0.0 : va;
+            Bs[0][kb(r) * T + (jb(r) ^ gemm_sw<GK>(kb(r)))] = db ? 0.0 : vb;
+        }
     }
     __syncthreads();
-    for (int k0 = klo; k0 < khi; k0 += G2_BK) {
-        const bool more = k0 + G2_BK < khi;
-        if (more) gload(k0 + G2_BK);
-#pragma unroll
-        for (int ks = 0; ks < G2_BK; ks += 4) {
-            double av[4], bv[4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const double x = As[s][ks + (lane >> 4)][wi + a * 16 + (lane & 15)];
-                av[a] = cacc ? -x : x;
-            }
-#pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = Bs[s][ks + (lane >> 4)][wj + b * 16 + (lane & 15)];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[b], av[a], acc[a][b], 0, 0, 0);
-        }
-        if (more) swrite(s ^ 1);
+    auto stage = [&](int st, int q) {  // stage st in LDS buffer q, st + 1 in registers 1 - q, st + 2 asked for
+        if (st + 2 < ns) gload(st + 2, q);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(q, st + 1);
         __syncthreads();
-        s ^= 1;
+    };
+    for (int st = 0; st < ns; st += 2) {
+        stage(st, 0);
+        if (st + 1 < ns) stage(st + 1, 1);
     }
-    if (g.lower_only && (i0 + wi) / TILE < (j0 + wj) / TILE) return;
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < MB; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < MB; ++b)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int gi = i0 + wi + a * 16 + (lane & 15);
-                const int gj = j0 + wj + b * 16 + (lane >> 4) + 4 * v;
+                const int gi = i0 + wi + a * 16 + lr, gj = j0 + wj + b * 16 + lk + 4 * v;
                 if (gi < g.M && gj < g.N) {
                     const long idx = gi + g.ldc * (long)gj;
                     if (cacc) {
@@ -254,183 +192,272 @@ __device__ __forceinline__ void gemm128_tile(const Gemm& g, int bi, int bj, int 
             }
 }
 
-// A workgroup computes one tile, or with g.pair two tiles whose k ranges add up
-// to the same length (row tiles i and n-1-i of a triangular k range, or the
-// same for columns): every workgroup then does equal work, which a one-tile
-// grid cannot give when the heavy tiles land on a few XCDs.
-template <int TA, int TB>
-__global__ __launch_bounds__(256, 2) void gemm128_f64_kernel(Gemm g) {
-    __shared__ double As[2][G2_BK][G2_PAD];
-    __shared__ double Bs[2][G2_BK][G2_PAD];
-    const int z = blockIdx.z;
-    int bi, bj;
-    gemm_tile_of(g, bi, bj);
-    int npass = 1;
-    if (g.pair) {
-        const int rows = g.pair == 1;
-        const int n = rows ? (g.M + G2_T - 1) / G2_T : (g.N + G2_T - 1) / G2_T;
-        bi = blockIdx.x;
-        bj = blockIdx.y;
-        npass = (rows ? n - 1 - bi : n - 1 - bj) != (rows ? bi : bj) ? 2 : 1;
-    }
-#pragma unroll 1
-    for (int pass = 0; pass < npass; ++pass) {
-        if (pass == 1) {
-            __syncthreads();  // the first tile's LDS readers are done
-            if (g.pair == 1) bi = (g.M + G2_T - 1) / G2_T - 1 - bi;
-            else bj = (g.N + G2_T - 1) / G2_T - 1 - bj;
-        }
-        gemm128_tile<TA, TB>(g, bi, bj, z, As, Bs);
-    }
+template <int T, int GK>
+static void gemm_tiles(const Gemm& g, hipStream_t st) {
+    const unsigned nr = (g.M + T - 1) / T, nc = (g.N + T - 1) / T, nz = g.batch > 0 ? g.batch : 1;
+    const bool rows_fast = g.kmode == K_BELOW_COLTILE || g.kmode == K_FROM_COLTILE || g.kmode == K_FULL;
+    const dim3 grid(rows_fast ? nr : nc, rows_fast ? nc : nr, nz);
+    if (!g.transA && !g.transB) hipLaunchKernelGGL((gemm_f64_kernel<T, GK, 0, 0>), grid, dim3(256), 0, st, g);
+    else if (!g.transA) hipLaunchKernelGGL((gemm_f64_kernel<T, GK, 0, 1>), grid, dim3(256), 0, st, g);
+    else if (!g.transB) hipLaunchKernelGGL((gemm_f64_kernel<T, GK, 1, 0>), grid, dim3(256), 0, st, g);
+    else hipLaunchKernelGGL((gemm_f64_kernel<T, GK, 1, 1>), grid, dim3(256), 0, st, g);
 }
 
-void launch_gemm(const Gemm& g, hipStream_t st) {
-    if (g.M <= 0 || g.N <= 0) return;
-    const unsigned nz = g.batch > 0 ? g.batch : 1;
-    if (g.M >= 2 * G2_T && g.N >= 2 * G2_T) {
-        Gemm p = g;
-        dim3 grid((g.M + G2_T - 1) / G2_T, (g.N + G2_T - 1) / G2_T, nz);
-        p.pair = 0;
-        p.c_acc = g.alpha == -1.0 && g.beta == 1.0;
-        if (!g.lower_only && (g.kmode == K_BELOW_ROWTILE || g.kmode == K_FROM_ROWTILE)) {
-            p.pair = 1;
-            grid.x = (grid.x + 1) / 2;
-        } else if (!g.lower_only && (g.kmode == K_BELOW_COLTILE || g.kmode == K_FROM_COLTILE)) {
-            p.pair = 2;
-            grid.y = (grid.y + 1) / 2;
-        }
-        if (!g.transA && !g.transB) hipLaunchKernelGGL((gemm128_f64_kernel<0, 0>), grid, dim3(256), 0, st, p);
-        else if (!g.transA) hipLaunchKernelGGL((gemm128_f64_kernel<0, 1>), grid, dim3(256), 0, st, p);
-        else if (!g.transB) hipLaunchKernelGGL((gemm128_f64_kernel<1, 0>), grid, dim3(256), 0, st, p);
-        else hipLaunchKernelGGL((gemm128_f64_kernel<1, 1>), grid, dim3(256), 0, st, p);
-        return;
-    }
-    dim3 grid((g.M + TILE - 1) / TILE, (g.N + TILE - 1) / TILE, nz);
-    hipLaunchKernelGGL(gemm_f64_kernel, grid, dim3(256), 0, st, g);
+// 64 x 64 tiles carry twice the arithmetic per byte fetched, 32 x 32 ones fill
+// the chip earlier and leave a shorter tail.  Measured, us (64, 32): L^-1 h at
+// N = 1024: 64, 41; 1792: 170, 151; 2112: 210, 223; 4096: 1257, 1624.  With
+// half the tiles and the longest k ranges on the few full columns the tail
+// weighs more: W L^-T at 2112: 176, 89; 4096: 741, 661; 7040: 2285, 2826.
+constexpr long GEMM_TILES = 1024, GEMM_TILES_LOWER = 5120;  // whole grids of 64 x 64 tiles from which they are used
+
+void launch_gemm(const Gemm& g0, hipStream_t st) {
+    if (g0.M <= 0 || g0.N <= 0) return;
+    Gemm g = g0;
+    g.c_acc = g.alpha == -1.0 && g.beta == 1.0;
+    const long tiles = (long)((g.M + 63) / 64) * ((g.N + 63) / 64) * (g.batch > 0 ? g.batch : 1);
+    if (tiles >= (g.lower_only && g.kmode != K_FULL ? GEMM_TILES_LOWER : GEMM_TILES)) gemm_tiles<64, 16>(g, st);
+    else gemm_tiles<32, 32>(g, st);
 }
 
-// Factor the 64 x 64 diagonal block at (j0, j0) in place (lower) and write its
-// inverse to Dinv[blk].  1024 threads, the block in LDS (column-major, padded),
-// blocked by 16 so that only 20 barriers separate the serial parts:
-//   factor, for each 16-column sub-panel k0:
-//     1. wave 0 factors the 16 x 16 diagonal sub-block, lane r holding row r in
-//        registers and taking column entries of other rows by shuffles;
-//     2. one thread per row below solves L_i,panel = A_i,panel L_D^-T by forward
-//        substitution over the 16 columns;
-//     3. all threads apply the rank-16 update to the lower part below;
-//   inverse X = L^-1:
-//     4. waves 0..3 invert the four 16 x 16 diagonal sub-blocks (lane c solves
-//        column c by forward substitution);
-//     5. sub-diagonal d = 1, 2, 3: T_IJ = sum_{K=J..I-1} L_IK X_KJ, then
-//        X_IJ = -X_II T_IJ, for all sub-blocks I - J = d at once.
+// Element (r, c) of a 64 x 64 block in LDS: columns of 64, odd ones with their
+// halves of 32 swapped by 16s, so that a 16 x 4 MFMA operand is read without
+// bank conflicts.
+__device__ __forceinline__ int blk_at(int r, int c) { return c * TILE + (r ^ ((c & 1) << 4)); }
+
+// 16 x 16 x 16 product of two sub-blocks held in LDS (A: rows ar.., columns ac..;
+// B: rows br.., columns bc..), added to acc in the plain layout (result v of
+// lane l: row l/16 + 4v, column l%16), which is also the layout of a B operand:
+// a product can be multiplied from the left by another without leaving the
+// registers (blk_mul_reg).
+__device__ __forceinline__ void blk_mul(v4d& acc, const double* A, int ar, int ac, const double* B, int br, int bc,
+                                        int lane) {
+    const int i = lane & 15, k = lane >> 4;
+#pragma unroll
+    for (int ks = 0; ks < 16; ks += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[blk_at(ar + i, ac + ks + k)], B[blk_at(br + ks + k, bc + i)], acc, 0,
+                                                   0, 0);
+}
+__device__ __forceinline__ void blk_mul_reg(v4d& acc, const double* A, int ar, int ac, v4d b, int lane) {
+    const int i = lane & 15, k = lane >> 4;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(A[blk_at(ar + i, ac + 4 * ks + k)], b[ks], acc, 0, 0, 0);
+}
+
+__device__ __forceinline__ double lane_value(double x, int l) {  // x of lane l (uniform), to a scalar register pair
+    const long u = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readlane((int)u, l), hi = __builtin_amdgcn_readlane((int)(u >> 32), l);
+    return __longlong_as_double((long)(((unsigned long)hi << 32) | lo));
+}
+
+// sqrt(d) and its reciprocal for a normal d > 0 by Goldschmidt's coupled
+// iteration from the hardware's estimate, with one residual correction of the
+// root: both are good to an ulp.
+__device__ __forceinline__ void root_and_inverse(double d, double& root, double& inv) {
+    const double y = __builtin_amdgcn_rsq(d);
+    double g = d * y, h = 0.5 * y;
+    double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    root = fma(fma(-g, g, d), h, g);
+    inv = 2.0 * h;
+}
+__device__ __forceinline__ double quotient(double a, double b, double binv) {  // a / b, 1/b known to an ulp
+    const double q = a * binv;
+    return fma(fma(-q, b, a), binv, q);
+}
+
+// inverse of the lower triangular 16 x 16 sub-block at (b0, b0) of L, column
+// `lane` of it by forward substitution
+__device__ __forceinline__ void invert_16(const double* L, const double* rinv, double* X, int b0, int lane) {
+    if (lane >= 16) return;
+    double x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        double v = i == lane ? 1.0 : 0.0;
+#pragma unroll
+        for (int k = 0; k < i; ++k) v = fma(-L[blk_at(b0 + i, b0 + k)], x[k], v);
+        x[i] = quotient(v, L[blk_at(b0 + i, b0 + i)], rinv[b0 + i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) X[blk_at(b0 + i, b0 + lane)] = x[i];
+}
+
+// Block b of a panel that starts at block p0: take the panel's earlier columns
+// off the 64 x 64 diagonal block (j0 = 64 b), factor it in place (lower) and
+// write its inverse to Dinv[b].  One workgroup of 10 waves; bound by the serial
+// chain of 64 columns, so that chain is kept short:
+//   wave 0 factors 16 columns at a time with the 64 rows as its lanes and the 16
+//   columns in registers: a column costs one root (root_and_inverse), one
+//   quotient and, per later column, a scalar broadcast (v_readlane) and an fma;
+//   the rank-16 update of the rest is one 16 x 16 MFMA block per wave;
+//   while wave 0 is at columns 16 p .., wave 1 inverts diagonal sub-block p - 1
+//   and wave 2 forms the (1, 0) block of the inverse; after the last columns the
+//   remaining blocks follow, X_IJ = -X_II (L_IJ X_JJ ..), T = L X formed while
+//   the last sub-block is inverted, products chained in registers.
 // The first non-positive pivot is reported as in LAPACK's potrf (1-based).
-constexpr int PD_P = TILE + 1;  // padded LDS column
-constexpr int PD_B = 16;        // sub-block size
-__global__ __launch_bounds__(1024) void potrf_diag_kernel(double* A, int ld, int j0, double* Dinv, int* info) {
-    __shared__ double Ls[TILE * PD_P];  // Ls[c * PD_P + r] = block (r, c)
-    __shared__ double Xs[TILE * PD_P];  // inverse, same layout
-    __shared__ double Ts[TILE * PD_P];  // products of step 5
-    __shared__ int bad;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    if (t == 0) bad = TILE + 1;
-    for (int e = t; e < TILE * TILE; e += 1024) {
-        const int r = e % TILE, c = e / TILE;
-        Ls[c * PD_P + r] = A[(long)(j0 + r) + (long)ld * (j0 + c)];
-        Xs[c * PD_P + r] = 0.0;
+__global__ __launch_bounds__(640) void potrf_diag_kernel(double* A, int ld, int p0, int b, double* Dinv, int* info) {
+    __shared__ double Ls[TILE * TILE];
+    __shared__ double Xs[TILE * TILE];
+    __shared__ double rinv[TILE];
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int lr = lane & 15, lk = lane >> 4;
+    const int j0 = b * TILE;
+    int bad = 0;  // wave 0: first bad column + 1
+    if (w < 10) {  // lower sub-blocks (I, J), minus the products of the panel's earlier columns
+        const int I = w >= 6 ? 3 : w >= 3 ? 2 : w >= 1 ? 1 : 0, J = w - I * (I + 1) / 2;
+        const double* D = A + (j0 + 16 * I + lr) + (long)ld * (j0 + 16 * J + lk);
+        v4d acc;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[v] = D[(long)ld * (4 * v)];
+        for (int k0 = p0 * TILE; k0 < j0; k0 += TILE) {
+            const double* LI = A + (j0 + 16 * I + lr) + (long)ld * (k0 + lk);
+            const double* LJ = A + (j0 + 16 * J + lr) + (long)ld * (k0 + lk);
+            double a[16], c[16];
+#pragma unroll
+            for (int ks = 0; ks < 16; ++ks) {
+                a[ks] = LI[(long)ld * (4 * ks)];
+                c[ks] = LJ[(long)ld * (4 * ks)];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // every load is issued before the first product waits
+#pragma unroll
+            for (int ks = 0; ks < 16; ++ks) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(c[ks], -a[ks], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Ls[blk_at(16 * I + lr, 16 * J + lk + 4 * v)] = acc[v];
+    }
+    for (int e = t; e < TILE * TILE; e += 640) Xs[e] = 0.0;
+    __syncthreads();
+    for (int p = 0; p < 4; ++p) {
+        const int k0 = 16 * p;
+        if (w == 0) {
+            const int row = (lane + k0) & 63;  // lanes 0..15: the diagonal sub-block; rows above it wrap to the last lanes
+            double a[16], piv = 1.0, ri = 1.0;
+            int ln = lane;
+            asm volatile("" : "+v"(ln));  // keeps the 16 lane masks below from living in scalar registers throughout
+#pragma unroll
+            for (int c = 0; c < 16; ++c) a[c] = Ls[blk_at(row, k0 + c)];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const double d = lane_value(a[j], j);
+                double sd, inv;
+                root_and_inverse(d > 0.0 ? d : 1.0, sd, inv);
+                const double l = ln == j ? sd : quotient(a[j], sd, inv);
+                piv = ln == j ? d : piv;
+                ri = ln == j ? inv : ri;
+                a[j] = l;
+#pragma unroll
+                for (int c = j + 1; c < 16; ++c) a[c] = fma(-l, lane_value(l, c), a[c]);
+            }
+            const unsigned long long failed = __ballot(lane < 16 && !(piv > 0.0));
+            if (failed && !bad) bad = k0 + __ffsll(failed);
+            if (lane < 16) rinv[k0 + lane] = ri;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) Ls[blk_at(row, k0 + c)] = a[c];
+        } else if (w == 1 && p > 0) {
+            invert_16(Ls, rinv, Xs, k0 - 16, lane);
+        } else if (w == 2 && p == 3) {  // X_10 = -X_11 (L_10 X_00)
+            v4d T = {0.0, 0.0, 0.0, 0.0}, X = {0.0, 0.0, 0.0, 0.0};
+            blk_mul(T, Ls, 16, 0, Xs, 0, 0, lane);
+            blk_mul_reg(X, Xs, 16, 16, T, lane);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Xs[blk_at(16 + lk + 4 * v, lr)] = -X[v];
+        }
+        __syncthreads();
+        const int n2 = 3 - p;  // sub-block rows below
+        if (w < n2 * (n2 + 1) / 2) {
+            const int i2 = w >= 3 ? 2 : w >= 1 ? 1 : 0, I = p + 1 + i2, J = p + 1 + w - i2 * (i2 + 1) / 2;
+            v4d acc;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[v] = Ls[blk_at(16 * I + lr, 16 * J + lk + 4 * v)];
+#pragma unroll
+            for (int ks = 0; ks < 16; ks += 4)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Ls[blk_at(16 * J + lr, k0 + ks + lk)],
+                                                           -Ls[blk_at(16 * I + lr, k0 + ks + lk)], acc, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) Ls[blk_at(16 * I + lr, 16 * J + lk + 4 * v)] = acc[v];
+        }
+        __syncthreads();
+    }
+    // waves 4..7: T_2J, T_3J = sum_K L_IK X_KJ over K = J..1 for the lower left
+    // 32 x 32 of the inverse; wave 1 inverts the last sub-block meanwhile, and
+    // wave 0 then closes X_32
+    v4d T2 = {0.0, 0.0, 0.0, 0.0}, T3 = {0.0, 0.0, 0.0, 0.0};
+    const int J = w & 1, low = (w >> 1) & 1;  // waves 4..7: block (2 + low, J)
+    if (w == 1) {
+        invert_16(Ls, rinv, Xs, 48, lane);
+    } else if (w >= 4 && w < 8) {
+        for (int K = J; K < 2; ++K) {
+            blk_mul(T2, Ls, 32, 16 * K, Xs, 16 * K, 16 * J, lane);
+            if (low) blk_mul(T3, Ls, 48, 16 * K, Xs, 16 * K, 16 * J, lane);
+        }
+    }
+    v4d T32 = {0.0, 0.0, 0.0, 0.0};
+    if (w == 0) blk_mul(T32, Ls, 48, 32, Xs, 32, 32, lane);
+    __syncthreads();
+    if (w == 0) {
+        v4d X = {0.0, 0.0, 0.0, 0.0};
+        blk_mul_reg(X, Xs, 48, 48, T32, lane);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) Xs[blk_at(48 + lk + 4 * v, 32 + lr)] = -X[v];
     }
     __syncthreads();
-    for (int k0 = 0; k0 < TILE; k0 += PD_B) {
-        if (w == 0) {  // 1. diagonal sub-block (wave-uniform branch: no barrier inside)
-            const int r = lane < PD_B ? lane : 0;
-            double a[PD_B];
+    if (w >= 4 && w < 8) {
+        v4d X = {0.0, 0.0, 0.0, 0.0};
+        blk_mul_reg(X, Xs, 32 + 16 * low, 32, T2, lane);
+        if (low) blk_mul_reg(X, Xs, 48, 48, T3, lane);
 #pragma unroll
-            for (int c = 0; c < PD_B; ++c) a[c] = Ls[(k0 + c) * PD_P + k0 + r];
-#pragma unroll
-            for (int j = 0; j < PD_B; ++j) {
-                const double d = __shfl(a[j], j);
-                const bool ok = d > 0.0;
-                if (!ok && lane == 0) atomicMin(&bad, k0 + j + 1);
-                const double sd = ok ? sqrt(d) : 1.0;
-                a[j] = lane == j ? sd : (lane > j ? a[j] / sd : a[j]);
-#pragma unroll
-                for (int c = j + 1; c < PD_B; ++c) {
-                    const double lcj = __shfl(a[j], c);  // L_cj from row c
-                    if (lane >= c) a[c] -= a[j] * lcj;
-                }
-            }
-            if (lane < PD_B) {
-#pragma unroll
-                for (int c = 0; c < PD_B; ++c) Ls[(k0 + c) * PD_P + k0 + lane] = c <= lane ? a[c] : 0.0;
-            }
-        }
-        __syncthreads();
-        const int n2 = TILE - k0 - PD_B;  // rows below the sub-block
-        if (n2 <= 0) break;
-        if (t < n2) {  // 2. sub-panel solve, one row per thread
-            const int i = k0 + PD_B + t;
-            double x[PD_B];
-#pragma unroll
-            for (int c = 0; c < PD_B; ++c) {
-                double v = Ls[(k0 + c) * PD_P + i];
-#pragma unroll
-                for (int k = 0; k < c; ++k) v -= x[k] * Ls[(k0 + k) * PD_P + k0 + c];
-                x[c] = v / Ls[(k0 + c) * PD_P + k0 + c];
-            }
-#pragma unroll
-            for (int c = 0; c < PD_B; ++c) Ls[(k0 + c) * PD_P + i] = x[c];
-        }
-        __syncthreads();
-        for (int e = t; e < n2 * n2; e += 1024) {  // 3. rank-16 update, lower part
-            const int i = k0 + PD_B + e % n2, j = k0 + PD_B + e / n2;
-            if (i < j) continue;
-            double v = Ls[j * PD_P + i];
-#pragma unroll
-            for (int k = 0; k < PD_B; ++k) v -= Ls[(k0 + k) * PD_P + i] * Ls[(k0 + k) * PD_P + j];
-            Ls[j * PD_P + i] = v;
-        }
-        __syncthreads();
-    }
-    if (w < TILE / PD_B && lane < PD_B) {  // 4. diagonal sub-block inverses
-        const int b0 = PD_B * w, c = lane;
-        double x[PD_B];
-#pragma unroll
-        for (int i = 0; i < PD_B; ++i) {
-            double v = i == c ? 1.0 : 0.0;
-#pragma unroll
-            for (int k = 0; k < i; ++k) v -= Ls[(b0 + k) * PD_P + b0 + i] * x[k];
-            x[i] = v / Ls[(b0 + i) * PD_P + b0 + i];
-        }
-#pragma unroll
-        for (int i = 0; i < PD_B; ++i) Xs[(b0 + c) * PD_P + b0 + i] = x[i];
+        for (int v = 0; v < 4; ++v) Xs[blk_at(32 + 16 * low + lk + 4 * v, 16 * J + lr)] = -X[v];
     }
     __syncthreads();
-    constexpr int NBK = TILE / PD_B;
-    for (int d = 1; d < NBK; ++d) {  // 5. off-diagonal sub-blocks by sub-diagonal
-        const int nblk = NBK - d;
-        for (int e = t; e < nblk * PD_B * PD_B; e += 1024) {
-            const int J = e / (PD_B * PD_B), I = J + d, i = e % PD_B, j = (e / PD_B) % PD_B;
-            double v = 0.0;
-            for (int k = PD_B * J; k < PD_B * I; ++k) v += Ls[k * PD_P + PD_B * I + i] * Xs[(PD_B * J + j) * PD_P + k];
-            Ts[(PD_B * J + j) * PD_P + PD_B * I + i] = v;
-        }
-        __syncthreads();
-        for (int e = t; e < nblk * PD_B * PD_B; e += 1024) {
-            const int J = e / (PD_B * PD_B), I = J + d, i = e % PD_B, j = (e / PD_B) % PD_B;
-            double v = 0.0;
-#pragma unroll
-            for (int k = 0; k < PD_B; ++k)
-                v -= Xs[(PD_B * I + k) * PD_P + PD_B * I + i] * Ts[(PD_B * J + j) * PD_P + PD_B * I + k];
-            Xs[(PD_B * J + j) * PD_P + PD_B * I + i] = v;
-        }
-        __syncthreads();
-    }
-    const int blk = j0 / TILE;
-    for (int e = t; e < TILE * TILE; e += 1024) {
+    for (int e = t; e < TILE * TILE; e += 640) {
         const int r = e % TILE, c = e / TILE;
-        A[(long)(j0 + r) + (long)ld * (j0 + c)] = r >= c ? Ls[c * PD_P + r] : 0.0;
-        Dinv[(long)blk * TILE * TILE + r + (long)TILE * c] = r >= c ? Xs[c * PD_P + r] : 0.0;
+        A[(long)(j0 + r) + (long)ld * (j0 + c)] = r >= c ? Ls[blk_at(r, c)] : 0.0;
+        Dinv[(long)b * TILE * TILE + e] = r >= c ? Xs[blk_at(r, c)] : 0.0;
     }
-    if (t == 0 && bad <= TILE && *info == 0) *info = j0 + bad;
+    if (t == 0 && bad && *info == 0) *info = j0 + bad;
+}
+
+// The column below diagonal block b of a panel that starts NK blocks earlier:
+// A_ib <- (A_ib - sum_k L_ik L_bk^T) L_bb^-T over the panel's columns k before
+// b.  A workgroup has 16 rows and its wave w the columns 16 w .. of the block;
+// all operands come straight from memory in MFMA layout and are in flight
+// together, so a launch costs one latency plus 16 (NK + 1) MFMA.  Bound by
+// that latency: rest / 16 workgroups (252 at ld = 4096) of at most 64 MFMA.
+template <int NK>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void chol_column_kernel(double* A, int ld, int b, const double* Dinv) {
+    __shared__ double Ts[TILE * 16];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+    const int j0 = b * TILE, i0 = j0 + TILE + 16 * blockIdx.x;
+    double* X = A + (i0 + lr) + (long)ld * (j0 + 16 * w + lk);  // value v: column + 4 v
+    const double* Di = Dinv + (long)b * TILE * TILE + (16 * w + lr) + TILE * lk;
+    v4d acc;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = X[(long)ld * (4 * v)];
+    double a[16 * NK + 1], c[16 * NK + 1], di[16];
+#pragma unroll
+    for (int ks = 0; ks < 16 * NK; ++ks) {
+        const long col = (long)ld * (j0 - NK * TILE + 4 * ks + lk);
+        a[ks] = A[(i0 + lr) + col];
+        c[ks] = A[(j0 + 16 * w + lr) + col];
+    }
+#pragma unroll
+    for (int ks = 0; ks < 16; ++ks) di[ks] = Di[TILE * (4 * ks)];
+    __builtin_amdgcn_sched_barrier(0);  // every load is issued before the first product waits
+#pragma unroll
+    for (int ks = 0; ks < 16 * NK; ++ks) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(c[ks], -a[ks], acc, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Ts[(16 * w + lk + 4 * v) * 16 + lr] = acc[v];
+    __syncthreads();
+    acc = (v4d){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int ks = 0; ks < 16; ++ks)  // the inverse is lower triangular: columns past 16 w + 15 are zero
+        if (ks < 4 * (w + 1)) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(di[ks], Ts[(4 * ks + lk) * 16 + lr], acc, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) X[(long)ld * (4 * v)] = acc[v];
 }
 
 // zero the blocks above the diagonal blocks (column j: rows 0 .. 64 floor(j / 64) - 1),
@@ -442,13 +469,12 @@ __global__ void zero_upper_blocks_kernel(double* A, int ld) {
     for (int i = threadIdx.x; i < top; i += blockDim.x) A[(long)i + (long)ld * j] = 0.0;
 }
 
-// Right-looking blocked Cholesky in panels of CHOL_PANEL 64-column blocks:
-// within a panel, block b is factored (potrf_diag_kernel), its column below is
-// solved against it, and the rank-64 update reaches only the panel's later
-// columns; the matrix right of the panel then takes one rank-256 update.  The
-// trailing matrix is read and written once per 256 columns instead of once per
-// 64 (at N = 4096 about 1.4 GB of update traffic instead of 5.7 GB), and its
-// GEMMs run with K = 256.
+// Blocked Cholesky in panels of CHOL_PANEL 64-column blocks, left-looking inside
+// a panel and right-looking between panels: a block takes two launches
+// (potrf_diag_kernel, chol_column_kernel), which apply the panel's earlier
+// columns on the fly, and the matrix right of the panel then takes one rank-256
+// update: it is read and written once per 256 columns and its GEMMs run with
+// K = 256.
 constexpr int CHOL_PANEL = 4;
 
 void launch_cholesky(double* A, int ld, double* Dinv, int* info, hipStream_t st) {
@@ -456,30 +482,13 @@ void launch_cholesky(double* A, int ld, double* Dinv, int* info, hipStream_t st)
     for (int p0 = 0; p0 < nb; p0 += CHOL_PANEL) {
         const int pe = std::min(nb, p0 + CHOL_PANEL);  // blocks p0 .. pe-1
         for (int b = p0; b < pe; ++b) {
-            const int j0 = b * TILE;
-            hipLaunchKernelGGL(potrf_diag_kernel, dim3(1), dim3(1024), 0, st, A, ld, j0, Dinv, info);
-            const int rest = ld - j0 - TILE;
-            if (rest <= 0) continue;
-            // column: A21 <- A21 * L11^-T (Dinv holds L11^-1).  In place is
-            // safe: N = 64 gives one column tile per row tile, and a tile reads
-            // all 64 k-columns of its own rows before it writes them.
-            Gemm g{};
-            g.M = rest; g.N = TILE; g.K = TILE;
-            g.A = A + (j0 + TILE) + (long)ld * j0; g.lda = ld;
-            g.B = Dinv + (long)b * TILE * TILE; g.ldb = TILE; g.transB = 1;
-            g.C = A + (j0 + TILE) + (long)ld * j0; g.ldc = ld;
-            g.alpha = 1.0; g.beta = 0.0; g.batch = 1;
-            launch_gemm(g, st);
-            // the panel's later columns (lower tiles only): A22[:, :w] -= A21 A21[:w]^T
-            const int w = pe * TILE - (j0 + TILE);
-            if (w <= 0) continue;
-            Gemm u{};
-            u.M = rest; u.N = w; u.K = TILE;
-            u.A = A + (j0 + TILE) + (long)ld * j0; u.lda = ld;
-            u.B = A + (j0 + TILE) + (long)ld * j0; u.ldb = ld; u.transB = 1;
-            u.C = A + (j0 + TILE) + (long)ld * (j0 + TILE); u.ldc = ld;
-            u.alpha = -1.0; u.beta = 1.0; u.lower_only = 1; u.batch = 1;
-            launch_gemm(u, st);
+            hipLaunchKernelGGL(potrf_diag_kernel, dim3(1), dim3(640), 0, st, A, ld, p0, b, Dinv, info);
+            const dim3 grid((ld - (b + 1) * TILE) / 16), block(256);
+            if (grid.x == 0) continue;
+            if (b == p0) hipLaunchKernelGGL(chol_column_kernel<0>, grid, block, 0, st, A, ld, b, Dinv);
+            else if (b == p0 + 1) hipLaunchKernelGGL(chol_column_kernel<1>, grid, block, 0, st, A, ld, b, Dinv);
+            else if (b == p0 + 2) hipLaunchKernelGGL(chol_column_kernel<2>, grid, block, 0, st, A, ld, b, Dinv);
+            else hipLaunchKernelGGL(chol_column_kernel<3>, grid, block, 0, st, A, ld, b, Dinv);
         }
         // right of the panel (lower tiles only): A33 -= L31 L31^T, K = the panel's width
         const int t0 = pe * TILE, rest = ld - t0;

@@ -187,3 +187,47 @@ def test_symmetric_half_storage_variant_large(n, n_wp, variant):
         ctx.close()
     finally:
         hip.force_matvec_variant(-1)
+
+
+@pytest.mark.parametrize("transA,transB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (31, 33, 15), (32, 65, 32), (63, 1, 33), (65, 129, 100),
+                                   (2049, 2047, 15), (2050, 2111, 16), (2047, 2049, 41)])
+def test_gemm_tile_edges(M, N, K, transA, transB):
+    """Tiles of 32 and (from 1024 tiles of 64 on) of 64; k ranges below, at and past a stage's depth."""
+    rng = np.random.default_rng(M + N + K)
+    _say(f"gemm edges M={M} N={N} K={K} tA={transA} tB={transB}")
+    A = rng.normal(size=(K, M) if transA else (M, K))
+    B = rng.normal(size=(N, K) if transB else (K, N))
+    C = rng.normal(size=(M, N))
+    oA, oB = (A.T if transA else A), (B.T if transB else B)
+    bound = 4.0 * (K + 3) * np.finfo(np.float64).eps * (np.abs(oA) @ np.abs(oB) + np.abs(C))
+    for alpha, beta in ((1.0, 0.0), (-1.0, 1.0)):  # the second starts from C in the accumulators
+        out = hip.run_gemm(A, B, C, alpha=alpha, beta=beta, transA=transA, transB=transB)
+        assert (np.abs(out - (alpha * (oA @ oB) + beta * C)) <= bound).all()
+
+
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 320, 576])
+def test_cholesky_panels(n):
+    """Panels of one to four blocks and the blocks after them; backward error as of the textbook algorithm."""
+    rng = np.random.default_rng(n)
+    _say(f"cholesky panels n={n}")
+    X = rng.normal(size=(n, n))
+    S = X @ X.T / n + 0.01 * np.eye(n)
+    L, Li, info = hip.run_cholesky(S)
+    eps = np.finfo(np.float64).eps
+    assert info == 0
+    assert (np.abs(L @ L.T - S) <= 4.0 * (n + 1) * eps * (np.abs(L) @ np.abs(L).T)).all()
+    Li = np.tril(Li)
+    assert np.abs(Li @ L - np.eye(n)).max() <= 4.0 * n * eps * np.linalg.cond(L)
+
+
+@pytest.mark.parametrize("col", [1, 16, 17, 63, 64, 65, 128, 200, 256, 257, 320])
+def test_cholesky_reports_first_bad_pivot(col):
+    rng = np.random.default_rng(col)
+    n = 320
+    _say(f"cholesky bad pivot {col}")
+    L = np.tril(rng.normal(size=(n, n))) * 0.05 + np.eye(n)
+    S = L @ L.T
+    S[col - 1, col - 1] -= 2.0 * L[col - 1, col - 1] ** 2  # the pivot becomes about -L_jj^2
+    _, _, info = hip.run_cholesky(S)
+    assert info == col
