@@ -111,6 +111,10 @@ struct dh_system {
     cplx* coef = nullptr;
     int* kout = nullptr;
     cplx* coef_h = nullptr;         // pinned staging of the coefficients
+    double* pin = nullptr;          // pinned host memory results are read through (host_buffer)
+    size_t pin_n = 0;
+    char* steps_mem = nullptr;      // device buffers of dh_propagate_steps, kept for its next call
+    size_t steps_bytes = 0;
     hipEvent_t coef_ev = nullptr;   // the last copy out of coef_h
     bool coef_pending = false;
     // multi-step series of dh_propagate_steps: MULTI_MAX accumulators and their
@@ -295,6 +299,8 @@ extern "C" int dh_system_destroy(dh_system* s) {
     if (s->ev1) hipEventDestroy(s->ev1);
     if (s->coef_ev) hipEventDestroy(s->coef_ev);
     if (s->coef_h) hipHostFree(s->coef_h);
+    if (s->pin) hipHostFree(s->pin);
+    if (s->steps_mem) hipFree(s->steps_mem);
     if (s->coefm_ev) hipEventDestroy(s->coefm_ev);
     if (s->coefm_h) hipHostFree(s->coefm_h);
     if (s->kq_h) hipHostFree(s->kq_h);
@@ -861,11 +867,16 @@ static int put_column(dh_system* s, cplx* dst, long dst_stride, const double* ho
     return DH_OK;
 }
 
-static int get_column(dh_system* s, double* host, const cplx* src, long src_stride, int slot) {
-    hipStream_t st = s->ctx->stream;
-    cplx* stg = s->stage + (size_t)slot * s->ld;
-    launch_strided_copy(stg, 1, src, src_stride, s->N, st);
-    DH_HIP(hipMemcpyAsync(host, stg, sizeof(cplx) * s->N, hipMemcpyDeviceToHost, st));
+// Pinned host memory of n doubles for this system's results, kept until the
+// system goes.  Its users wait for the stream before they return, so no device
+// write is outstanding here.
+static int host_buffer(dh_system* s, size_t n) {
+    if (n <= s->pin_n) return DH_OK;
+    if (s->pin) hipHostFree(s->pin);
+    s->pin = nullptr;
+    s->pin_n = 0;
+    DH_HIP(hipHostMalloc((void**)&s->pin, sizeof(double) * n, hipHostMallocDefault));
+    s->pin_n = n;
     return DH_OK;
 }
 
@@ -1017,11 +1028,19 @@ extern "C" int dh_get_wavepacket(dh_system* s, int wp, double* bra, double* ket)
     DH_HIP(hipSetDevice(s->ctx->device));
     const int W = s->W;
     hipStream_t st = s->ctx->stream;
-    int rc = DH_OK;
-    if (bra && (rc = get_column(s, bra, s->out + wp, 3 * W, 0))) return rc;
-    if (ket && (rc = get_column(s, ket, s->out + 2 * W + wp, 3 * W, 1))) return rc;
+    const size_t n = 2 * (size_t)s->N;
+    if (int rc = host_buffer(s, 2 * n)) return rc;
+    ExportArgs e{};
+    e.n = s->N;
+    e.stride = 3 * W;
+    if (bra) e.col[0] = s->out + wp;
+    if (ket) e.col[1] = s->out + 2 * W + wp;
+    e.dst = s->pin;
+    launch_export(e, st);
     DH_HIP(hipGetLastError());
     DH_HIP(hipStreamSynchronize(st));
+    if (bra) std::memcpy(bra, s->pin, sizeof(double) * n);
+    if (ket) std::memcpy(ket, s->pin + (bra ? n : 0), sizeof(double) * n);
     return DH_OK;
 }
 
@@ -1316,7 +1335,7 @@ static int chebyshev_series(dh_system* s, bool one_launch = true) {
     return DH_OK;
 }
 
-static void launch_outputs(dh_system* s) {
+static void launch_outputs(dh_system* s, double* pops, double* erg) {
     hipStream_t st = s->ctx->stream;
     const int W = s->W;
     MatvecArgs a{};
@@ -1340,8 +1359,9 @@ static void launch_outputs(dh_system* s) {
     a.x = s->phi; a.x_stride = 2 * W; a.x_off = 0;
     a.out = s->out; a.out_stride = 3 * W; a.out_off = W;
     launch_matvec(a, st);
-    launch_observables(s->N, W, s->n_frag, s->frag, s->out, s->phi, s->hk, s->pops, s->erg, s->norms, st);
+    launch_observables(s->N, W, s->n_frag, s->frag, s->out, s->phi, s->hk, pops, erg, s->norms, st);
 }
+static void launch_outputs(dh_system* s) { launch_outputs(s, s->pops, s->erg); }
 
 // One step of dt (eV^-1) with the norm check: the term series, the new state's
 // norms and the outputs, then one host wait; a step whose norm drifts is
@@ -1349,8 +1369,9 @@ static void launch_outputs(dh_system* s) {
 static int propagate_checked(dh_system* s, double dt, int* n_terms, bool one_launch = true) {
     hipStream_t st = s->ctx->stream;
     const int R = 2 * s->W;
+    if (int rc = host_buffer(s, 2 * (size_t)R)) return rc;
+    const double *n0 = s->pin, *n1 = s->pin + R;
     launch_column_norms(s->N, R, s->phi, s->norms0, st);
-    std::vector<double> n0(R), n1(R);
     // FP64 norm drift of one step that signals bounds not enclosing the
     // spectrum; the mixed mode's FP32 products drift ~1e-7 per step by themselves
     // (mode 2 propagates with the exactly symmetric FP32-rounded H: FP64 drift)
@@ -1370,8 +1391,13 @@ static int propagate_checked(dh_system* s, double dt, int* n_terms, bool one_lau
         // an attempt that fails the drift check below recomputes them
         if (fp32_products(s)) launch_renorm_columns(s->phi, s->N, R, s->norms0, s->norms1, st);
         launch_outputs(s);
-        DH_HIP(hipMemcpyAsync(n0.data(), s->norms0, sizeof(double) * R, hipMemcpyDeviceToHost, st));
-        DH_HIP(hipMemcpyAsync(n1.data(), s->norms1, sizeof(double) * R, hipMemcpyDeviceToHost, st));
+        ExportArgs e{};
+        e.arr[0] = s->norms0;
+        e.arr[1] = s->norms1;
+        e.count[0] = e.count[1] = R;
+        e.dst = s->pin;
+        launch_export(e, st);
+        DH_HIP(hipGetLastError());
         DH_HIP(hipStreamSynchronize(st));
         double drift = 0.0;
         for (int c = 0; c < R; ++c) {
@@ -1697,16 +1723,36 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     return DH_OK;
 }
 
-// Device buffers of one dh_propagate_steps call, freed on every return path
-// (after the side stream, whose launched build reads geo, has drained).
+// Device buffers of one dh_propagate_steps call, in the system's kept block (a
+// block per call costs seven allocations and frees); the side stream, whose
+// launched build reads geo, has drained on every return path.
 struct StepsScratch {
     double *geo = nullptr, *n0 = nullptr, *n1 = nullptr, *pops = nullptr, *erg = nullptr;
     cplx *ck_phi = nullptr, *ck_out = nullptr;
     hipStream_t side = nullptr;
     ~StepsScratch() {
         if (side) hipStreamSynchronize(side);
-        for (void* p : {(void*)geo, (void*)n0, (void*)n1, (void*)pops, (void*)erg, (void*)ck_phi, (void*)ck_out})
-            if (p) hipFree(p);
+    }
+    int take(dh_system* s, int n_steps, size_t geo_n) {
+        const size_t R = 2 * (size_t)s->W, ld = s->ld, n = n_steps;
+        const size_t doubles = 2 * n * R + n * s->W * (s->n_frag + 1) + n * s->W * 2 + geo_n;
+        const size_t bytes = sizeof(cplx) * ld * (R + 3 * s->W) + sizeof(double) * doubles;
+        if (bytes > s->steps_bytes) {
+            DH_HIP(hipStreamSynchronize(s->ctx->stream));
+            if (s->steps_mem) hipFree(s->steps_mem);
+            s->steps_mem = nullptr;
+            s->steps_bytes = 0;
+            DALLOC(s->steps_mem, bytes);
+            s->steps_bytes = bytes;
+        }
+        ck_phi = (cplx*)s->steps_mem;
+        ck_out = ck_phi + ld * R;
+        n0 = (double*)(ck_out + ld * 3 * s->W);
+        n1 = n0 + n * R;
+        pops = n1 + n * R;
+        erg = pops + n * s->W * (s->n_frag + 1);
+        geo = erg + n * s->W * 2;
+        return DH_OK;
     }
 };
 
@@ -1725,22 +1771,16 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
     const int W = s->W, R = 2 * W, NP = s->n_frag + 1;
     const double dt = dt_ps / H_BAR;
     StepsScratch d;
-    DALLOC(d.n0, (size_t)n_steps * R);
-    DALLOC(d.n1, (size_t)n_steps * R);
-    DALLOC(d.pops, (size_t)n_steps * W * NP);
-    DALLOC(d.erg, (size_t)n_steps * W * 2);
-    DALLOC(d.ck_phi, (size_t)s->ld * R);
-    DALLOC(d.ck_out, (size_t)s->ld * 3 * W);
     const size_t geo_n = (size_t)s->n_atoms * 3;
+    if ((rc = d.take(s, n_steps, geo_n * n_geo))) return rc;
+    if ((rc = host_buffer(s, (size_t)n_steps * W * std::max(4, NP + 2)))) return rc;
     if (n_geo > 0) {
         if ((rc = ensure_side(s))) return rc;
         d.side = s->ctx->side;
-        DALLOC(d.geo, geo_n * n_geo);
         // every geometry goes to the device once; a rebuild reads its slice there
         DH_HIP(hipMemcpyAsync(d.geo, coords, sizeof(double) * geo_n * n_geo, hipMemcpyHostToDevice, st));
         DH_HIP(hipStreamSynchronize(st));  // the side stream reads them
     }
-    std::vector<double> h0((size_t)n_steps * R), h1((size_t)n_steps * R);
     const double drift_tol = fp32_products(s) ? 1e-4 : 1e-9;
     int last_terms = 0;
     for (int j = 0; j < n_steps;) {
@@ -1797,12 +1837,8 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
                     launch_column_norms(s->N, R, st_q, d.n1 + (size_t)(i + q) * R, st);
                     if (f32p) launch_renorm_columns(st_q, s->N, R, d.n0 + (size_t)(i + q) * R, d.n1 + (size_t)(i + q) * R, st);
                     s->phi = st_q;  // the outputs of step i + q
-                    launch_outputs(s);
+                    launch_outputs(s, d.pops + (size_t)(i + q) * W * NP, d.erg + (size_t)(i + q) * W * 2);
                     s->phi = keep;
-                    DH_HIP(hipMemcpyAsync(d.pops + (size_t)(i + q) * W * NP, s->pops, sizeof(double) * W * NP,
-                                          hipMemcpyDeviceToDevice, st));
-                    DH_HIP(hipMemcpyAsync(d.erg + (size_t)(i + q) * W * 2, s->erg, sizeof(double) * W * 2,
-                                          hipMemcpyDeviceToDevice, st));
                 }
                 DH_HIP(hipMemcpyAsync(s->phi, s->accm + (size_t)(mc - 1) * acc_n, sizeof(cplx) * acc_n,
                                       hipMemcpyDeviceToDevice, st));
@@ -1821,11 +1857,7 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
                 launch_column_norms(s->N, R, s->phi, d.n1 + (size_t)i * R, st);
                 if (fp32_products(s))
                     launch_renorm_columns(s->phi, s->N, R, d.n0 + (size_t)i * R, d.n1 + (size_t)i * R, st);
-                launch_outputs(s);
-                DH_HIP(hipMemcpyAsync(d.pops + (size_t)i * W * NP, s->pops, sizeof(double) * W * NP,
-                                      hipMemcpyDeviceToDevice, st));
-                DH_HIP(hipMemcpyAsync(d.erg + (size_t)i * W * 2, s->erg, sizeof(double) * W * 2,
-                                      hipMemcpyDeviceToDevice, st));
+                launch_outputs(s, d.pops + (size_t)i * W * NP, d.erg + (size_t)i * W * 2);
             }
             // the next geometry's operators, on the side stream, while this
             // interval's steps run; launched once the first series is queued so
@@ -1836,13 +1868,21 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
             }
             i += mc;
         }
+        // the last step's observables are also the system's current ones
+        DH_HIP(hipMemcpyAsync(s->pops, d.pops + (size_t)(jend - 1) * W * NP, sizeof(double) * W * NP,
+                              hipMemcpyDeviceToDevice, st));
+        DH_HIP(hipMemcpyAsync(s->erg, d.erg + (size_t)(jend - 1) * W * 2, sizeof(double) * W * 2,
+                              hipMemcpyDeviceToDevice, st));
+        const long cnt = (long)(jend - j) * R;
+        ExportArgs e{};
+        e.arr[0] = d.n0 + (size_t)j * R;
+        e.arr[1] = d.n1 + (size_t)j * R;
+        e.count[0] = e.count[1] = cnt;
+        e.dst = s->pin;
+        launch_export(e, st);
         DH_HIP(hipGetLastError());
-        const size_t cnt = (size_t)(jend - j) * R;
-        DH_HIP(hipMemcpyAsync(h0.data() + (size_t)j * R, d.n0 + (size_t)j * R, sizeof(double) * cnt,
-                              hipMemcpyDeviceToHost, st));
-        DH_HIP(hipMemcpyAsync(h1.data() + (size_t)j * R, d.n1 + (size_t)j * R, sizeof(double) * cnt,
-                              hipMemcpyDeviceToHost, st));
         DH_HIP(hipStreamSynchronize(st));
+        const double *h0 = s->pin, *h1 = s->pin + cnt;
         float series_ms = 0.0f;
         if (s->timing)
             for (int i = 0; i < n_timed; ++i) {
@@ -1851,9 +1891,9 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
                 series_ms += ms;
             }
         double drift = 0.0;
-        for (size_t e = (size_t)j * R; e < (size_t)jend * R; ++e) {
-            if (h0[e] > 0) drift = std::max(drift, std::fabs(h1[e] - h0[e]) / h0[e]);
-            if (!std::isfinite(h1[e])) drift = INFINITY;
+        for (long c = 0; c < cnt; ++c) {
+            if (h0[c] > 0) drift = std::max(drift, std::fabs(h1[c] - h0[c]) / h0[c]);
+            if (!std::isfinite(h1[c])) drift = INFINITY;
         }
         if (drift < drift_tol) {
             s->stats[4] = drift;
@@ -1880,9 +1920,19 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
         }
         j = jend;
     }
-    if (pops) DH_HIP(hipMemcpyAsync(pops, d.pops, sizeof(double) * n_steps * W * NP, hipMemcpyDeviceToHost, st));
-    if (erg) DH_HIP(hipMemcpyAsync(erg, d.erg, sizeof(double) * n_steps * W * 2, hipMemcpyDeviceToHost, st));
+    if (pops || erg) {
+        ExportArgs e{};
+        e.arr[0] = d.pops;
+        e.arr[1] = d.erg;
+        e.count[0] = (long)n_steps * W * NP;
+        e.count[1] = (long)n_steps * W * 2;
+        e.dst = s->pin;
+        launch_export(e, st);
+        DH_HIP(hipGetLastError());
+    }
     DH_HIP(hipStreamSynchronize(st));
+    if (pops) std::memcpy(pops, s->pin, sizeof(double) * (size_t)n_steps * W * NP);
+    if (erg) std::memcpy(erg, s->pin + (size_t)n_steps * W * NP, sizeof(double) * (size_t)n_steps * W * 2);
     if (n_terms) *n_terms = last_terms;
     return DH_OK;
 }
@@ -1892,15 +1942,23 @@ extern "C" int dh_get_observables(dh_system* s, int wp, double* ao_bra, double* 
     DH_HIP(hipSetDevice(s->ctx->device));
     hipStream_t st = s->ctx->stream;
     const int W = s->W;
-    if (ao_bra) {
-        const int rc = get_column(s, ao_bra, s->out + W + wp, 3 * W, 0);
-        if (rc) return rc;
-    }
-    if (pops)
-        DH_HIP(hipMemcpyAsync(pops, s->pops + (size_t)wp * (s->n_frag + 1), sizeof(double) * (s->n_frag + 1),
-                              hipMemcpyDeviceToHost, st));
-    if (erg) DH_HIP(hipMemcpyAsync(erg, s->erg + 2 * wp, sizeof(double) * 2, hipMemcpyDeviceToHost, st));
+    const size_t n = ao_bra ? 2 * (size_t)s->N : 0, np = pops ? s->n_frag + 1 : 0, ne = erg ? 2 : 0;
+    if (int rc = host_buffer(s, n + np + ne)) return rc;
+    ExportArgs e{};
+    e.n = s->N;
+    e.stride = 3 * W;
+    if (ao_bra) e.col[0] = s->out + W + wp;
+    e.arr[0] = s->pops + (size_t)wp * (s->n_frag + 1);
+    e.arr[1] = s->erg + 2 * wp;
+    e.count[0] = (long)np;
+    e.count[1] = (long)ne;
+    e.dst = s->pin;
+    launch_export(e, st);
+    DH_HIP(hipGetLastError());
     DH_HIP(hipStreamSynchronize(st));
+    if (ao_bra) std::memcpy(ao_bra, s->pin, sizeof(double) * n);
+    if (pops) std::memcpy(pops, s->pin + n, sizeof(double) * np);
+    if (erg) std::memcpy(erg, s->pin + n + np, sizeof(double) * ne);
     return DH_OK;
 }
 

@@ -198,6 +198,15 @@ int matvec_split_for(int N, int R);
 // complex elements of a.partial the symmetric two-phase variant needs at (ld, R)
 long sym_partial_cplx(int ld, int R);
 long sym2_partial_cplx(int ld, int R);
+struct ExportArgs {
+    int n;                // rows of a column
+    long stride;          // between a column's elements
+    const cplx* col[2];   // null: left out
+    const double* arr[3];
+    long count[3];        // 0: left out
+    double* dst;          // pinned host memory, 4 n + the counts
+};
+void launch_export(const ExportArgs& e, hipStream_t st);
 void launch_strided_copy(cplx* dst, long ds, const cplx* src, long ss, int n, hipStream_t st);
 bool sym_supported(int R, int tri);
 void launch_matvec(const MatvecArgs& a, hipStream_t st);
