@@ -17,6 +17,7 @@
 // order and applies the fused epilogue.  The summation order is fixed, so
 // results are bitwise reproducible run to run.
 #include "common.hpp"
+#include "gemm.hpp"
 #include "kernels.hpp"
 
 #include <cmath>
@@ -863,29 +864,17 @@ void launch_multi_panel_grouped(const PanelArgs* d_args, const int* task_desc, c
                            k0, k1);
 }
 
-// Split-K multi-RHS term GEMM: Y = H X with H N x N (FP64, or its FP32 copy
-// for PREC 1) and X the 2R real columns of the RHS.  A workgroup computes a
-// 128 (orbitals) x 128 (real columns) tile over one K slice; 4 waves in 2 x 2,
-// each a 64 x 64 quadrant of 4 x 4 MFMA 16x16x4 blocks.  16-deep k stages are
-// double-buffered in LDS and prefetched into registers.  The MFMA runs with
-// the operands swapped (D^T = X^T H^T), so a lane's results lie in 16
-// consecutive orbitals of one column.  Slice z writes its FP64 partial
-// product to P[z][c][i]; gemm3_reduce_kernel adds the slices in order and runs
-// the Chebyshev epilogue.  The FP32 path accumulates each K slice in FP32 and
-// adds the slices in FP64.
+// The operator on many columns as a matrix product, Y = op(M) X with M N x N
+// and X the C = 2R real columns of the right-hand sides: FP64 products
+// (panel_kernel; M stored in FP64 or FP32) or FP32 ones (panel_f32_kernel, the
+// mixed modes).  A tile of rows and columns is split over its k range into S
+// slices; slice z goes to P[z][c][i], and panel_reduce_kernel adds the slices in
+// order and runs the epilogue.
 constexpr int G3_T = 128;
-// k-stage depth: 16 (FP64) / 32 (FP32) keeps the double-buffered tiles at 74 KB of
-// LDS, so two workgroups share a CU and hide each other's barrier and load waits
-// PREC: 0 = FP64, 1 = FP32 products and slice sums (mixed), 2 = FP32-stored H
-// widened to FP64 on load, FP64 products (the arithmetic of PREC 0)
-template <int PREC> struct G3 { static constexpr int BK = PREC == 1 ? 32 : 16; };
-// row pad: successive k-rows of an operand read start 32 banks apart (FP64) or
-// 16 banks apart (FP32), so the four rows a wave reads do not collide
-constexpr int G3_PAD = 16;
-
+// rows from which a slice is worth its partial product, and the bound of P
 int gemm3_splits(int N, int R) {
     const int tiles = ((N + G3_T - 1) / G3_T) * ((2 * R + G3_T - 1) / G3_T);
-    int S = (512 + tiles - 1) / tiles;  // two workgroups per CU
+    int S = (512 + tiles - 1) / tiles;  // two workgroups of the FP32 kernel per CU
     const int kmax = (N + 255) / 256;  // at least 256 k per slice
     if (S > kmax) S = kmax;
     return S < 1 ? 1 : S;
@@ -893,50 +882,93 @@ int gemm3_splits(int N, int R) {
 
 long gemm3_partial_doubles(int N, int ld, int R) { return (long)gemm3_splits(N, R) * ld * 2 * R; }
 
-template <int PREC>
-__global__ __launch_bounds__(256) void gemm3_kernel(MatvecArgs a, double* __restrict__ P, int KS) {
-    constexpr bool F32 = PREC == 1;
-    using T = typename std::conditional<F32, float, double>::type;
-    constexpr int G3_BK = G3<PREC>::BK;
-    __shared__ T As[2][G3_BK][G3_T + G3_PAD];
-    __shared__ T Bs[2][G3_BK][G3_T + G3_PAD];
+// FP64 tile T x T, T = 64 or 32 (gemm_accumulate).  TRI: the triangle j <= i
+// (a.tri = TRI_UPPER) or j >= i of the mirrored storage, whose row tiles have k
+// ranges of their own: the part off the diagonal tile without a mask, the
+// diagonal tile with one.  Every row tile's range is cut into the same number of
+// slices, longest ranges first, so the launch ends evenly.
+template <int T, typename EA, bool TRI>
+__global__ __launch_bounds__(256) void panel_kernel(MatvecArgs a, double* __restrict__ P, int S) {
+    __shared__ double As[2][16 * T];
+    __shared__ double Bs[2][16 * T];
+    constexpr int MB = T / 32;
+    const int N = a.N, C = 2 * a.R;
+    const bool upper = TRI && a.tri == TRI_UPPER;
+    const int i0 = (upper ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * T, c0 = blockIdx.y * T, z = blockIdx.z;
+    const int lo = TRI && !upper ? i0 : 0, hi = upper ? min(N, i0 + T) : N;
+    const int per = ((hi - lo + S - 1) / S + 15) & ~15;
+    const int klo = min(hi, lo + z * per), khi = min(hi, klo + per);
+    const EA* A = (sizeof(EA) == 8 ? reinterpret_cast<const EA*>(a.M) : reinterpret_cast<const EA*>(a.M32)) + i0;
+    const double* B = reinterpret_cast<const double*>(a.x) + 2L * a.x_off + c0;
+    const long xs = 2L * a.x_stride;
+    v4d acc[MB][MB];
+#pragma unroll
+    for (int p = 0; p < MB; ++p)
+#pragma unroll
+        for (int q = 0; q < MB; ++q) acc[p][q] = (v4d){0.0, 0.0, 0.0, 0.0};
+    int ulo = klo, uhi = khi;  // without a mask
+    if constexpr (TRI) {
+        const int mlo = upper ? max(klo, i0) : klo, mhi = upper ? khi : min(khi, i0 + T);
+        gemm_accumulate<T, 16, 0, 1, true>(acc, A, a.ld, N - i0, B, xs, C - c0, mlo, mhi, As, Bs,
+                                           [&](int i, int k) { return upper ? k <= i0 + i : k >= i0 + i; });
+        if (upper) uhi = min(khi, i0);
+        else ulo = max(klo, i0 + T);
+    }
+    gemm_accumulate<T, 16, 0, 1, false>(acc, A, a.ld, N - i0, B, xs, C - c0, ulo, uhi, As, Bs,
+                                        [](int, int) { return true; });
+    double* Pz = P + (long)z * C * a.ld;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int ib = i0 + (w >> 1) * (T / 2) + (lane & 15), cb = c0 + (w & 1) * (T / 2) + (lane >> 4);
+#pragma unroll
+    for (int p = 0; p < MB; ++p)
+#pragma unroll
+        for (int q = 0; q < MB; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int gi = ib + p * 16, gc = cb + q * 16 + 4 * v;
+                if (gi < N && gc < C) Pz[(long)gc * a.ld + gi] = acc[p][q][v];
+            }
+}
+
+// FP32 products and slice sums on the FP32 copies: 128 x 128 tiles, 4 waves in
+// 2 x 2, each a 64 x 64 quadrant of 4 x 4 MFMA 16x16x4 blocks, operands swapped
+// as above; 32-deep k stages double-buffered in LDS (74 KB: two workgroups a CU)
+// and fetched into registers a stage ahead.
+constexpr int G3_BK = 32;
+constexpr int G3_PAD = 16;  // the four k rows of an operand read start 16 banks apart
+
+__global__ __launch_bounds__(256) void panel_f32_kernel(MatvecArgs a, float* __restrict__ P, int KS) {
+    __shared__ float As[2][G3_BK][G3_T + G3_PAD];
+    __shared__ float Bs[2][G3_BK][G3_T + G3_PAD];
     const int N = a.N, C = 2 * a.R;
     const int i0 = blockIdx.x * G3_T, c0 = blockIdx.y * G3_T, z = blockIdx.z;
     const int klo = z * KS, khi = min(N, klo + KS);
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int wi = (w >> 1) * 64, wc = (w & 1) * 64;
     const double* X = reinterpret_cast<const double*>(a.x);
-    const float* X32 = F32 ? a.x32 : nullptr;  // FP32 copy of x when the caller keeps one
+    const float* X32 = a.x32;  // FP32 copy of x when the caller keeps one
     const long xs = 2L * a.x_stride, xo = 2L * a.x_off;
-    using acc_t = typename std::conditional<F32, v4f, v4d>::type;
-    acc_t acc[4][4];
+    v4f acc[4][4];
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) acc[p][q][v] = (T)0;
+        for (int q = 0; q < 4; ++q) acc[p][q] = (v4f){0.f, 0.f, 0.f, 0.f};
     constexpr int LPT = G3_BK * G3_T / 256;  // elements of each tile per thread per stage
-    T ra[LPT], rb[LPT];
+    float ra[LPT], rb[LPT];
     // H tile: rows i0..i0+127 (lane-contiguous), k0..k0+BK-1; X tile: k0..k0+BK-1, columns c0..c0+127
     auto gload = [&](int k0) {
 #pragma unroll
         for (int r = 0; r < LPT; ++r) {
             const int ii = t & 127, kk = (t >> 7) + 2 * r;
             const int gi = i0 + ii, gk = k0 + kk;
-            T v = (T)0;
-            if (gi < N && gk < khi) {
-                if constexpr (PREC == 0) v = a.M[gi + (long)a.ld * gk];
-                else v = (T)a.M32[gi + (long)a.ld * gk];
-            }
-            ra[r] = v;
+            ra[r] = gi < N && gk < khi ? a.M32[gi + (long)a.ld * gk] : 0.f;
         }
 #pragma unroll
         for (int r = 0; r < LPT; ++r) {
             const int cc = t & 127, kk = (t >> 7) + 2 * r;
             const int gc = c0 + cc, gk = k0 + kk;
-            T v = (T)0;
-            if (gc < C && gk < khi) v = X32 ? (T)X32[gk * xs + xo + gc] : (T)X[gk * xs + xo + gc];
+            float v = 0.f;
+            if (gc < C && gk < khi) v = X32 ? X32[gk * xs + xo + gc] : (float)X[gk * xs + xo + gc];
             rb[r] = v;
         }
     };
@@ -959,7 +991,7 @@ __global__ __launch_bounds__(256) void gemm3_kernel(MatvecArgs a, double* __rest
         if (more) gload(k0 + G3_BK);
 #pragma unroll
         for (int ks = 0; ks < G3_BK; ks += 4) {
-            T av[4], bv[4];
+            float av[4], bv[4];
 #pragma unroll
             for (int p = 0; p < 4; ++p) av[p] = As[s][ks + (lane >> 4)][wi + p * 16 + (lane & 15)];
 #pragma unroll
@@ -967,22 +999,15 @@ __global__ __launch_bounds__(256) void gemm3_kernel(MatvecArgs a, double* __rest
 #pragma unroll
             for (int p = 0; p < 4; ++p)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    if constexpr (!F32)
-                        acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[q], av[p], acc[p][q], 0, 0, 0);
-                    else
-                        acc[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[q], av[p], acc[p][q], 0, 0, 0);
-                }
+                for (int q = 0; q < 4; ++q)
+                    acc[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[q], av[p], acc[p][q], 0, 0, 0);
         }
         if (more) swrite(s ^ 1);
         __syncthreads();
         s ^= 1;
     }
-    // D^T layout: f64 lane l, value v -> column (l >> 4) + 4v, orbital l & 15;
-    //             f32 lane l, value v -> column 4 (l >> 4) + v, orbital l & 15.
-    // PREC 1 stores its FP32 slice sums as FP32 (exact, half the bytes).
-    using part_t = typename std::conditional<PREC == 1, float, double>::type;
-    part_t* Pz = reinterpret_cast<part_t*>(P) + (long)z * C * a.ld;
+    // D^T layout: lane l, value v -> column 4 (l >> 4) + v, orbital l & 15
+    float* Pz = P + (long)z * C * a.ld;
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
@@ -990,77 +1015,86 @@ __global__ __launch_bounds__(256) void gemm3_kernel(MatvecArgs a, double* __rest
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int gi = i0 + wi + p * 16 + (lane & 15);
-                const int gc = c0 + wc + q * 16 + (!F32 ? (lane >> 4) + 4 * v : 4 * (lane >> 4) + v);
-                if (gi < N && gc < C) Pz[(long)gc * a.ld + gi] = (part_t)acc[p][q][v];
+                const int gc = c0 + wc + q * 16 + 4 * (lane >> 4) + v;
+                if (gi < N && gc < C) Pz[(long)gc * a.ld + gi] = acc[p][q][v];
             }
 }
 
-// slices added in order, in FP64 (PT: how the slices were stored)
+// Slices added in order, in FP64 (PT: how they were stored), then, with Plo,
+// those of the residual's products (mode 3) likewise, and the epilogue.  The
+// slices have a column's rows together, x and the outputs a row's columns: a
+// workgroup turns 16 rows of 8 complex columns through LDS, so both sides are
+// read and written in whole lines.  Bound by the latency of the slices' loads,
+// hence one sum per thread and small workgroups.
 template <typename PT>
-__global__ __launch_bounds__(256) void gemm3_reduce_kernel(MatvecArgs a, const PT* __restrict__ P, int S) {
-    const long n = (long)a.N * a.R;
-    const long e = blockIdx.x * 256L + threadIdx.x;
-    if (e >= n) return;
-    const int r = (int)(e / a.N), i = (int)(e % a.N);
-    const long C = 2L * a.R;
-    cplx y{0.0, 0.0};
-    for (int z = 0; z < S; ++z) {
-        const PT* Pz = P + (long)z * C * a.ld;
-        y.re += (double)Pz[(2L * r) * a.ld + i];
-        y.im += (double)Pz[(2L * r + 1) * a.ld + i];
-    }
-    term_epilogue(a, i, r, y);
+__global__ __launch_bounds__(256) void panel_reduce_kernel(MatvecArgs a, const PT* __restrict__ P,
+                                                           const PT* __restrict__ Plo, int S) {
+    __shared__ double y[16][17];  // y[column][row]
+    const int i0 = blockIdx.x * 16, r0 = blockIdx.y * 8, t = threadIdx.x;
+    const long C = 2L * a.R, slice = C * a.ld;
+    const int c = t >> 4, i = min(i0 + (t & 15), a.N - 1);
+    const long o = min(2L * r0 + c, C - 1) * a.ld + i;
+    auto sum = [&](const PT* p) {
+        double v = 0.0;
+        int z = 0;
+        for (; z + 4 <= S; z += 4) {
+            const double p0 = (double)p[z * slice + o], p1 = (double)p[(z + 1) * slice + o];
+            const double p2 = (double)p[(z + 2) * slice + o], p3 = (double)p[(z + 3) * slice + o];
+            v += p0;
+            v += p1;
+            v += p2;
+            v += p3;
+        }
+        for (; z < S; ++z) v += (double)p[z * slice + o];
+        return v;
+    };
+    double v = sum(P);
+    if (Plo) v += sum(Plo);
+    y[c][t & 15] = v;
+    __syncthreads();
+    const int r = t & 7, ii = t >> 3;
+    if (t < 128 && i0 + ii < a.N && r0 + r < a.R)
+        term_epilogue(a, i0 + ii, r0 + r, cplx{y[2 * r][ii], y[2 * r + 1][ii]});
 }
 
-// Slices of the library GEMMs of the mixed modes, added in FP64 in slice order:
-// the FP32 products Phi[z] and (mode 3) the residual's products Plo[z], both
-// laid out as gemm3's slices ([z][c][i], ld rows)
-__global__ __launch_bounds__(256) void lib_reduce_kernel(MatvecArgs a, const float* __restrict__ Phi,
-                                                          const float* __restrict__ Plo, int S) {
-    const long n = (long)a.N * a.R;
-    const long e = blockIdx.x * 256L + threadIdx.x;
-    if (e >= n) return;
-    const int r = (int)(e / a.N), i = (int)(e % a.N);
-    const long C = 2L * a.R;
-    cplx y{0.0, 0.0};
-    for (int z = 0; z < S; ++z) {
-        const long o = (long)z * C * a.ld;
-        y.re += (double)Phi[o + (2L * r) * a.ld + i];
-        y.im += (double)Phi[o + (2L * r + 1) * a.ld + i];
-    }
-    if (Plo) {
-        cplx lo{0.0, 0.0};
-        for (int z = 0; z < S; ++z) {
-            const long o = (long)z * C * a.ld;
-            lo.re += (double)Plo[o + (2L * r) * a.ld + i];
-            lo.im += (double)Plo[o + (2L * r + 1) * a.ld + i];
-        }
-        y.re += lo.re;
-        y.im += lo.im;
-    }
-    term_epilogue(a, i, r, y);
-}
+static dim3 panel_reduce_grid(const MatvecArgs& a) { return dim3((a.N + 15) / 16, (a.R + 7) / 8); }
 
 void launch_lib_reduce(const MatvecArgs& a, const float* Phi, const float* Plo, int S, hipStream_t st) {
-    const long n = (long)a.N * a.R;
-    hipLaunchKernelGGL(lib_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, Phi, Plo, S);
+    hipLaunchKernelGGL((panel_reduce_kernel<float>), panel_reduce_grid(a), dim3(256), 0, st, a, Phi, Plo, S);
+}
+
+// Slices of the FP64 kernel: 3 (T = 64) or 4 (T = 32) workgroups a CU, at least
+// 256 k each, and no more than P is sized for.
+template <int T, typename EA, bool TRI>
+static int panel_tiles(const MatvecArgs& a, double* P, hipStream_t st) {
+    const int tr = (a.N + T - 1) / T, tc = (2 * a.R + T - 1) / T, want = T == 64 ? 768 : 1024;
+    const int S = std::max(1, std::min(want / (tr * tc), gemm3_splits(a.N, a.R)));
+    hipLaunchKernelGGL((panel_kernel<T, EA, TRI>), dim3(tr, tc, S), dim3(256), 0, st, a, P, S);
+    return S;
+}
+
+// up to 32 real columns a tile of 64 would be half empty
+template <typename EA, bool TRI>
+static int panel_f64(const MatvecArgs& a, double* P, hipStream_t st) {
+    return 2 * a.R <= 32 ? panel_tiles<32, EA, TRI>(a, P, st) : panel_tiles<64, EA, TRI>(a, P, st);
 }
 
 void launch_gemm3(const MatvecArgs& a, int prec, double* P, hipStream_t st) {
-    const int S = gemm3_splits(a.N, a.R);
-    const int BK = prec == 1 ? G3<1>::BK : G3<0>::BK;
-    const int KS = (((a.N + S - 1) / S) + BK - 1) / BK * BK;
-    const int Sr = (a.N + KS - 1) / KS;
-    dim3 grid((a.N + G3_T - 1) / G3_T, (2 * a.R + G3_T - 1) / G3_T, Sr);
-    if (prec == 0) hipLaunchKernelGGL((gemm3_kernel<0>), grid, dim3(256), 0, st, a, P, KS);
-    else if (prec == 1) hipLaunchKernelGGL((gemm3_kernel<1>), grid, dim3(256), 0, st, a, P, KS);
-    else hipLaunchKernelGGL((gemm3_kernel<2>), grid, dim3(256), 0, st, a, P, KS);
-    const long n = (long)a.N * a.R;
-    const dim3 rg((unsigned)((n + 255) / 256));
-    if (prec == 1)
-        hipLaunchKernelGGL((gemm3_reduce_kernel<float>), rg, dim3(256), 0, st, a, reinterpret_cast<const float*>(P), Sr);
-    else
-        hipLaunchKernelGGL((gemm3_reduce_kernel<double>), rg, dim3(256), 0, st, a, (const double*)P, Sr);
+    if (prec == 1) {
+        const int S = gemm3_splits(a.N, a.R);
+        const int KS = (((a.N + S - 1) / S) + G3_BK - 1) / G3_BK * G3_BK;
+        const int Sr = (a.N + KS - 1) / KS;
+        const dim3 grid((a.N + G3_T - 1) / G3_T, (2 * a.R + G3_T - 1) / G3_T, Sr);
+        hipLaunchKernelGGL(panel_f32_kernel, grid, dim3(256), 0, st, a, reinterpret_cast<float*>(P), KS);
+        launch_lib_reduce(a, reinterpret_cast<const float*>(P), nullptr, Sr, st);
+        return;
+    }
+    int S;
+    if (prec == 2) S = panel_f64<float, false>(a, P, st);
+    else if (a.tri == TRI_FULL) S = panel_f64<double, false>(a, P, st);
+    else S = panel_f64<double, true>(a, P, st);
+    hipLaunchKernelGGL((panel_reduce_kernel<double>), panel_reduce_grid(a), dim3(256), 0, st, a, (const double*)P,
+                       (const double*)nullptr, S);
 }
 
 static int g_gemm_bn = 0;  // 0: choose by size; 16 or 32 forces the tile width
@@ -2361,9 +2395,8 @@ void launch_matvec_variant(const MatvecArgs& a, int variant, hipStream_t st) {
         return;
     }
     if (variant == 15) {
-        // matrix-core split-K GEMM; triangular shapes use the column-block kernel
-        if (a.tri == TRI_FULL) launch_gemm3(a, 0, reinterpret_cast<double*>(a.partial), st);
-        else launch_matvec_variant(a, 9, st);
+        // matrix-core split-K product
+        launch_gemm3(a, 0, reinterpret_cast<double*>(a.partial), st);
         return;
     }
     switch (a.R) {

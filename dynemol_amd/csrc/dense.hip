@@ -8,182 +8,70 @@
 // of 64; the padding of S carries an identity block, so every blocked
 // routine runs on whole 64 x 64 tiles.
 #include "common.hpp"
+#include "gemm.hpp"
 #include "kernels.hpp"
 
 #include <algorithm>
 
 namespace dh {
 
-// C = alpha * opA(A) opB(B) + beta * C on T x T tiles, T = 64 or 32: 256 threads
-// = 4 waves in a 2 x 2 arrangement, each wave a T/2 x T/2 quadrant of 16 x 16
-// MFMA blocks (v_mfma_f64_16x16x4f64: lane l holds A[l%16][l/16] and
-// B[l/16][l%16]; result v of lane l is D[l/16 + 4v][l%16]).  The MFMA is issued
-// with the operands swapped (D^T = B^T A^T), so a lane's four results lie in
-// four columns and each column's 16 rows are contiguous in C.
-//
-// Bound: the matrix cores (64 cycles per instruction and SIMD).  A GK-deep k
-// stage is double-buffered in LDS; the stage after next is fetched into
-// registers while the current one is multiplied, and the next one goes from
-// registers to LDS half way through, so that its writes overlap products (one
-// barrier per stage).  The LDS rows are XOR-swizzled (gemm_sw) instead of
-// padded: operand reads (16 rows x 4 k), row-wise stores and k-wise stores
-// (transposed operands) are all free of bank conflicts.  Full products of 4096:
-// 55 TFLOP/s with T = 64 (3 workgroups a CU); 72 without the fetches, 75 for
-// the bare instructions.  A pair of 128 x 128 tiles per workgroup, which this
-// replaces, took 112 us where N = 576 now takes 18, 474 for L^-1 h at 2112
-// (210 now) and 1416 at 4096 (1257 now).
+// C = alpha * opA(A) opB(B) + beta * C on T x T tiles, T = 64 or 32
+// (gemm_accumulate).  A pair of 128 x 128 tiles per workgroup, which this
+// replaces, took 112 us where N = 576 now takes 14, 474 for L^-1 h at 2112 (175
+// now) and 1416 at 4096 (1110 now).
 //
 // Workgroups start in blockIdx order (x fastest).  With a k range that grows
 // with the row (column) tile, columns (rows) run fastest and the longest tiles
 // start first, so that the last ones to start are short; consecutive
 // workgroups go round the XCDs, so an XCD keeps to an eighth of the fast
 // dimension where that divides by 8 and its tiles share operands in its L2.
-template <int GK>
-__device__ __forceinline__ int gemm_sw(int k) {
-    return ((k & 1) << 4) | (k & 14) | (GK > 16 ? (k >> 4) & 1 : 0);
-}
-
 template <int T, int GK, int TA, int TB>
 __global__ __launch_bounds__(256) void gemm_f64_kernel(Gemm g) {
-    __shared__ double As[2][GK * T];  // As[s][k * T + (i ^ gemm_sw(k))]
+    __shared__ double As[2][GK * T];
     __shared__ double Bs[2][GK * T];
-    constexpr int MB = T / 32;        // 16 x 16 blocks of a wave per direction
-    constexpr int NL = GK * T / 256;  // values a thread fetches per operand and stage
+    constexpr int MB = T / 32;
     const bool rows_fast = g.kmode == K_BELOW_COLTILE || g.kmode == K_FROM_COLTILE || g.kmode == K_FULL;
     int bi = rows_fast ? blockIdx.x : blockIdx.y, bj = rows_fast ? blockIdx.y : blockIdx.x;
     if (g.kmode == K_BELOW_ROWTILE) bi = gridDim.y - 1 - bi;
     else if (g.kmode == K_BELOW_COLTILE) bj = gridDim.y - 1 - bj;
     const int i0 = bi * T, j0 = bj * T;
     if (g.lower_only && i0 / TILE < j0 / TILE) return;
-    const double* A = g.A + (long)blockIdx.z * g.strideA;
-    const double* B = g.B + (long)blockIdx.z * g.strideB;
+    const double* A = g.A + (long)blockIdx.z * g.strideA + (TA ? g.lda * (long)i0 : (long)i0);
+    const double* B = g.B + (long)blockIdx.z * g.strideB + (TB ? (long)j0 : g.ldb * (long)j0);
     double* C = g.C + (long)blockIdx.z * g.strideC;
     int klo = 0, khi = g.K;
     if (g.kmode == K_BELOW_ROWTILE) khi = min(g.K, i0 + T);
     else if (g.kmode == K_BELOW_COLTILE) khi = min(g.K, j0 + T);
     else if (g.kmode == K_FROM_ROWTILE) klo = i0;
     else if (g.kmode == K_FROM_COLTILE) klo = j0;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wi = (w >> 1) * (T / 2), wj = (w & 1) * (T / 2);
-    const int lr = lane & 15, lk = lane >> 4;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int ib = i0 + (w >> 1) * (T / 2) + (lane & 15), jb = j0 + (w & 1) * (T / 2) + (lane >> 4);
     v4d acc[MB][MB];
-#pragma unroll
-    for (int a = 0; a < MB; ++a)
-#pragma unroll
-        for (int b = 0; b < MB; ++b) acc[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
-    // C <- C - A B: C is read into the accumulators before the k loop, where its
-    // latency overlaps the operand loads, and the products are subtracted (A
-    // negated on its way out of LDS, exactly)
+    // C <- C - A B: the accumulators start at -C, whose latency overlaps the
+    // first operand loads, and their negative is stored (exact either way)
     const bool cacc = g.c_acc != 0;
-    if (cacc) {
-#pragma unroll
-        for (int a = 0; a < MB; ++a)
-#pragma unroll
-            for (int b = 0; b < MB; ++b)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int gi = min(i0 + wi + a * 16 + lr, g.M - 1), gj = min(j0 + wj + b * 16 + lk + 4 * v, g.N - 1);
-                    acc[a][b][v] = C[gi + g.ldc * (long)gj];
-                }
-    }
-    // value r of this thread: row (column) ia, depth ka (kb) of the stage; rows
-    // past the edge are read from the last one and their results not stored
-    auto ia = [&](int r) { return TA ? t / GK + (256 / GK) * r : t % T; };
-    auto ka = [&](int r) { return TA ? t % GK : t / T + (256 / T) * r; };
-    auto jb = [&](int r) { return TB ? t % T : t / GK + (256 / GK) * r; };
-    auto kb = [&](int r) { return TB ? t / T + (256 / T) * r : t % GK; };
-    const long sa = TA ? 1 : g.lda, sb = TB ? g.ldb : 1;  // strides of one k
-    unsigned oa[NL], ob[NL];                              // byte offsets from the stage's first k
-#pragma unroll
-    for (int r = 0; r < NL; ++r) {
-        oa[r] = 8u * (unsigned)(min(ia(r), g.M - 1 - i0) * (TA ? (int)g.lda : 1) + ka(r) * (int)sa);
-        ob[r] = 8u * (unsigned)(min(jb(r), g.N - 1 - j0) * (TB ? 1 : (int)g.ldb) + kb(r) * (int)sb);
-    }
-    const double* At = A + (TA ? g.lda * (long)i0 : (long)i0);
-    const double* Bt = B + (TB ? (long)j0 : g.ldb * (long)j0);
-    const int ns = (khi - klo + GK - 1) / GK;  // stages; a last one that is not whole starts earlier,
-    const int skip = ns * GK - (khi - klo);    // its first `skip` depths, done before, count as zero
-    double ra[2][NL], rb[2][NL];
-    auto at = [](const double* base, unsigned o) { return *(const double*)((const char*)base + o); };
-    auto gload = [&](int st, int q) {
-        const int k0 = klo + st * GK - (st == ns - 1 ? skip : 0);
-        const double* Ak = At + sa * k0;
-        const double* Bk = Bt + sb * k0;
-#pragma unroll
-        for (int r = 0; r < NL; ++r) {
-            ra[q][r] = at(Ak, oa[r]);
-            rb[q][r] = at(Bk, ob[r]);
-        }
-    };
-    auto swrite = [&](int st, int q) {
-        const int z = st == ns - 1 ? skip : 0;
-#pragma unroll
-        for (int r = 0; r < NL; ++r) {
-            As[q][ka(r) * T + (ia(r) ^ gemm_sw<GK>(ka(r)))] = ka(r) < z ? 0.0 : ra[q][r];
-            Bs[q][kb(r) * T + (jb(r) ^ gemm_sw<GK>(kb(r)))] = kb(r) < z ? 0.0 : rb[q][r];
-        }
-    };
-    auto multiply = [&](int q, int st) {  // and, half way, stage st (if there is one) from the registers to the other buffer
-        double av[2][MB], bv[2][MB];
-        auto fetch = [&](int ks) {
-            const int k = ks + lk, x = gemm_sw<GK>(k), p = (ks >> 2) & 1;
-#pragma unroll
-            for (int a = 0; a < MB; ++a) av[p][a] = As[q][k * T + ((wi + a * 16 + lr) ^ x)];
-#pragma unroll
-            for (int b = 0; b < MB; ++b) bv[p][b] = Bs[q][k * T + ((wj + b * 16 + lr) ^ x)];
-        };
-        fetch(0);
-#pragma unroll
-        for (int ks = 0; ks < GK; ks += 4) {
-            if (ks + 4 < GK) fetch(ks + 4);
-            if (ks == GK / 2 && st < ns) swrite(st, 1 - q);
-            __builtin_amdgcn_sched_barrier(0);  // the next operands are on their way before these products start
-            const int p = (ks >> 2) & 1;
-#pragma unroll
-            for (int a = 0; a < MB; ++a)
-#pragma unroll
-                for (int b = 0; b < MB; ++b)
-                    acc[a][b] =
-                        __builtin_amdgcn_mfma_f64_16x16x4f64(bv[p][b], cacc ? -av[p][a] : av[p][a], acc[a][b], 0, 0, 0);
-        }
-    };
-    if (khi - klo >= GK) {
-        gload(0, 0);
-        if (ns > 1) gload(1, 1);
-        swrite(0, 0);
-    } else if (khi > klo) {  // one short stage: depths past the end are read from the last one and set to zero
-        const int last = khi - 1 - klo;
-#pragma unroll
-        for (int r = 0; r < NL; ++r) {
-            const int da = max(ka(r) - last, 0), db = max(kb(r) - last, 0);
-            const double va = at(At + sa * klo, oa[r] - 8u * (unsigned)(da * (int)sa));
-            const double vb = at(Bt + sb * klo, ob[r] - 8u * (unsigned)(db * (int)sb));
-            As[0][ka(r) * T + (ia(r) ^ gemm_sw<GK>(ka(r)))] = da ? 0.0 : va;
-            Bs[0][kb(r) * T + (jb(r) ^ gemm_sw<GK>(kb(r)))] = db ? 0.0 : vb;
-        }
-    }
-    __syncthreads();
-    auto stage = [&](int st, int q) {  // stage st in LDS buffer q, st + 1 in registers 1 - q, st + 2 asked for
-        if (st + 2 < ns) gload(st + 2, q);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(q, st + 1);
-        __syncthreads();
-    };
-    for (int st = 0; st < ns; st += 2) {
-        stage(st, 0);
-        if (st + 1 < ns) stage(st + 1, 1);
-    }
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll
         for (int b = 0; b < MB; ++b)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int gi = i0 + wi + a * 16 + lr, gj = j0 + wj + b * 16 + lk + 4 * v;
+                const int gi = min(ib + a * 16, g.M - 1), gj = min(jb + b * 16 + 4 * v, g.N - 1);
+                acc[a][b][v] = cacc ? -C[gi + g.ldc * (long)gj] : 0.0;
+            }
+    gemm_accumulate<T, GK, TA, TB, false>(acc, A, g.lda, g.M - i0, B, g.ldb, g.N - j0, klo, khi, As, Bs,
+                                          [](int, int) { return true; });
+#pragma unroll
+    for (int a = 0; a < MB; ++a)
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int gi = ib + a * 16, gj = jb + b * 16 + 4 * v;
                 if (gi < g.M && gj < g.N) {
                     const long idx = gi + g.ldc * (long)gj;
                     if (cacc) {
-                        C[idx] = acc[a][b][v];
+                        C[idx] = -acc[a][b][v];
                     } else {
                         const double old = g.beta == 0.0 ? 0.0 : g.beta * C[idx];
                         C[idx] = g.alpha * acc[a][b][v] + old;
@@ -205,18 +93,22 @@ static void gemm_tiles(const Gemm& g, hipStream_t st) {
 
 // 64 x 64 tiles carry twice the arithmetic per byte fetched, 32 x 32 ones fill
 // the chip earlier and leave a shorter tail.  Measured, us (64, 32): L^-1 h at
-// N = 1024: 64, 41; 1792: 170, 151; 2112: 210, 223; 4096: 1257, 1624.  With
+// N = 1024: 49, 32; 2112: 175, 189; 4096: 1135, 1229; 7040: 5442, 7696.  With
 // half the tiles and the longest k ranges on the few full columns the tail
-// weighs more: W L^-T at 2112: 176, 89; 4096: 741, 661; 7040: 2285, 2826.
+// weighs more: W L^-T at 2112: 181, 84; 4096: 657, 531; 7040: 1883, 2417; and
+// on a short k (rank 256 on the lower tiles, 4096: 131, 113; 7040: 293, 276)
+// the start does.
 constexpr long GEMM_TILES = 1024, GEMM_TILES_LOWER = 5120;  // whole grids of 64 x 64 tiles from which they are used
+constexpr int GEMM_SHORT_K = 256;
 
 void launch_gemm(const Gemm& g0, hipStream_t st) {
     if (g0.M <= 0 || g0.N <= 0) return;
     Gemm g = g0;
     g.c_acc = g.alpha == -1.0 && g.beta == 1.0;
     const long tiles = (long)((g.M + 63) / 64) * ((g.N + 63) / 64) * (g.batch > 0 ? g.batch : 1);
-    if (tiles >= (g.lower_only && g.kmode != K_FULL ? GEMM_TILES_LOWER : GEMM_TILES)) gemm_tiles<64, 16>(g, st);
-    else gemm_tiles<32, 32>(g, st);
+    const bool large = g.lower_only ? tiles >= GEMM_TILES_LOWER && g.K > GEMM_SHORT_K : tiles >= GEMM_TILES;
+    if (large) gemm_tiles<64, 16>(g, st);
+    else gemm_tiles<32, 16>(g, st);
 }
 
 // Element (r, c) of a 64 x 64 block in LDS: columns of 64, odd ones with their
