@@ -614,15 +614,29 @@ static OpsTarget main_target(dh_system* s) {
                      s->lv, s->lvp, s->lw, s->partial, s->lal, s->lbe, s->counters, s->bounds_h};
 }
 
-// Lanczos spectral bounds of t.Hth into t.bounds (host wait on t.st)
-// With al_host/be_host (pinned), the coefficients are only copied there on
-// t.st and the host part (lanczos_bounds_host) is left to the caller, after
-// the stream has passed them; *m_out gets their count.
-static int bounds_into(dh_system* s, const OpsTarget& t, double* al_host = nullptr, double* be_host = nullptr,
-                       int* m_out = nullptr) {
+// the shadow set that a side build fills
+static OpsTarget side_target(dh_system* s) {
+    dh_context* c = s->ctx;
+    auto& h = s->sh;
+    return OpsTarget{c->side, c->S2, c->h2, c->W2, c->Dinv2, c->info2, h.Q1, h.Q2, h.Hth, h.H32, h.Hlo,
+                     h.lv, h.lvp, h.lw, h.partial, h.lal, h.lbe, h.counters, h.bounds};
+}
+
+constexpr unsigned LANCZOS_SEED = 0x9e3779b9u;
+
+static int lanczos_count(const dh_system* s) { return std::min(s->lanczos_steps, std::min(LANCZOS_MAX, s->N)); }
+
+// The Lanczos recurrence on t.Hth, its coefficients to t.lal and t.lbe: in one
+// launch where that fits (the exchange goes through t.Dinv, free by now), else,
+// and always with one_launch off, step by step.
+static int lanczos_into(dh_system* s, const OpsTarget& t, bool one_launch) {
     hipStream_t st = t.st;
-    const int m = std::min(s->lanczos_steps, std::min(LANCZOS_MAX, s->N));
-    launch_lanczos_start(s->N, t.lv, t.lvp, 0x9e3779b9u, st);
+    const int m = lanczos_count(s);
+    if (one_launch && !matvec_forced() &&
+        launch_lanczos_resident(t.Hth, s->ld, s->N, m, LANCZOS_SEED, t.lal, t.lbe, t.Dinv,
+                                (long)sizeof(double) * s->ld * TILE, s->ctx->cus, st))
+        return DH_OK;
+    launch_lanczos_start(s->N, t.lv, t.lvp, LANCZOS_SEED, st);
     MatvecArgs a{};
     a.M = t.Hth;
     a.ld = s->ld;
@@ -640,18 +654,38 @@ static int bounds_into(dh_system* s, const OpsTarget& t, double* al_host = nullp
         launch_lanczos_step(s->N, t.lv, t.lvp, t.lw, t.lal, t.lbe, j, st);
     }
     DH_HIP(hipGetLastError());
-    if (al_host) {
-        DH_HIP(hipMemcpyAsync(al_host, t.lal, sizeof(double) * m, hipMemcpyDeviceToHost, st));
-        DH_HIP(hipMemcpyAsync(be_host, t.lbe, sizeof(double) * (m + 1), hipMemcpyDeviceToHost, st));
-        *m_out = m;
-        return DH_OK;
+    return DH_OK;
+}
+
+static int lanczos_read(const OpsTarget& t, double* al, double* be, int m) {
+    DH_HIP(hipMemcpyAsync(al, t.lal, sizeof(double) * m, hipMemcpyDeviceToHost, t.st));
+    DH_HIP(hipMemcpyAsync(be, t.lbe, sizeof(double) * (m + 1), hipMemcpyDeviceToHost, t.st));
+    return DH_OK;
+}
+
+// Spectral bounds into t.bounds from coefficients that have arrived in al and be.
+// Coefficients that are not finite (a launch that gave up waiting, or an
+// operator that is not finite itself) are formed again step by step.
+static int bounds_from(dh_system* s, const OpsTarget& t, double* al, double* be, int m) {
+    bool finite = true;
+    for (int j = 0; j < m; ++j) finite = finite && std::isfinite(al[j]) && std::isfinite(be[j + 1]);
+    if (!finite) {
+        if (int rc = lanczos_into(s, t, false)) return rc;
+        if (int rc = lanczos_read(t, al, be, m)) return rc;
+        DH_HIP(hipStreamSynchronize(t.st));
     }
-    double al[LANCZOS_MAX], be[LANCZOS_MAX + 1];
-    DH_HIP(hipMemcpyAsync(al, t.lal, sizeof(double) * m, hipMemcpyDeviceToHost, st));
-    DH_HIP(hipMemcpyAsync(be, t.lbe, sizeof(double) * (m + 1), hipMemcpyDeviceToHost, st));
-    DH_HIP(hipStreamSynchronize(st));
     lanczos_bounds_host(al, be, m, s->rel_margin, t.bounds);
     return DH_OK;
+}
+
+// Lanczos spectral bounds of t.Hth into t.bounds (host wait on t.st)
+static int bounds_into(dh_system* s, const OpsTarget& t) {
+    double al[LANCZOS_MAX], be[LANCZOS_MAX + 1];
+    const int m = lanczos_count(s);
+    if (int rc = lanczos_into(s, t, true)) return rc;
+    if (int rc = lanczos_read(t, al, be, m)) return rc;
+    DH_HIP(hipStreamSynchronize(t.st));
+    return bounds_from(s, t, al, be, m);
 }
 
 // the bounds of a finished build become the system's
@@ -1533,13 +1567,13 @@ static int side_launch(dh_system* s, const double* d_geo, double cutoff, double 
         dh::set_error("dh_propagate_steps: kernel launch failed: %s", hipGetErrorString(hipGetLastError()));
         return DH_ERR_HIP;
     }
-    OpsTarget t{c->side, c->S2, c->h2, c->W2, c->Dinv2, c->info2, h.Q1, h.Q2, h.Hth, h.H32, h.Hlo,
-                h.lv, h.lvp, h.lw, h.partial, h.lal, h.lbe, h.counters, h.bounds};
+    const OpsTarget t = side_target(s);
     int rc = factor_into(s, t, false, h.h_info);
     if (rc) return rc;
     f32_copies_into(s, t);
-    rc = bounds_into(s, t, h.h_al, h.h_be, &h.m);
-    if (rc) return rc;
+    h.m = lanczos_count(s);
+    if ((rc = lanczos_into(s, t, true))) return rc;
+    if ((rc = lanczos_read(t, h.h_al, h.h_be, h.m))) return rc;
     DH_HIP(hipEventRecord(h.done, c->side));
     h.pending = true;
     s->stats[8] += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1560,8 +1594,7 @@ static int side_finish(dh_system* s) {
                       "column %d)", *h.h_info);
         return DH_ERR_NOT_SPD;
     }
-    lanczos_bounds_host(h.h_al, h.h_be, h.m, s->rel_margin, h.bounds);
-    return DH_OK;
+    return bounds_from(s, side_target(s), h.h_al, h.h_be, h.m);
 }
 
 // The shadow operators become the system's (host pointer swaps; both streams

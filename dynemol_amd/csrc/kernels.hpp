@@ -247,6 +247,9 @@ void launch_lanczos_step(int N, cplx* v, cplx* vprev, const cplx* w, double* alp
                          hipStream_t st);
 // extreme-eigenvalue bounds of the Lanczos tridiagonal (al[0..m-1], be[1..m]),
 // on the host: bounds = [emin, emax, theta_min, theta_max, res_min, res_max]
+// the whole recurrence in one launch (lanczos.hip); false: not launched
+bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned seed, double* alpha, double* beta,
+                             void* scratch, long scratch_bytes, int cus, hipStream_t st);
 void lanczos_bounds_host(const double* al, const double* be, int m, double rel_margin, double* bounds);
 int bessel_coef_host(double x, double phase, int kmax_alloc, double tol, cplx* coef);
 void launch_bessel(double x, double phase, int kmax_alloc, double tol, double* J, cplx* coef, int* out_k,
