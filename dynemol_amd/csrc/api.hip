@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -226,6 +227,27 @@ static int round_ld(int N) { return ((N + TILE - 1) / TILE) * TILE; }
 extern "C" const char* dh_last_error(void) { return dh::last_error(); }
 extern "C" int dh_version(void) { return 100; }
 
+// Contexts alive in this process.  The Lanczos recurrence is launched
+// cooperatively only while there is one: builds are where threads that drive
+// their own contexts meet first, and a traced run of two such threads, both
+// with a cooperative launch in their builds, did not come back (the kernel's own
+// waits are bounded; the cause was not found).
+static std::atomic<int> g_contexts{0};
+
+__global__ void first_cooperative_kernel() {}
+
+// The runtime sets up its queue for cooperative launches at the first one: done
+// here, one thread at a time, and not by whichever threads come first.
+static void first_cooperative_launch(hipStream_t st) {
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lk(mu);
+    void* params[] = {nullptr};
+    if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&first_cooperative_kernel), dim3(1), dim3(64), params,
+                                   0, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+        (void)hipGetLastError();
+}
+
 extern "C" int dh_init(int device, dh_context** out) {
     CHECK_ARG(out != nullptr, "dh_init: null output");
     int n = 0;
@@ -245,6 +267,8 @@ extern "C" int dh_init(int device, dh_context** out) {
         delete c;
         return DH_ERR_NOMEM;
     }
+    if (c->cus) first_cooperative_launch(c->stream);
+    g_contexts.fetch_add(1);
     *out = c;
     return DH_OK;
 }
@@ -337,6 +361,7 @@ extern "C" int dh_finalize(dh_context* c) {
     hipFree(c->d_info);
     if (c->side) hipStreamDestroy(c->side);
     hipStreamDestroy(c->stream);
+    g_contexts.fetch_sub(1);
     delete c;
     return DH_OK;
 }
@@ -632,7 +657,7 @@ static int lanczos_count(const dh_system* s) { return std::min(s->lanczos_steps,
 static int lanczos_into(dh_system* s, const OpsTarget& t, bool one_launch) {
     hipStream_t st = t.st;
     const int m = lanczos_count(s);
-    if (one_launch && !matvec_forced() &&
+    if (one_launch && !matvec_forced() && g_contexts.load() == 1 &&
         launch_lanczos_resident(t.Hth, s->ld, s->N, m, LANCZOS_SEED, t.lal, t.lbe, t.Dinv,
                                 (long)sizeof(double) * s->ld * TILE, s->ctx->cus, st))
         return DH_OK;
