@@ -513,15 +513,17 @@ bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, i
 // ------------------------------------------------------------------ batches
 // A batch fills the chip with many systems, so its kernels are chosen for
 // throughput: 16 rows per workgroup, both passes of R > 4 together, and 4 waves
-// per workgroup up to ld = 1024, so that two or more workgroups share a CU and
-// cover each other's exchange.  The split of a system's sums depends on its ld
-// and R alone: its bits are the same in every batch.  64 systems of N 256-2048
-// with 4 wavepackets, 40 steps: 214 ms with one grouped launch per term, 152 ms
-// here; a launch of 8 systems of N = 1000 takes 7.7 us per term, 3.4 of them
-// matrix-core time (both workgroups of a CU wait at the same time).
-static int batch_waves(int ld) { return ld <= 1024 ? 4 : 8; }
-static int batch_lds(int nw, int R) {
-    return (R > 4 ? 2 : 1) * nw * 16 * 4 * 16 + 3 * 16 * R * 16;
+// per workgroup as far as two such workgroups share a CU and cover each other's
+// exchange (up to 256 registers a lane each and half of the LDS: ld = 2048, at
+// R > 4 1920); 8 waves, one workgroup a CU, above.  The split of a system's sums
+// depends on its ld and R alone: its bits are the same in every batch.  64
+// systems of N 256-2048 with 4 wavepackets, 40 steps: 214 ms with one grouped
+// launch per term, 153 ms with 4 waves up to ld = 1024 only, 138 up to 1408, 123
+// here (1 wavepacket: 85 ms up to 1024, 63 here).
+static int batch_waves(int ld, int R) { return ld <= (R > 4 ? 1920 : 2048) ? 4 : 8; }
+static int batch_lds(int nw, int nt, int R) {
+    const int nl = std::max(0, nt - rs_most(R <= 2 ? 0 : R <= 4 ? 1 : 2));
+    return nl * nw * 4 * 64 * 8 + (R > 4 ? 2 : 1) * nw * 16 * 4 * 16 + 3 * 16 * R * 16;
 }
 
 // the grouped kernel for (waves, most groups per wave, columns), its workgroups
@@ -540,23 +542,35 @@ static GroupedKernel grouped_pick(int n) {
         DH_GROUPED(6);
         DH_GROUPED(8);
     }
-    DH_GROUPED(10);
-    DH_GROUPED(12);
-    DH_GROUPED(14);
+    if constexpr (NW == 4) {
+        DH_GROUPED(10);
+        DH_GROUPED(12);
+        DH_GROUPED(14);
+    }
     DH_GROUPED(16);
+    if constexpr (NW == 4) {
+        DH_GROUPED(18);
+        DH_GROUPED(20);
+        DH_GROUPED(22);
+        DH_GROUPED(24);
+        DH_GROUPED(26);
+        DH_GROUPED(28);
+        DH_GROUPED(30);
+        if constexpr (RC < 2) DH_GROUPED(32);
+    }
 #undef DH_GROUPED
     return GroupedKernel{};
 }
 static GroupedKernel grouped_kernel(int nw, int n, int R) {
     const int rc = R <= 2 ? 0 : R <= 4 ? 1 : 2;
     if (nw == 4) return rc == 0 ? grouped_pick<4, 0>(n) : rc == 1 ? grouped_pick<4, 1>(n) : grouped_pick<4, 2>(n);
-    return rc == 0 ? grouped_pick<8, 0>(n) : rc == 1 ? grouped_pick<8, 1>(n) : grouped_pick<8, 2>(n);
+    return grouped_pick<8, 2>(n);
 }
 
 bool resident_batch_member(ResidentArgs* a, void* scratch, long scratch_bytes, int cus) {
     if (cus <= 0 || a->ld > 2048 || a->R > 8 || a->ld / 16 > cus) return false;
     if (!resident_scratch(a, scratch, scratch_bytes)) return false;
-    const int nw = batch_waves(a->ld);
+    const int nw = batch_waves(a->ld, a->R);
     a->groups = (a->ld / 16 + nw - 1) / nw;
     return true;
 }
@@ -578,10 +592,10 @@ bool resident_batch_rounds(const std::vector<ResidentArgs>& members, int cus, st
     int room = 0, nw = 0;
     for (int i : order) {
         const ResidentArgs& a = members[i];
-        const int wgs = a.ld / 16, w = batch_waves(a.ld);
+        const int wgs = a.ld / 16, w = batch_waves(a.ld, a.R);
         if (w != nw || wgs > room) {
             const GroupedKernel k = grouped_kernel(w, a.groups, a.R);
-            const int lds = batch_lds(w, a.R);
+            const int lds = batch_lds(w, k.nt, a.R);
             int per_cu = 0;
             if (!k.f || hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess ||
                 hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k.f, w * 64, (size_t)lds) != hipSuccess ||

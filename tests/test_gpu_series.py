@@ -150,3 +150,35 @@ def test_batch_series_matches_terms(ctx, n_wp):
     for N, x, y in zip(sizes, *out):
         for w in range(n_wp):
             assert np.linalg.norm(x[w] - y[w]) <= 1e-11 * np.linalg.norm(y[w]), N
+
+
+# 4 waves per workgroup up to ld = 2048 (1920 for 4 wavepackets): every count of groups per wave from 18 on,
+# with and without part of the operator in LDS
+@pytest.mark.parametrize("n_wp,sizes", [(1, [1100, 1409, 1537, 1700, 1985, 2048]), (2, [1088, 1473, 1600, 1793, 2000]),
+                                        (4, [1150, 1280, 1408, 1530, 1660, 1792, 1920, 1921])])
+def test_batch_series_four_waves(ctx, n_wp, sizes):
+    out = []
+    for family in (-1, 0):
+        hip.force_batch_family(2 * n_wp, family)
+        try:
+            systems = []
+            for N in sizes:
+                rng = np.random.default_rng(N)
+                b = rng.normal(size=(N, N)) / np.sqrt(N)
+                s = hip.System(ctx, n_orb=N, n_wp=n_wp)
+                s.load_operators(np.eye(N), 8.0 * (b + b.T) - 10.0 * np.eye(N))
+                for w in range(n_wp):
+                    c = (rng.normal(size=N) + 1j * rng.normal(size=N)) / np.sqrt(2.0 * N)
+                    s.set_initial_state(w, c, c)
+                systems.append(s)
+            batch = hip.Batch(ctx, systems)
+            batch.propagate_steps(4, DT)
+            out.append([[s.wavepacket(w)[1] for w in range(n_wp)] for s in systems])
+            batch.close()
+            for s in systems:
+                s.close()
+        finally:
+            hip.force_batch_family(2 * n_wp, -1)
+    for N, x, y in zip(sizes, *out):
+        for w in range(n_wp):
+            assert np.linalg.norm(x[w] - y[w]) <= 1e-11 * np.linalg.norm(y[w]), N
