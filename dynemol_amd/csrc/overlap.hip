@@ -13,15 +13,15 @@
 // rounding: 16 points for |t| < 4, 24 for |t| < 16, else 32 on the part of
 // [-1, 1] where exp(-|t| ...) > e^-80.  The polynomial is evaluated in factored
 // form (radii and heights over both centres), so nothing cancels, and a
-// thread needs no tables: the recursions of the published scheme kept 7 KB of
+// lane needs no tables: the recursions of the published scheme kept 7 KB of
 // them per lane in scratch memory, whose traffic bound the kernel (N = 4096: 3.9
 // ms; N = 514: 1.4 ms).
 //
 // Work decomposition: the atom pairs within the cutoff are collected into a
-// list, and one thread takes one (pair, shell pair).  A shell is the set of
-// 2l+1 orbitals sharing (n, l, zeta, coef) on one atom; a thread evaluates the
-// min(la, lb) + 1 lined-up overlaps together and writes the (2la+1) x (2lb+1)
-// block of S and h (and the mirrored block).
+// list, and eight lanes take one (pair, shell pair).  A shell is the set of
+// 2l+1 orbitals sharing (n, l, zeta, coef) on one atom; the lanes share the eta
+// nodes of its min(la, lb) + 1 lined-up overlaps, and each writes a column of
+// the (2la+1) x (2lb+1) block of S and h (and of the mirrored block).
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -58,10 +58,32 @@ __constant__ double LAG_W[8] = {
     0.3691885893416375, 0.41878678081434295, 0.1757949866371718, 0.03334349226121565, 0.0027945362352256725,
     9.076508773358213e-05, 8.485746716272531e-07, 1.0480011748715104e-09};
 
+// Lanes that share one pair of shells.  With a lane per pair of shells a small
+// system leaves most of the chip idle and takes the length of one lane's
+// quadrature, and a wave runs every eta tier that any of its 64 pairs needs.
+// Eight lanes take the eta nodes in turn, and a column of the block each: N =
+// 514: 256 -> 40 us, 2078: 415 -> 159, 4096: 692 -> 364 (three waves a SIMD; with
+// four the spills cost more: 50, 203, 459).
+constexpr int SUB = 8;
+
+template <int CTRL>
+__device__ __forceinline__ double ov_dpp(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double sub_sum(double v) {  // over the eight lanes, the same in each
+    v += ov_dpp<0xB1>(v);         // quad lanes 1, 0, 3, 2
+    v += ov_dpp<0x4E>(v);         // quad lanes 2, 3, 0, 1
+    return v + ov_dpp<0x141>(v);  // the other quad of the half row
+}
+
 // Lined-up overlaps of two normalised STOs (A at the origin, B at R on z, both
-// along the same axes), acc[m] += cc <n l m | n' l' m>, m = 0..min(LA, LB).
+// along the same axes), acc[m] += cc <n l m | n' l' m>, m = 0..min(LA, LB): the
+// share of lane sub of SUB.
 template <int LA, int LB>
-__device__ __forceinline__ void lined_up(int na, double za, int nb, double zb, double R, double cc, double* acc) {
+__device__ __forceinline__ void lined_up(int na, double za, int nb, double zb, double R, double cc, int sub,
+                                         double* acc) {
     constexpr int MS = LA < LB ? LA : LB;
     const double hr = 0.5 * R, p = (za + zb) * hr, t = (za - zb) * hr, at = fabs(t);
     const double sg = t < 0.0 ? -1.0 : 1.0;  // exp(-t eta) is largest at eta = -sg
@@ -71,15 +93,9 @@ __device__ __forceinline__ void lined_up(int na, double za, int nb, double zb, d
     double sum[MS + 1];
 #pragma unroll
     for (int m = 0; m <= MS; ++m) sum[m] = 0.0;
-    // one pass per point count that any lane of the wave needs: the nodes are then
-    // the same for the whole wave (scalar loads); a lane adds its own pass only
-    for (int tr = 0; tr < 3; ++tr) {
-        if (__ballot(tier == tr) == 0) continue;
-        const int o = tr == 0 ? 0 : tr == 1 ? 8 : 20, half = tr == 0 ? 8 : tr == 1 ? 12 : 16;
-        double part[MS + 1];
-#pragma unroll
-        for (int m = 0; m <= MS; ++m) part[m] = 0.0;
-        for (int j = 0; j < 2 * half; ++j) {
+    {
+        const int o = tier == 0 ? 0 : tier == 1 ? 8 : 20, half = tier == 0 ? 8 : tier == 1 ? 12 : 16;
+        for (int j = sub; j < 2 * half; j += SUB) {
             const double x = j < half ? GL_X[o + j] : -GL_X[o + j - half];
             const double u = len * (1.0 + x);             // distance from the heavy end
             const double eta = sg * (u - 1.0);
@@ -114,11 +130,8 @@ __device__ __forceinline__ void lined_up(int na, double za, int nb, double zb, d
                 }
             }
 #pragma unroll
-            for (int m = 0; m <= MS; ++m) part[m] += we * in[m];
+            for (int m = 0; m <= MS; ++m) sum[m] += we * in[m];
         }
-#pragma unroll
-        for (int m = 0; m <= MS; ++m)
-            if (tier == tr) sum[m] = part[m];
     }
     // (R/2)^(na + nb + 1) / p, the radial norms and the norms of the harmonics
     double fa = 1.0, fb = 1.0;
@@ -234,7 +247,7 @@ __global__ __launch_bounds__(256) void pair_list_kernel(const BasisDev b, double
 
 template <int LA, int LB>
 __device__ __forceinline__ void shell_block(const BasisDev& b, int shA, int shB, const Axes& ax, double R, double* S,
-                                            double* h, int ld, double s_drop) {
+                                            double* h, int ld, double s_drop, int sub) {
     constexpr int MS = LA < LB ? LA : LB;
     double sig[MS + 1];
 #pragma unroll
@@ -242,42 +255,44 @@ __device__ __forceinline__ void shell_block(const BasisDev& b, int shA, int shB,
     for (int j = 0; j < b.sh_nzeta[shB]; ++j)
         for (int i = 0; i < b.sh_nzeta[shA]; ++i)
             lined_up<LA, LB>(b.sh_n[shA], b.sh_zeta[2 * shA + i], b.sh_n[shB], b.sh_zeta[2 * shB + j], R,
-                             b.sh_coef[2 * shA + i] * b.sh_coef[2 * shB + j], sig);
-    double blk[2 * LA + 1][2 * LB + 1];
+                             b.sh_coef[2 * shA + i] * b.sh_coef[2 * shB + j], sub, sig);
+#pragma unroll
+    for (int m = 0; m <= MS; ++m) sig[m] = sub_sum(sig[m]);
+    double col[2 * LA + 1];  // column sub of the block (lanes past its last repeat it and store nothing)
 #pragma unroll
     for (int m = -MS; m <= MS; ++m) {
         double ra[2 * LA + 1], rb[2 * LB + 1];
         rotation_column<LA>(ax, m, ra);
         rotation_column<LB>(ax, m, rb);
+        double sb = rb[0];
+#pragma unroll
+        for (int j = 1; j <= 2 * LB; ++j) sb = sub == j ? rb[j] : sb;
         const double s = sig[m < 0 ? -m : m];
 #pragma unroll
-        for (int i = 0; i <= 2 * LA; ++i)
-#pragma unroll
-            for (int j = 0; j <= 2 * LB; ++j) {
-                const double v = s * ra[i] * rb[j];
-                blk[i][j] = m == -MS ? v : blk[i][j] + v;
-            }
+        for (int i = 0; i <= 2 * LA; ++i) {
+            const double v = s * ra[i] * sb;
+            col[i] = m == -MS ? v : col[i] + v;
+        }
     }
-    const int a0 = b.sh_orb0[shA], b0 = b.sh_orb0[shB];
+    if (sub > 2 * LB) return;
+    const int a0 = b.sh_orb0[shA], bo = b.sh_orb0[shB] + sub;
     // X of the block: IP, k_WH and V_shift per orbital
 #pragma unroll
-    for (int j = 0; j <= 2 * LB; ++j)
-#pragma unroll
-        for (int i = 0; i <= 2 * LA; ++i) {
-            double s = blk[i][j];
-            if (fabs(s) < s_drop) s = 0.0;
-            const int a = a0 + i, bo = b0 + j;
-            const double hv = huckel_x(b.ip[a], b.ip[bo], b.kwh[a], b.kwh[bo], b.vshift[a], b.vshift[bo]) * s;
-            S[(long)a + (long)ld * bo] = s;
-            S[(long)bo + (long)ld * a] = s;
-            h[(long)a + (long)ld * bo] = hv;
-            h[(long)bo + (long)ld * a] = hv;
-        }
+    for (int i = 0; i <= 2 * LA; ++i) {
+        double s = col[i];
+        if (fabs(s) < s_drop) s = 0.0;
+        const int a = a0 + i;
+        const double hv = huckel_x(b.ip[a], b.ip[bo], b.kwh[a], b.kwh[bo], b.vshift[a], b.vshift[bo]) * s;
+        S[(long)a + (long)ld * bo] = s;
+        S[(long)bo + (long)ld * a] = s;
+        h[(long)a + (long)ld * bo] = hv;
+        h[(long)bo + (long)ld * a] = hv;
+    }
 }
 
-__global__ __launch_bounds__(64) void build_SH_kernel(const BasisDev b, const int* count, const int2* list, double* S,
+__global__ __launch_bounds__(64, 3) void build_SH_kernel(const BasisDev b, const int* count, const int2* list, double* S,
                                                       double* h, int ld, double s_drop) {
-    const int q = blockIdx.x * 64 + threadIdx.x;
+    const int q = blockIdx.x * (64 / SUB) + threadIdx.x / SUB, sub = threadIdx.x % SUB;
     if (q >= *count) return;
     const int2 pr = list[q];
     const int sp = blockIdx.y;
@@ -314,15 +329,15 @@ __global__ __launch_bounds__(64) void build_SH_kernel(const BasisDev b, const in
     ax.e2[2] = ax.u[0] * ax.e1[1] - ax.u[1] * ax.e1[0];
     const int shA = b.atom_shell0[ia] + sa, shB = b.atom_shell0[ib] + sb;
     switch (3 * b.sh_l[shA] + b.sh_l[shB]) {
-        case 0: shell_block<0, 0>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 1: shell_block<0, 1>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 2: shell_block<0, 2>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 3: shell_block<1, 0>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 4: shell_block<1, 1>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 5: shell_block<1, 2>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 6: shell_block<2, 0>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        case 7: shell_block<2, 1>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
-        default: shell_block<2, 2>(b, shA, shB, ax, R, S, h, ld, s_drop); break;
+        case 0: shell_block<0, 0>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 1: shell_block<0, 1>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 2: shell_block<0, 2>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 3: shell_block<1, 0>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 4: shell_block<1, 1>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 5: shell_block<1, 2>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 6: shell_block<2, 0>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        case 7: shell_block<2, 1>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
+        default: shell_block<2, 2>(b, shA, shB, ax, R, S, h, ld, s_drop, sub); break;
     }
 }
 
@@ -340,7 +355,7 @@ int launch_build_SH(const BasisDev& b, int N, int ld, double* S, double* h, doub
     if (npair > 0) {
         hipLaunchKernelGGL(pair_list_kernel, dim3((unsigned)((npair + 255) / 256)), dim3(256), 0, st, b, cutoff, count,
                            list);
-        hipLaunchKernelGGL(build_SH_kernel, dim3((unsigned)((npair + 63) / 64), MAX_SHELLS * MAX_SHELLS), dim3(64), 0, st,
+        hipLaunchKernelGGL(build_SH_kernel, dim3((unsigned)((npair + 64 / SUB - 1) / (64 / SUB)), MAX_SHELLS * MAX_SHELLS), dim3(64), 0, st,
                            b, count, list, S, h, ld, s_drop);
     }
     return hipGetLastError() == hipSuccess ? 0 : -1;
