@@ -102,8 +102,24 @@ constexpr int rs_depth(int rg, int nt, int nreg, int rc) {
                              : (184 - 8 * nreg) / 4;
     return d < 2 ? std::min(2, nt) : std::min(d, nt);
 }
+// EAGER, up to 640 columns (NW NT groups of 16): a term is latency there, and the
+// data are their own flags.  A slot holds RS_UNSET in every word until its term
+// is published; a wave loads all its groups of x at device scope (past the L2)
+// until none of them is unset, which saves the wait for the stores, the flag's
+// way and the second read.  A workgroup that publishes T_k sets its rows of slot
+// k + 2 back: every workgroup has published T_{k-1}, so all are past reading
+// T_{k-2}, the last term that slot may hold; and it waits for those stores before
+// it publishes T_{k+1}, without which nobody looks for T_{k+2}.  Slots 0 and 1 are
+// set before the launch.  A value that is itself this NaN ends in the bounded wait.
+constexpr bool rs_eager(int nw, int nt) { return nw * nt <= 40; }
+constexpr int RS_UNSET = 0x7ffba5c3;
+__device__ __forceinline__ bool rs_unset(double x, double y) {
+    return (__double2hiint(x) == RS_UNSET) | (__double2hiint(y) == RS_UNSET);
+}
+
 template <int NW, int RG, int NT, int RC>
 __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int blk, const int nblk) {
+    constexpr bool EAGER = rs_eager(NW, NT);
     constexpr int NREG = RG == 4 && NT > rs_most(RC) ? rs_most(RC) : NT, NL = NT - NREG;
     constexpr int NQ = (MULTI_MAX + NW - 1) / NW;  // accumulators per wave
     constexpr bool PAIR = RC > 0, WIDE = RC == 2 && RG == 4;
@@ -111,7 +127,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
     constexpr int PT = RC == 2 && !WIDE ? 2 : 1;  // column sets
     constexpr int XL = WIDE ? 2 : PT;             // loads of x per group
     constexpr int PC = WIDE ? 8 : 4;              // columns per row of a wave's partial sums
-    constexpr int DEPTH = rs_depth(RG, NT, NREG, RC);
+    constexpr int DEPTH = EAGER ? NT : rs_depth(RG, NT, NREG, RC);
     using xv_t = typename std::conditional<PAIR, double2, double>::type;
     extern __shared__ double smem[];
     const int R = a.R;
@@ -163,14 +179,9 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
     constexpr int gbytes = XL * 64 * (int)sizeof(xv_t);  // a group's part of a slot
     // element e of the workgroup's rows goes to its lane's place (WIDE: load q
     // holds rows 8 q + k and 8 q + 4 + k of lane 16k + real column side by side)
-    auto publish = [&](int e, cplx T, int slot) {
+    auto put = [&](int e, v4i bits, int slot) {
         const int row = r0 + e / R, col = e % R;
         const int to = (row >> 4) * gbytes, so = slot * a.slot_bytes;
-        v4i bits;
-        bits[0] = __double2loint(T.re);
-        bits[1] = __double2hiint(T.re);
-        bits[2] = __double2loint(T.im);
-        bits[3] = __double2hiint(T.im);
         if constexpr (WIDE) {
             const int at = to + (row >> 3 & 1) * 1024 + (16 * (row & 3) + 2 * col) * 16 + (row >> 2 & 1) * 8;
             __builtin_amdgcn_raw_buffer_store_b64(bits.xy, ring, at, so, AUX_DEVICE_SCOPE);
@@ -180,10 +191,21 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
             __builtin_amdgcn_raw_buffer_store_b128(bits, ring, to + at * (int)sizeof(xv_t), so, AUX_DEVICE_SCOPE);
         }
     };
+    auto publish = [&](int e, cplx T, int k) {  // T_k
+        v4i bits;
+        bits[0] = __double2loint(T.re);
+        bits[1] = __double2hiint(T.re);
+        bits[2] = __double2loint(T.im);
+        bits[3] = __double2hiint(T.im);
+        if constexpr (EAGER) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last term's put of RS_UNSET
+        put(e, bits, k % a.slots);
+        if constexpr (EAGER) put(e, v4i{RS_UNSET, RS_UNSET, RS_UNSET, RS_UNSET}, (k + 2) % a.slots);
+    };
     // waves 0..SW-1 add up the waves' sums and publish 64 elements each; a flag per
     // publishing wave
     constexpr int SW = RB * (PAIR ? 4 * RC : 2) > 64 ? 2 : 1;
     auto raise = [&](unsigned v) {  // after this wave's stores have arrived
+        if constexpr (EAGER) return;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (lane < RS_COPIES)
             __hip_atomic_store(a.flags + (lane * nblk + blk) * SW + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -221,7 +243,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
         for (int v = 0; v < NQ; ++v)
             if (k <= kq[v]) ck[v] = rs_coef(a.coef + (long)(w + NW * v) * a.coef_stride + k);
         if (active) {
-            if (!dead) {
+            if (!EAGER && !dead) {
                 unsigned long long t0 = 0;
                 for (int spin = 0;; ++spin) {
                     const unsigned v = __hip_atomic_load(myflag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -238,17 +260,18 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
             }
             asm volatile("" ::: "memory");
             const int slot = (k - 1) % a.slots;
-            if (slot == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (!EAGER && slot == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             // (columns past the last are not written: their sums are not kept;
             // groups past ld read the last one: their H is zero)
             const int xoff = lane * (int)sizeof(xv_t);
             const int soff = slot * a.slot_bytes + (k0 >> 4) * gbytes;
             auto xload = [&](int g, int p) -> xv_t {
                 const int so = soff + min(g, max(ng, 1) - 1) * gbytes;
+                constexpr int aux = EAGER ? AUX_DEVICE_SCOPE : 0;
                 if constexpr (PAIR)
-                    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(ring, xoff + p * 1024, so, 0));
+                    return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(ring, xoff + p * 1024, so, aux));
                 else
-                    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ring, xoff, so, 0));
+                    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ring, xoff, so, aux));
             };
             double yr[PT][RG], yi[PT][RG];
             v4d yw[2];  // WIDE: even and odd steps of 4 columns
@@ -281,10 +304,31 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
                 return st < RONLY ? st : (st - RONLY) % 2 == 0 ? RONLY + (st - RONLY) / 2 : NREG + (st - RONLY) / 2;
             };
             xv_t xb[DEPTH][XL];
+            unsigned long long t0 = 0;
+            for (int spin = 0;; ++spin) {
+                if constexpr (EAGER) asm volatile("" ::: "memory");  // every look reads memory again
 #pragma unroll
-            for (int d = 0; d < DEPTH; ++d)
+                for (int d = 0; d < DEPTH; ++d)
 #pragma unroll
-                for (int p = 0; p < XL; ++p) xb[d][p] = xload(group(d), p);
+                    for (int p = 0; p < XL; ++p) xb[d][p] = xload(group(d), p);
+                if (!EAGER || dead) break;
+                bool unset = false;
+#pragma unroll
+                for (int d = 0; d < DEPTH; ++d)
+#pragma unroll
+                    for (int p = 0; p < XL; ++p) {
+                        // columns past the last are never written
+                        if constexpr (WIDE) unset |= ((lane & 15) < 2 * R) & rs_unset(xb[d][p].x, xb[d][p].y);
+                        else if constexpr (PAIR) unset |= (lj + 4 * p < R) & rs_unset(xb[d][p].x, xb[d][p].y);
+                        else unset |= (lj < 2 * R) & rs_unset(xb[d][p], xb[d][p]);
+                    }
+                if (__ballot(unset) == 0) break;
+                if ((spin & 255) == 255) {
+                    const unsigned long long now = wall_clock64();
+                    if (t0 == 0) t0 = now;
+                    else if (now - t0 > RS_WAIT_TICKS) dead = true;
+                }
+            }
             double hl[RG];
 #pragma unroll
             for (int st = 0; st < NT; ++st) {
@@ -361,7 +405,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
                     T.re -= x2.re;
                     T.im -= x2.im;
                 }
-                if (k < K) publish(e, T, k % a.slots);
+                if (k < K) publish(e, T, k);
                 tk[e] = T;
             }
             if (k < K) raise((unsigned)k + 1u);
@@ -423,10 +467,18 @@ __global__ __launch_bounds__(NW * 64, 2) void resident_grouped_kernel(const Resi
     resident_body<NW, 4, NT, RC>(a, mp[1], a.ld / 16);
 }
 
-__global__ __launch_bounds__(256) void resident_clear_kernel(const ResidentArgs* members) {
+// Before a launch: flags to zero, and slots 0 and 1 of the ring, which lie behind
+// them, to RS_UNSET.
+__device__ __forceinline__ void resident_clear(const ResidentArgs& a, int first, int step) {
+    const int nf = (int)(a.ring - reinterpret_cast<char*>(a.flags)) / 4, n = nf + 2 * a.slot_bytes / 4;
+    for (int i = first; i < n; i += step) a.flags[i] = i < nf ? 0u : (unsigned)RS_UNSET;
+}
+__global__ __launch_bounds__(256) void resident_clear_kernel(ResidentArgs a) {
+    resident_clear(a, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256);
+}
+__global__ __launch_bounds__(256) void resident_clear_grouped_kernel(const ResidentArgs* members) {
     const ResidentArgs a = members[blockIdx.x];
-    const int n = (int)(a.ring - reinterpret_cast<char*>(a.flags)) / 4;
-    for (int i = threadIdx.x; i < n; i += 256) a.flags[i] = 0u;
+    resident_clear(a, blockIdx.y * 256 + threadIdx.x, gridDim.y * 256);
 }
 
 // ------------------------------------------------------------------ plan
@@ -503,7 +555,7 @@ bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, i
     const ResidentPlan p = resident_plan(a.ld, a.R, cus);
     if (!p.ok || !resident_scratch(&a, scratch, scratch_bytes)) return false;
     a.groups = p.groups;
-    launch_zero_u32(a.flags, (int)(resident_flag_bytes(a.ld) / 4), st);
+    hipLaunchKernelGGL(resident_clear_kernel, dim3(32), dim3(256), 0, st, a);
     const hipError_t e = resident_launch(a, p, st);
     if (e == hipSuccess) return true;
     (void)hipGetLastError();  // not launched: the caller runs the series term by term
@@ -617,7 +669,7 @@ bool resident_batch_rounds(const std::vector<ResidentArgs>& members, int cus, st
 int launch_resident_rounds(const ResidentArgs* d_members, int n, const int2* d_map,
                            const std::vector<ResidentRound>& rounds, hipStream_t st) {
     if (n <= 0) return 0;
-    hipLaunchKernelGGL(resident_clear_kernel, dim3(n), dim3(256), 0, st, d_members);
+    hipLaunchKernelGGL(resident_clear_grouped_kernel, dim3(n, 8), dim3(256), 0, st, d_members);
     for (const ResidentRound& r : rounds) {
         const int2* map = d_map + r.first;
         void* params[] = {&d_members, &map};
