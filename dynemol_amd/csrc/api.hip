@@ -2107,7 +2107,7 @@ static size_t apply_layout(int N, int R, char* base, ApplyWork* w) {
     t.partial = (cplx*)take(sizeof(cplx) * part);
     t.partial_cplx = part;
     t.counters = (unsigned*)take(sizeof(unsigned) * ld);
-    t.J = (double*)take(sizeof(double) * (KMAX_ALLOC + 2));
+    t.J = (double*)take(sizeof(double) * (KMAX_ALLOC + 2));  // not used any more: keeps the size callers know
     t.coef = (cplx*)take(sizeof(cplx) * (KMAX_ALLOC + 2));
     t.kout = (int*)take(sizeof(int) * 4);
     t.norms0 = (double*)take(sizeof(double) * R);
@@ -2161,7 +2161,7 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
     for (int attempt = 0; attempt < 4; ++attempt) {
         const double c = 0.5 * (bounds[1] + bounds[0]);
         const double r = 0.5 * (bounds[1] - bounds[0]) * widen;
-        launch_bessel(r * dt, c * dt, KMAX_ALLOC, BESSEL_TOL, w.J, w.coef, w.kout, st);
+        launch_bessel(r * dt, c * dt, KMAX_ALLOC, BESSEL_TOL, w.coef, w.kout, st);
         int K = 0;
         DH_HIP(hipGetLastError());
         DH_HIP(hipMemcpyAsync(&K, w.kout, sizeof(int), hipMemcpyDeviceToHost, st));

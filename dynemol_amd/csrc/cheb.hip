@@ -2583,40 +2583,79 @@ void lanczos_bounds_host(const double* al, const double* be, int m, double rel_m
 // J_k(x), k = 0..K, by Miller's backward recurrence J_{k-1} = (2k/x) J_k - J_{k+1}
 // normalised with J_0 + 2 sum J_{2k} = 1; K = last k with |J_k| > tol.
 // coef[k] = (2 - delta_k0) (-i)^k J_k(x) e^{-i c dt};  out_k[0] = K (number of terms - 1).
-__global__ void bessel_coef_kernel(double x, double phase, int kmax_alloc, double tol, double* J, cplx* coef, int* out_k) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+//
+// One wave.  The recurrence and the normalisation are serial: every lane runs
+// them (the values go to LDS once), eight steps' factors 2k/x read ahead, so a
+// step costs its multiply and add; divisions, magnitudes and coefficients are
+// the lanes'.  With all of it in one lane and through global memory the table of
+// 85 terms took 53 us, a tenth of a short dh_chebyshev_apply; here 9.
+constexpr int BESSEL_MAX = 4098;
+__global__ __launch_bounds__(64) void bessel_coef_kernel(double x, double phase, int kmax_alloc, double tol, cplx* coef,
+                                                         int* out_k) {
+    __shared__ double J[BESSEL_MAX];
+    const int lane = threadIdx.x;
     int K = 0;
     if (x < 1e-12) {
-        J[0] = 1.0;
-        K = 0;
+        if (lane == 0) J[0] = 1.0;
+        __syncthreads();
     } else {
         int M = (int)(x + 15.0 * cbrt(x) + 40.0);
         M += M & 1;
         if (M > kmax_alloc - 2) M = kmax_alloc - 2;
+        // J[k - 1] holds 2k/x until step k replaces it
+        for (int k = 1 + lane; k <= M; k += 64) J[k - 1] = 2.0 * k / x;
+        if (lane == 0) J[M] = 1e-300;
+        __syncthreads();
         double jp1 = 0.0, jk = 1e-300;
-        for (int k = 0; k <= M + 1; ++k) J[k] = 0.0;
-        J[M] = jk;
-        for (int k = M; k >= 1; --k) {
-            const double jm1 = (2.0 * k / x) * jk - jp1;
-            J[k - 1] = jm1;
-            jp1 = jk;
-            jk = jm1;
-            if (fabs(jk) > 1e250) {
-                for (int q = k - 1; q <= M; ++q) J[q] *= 1e-250;
-                jk *= 1e-250;
-                jp1 *= 1e-250;
+        constexpr int AHEAD = 8;
+        double f[AHEAD];
+        for (int k = M; k >= 1; k -= AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) f[u] = J[max(k - u - 1, 0)];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {
+                if (k - u < 1) break;
+                const double jm1 = f[u] * jk - jp1;
+                if (lane == 0) J[k - u - 1] = jm1;
+                jp1 = jk;
+                jk = jm1;
+                if (fabs(jk) > 1e250) {
+                    __syncthreads();
+                    for (int q = k - u - 1 + lane; q <= M; q += 64) J[q] *= 1e-250;
+                    __syncthreads();
+                    jk *= 1e-250;
+                    jp1 *= 1e-250;
+                }
             }
         }
+        __syncthreads();
         double norm = J[0];
-        for (int k = 2; k <= M; k += 2) norm += 2.0 * J[k];
-        for (int k = 0; k <= M; ++k) J[k] /= norm;
-        K = M;
-        while (K > 0 && fabs(J[K]) < tol) --K;
+        int k = 2;
+        for (; k + 14 <= M; k += 16) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = J[k + 2 * u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) norm += 2.0 * v[u];
+        }
+        for (; k <= M; k += 2) norm += 2.0 * J[k];
+        __syncthreads();
+        for (int q = lane; q <= M; q += 64) J[q] /= norm;
+        __syncthreads();
+        // the last k with |J_k| >= tol, or 0
+        for (int top = M; top > 0; top -= 64) {
+            const int q = top - lane;
+            const unsigned long long keep = __ballot(q > 0 && !(fabs(J[max(q, 0)]) < tol));
+            if (keep) {
+                K = top - (__ffsll(keep) - 1);
+                break;
+            }
+        }
         K += 1;
         if (K > M) K = M;
     }
     const double cp = cos(phase), sp = -sin(phase);  // e^{-i phase}
-    for (int k = 0; k <= K; ++k) {
+    for (int k = lane; k <= K; k += 64) {
         const double f = (k == 0 ? 1.0 : 2.0) * J[k];
         // (-i)^k
         double re, im;
@@ -2628,8 +2667,10 @@ __global__ void bessel_coef_kernel(double x, double phase, int kmax_alloc, doubl
         }
         coef[k] = cplx{re * cp - im * sp, re * sp + im * cp};
     }
-    coef[K + 1] = cplx{0.0, 0.0};
-    out_k[0] = K;
+    if (lane == 0) {
+        coef[K + 1] = cplx{0.0, 0.0};
+        out_k[0] = K;
+    }
 }
 
 // The same coefficients on the host (the recurrence above, operation for
@@ -2863,9 +2904,10 @@ void launch_lanczos_step(int N, cplx* v, cplx* vprev, const cplx* w, double* alp
                          hipStream_t st) {
     hipLaunchKernelGGL(lanczos_step_kernel, dim3(1), dim3(1024), 0, st, N, v, vprev, w, alpha, beta, j);
 }
-void launch_bessel(double x, double phase, int kmax_alloc, double tol, double* J, cplx* coef, int* out_k,
+void launch_bessel(double x, double phase, int kmax_alloc, double tol, cplx* coef, int* out_k,
                    hipStream_t st) {
-    hipLaunchKernelGGL(bessel_coef_kernel, dim3(1), dim3(64), 0, st, x, phase, kmax_alloc, tol, J, coef, out_k);
+    hipLaunchKernelGGL(bessel_coef_kernel, dim3(1), dim3(64), 0, st, x, phase, std::min(kmax_alloc, BESSEL_MAX), tol,
+                       coef, out_k);
 }
 void launch_observables(int N, int W, int n_frag, const int* frag, const cplx* out, const cplx* phi, const cplx* hk,
                         double* pops, double* erg, double* norms, hipStream_t st) {

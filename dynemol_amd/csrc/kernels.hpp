@@ -252,7 +252,7 @@ bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned see
                              void* scratch, long scratch_bytes, int cus, hipStream_t st);
 void lanczos_bounds_host(const double* al, const double* be, int m, double rel_margin, double* bounds);
 int bessel_coef_host(double x, double phase, int kmax_alloc, double tol, cplx* coef);
-void launch_bessel(double x, double phase, int kmax_alloc, double tol, double* J, cplx* coef, int* out_k,
+void launch_bessel(double x, double phase, int kmax_alloc, double tol, cplx* coef, int* out_k,
                    hipStream_t st);
 void launch_observables(int N, int W, int n_frag, const int* frag, const cplx* out, const cplx* phi, const cplx* hk,
                         double* pops, double* erg, double* norms, hipStream_t st);
