@@ -8,12 +8,13 @@
 // (134 MB), so this kernel loads H once, keeps each workgroup's rows of it in
 // registers and LDS, and runs every term of the series with nothing read from
 // memory but the previous term's vectors, which the workgroups exchange
-// through global memory behind one flag per workgroup and term.  Per term, one
-// launch per term against this kernel: N = 4096, R = 4: 21.6 -> 6.9 us; N =
-// 2048: 10.3 -> 4.7 us (R = 4), 17 -> 5.5 us (R = 8); N = 416: 7.2 -> 2.9 us.
-// At N = 4096 a term is now 3.4 us of matrix-core time, about 1.4 us of waiting
-// for the other workgroups' flags and 1.5 us of latencies (first loads of x,
-// the sum over the waves, the store); at N = 416 it is latency alone.
+// through global memory: behind one flag per workgroup and term, or (EAGER below)
+// with the data as their own flags.  Per term, one launch per term against this
+// kernel: N = 4096, R = 4: 21.6 -> 6.9 us; N = 2048: 10.3 -> 4.1 us (R = 4), 17 ->
+// 5.2 us (R = 8); N = 416: 7.2 -> 2.3 us.  At N = 4096 a term is now 3.4 us of
+// matrix-core time, about 1.4 us of waiting for the other workgroups' flags and
+// 1.5 us of latencies (first loads of x, the sum over the waves, the store); at N
+// = 416 it is the latency of one exchange.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -28,9 +29,8 @@ namespace dh {
 // 12 + b of the group, so a B operand (x) feeds every row group without
 // replication: lane 16k + 4b + j takes x[16g + 4k + b][j], 16 bytes (re, im).
 // The ring keeps the vectors in this order (per group of 16 rows and pass of 4
-// columns, the 64 lanes' values), so a load is 1 KB contiguous: in row-major
-// order its quarter-waves touched 4 half-used lines each, and a CU got 22 bytes
-// per clock.  A operands (H) stay in the lane's registers, up to what
+// columns, the 64 lanes' values), so a load is 1 KB contiguous (as fast as
+// row-major order measured, and the addresses are simpler).  A operands (H) stay in the lane's registers, up to what
 // 256 registers hold beside the products (23 groups at R = 4), and in LDS from
 // there on.  At R = 4 a group is 8 MFMAs of 16 cycles on one load; N = 4096: 32
 // groups per wave, 3.4 us of matrix-core time per term.
@@ -102,16 +102,23 @@ constexpr int rs_depth(int rg, int nt, int nreg, int rc) {
                              : (184 - 8 * nreg) / 4;
     return d < 2 ? std::min(2, nt) : std::min(d, nt);
 }
-// EAGER, up to 640 columns (NW NT groups of 16): a term is latency there, and the
-// data are their own flags.  A slot holds RS_UNSET in every word until its term
-// is published; a wave loads all its groups of x at device scope (past the L2)
-// until none of them is unset, which saves the wait for the stores, the flag's
-// way and the second read.  A workgroup that publishes T_k sets its rows of slot
-// k + 2 back: every workgroup has published T_{k-1}, so all are past reading
-// T_{k-2}, the last term that slot may hold; and it waits for those stores before
-// it publishes T_{k+1}, without which nobody looks for T_{k+2}.  Slots 0 and 1 are
-// set before the launch.  A value that is itself this NaN ends in the bounded wait.
-constexpr bool rs_eager(int nw, int nt) { return nw * nt <= 40; }
+// EAGER, while a wave's whole share of x fits its registers beside H: the data
+// are their own flags.  A slot holds RS_UNSET in every word until its term is
+// published; a wave loads all its groups of x at device scope (past the L2) until
+// none of them is unset, which saves the wait for the stores, the flag's way and
+// the second read.  A workgroup that publishes T_k sets its rows of slot k + 2
+// back: every workgroup has published T_{k-1}, so all are past reading T_{k-2},
+// the last term that slot may hold; and it waits for those stores before it
+// publishes T_{k+1}, without which nobody looks for T_{k+2}.  Slots 0 and 1 are set
+// before the launch.  A value that is itself this NaN ends in the bounded wait.
+// Per term, us with flags / eager: N = 416, R = 4: 3.3 / 2.3; 1024: 3.5 / 2.6; 2048:
+// 4.7 / 4.1; 2304: 4.9 / 4.5, but 2560: 5.1 / 5.7 (x no longer fits); R = 2: 2048:
+// 3.7 / 2.9, 2560: 4.1 / 3.5, 3072: 4.6 / 4.4 with spills; R = 8: 1024: 4.1 / 3.3,
+// 2048: 5.4 / 5.2.  A batch fills the chip, and its kernels read x past the L2
+// only where that is little (640 columns).
+constexpr bool rs_eager(int nw, int rg, int nt, int rc) {
+    return nw == 4 ? nt <= 10 : rc == 0 ? nt <= 22 : rc == 1 ? nt <= 18 : rg == 2;
+}
 constexpr int RS_UNSET = 0x7ffba5c3;
 __device__ __forceinline__ bool rs_unset(double x, double y) {
     return (__double2hiint(x) == RS_UNSET) | (__double2hiint(y) == RS_UNSET);
@@ -119,7 +126,7 @@ __device__ __forceinline__ bool rs_unset(double x, double y) {
 
 template <int NW, int RG, int NT, int RC>
 __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int blk, const int nblk) {
-    constexpr bool EAGER = rs_eager(NW, NT);
+    constexpr bool EAGER = rs_eager(NW, RG, NT, RC);
     constexpr int NREG = RG == 4 && NT > rs_most(RC) ? rs_most(RC) : NT, NL = NT - NREG;
     constexpr int NQ = (MULTI_MAX + NW - 1) / NW;  // accumulators per wave
     constexpr bool PAIR = RC > 0, WIDE = RC == 2 && RG == 4;

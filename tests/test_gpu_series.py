@@ -182,3 +182,38 @@ def test_batch_series_four_waves(ctx, n_wp, sizes):
     for N, x, y in zip(sizes, *out):
         for w in range(n_wp):
             assert np.linalg.norm(x[w] - y[w]) <= 1e-11 * np.linalg.norm(y[w]), N
+
+
+# edges of the sizes whose data are their own flags (2816 at R = 1 and 2, 2304 at 4, 2048 at 8), and counts of
+# columns that leave part of a lane's share unwritten
+@pytest.mark.parametrize("N,R", [(385, 4), (448, 1), (641, 8), (1024, 2), (1409, 4), (1990, 1), (2047, 8), (2304, 4),
+                                 (2305, 4), (2816, 2), (2816, 1), (2817, 2)])
+def test_series_without_flags(ctx, operator, N, R):
+    print(f"[gpu] series without flags, N={N}, R={R}", flush=True)
+    a, ka = _apply(ctx, operator, N, R, -1)
+    b, kb = _apply(ctx, operator, N, R, 18 if R <= 8 else 15)
+    assert ka == kb
+    assert np.linalg.norm(a[:N] - b[:N]) <= 1e-11 * np.linalg.norm(b[:N])
+
+
+@pytest.mark.parametrize("n_wp,N", [(3, 500), (3, 1500), (3, 2100), (1, 300), (2, 2304)])
+def test_steps_without_flags(ctx, operator, n_wp, N):
+    """Several long series one after another on one system (stale ring slots of the last one), R = 2, 4 and 6."""
+    print(f"[gpu] steps without flags, N={N}, n_wp={n_wp}", flush=True)
+    out = []
+    for variant in (-1, 9):
+        hip.force_matvec_variant(variant)
+        try:
+            s = hip.System(ctx, n_orb=N, n_wp=n_wp)
+            s.load_operators(np.eye(N), operator[:N, :N] * (34.0 / np.sqrt(8.0 * N)))
+            rng = np.random.default_rng(N)
+            for w in range(n_wp):
+                c = (rng.normal(size=N) + 1j * rng.normal(size=N)) / np.sqrt(2.0 * N)
+                s.set_initial_state(w, c, c)
+            for m in (1, 7, 3, 10):
+                s.propagate_steps(m, DT)
+            out.append(np.stack([s.wavepacket(w)[1] for w in range(n_wp)]))
+            s.close()
+        finally:
+            hip.force_matvec_variant(-1)
+    assert np.linalg.norm(out[0] - out[1]) <= 1e-11 * np.linalg.norm(out[1])
