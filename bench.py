@@ -25,6 +25,7 @@ sys.path.insert(0, ROOT)
 DT_PS = 5.0e-4
 REBUILD_EVERY = 10
 JITTER = 0.02
+FP64_PEAK_TFLOPS = 78.6  # matrix cores, dense
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per Chebyshev term (both kernels of the symmetric variant, N=4096,
 # 4 RHS) from rocprofv3 FETCH_SIZE and WRITE_SIZE, each scaled by what the same
@@ -627,20 +628,41 @@ def main():
 
     R = 4  # complex columns: electron and hole, bra and ket each
     variant = g["tuning"]["term"]
-    sym = variant in SYM_VARIANTS
-    # algorithmic bytes of the kernel that ran: the symmetric variants read H's
-    # lower-triangle tiles once (half storage), the dense ones all of H
-    bytes_term = half_storage_bytes(N, R) if sym else term_bytes(N, R)
-    avg_launch_s = g["series_ms"] / 1e3 / max(1, g["series_launches"])
-    achieved = bytes_term / avg_launch_s / 1e9
-    traffic = MEASURED_TRAFFIC_BYTES.get(variant) if N == 4096 else None
+    avg_term_s = g["series_ms"] / 1e3 / max(1, g["series_launches"])
     value = 2 * args.steps / g["elapsed"]
     prop_only = g["prop_only"]
-    # the same term alone (HIP events around repeated launches on a zero-filled
-    # operator of the same shape, one accumulator, nothing beside it): the
-    # figure a kernel trace's phase 1 + phase 2 averages compare with
-    from dynemol_amd import hip
-    alone_us = hip.time_matvec(N, R, variant, reps=50)
+    flops_term = 4 * R * N * N
+    # a series of up to 8 columns and 4096 orbitals runs in one launch with H on the chip (H is read once per
+    # series): its products are the bound, H's bytes are spread over the series' terms
+    if args.term_variant < 0 and N <= 4096:
+        terms = float(np.median(g["terms"]))
+        achieved = flops_term / avg_term_s / 1e12
+        roofline = {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                    "frac": round(achieved / FP64_PEAK_TFLOPS, 4), "traffic": None,
+                    "kernel": "Chebyshev series in one launch, FP64, 4 RHS, H resident in registers and LDS",
+                    "flops_per_term": flops_term, "bytes_per_term": round(8 * N * N / terms + 32 * N * R),
+                    "avg_term_us": round(avg_term_s * 1e6, 3)}
+    else:
+        sym = variant in SYM_VARIANTS
+        # algorithmic bytes of the kernel that ran: the symmetric variants read H's
+        # lower-triangle tiles once (half storage), the dense ones all of H
+        bytes_term = half_storage_bytes(N, R) if sym else term_bytes(N, R)
+        achieved = bytes_term / avg_term_s / 1e9
+        traffic = MEASURED_TRAFFIC_BYTES.get(variant) if N == 4096 else None
+        # the same term alone (HIP events around repeated launches on a zero-filled
+        # operator of the same shape, one accumulator, nothing beside it): the
+        # figure a kernel trace's phase 1 + phase 2 averages compare with
+        from dynemol_amd import hip
+        alone_us = hip.time_matvec(N, R, variant, reps=50)
+        roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
+                    "kernel": f"Chebyshev term, FP64, 4 RHS (variant {variant}: "
+                              f"{'lower-triangle tiles of symmetric H' if sym else 'dense H'})",
+                    "bytes_per_term": bytes_term, "avg_term_us": round(avg_term_s * 1e6, 3),
+                    # measured HBM bytes per term over the same time
+                    "traffic_frac": round(traffic / avg_term_s / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
+                    "alone_us": round(alone_us, 3),
+                    "alone_frac": round(bytes_term / (alone_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)}
     out = {
         "metric": "wavepacket-steps/s at N=4096 (mixed vs FP64, pop.err<=1e-6) + serve p50/p99",
         "value": round(value, 3),
@@ -658,21 +680,7 @@ def main():
                                "hole HOMO), 0.5 fs steps, S/h/Cholesky/Lanczos rebuilt every 10 steps (jitter 0.02 A), "
                                "the step loop on the device (dh_propagate_steps)",
                    "n_orbitals": N, "wavepackets": 2, "rebuild_every": REBUILD_EVERY},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": f"Chebyshev term, FP64, 4 RHS (autotuned variant {variant}: "
-                               f"{'lower-triangle tiles of symmetric H' if sym else 'dense H'})",
-                     "bytes_per_launch": bytes_term, "avg_launch_us": round(avg_launch_s * 1e6, 3),
-                     # measured HBM bytes per term over the same time
-                     "traffic_frac": round(traffic / avg_launch_s / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
-                     # the same time against a dense term's bytes (H read in full, 8 N^2 + 80 N R): the rate a
-                     # dense-storage kernel would need to match this one, not an HBM rate
-                     # the timed region's rebuilds run on a second stream beside the terms (dh_propagate_steps),
-                     # so this average includes their interference
-                     "dense_equivalent_bytes": term_bytes(N, R),
-                     "dense_equivalent_frac": round(term_bytes(N, R) / avg_launch_s / 1e9 / HBM_PEAK_GBS, 4),
-                     "alone_us": round(alone_us, 3),
-                     "alone_frac": round(bytes_term / (alone_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4)},
+        "roofline": roofline,
         "propagation_only_value": round(prop_only, 3),
         # terms launched in the timed region per step (an interval's steps share recurrences)
         "chebyshev_terms_per_step": round(g["series_launches"] / args.steps, 1),

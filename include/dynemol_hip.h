@@ -198,10 +198,12 @@ int dh_set_timing(dh_system *sys, int on);
 /* Steps per Chebyshev recurrence in dh_propagate_steps (every precision mode
  * and term kernel): within a rebuild interval the operator is fixed and the
  * terms T_k(Hh) phi do not depend on time, so one recurrence to the last
- * step's K collects every step's state, each with its own coefficients (the
- * symmetric half-storage terms add each term to the step accumulators in
- * their epilogue; the other term kernels leave the terms in a 16-slot ring
- * that a pass adds to the accumulators every 16 terms).  m = 0
+ * step's K collects every step's state, each with its own coefficients (a
+ * series of up to 8 columns and 4096 orbitals in FP64 runs in one launch with
+ * the operator on the chip and keeps the accumulators there; the symmetric
+ * half-storage terms add each term to the step accumulators in their epilogue;
+ * the other term kernels leave the terms in a 16-slot ring that a pass adds to
+ * the accumulators every 16 terms).  m = 0
  * (default): up to 10 steps per recurrence, within the interval and the
  * 4096-term coefficient table; m = 1: one recurrence per step, the same
  * kernels and bits as dh_propagate.  The steps' states agree to rounding
@@ -212,7 +214,8 @@ int dh_set_steps_per_series(dh_system *sys, int m);
 /* Run each step's Chebyshev term series as one captured hipGraph (on = 1;
  * the default for N <= 2048) or as individual kernel launches (on = 0).  The graph is
  * captured on the first step with given spectral bounds, term count and buffer
- * assignment and replayed afterwards; results are identical either way.  No
+ * assignment and replayed afterwards; results are identical either way.  A
+ * series that runs in one launch (dh_set_steps_per_series) uses neither.  No
  * counterpart in the reference (one cuBLAS call per term, Taylor_gpu.cpp:295-330). */
 int dh_set_graph(dh_system *sys, int on);
 /* Matvec kernel variant chosen by the autotuner for this system's shapes:
@@ -223,9 +226,11 @@ int dh_matvec_tuning(dh_system *sys, int *out7);
 
 /*
  * Multi-system batch: n systems of possibly different N with the same number
- * of wavepackets (1, 2, 4, 8 or 16), advanced together by one grouped launch per
- * Chebyshev term (FP64 members; members in other precision modes run their own
- * term kernels in the same step).  The systems stay owned by the caller; results are read per
+ * of wavepackets (1, 2, 4, 8 or 16), advanced together: members of up to 4
+ * wavepackets and 2048 orbitals by a few launches per series, each over as many
+ * members as the chip holds with their operators in registers; the others by one
+ * grouped launch per Chebyshev term (FP64 members; members in other precision
+ * modes run their own term kernels in the same step).  The systems stay owned by the caller; results are read per
  * system with dh_get_wavepacket / dh_get_observables.  No counterpart in the
  * reference (one system per process, ElHl_Chebyshev.f:148-291).
  */
@@ -238,15 +243,16 @@ int dh_batch_propagate(dh_batch *batch, double t_init, double t_max, int *max_te
  * own coefficients, as dh_propagate_steps does for one system): one norm
  * check, commit and output pass per recurrence, and the outputs read
  * afterwards are those of the final state.  The states agree with n_steps
- * calls of dh_batch_propagate to rounding.  The grouped terms write each
- * member's ring of 16 terms, and a grouped pass adds them to the members'
- * accumulators every 16 terms.  Batches with members in other precision modes
+ * calls of dh_batch_propagate to rounding.  Members whose operators stay on the
+ * chip keep their accumulators there; the grouped terms write each member's
+ * ring of 16 terms, and a grouped pass adds them to the members' accumulators
+ * every 16 terms.  Batches with members in other precision modes
  * step one step at a time.  max_terms: the most terms of one recurrence.  No counterpart
  * in the reference. */
 int dh_batch_propagate_steps(dh_batch *batch, int n_steps, double dt, int *max_terms);
 /* Term kernel family the batch autotuner chose for this batch's wavepacket
- * count (once per process, by timing both on the first batch of that count):
- * 1 = symmetric half-storage tiles, 0 = dense column blocks.  Members in a
+ * count (once per process, by timing both on the first batch of that count that
+ * has grouped terms): 1 = symmetric half-storage tiles, 0 = dense column blocks.  Members in a
  * precision mode other than FP64 run their own term kernels inside the batch
  * step.  No counterpart in the reference. */
 int dh_batch_tuning(dh_batch *batch, int *family);
