@@ -892,15 +892,19 @@ __global__ __launch_bounds__(256) void panel_kernel(MatvecArgs a, double* __rest
     __shared__ double As[2][16 * T];
     __shared__ double Bs[2][16 * T];
     constexpr int MB = T / 32;
-    const int N = a.N, C = 2 * a.R;
+    const int N = a.N, C1 = 2 * a.R, C = C1 * max(a.steps, 1);
     const bool upper = TRI && a.tri == TRI_UPPER;
     const int i0 = (upper ? gridDim.x - 1 - blockIdx.x : blockIdx.x) * T, c0 = blockIdx.y * T, z = blockIdx.z;
     const int lo = TRI && !upper ? i0 : 0, hi = upper ? min(N, i0 + T) : N;
     const int per = ((hi - lo + S - 1) / S + 15) & ~15;
     const int klo = min(hi, lo + z * per), khi = min(hi, klo + per);
     const EA* A = (sizeof(EA) == 8 ? reinterpret_cast<const EA*>(a.M) : reinterpret_cast<const EA*>(a.M32)) + i0;
-    const double* B = reinterpret_cast<const double*>(a.x) + 2L * a.x_off + c0;
+    const double* B = reinterpret_cast<const double*>(a.x) + 2L * a.x_off;
     const long xs = 2L * a.x_stride;
+    auto bcol = [&](int j) {  // real column c0 + j: a step and a column of its state
+        const int c = c0 + j, q = a.steps > 1 ? c / C1 : 0;
+        return c - q * C1 + q * (int)(2 * a.x_step);
+    };
     v4d acc[MB][MB];
 #pragma unroll
     for (int p = 0; p < MB; ++p)
@@ -910,12 +914,12 @@ __global__ __launch_bounds__(256) void panel_kernel(MatvecArgs a, double* __rest
     if constexpr (TRI) {
         const int mlo = upper ? max(klo, i0) : klo, mhi = upper ? khi : min(khi, i0 + T);
         gemm_accumulate<T, 16, 0, 1, true>(acc, A, a.ld, N - i0, B, xs, C - c0, mlo, mhi, As, Bs,
-                                           [&](int i, int k) { return upper ? k <= i0 + i : k >= i0 + i; });
+                                           [&](int i, int k) { return upper ? k <= i0 + i : k >= i0 + i; }, bcol);
         if (upper) uhi = min(khi, i0);
         else ulo = max(klo, i0 + T);
     }
     gemm_accumulate<T, 16, 0, 1, false>(acc, A, a.ld, N - i0, B, xs, C - c0, ulo, uhi, As, Bs,
-                                        [](int, int) { return true; });
+                                        [](int, int) { return true; }, bcol);
     double* Pz = P + (long)z * C * a.ld;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int ib = i0 + (w >> 1) * (T / 2) + (lane & 15), cb = c0 + (w & 1) * (T / 2) + (lane >> 4);
@@ -1031,7 +1035,8 @@ __global__ __launch_bounds__(256) void panel_reduce_kernel(MatvecArgs a, const P
                                                            const PT* __restrict__ Plo, int S) {
     __shared__ double y[16][17];  // y[column][row]
     const int i0 = blockIdx.x * 16, r0 = blockIdx.y * 8, t = threadIdx.x;
-    const long C = 2L * a.R, slice = C * a.ld;
+    const int RT = a.R * max(a.steps, 1);
+    const long C = 2L * RT, slice = C * a.ld;
     const int c = t >> 4, i = min(i0 + (t & 15), a.N - 1);
     const long o = min(2L * r0 + c, C - 1) * a.ld + i;
     auto sum = [&](const PT* p) {
@@ -1053,30 +1058,45 @@ __global__ __launch_bounds__(256) void panel_reduce_kernel(MatvecArgs a, const P
     y[c][t & 15] = v;
     __syncthreads();
     const int r = t & 7, ii = t >> 3;
-    if (t < 128 && i0 + ii < a.N && r0 + r < a.R)
-        term_epilogue(a, i0 + ii, r0 + r, cplx{y[2 * r][ii], y[2 * r + 1][ii]});
+    if (t >= 128 || i0 + ii >= a.N || r0 + r >= RT) return;
+    const cplx v1{y[2 * r][ii], y[2 * r + 1][ii]};
+    if (a.steps > 1) {
+        const int q = (r0 + r) / a.R;
+        cplx* const out = q == a.steps - 1 ? a.out_last : a.out + q * a.out_step;
+        out[(long)(i0 + ii) * a.out_stride + a.out_off + (r0 + r - q * a.R)] = v1;
+    } else {
+        term_epilogue(a, i0 + ii, r0 + r, v1);
+    }
 }
 
-static dim3 panel_reduce_grid(const MatvecArgs& a) { return dim3((a.N + 15) / 16, (a.R + 7) / 8); }
+static dim3 panel_reduce_grid(const MatvecArgs& a) { return dim3((a.N + 15) / 16, (a.R * std::max(a.steps, 1) + 7) / 8); }
 
 void launch_lib_reduce(const MatvecArgs& a, const float* Phi, const float* Plo, int S, hipStream_t st) {
     hipLaunchKernelGGL((panel_reduce_kernel<float>), panel_reduce_grid(a), dim3(256), 0, st, a, Phi, Plo, S);
 }
 
-// Slices of the FP64 kernel: 3 (T = 64) or 4 (T = 32) workgroups a CU, at least
-// 256 k each, and no more than P is sized for.
+// Slices of the FP64 kernel: 3 (T = 64) or 4 (T = 32) workgroups a CU, at most
+// `most` (256 k each, and what P is sized for).
 template <int T, typename EA, bool TRI>
-static int panel_tiles(const MatvecArgs& a, double* P, hipStream_t st) {
-    const int tr = (a.N + T - 1) / T, tc = (2 * a.R + T - 1) / T, want = T == 64 ? 768 : 1024;
-    const int S = std::max(1, std::min(want / (tr * tc), gemm3_splits(a.N, a.R)));
+static int panel_tiles(const MatvecArgs& a, double* P, int most, hipStream_t st) {
+    const int tr = (a.N + T - 1) / T, tc = (2 * a.R * std::max(a.steps, 1) + T - 1) / T, want = T == 64 ? 768 : 1024;
+    const int S = std::max(1, std::min(want / (tr * tc), most));
     hipLaunchKernelGGL((panel_kernel<T, EA, TRI>), dim3(tr, tc, S), dim3(256), 0, st, a, P, S);
     return S;
 }
 
 // up to 32 real columns a tile of 64 would be half empty
 template <typename EA, bool TRI>
-static int panel_f64(const MatvecArgs& a, double* P, hipStream_t st) {
-    return 2 * a.R <= 32 ? panel_tiles<32, EA, TRI>(a, P, st) : panel_tiles<64, EA, TRI>(a, P, st);
+static int panel_f64(const MatvecArgs& a, double* P, int most, hipStream_t st) {
+    return 2 * a.R * std::max(a.steps, 1) <= 32 ? panel_tiles<32, EA, TRI>(a, P, most, st)
+                                                : panel_tiles<64, EA, TRI>(a, P, most, st);
+}
+
+void launch_panel_steps(const MatvecArgs& a, double* P, long p_doubles, hipStream_t st) {
+    const int most = (int)std::min<long>((a.N + 255) / 256, p_doubles / (2L * a.R * std::max(a.steps, 1) * a.ld));
+    const int S = a.tri == TRI_FULL ? panel_f64<double, false>(a, P, most, st) : panel_f64<double, true>(a, P, most, st);
+    hipLaunchKernelGGL((panel_reduce_kernel<double>), panel_reduce_grid(a), dim3(256), 0, st, a, (const double*)P,
+                       (const double*)nullptr, S);
 }
 
 void launch_gemm3(const MatvecArgs& a, int prec, double* P, hipStream_t st) {
@@ -1090,9 +1110,10 @@ void launch_gemm3(const MatvecArgs& a, int prec, double* P, hipStream_t st) {
         return;
     }
     int S;
-    if (prec == 2) S = panel_f64<float, false>(a, P, st);
-    else if (a.tri == TRI_FULL) S = panel_f64<double, false>(a, P, st);
-    else S = panel_f64<double, true>(a, P, st);
+    const int most = gemm3_splits(a.N, a.R);
+    if (prec == 2) S = panel_f64<float, false>(a, P, most, st);
+    else if (a.tri == TRI_FULL) S = panel_f64<double, false>(a, P, most, st);
+    else S = panel_f64<double, true>(a, P, most, st);
     hipLaunchKernelGGL((panel_reduce_kernel<double>), panel_reduce_grid(a), dim3(256), 0, st, a, (const double*)P,
                        (const double*)nullptr, S);
 }
@@ -2794,9 +2815,8 @@ __global__ __launch_bounds__(256) void grouped_observables_kernel(const ObsTask*
 }
 
 // Column norms |phi_c|^2 of an N x R complex block (one workgroup per column).
-__global__ __launch_bounds__(256) void column_norms_kernel(int N, int R, const cplx* x, double* out) {
+__device__ __forceinline__ double column_norm(int N, int R, const cplx* x, int c) {
     __shared__ double sh[4];
-    const int c = blockIdx.x;
     double s = 0.0;
 #pragma unroll 4
     for (int i = threadIdx.x; i < N; i += blockDim.x) {
@@ -2806,7 +2826,34 @@ __global__ __launch_bounds__(256) void column_norms_kernel(int N, int R, const c
     s = wave_sum(s);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) out[c] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    return ((sh[0] + sh[1]) + sh[2]) + sh[3];
+}
+
+__global__ __launch_bounds__(256) void column_norms_kernel(int N, int R, const cplx* x, double* out) {
+    const double s = column_norm(N, R, x, blockIdx.x);
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
+}
+
+__global__ __launch_bounds__(256) void step_norms_kernel(int N, int R, const cplx* keep, const cplx* accm, long acc_step,
+                                                         int steps, bool from_keep, double* n0, double* n1) {
+    const int c = blockIdx.x, q = blockIdx.y;  // q = 0: the input; else the result of step q - 1
+    const double s = column_norm(N, R, q ? accm + (q - 1) * acc_step : keep, c);
+    if (threadIdx.x != 0) return;
+    if (q > 0) n1[(q - 1) * R + c] = s;
+    if (from_keep) {
+        if (q == 0)
+            for (int p = 0; p < steps; ++p) n0[p * R + c] = s;
+    } else if (q < steps) {
+        n0[q * R + c] = s;
+    }
+}
+
+__global__ __launch_bounds__(256) void step_observables_kernel(StepObservables o) {
+    const int w = blockIdx.x, q = blockIdx.y;
+    const bool last = q == o.steps - 1;
+    observables_body(o.N, o.W, o.n_frag, o.frag, last ? o.out_last : o.out + q * o.out_step, o.phi + q * o.phi_step,
+                     last ? o.hk_last : o.hk + q * o.hk_step, o.pops + (long)q * o.W * (o.n_frag + 1),
+                     o.erg + (long)q * o.W * 2, o.norms + (long)q * o.W * 2, w);
 }
 
 __global__ __launch_bounds__(256) void grouped_norms_kernel(const NormTask* tasks) {
@@ -2916,6 +2963,15 @@ void launch_observables(int N, int W, int n_frag, const int* frag, const cplx* o
 }
 void launch_column_norms(int N, int R, const cplx* x, double* out, hipStream_t st) {
     hipLaunchKernelGGL(column_norms_kernel, dim3(R), dim3(256), 0, st, N, R, x, out);
+}
+
+void launch_step_norms(int N, int R, const cplx* keep, const cplx* accm, long acc_step, int steps, bool from_keep,
+                       double* n0, double* n1, hipStream_t st) {
+    hipLaunchKernelGGL(step_norms_kernel, dim3(R, steps + 1), dim3(256), 0, st, N, R, keep, accm, acc_step, steps,
+                       from_keep, n0, n1);
+}
+void launch_step_observables(const StepObservables& o, hipStream_t st) {
+    hipLaunchKernelGGL(step_observables_kernel, dim3(o.W, o.steps), dim3(256), 0, st, o);
 }
 
 }  // namespace dh

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void gemm_f64_kernel(Gemm g) {
                 acc[a][b][v] = cacc ? -C[gi + g.ldc * (long)gj] : 0.0;
             }
     gemm_accumulate<T, GK, TA, TB, false>(acc, A, g.lda, g.M - i0, B, g.ldb, g.N - j0, klo, khi, As, Bs,
-                                          [](int, int) { return true; });
+                                          [](int, int) { return true; }, [](int j) { return j; });
 #pragma unroll
     for (int a = 0; a < MB; ++a)
 #pragma unroll

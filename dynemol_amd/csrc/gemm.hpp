@@ -49,11 +49,12 @@ __device__ __forceinline__ void gemm_order() {
 // first column (columns contiguous with TB, else k contiguous); na and nb rows
 // and columns of the tile exist: those past them are read from the last one.
 // keep(i, k) says for MASKED products which elements of A count (i within the
-// tile).  Every thread of the workgroup calls it; it ends with a barrier.
-template <int T, int GK, int TA, int TB, bool MASKED, typename EA, typename Keep>
+// tile); bcol(j) is the place of column j of a TB tile, in elements from B.  Every thread of the workgroup calls it; it ends with a barrier.
+template <int T, int GK, int TA, int TB, bool MASKED, typename EA, typename Keep, typename BCol>
 __device__ __forceinline__ void gemm_accumulate(v4d (&acc)[T / 32][T / 32], const EA* A, long lda, int na,
                                                 const double* B, long ldb, int nb, int klo, int khi,
-                                                double (*As)[GK * T], double (*Bs)[GK * T], const Keep& keep) {
+                                                double (*As)[GK * T], double (*Bs)[GK * T], const Keep& keep,
+                                                const BCol& bcol) {
     constexpr int MB = T / 32;        // 16 x 16 blocks of a wave per direction
     constexpr int NL = GK * T / 256;  // values a thread fetches per operand and stage
     constexpr int EB = (int)sizeof(EA);
@@ -70,7 +71,7 @@ __device__ __forceinline__ void gemm_accumulate(v4d (&acc)[T / 32][T / 32], cons
 #pragma unroll
     for (int r = 0; r < NL; ++r) {
         oa[r] = EB * (min(ia(r), na - 1) * (TA ? (int)lda : 1) + ka(r) * (int)sa);
-        ob[r] = 8 * (min(jb(r), nb - 1) * (TB ? 1 : (int)ldb) + kb(r) * (int)sb);
+        ob[r] = 8 * ((TB ? bcol(min(jb(r), nb - 1)) : min(jb(r), nb - 1) * (int)ldb) + kb(r) * (int)sb);
     }
     const int ns = khi > klo ? (khi - klo + GK - 1) / GK : 0;  // stages; a last one that is not whole starts
     const int skip = ns * GK - (khi - klo);                    // earlier, its first `skip` depths count as zero

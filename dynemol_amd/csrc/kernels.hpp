@@ -183,6 +183,12 @@ struct MatvecArgs {
     const cplx* coefm;
     int coefm_stride;
     int m_lo, m_hi;
+    // Products on the states of several steps at once (launch_panel_steps): step
+    // q's columns are x + q * x_step, its results out + q * out_step, the last
+    // step's out_last.
+    int steps;
+    long x_step, out_step;
+    cplx* out_last;
     int m_pair;  // EPI_CHEB: 0 = adds nothing, 1 = c_k T_k, 2 = c_{k-1} x + c_k T_k (x = T_{k-1})
 };
 // true once after a term launch that accumulated a.accm itself
@@ -222,6 +228,21 @@ void launch_cheb_gemm(const MatvecArgs& a, int prec, hipStream_t st);
 // products on M32 widened to FP64); P holds
 // gemm3_partial_doubles(N, ld, R) doubles of partial products
 void launch_gemm3(const MatvecArgs& a, int prec, double* P, hipStream_t st);
+// EPI_PLAIN products of a.steps states; p_doubles: size of P, at least 2 R steps ld
+void launch_panel_steps(const MatvecArgs& a, double* P, long p_doubles, hipStream_t st);
+// norms of keep and of the steps' states accm + q * acc_step: n0[q] of step q's
+// input (keep's for every step with from_keep), n1[q] of its result
+void launch_step_norms(int N, int R, const cplx* keep, const cplx* accm, long acc_step, int steps, bool from_keep,
+                       double* n0, double* n1, hipStream_t st);
+struct StepObservables {
+    int N, W, n_frag, steps;
+    const int* frag;
+    const cplx *out, *hk, *phi;  // step q at + q * its step; the last step's out and hk apart
+    long out_step, hk_step, phi_step;
+    const cplx *out_last, *hk_last;
+    double *pops, *erg, *norms;  // norms: 2 W per step
+};
+void launch_step_observables(const StepObservables& o, hipStream_t st);
 void launch_term_f32h(const MatvecArgs& a, hipStream_t st);
 long gemm3_partial_doubles(int N, int ld, int R);
 // Grouped column-block matvec over many systems (R in {1, 2, 4, 8, 16}); each
