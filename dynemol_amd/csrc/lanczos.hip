@@ -6,10 +6,13 @@
 // 4096.  Here a workgroup keeps its rows of H in registers (and LDS at the
 // largest sizes) and every workgroup keeps the whole of v_j and v_{j-1}, spread
 // over its threads.  A step exchanges one vector, y = H v_j: each workgroup
-// publishes its rows of y behind a flag, reads the whole of it, and forms
-// alpha = v.y, w = y - alpha v - beta v_prev and beta = |w| for itself, in the
-// same order everywhere, so no second exchange is needed.  Bound by that
-// exchange and two workgroup-wide sums: about 3 us a step at any size.
+// publishes its rows of y, reads the whole of it, and forms alpha = v.y, w = y -
+// alpha v - beta v_prev and beta = |w| for itself, in the same order everywhere,
+// so no second exchange is needed.  The data are their own flags: every step has
+// a slot of its own, set to LZ_UNSET before the launch, and a wave loads its share
+// past the L2 until nothing in it is unset.  Bound by that exchange and two
+// workgroup-wide sums: 126 us for the 48 steps at N = 514, 172 at 2078, 347 at
+// 4096 (201, 234 and 512 with one flag per workgroup and step).
 //
 // All workgroups must be on the chip at once, so the launch is cooperative, and
 // every wait is bounded (wall clock): a wave that runs out of time goes on with
@@ -21,17 +24,16 @@
 
 namespace dh {
 
-constexpr int LZ_COPIES = 16;                               // of the flags, each polled by every 16th workgroup
 constexpr unsigned long long LZ_WAIT_TICKS = 200000000ull;  // 2 s of the 100 MHz wall clock
-constexpr int LZ_DEVICE_SCOPE = 16;                         // buffer store: sc1
+constexpr int LZ_DEVICE_SCOPE = 16;                         // buffer access: sc1
+constexpr int LZ_UNSET = 0x7ffba5c3;                        // high word of a value not there yet (a NaN)
 
 struct LanczosArgs {
     const double* H;
     int ld, N, m;
     unsigned seed;
     double *alpha, *beta;
-    unsigned* flags;  // [LZ_COPIES][workgroups], zero at the start
-    double* ring;     // y of step j at ring + j * ld: read once, so never stale in a cache
+    double* ring;  // y of step j at ring + j * ld
 };
 
 __device__ __forceinline__ void lz_swap32(double& a, double& b) {  // upper half of a <-> lower half of b
@@ -112,7 +114,7 @@ __global__ __launch_bounds__(512) void lanczos_resident_kernel(LanczosArgs a) {
     extern __shared__ double hs[];                    // [RL][M][512]
     __shared__ double part[8][RW], red[2][8];
     const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int blk = blockIdx.x, nblk = gridDim.x, r0 = blk * RW, c0 = 64 * M * w;
+    const int blk = blockIdx.x, r0 = blk * RW, c0 = 64 * M * w;
     const int N = a.N, ld = a.ld;
     double h[RR][M], v[M], vp[M];
     auto hval = [&](int i, int q) {
@@ -153,12 +155,8 @@ __global__ __launch_bounds__(512) void lanczos_resident_kernel(LanczosArgs a) {
 
     const __amdgpu_buffer_rsrc_t ring =
         __builtin_amdgcn_make_buffer_rsrc(a.ring, 0, a.m * ld * 8, 0x00020000);
-    // flags of the rows this wave reads
-    const int f0 = c0 / RW, nf = max(0, min((c0 + 64 * M) / RW, nblk) - f0);
-    const unsigned* const flag = a.flags + (blk % LZ_COPIES) * nblk + min(f0 + min(lane, max(nf - 1, 0)), nblk - 1);
     bool dead = false;
     double be = 0.0;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     for (int j = 0; j < a.m; ++j) {
         double s[RW];
 #pragma unroll
@@ -189,37 +187,28 @@ __global__ __launch_bounds__(512) void lanczos_resident_kernel(LanczosArgs a) {
                 bits[1] = __double2hiint(y);
                 __builtin_amdgcn_raw_buffer_store_b64(bits, ring, (j * ld + r0 + lane) * 8, 0, LZ_DEVICE_SCOPE);
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the rows have arrived
-            if (lane < LZ_COPIES)
-                __hip_atomic_store(a.flags + lane * nblk + blk, (unsigned)(j + 1), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (nf > 0 && !dead) {
-            unsigned long long t0 = 0;
-            for (int spin = 0;; ++spin) {
-                const unsigned f = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (__ballot(f < (unsigned)(j + 1)) == 0) break;
-                if ((spin & 255) == 255) {
-                    const unsigned long long now = wall_clock64();
-                    if (t0 == 0) t0 = now;
-                    else if (now - t0 > LZ_WAIT_TICKS) {
-                        dead = true;
-                        break;
-                    }
-                }
+        double y[M];
+        unsigned long long t0 = 0;
+        for (int spin = 0;; ++spin) {
+            asm volatile("" ::: "memory");  // every look reads memory again
+            bool unset = false;
+#pragma unroll
+            for (int q = 0; q < M; ++q) {
+                const int c = c0 + 64 * q + lane;
+                y[q] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(ring, (j * ld + min(c, N - 1)) * 8, 0,
+                                                                                       LZ_DEVICE_SCOPE));
+            }
+#pragma unroll
+            for (int q = 0; q < M; ++q) unset |= (c0 + 64 * q + lane < N) & (__double2hiint(y[q]) == LZ_UNSET);
+            if (dead || __ballot(unset) == 0) break;
+            if ((spin & 255) == 255) {
+                const unsigned long long now = wall_clock64();
+                if (t0 == 0) t0 = now;
+                else if (now - t0 > LZ_WAIT_TICKS) dead = true;
             }
         }
-        asm volatile("" ::: "memory");
-        double y[M], p = dead ? __builtin_nan("") : 0.0;
-#pragma unroll
-        for (int q = 0; q < M; ++q) {
-            // (a wave with no columns must not read: it has not waited, and the line
-            // would stay in the XCD's L2 as it was)
-            const int c = c0 + 64 * q + lane;
-            y[q] = nf > 0 ? __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
-                                                           ring, (j * ld + min(c, N - 1)) * 8, 0, 0))
-                          : 0.0;
-        }
+        double p = dead ? __builtin_nan("") : 0.0;
 #pragma unroll
         for (int q = 0; q < M; ++q) {
             if (c0 + 64 * q + lane >= N) y[q] = 0.0;
@@ -247,6 +236,10 @@ __global__ __launch_bounds__(512) void lanczos_resident_kernel(LanczosArgs a) {
     }
 }
 
+__global__ __launch_bounds__(256) void lanczos_clear_kernel(unsigned* ring, long n) {
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) ring[i] = LZ_UNSET;
+}
+
 template <int M>
 static hipError_t lanczos_go(LanczosArgs a, hipStream_t st) {
     constexpr int RW = M == 1 ? 2 : M == 2 ? 4 : M <= 4 ? 8 : 16;
@@ -254,7 +247,9 @@ static hipError_t lanczos_go(LanczosArgs a, hipStream_t st) {
     const void* f = reinterpret_cast<const void*>(&lanczos_resident_kernel<M>);
     if (hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds); e != hipSuccess) return e;
     const int wgs = (a.N + RW - 1) / RW;
-    launch_zero_u32(a.flags, LZ_COPIES * wgs, st);
+    const long words = 2L * a.m * a.ld;
+    hipLaunchKernelGGL(lanczos_clear_kernel, dim3((unsigned)std::min(512L, (words + 255) / 256)), dim3(256), 0, st,
+                       reinterpret_cast<unsigned*>(a.ring), words);
     void* params[] = {&a};
     return hipLaunchCooperativeKernel(f, dim3(wgs), dim3(512), params, lds, st);
 }
@@ -266,10 +261,8 @@ bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned see
                              void* scratch, long scratch_bytes, int cus, hipStream_t st) {
     const int M = (ld + 511) / 512, RW = M == 1 ? 2 : M == 2 ? 4 : M <= 4 ? 8 : 16;
     if (M > 8 || (N + RW - 1) / RW > cus) return false;
-    const long fb = LZ_COPIES * 256L * 4;
-    if (fb + 8L * m * ld > scratch_bytes) return false;
-    LanczosArgs a{H, ld, N, m, seed, alpha, beta, static_cast<unsigned*>(scratch),
-                  reinterpret_cast<double*>(static_cast<char*>(scratch) + fb)};
+    if (8L * m * ld > scratch_bytes) return false;
+    LanczosArgs a{H, ld, N, m, seed, alpha, beta, static_cast<double*>(scratch)};
     hipError_t e;
     switch (M) {
         case 1: e = lanczos_go<1>(a, st); break;
