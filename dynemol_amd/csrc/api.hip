@@ -1847,15 +1847,21 @@ struct StepsScratch {
     int take(dh_system* s, int n_steps, size_t geo_n) {
         const size_t R = 2 * (size_t)s->W, ld = s->ld, n = n_steps;
         const size_t doubles = 2 * n * R + n * s->W * (s->n_frag + 1) + n * s->W * 2 + geo_n;
-        const size_t extra = steps_outputs_bytes(s) ? steps_outputs_bytes(s) + steps_slices_bytes(s) : 0;
-        const size_t bytes = sizeof(cplx) * ld * (R + 3 * s->W) + extra + sizeof(double) * doubles;
-        if (bytes > s->steps_bytes) {
+        const size_t must = sizeof(cplx) * ld * (R + 3 * s->W) + sizeof(double) * doubles;
+        size_t extra = 0;
+        if (n_steps > 1 && s->steps_per_series != 1 && steps_outputs_bytes(s))
+            extra = steps_outputs_bytes(s) + steps_slices_bytes(s);
+        if (must + extra > s->steps_bytes) {
             DH_HIP(hipStreamSynchronize(s->ctx->stream));
             if (s->steps_mem) hipFree(s->steps_mem);
             s->steps_mem = nullptr;
             s->steps_bytes = 0;
-            DALLOC(s->steps_mem, bytes);
-            s->steps_bytes = bytes;
+            if (extra && dalloc(&s->steps_mem, must + extra)) {  // without them the outputs go step by step
+                (void)hipGetLastError();
+                extra = 0;
+            }
+            if (!s->steps_mem) DALLOC(s->steps_mem, must);
+            s->steps_bytes = must + extra;
         }
         ck_phi = (cplx*)s->steps_mem;
         ck_out = ck_phi + ld * R;
