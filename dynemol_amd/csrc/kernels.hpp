@@ -38,8 +38,8 @@ __host__ __device__ inline double huckel_x(double ipa, double ipb, double kwa, d
     return keff * c2 * 0.5 + c4;
 }
 
-// scratch: 256 bytes and 4 n_atoms (n_atoms - 1) more (an ld x ld matrix of
-// doubles holds that: ld >= 64 and ld >= n_atoms)
+// scratch: 256 bytes and 4 N (N - 1) more, the pairs of atoms with orbitals (an
+// ld x ld matrix of doubles holds that: ld >= 64 and ld >= N)
 int launch_build_SH(const BasisDev& b, int N, int ld, double* S, double* h, double cutoff, double s_drop, void* scratch,
                     hipStream_t st);
 

@@ -219,7 +219,9 @@ __global__ void init_SH_kernel(double* S, double* h, int N, int ld, const double
 
 // Pairs (ia > ib) within the cutoff, in about basis-signature order: the lanes of
 // a wave of the next kernel then share one element pair for the most part, and
-// none is idle for its distance.
+// none is idle for its distance.  Atoms without orbitals have no block, and at
+// most N atoms have orbitals, so the list holds at most N (N - 1) / 2 pairs
+// whatever n_atoms is.
 __global__ __launch_bounds__(256) void pair_list_kernel(const BasisDev b, double cutoff, int* count, int2* list) {
     const long npair = (long)b.n_atoms * (b.n_atoms - 1) / 2;
     const long q = blockIdx.x * 256L + threadIdx.x;
@@ -234,7 +236,7 @@ __global__ __launch_bounds__(256) void pair_list_kernel(const BasisDev b, double
         const int ap = b.atom_order[p], ar = b.atom_order[r];
         const double x = b.coords[3 * ap] - b.coords[3 * ar], y = b.coords[3 * ap + 1] - b.coords[3 * ar + 1],
                      z = b.coords[3 * ap + 2] - b.coords[3 * ar + 2];
-        near = !(sqrt(x * x + y * y + z * z) > cutoff);
+        near = b.atom_nshell[ap] > 0 && b.atom_nshell[ar] > 0 && !(sqrt(x * x + y * y + z * z) > cutoff);
         pr = make_int2(ap, ar);
     }
     const unsigned long long mask = __ballot(near);
@@ -341,7 +343,7 @@ __global__ __launch_bounds__(64, 3) void build_SH_kernel(const BasisDev b, const
     }
 }
 
-// scratch: a counter, then up to n_atoms (n_atoms - 1) / 2 pairs (8 bytes each)
+// scratch: a counter, then up to N (N - 1) / 2 pairs (8 bytes each)
 int launch_build_SH(const BasisDev& b, int N, int ld, double* S, double* h, double cutoff, double s_drop, void* scratch,
                     hipStream_t st) {
     int* const count = static_cast<int*>(scratch);
