@@ -85,6 +85,9 @@ template <int LA, int LB>
 __device__ __forceinline__ void lined_up(int na, double za, int nb, double zb, double R, double cc, int sub,
                                          double* acc) {
     constexpr int MS = LA < LB ? LA : LB;
+    // Two centres at one point: the limit R -> 0 is finite, and at 1e-20 the
+    // powers of 1 / p (up to the tenth) and of R still have room in the exponent
+    if (R < 1e-20) R = 1e-20;
     const double hr = 0.5 * R, p = (za + zb) * hr, t = (za - zb) * hr, at = fabs(t);
     const double sg = t < 0.0 ? -1.0 : 1.0;  // exp(-t eta) is largest at eta = -sg
     const double pinv = 1.0 / p, low = fmin(za, zb) * R;  // p - |t|
