@@ -72,6 +72,12 @@ __device__ __forceinline__ double rs_dpp(double v) {
     const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
     return __hiloint2double(hi, lo);
 }
+// z + c t with the fused operations spelt out: left to the compiler, the choice of
+// the product that is fused differed between instances (NT = 32 from the others),
+// and a batch member's last bits with it
+__device__ __forceinline__ cplx rs_cfma(cplx c, cplx t, cplx z) {
+    return cplx{fma(-c.im, t.im, fma(c.re, t.re, z.re)), fma(c.im, t.re, fma(c.re, t.im, z.im))};
+}
 // sum over the four blocks (lanes 4 apart of a row of 16)
 __device__ __forceinline__ double rs_block_sum(double v) {
     const double z = v + rs_dpp<0x128>(v);  // row rotate 8
@@ -88,10 +94,19 @@ __device__ __forceinline__ void rs_lds_barrier() { asm volatile("s_waitcnt lgkmc
 // per lane, no block sums; measured 64 cycles per 1024 products where the 4x4x4
 // form takes 80 to 88), or with 8 rows (RG = 2) two sets of 4 complex columns.
 // NT: the most groups per wave, a compile-time count so that the loads of x run
-// ahead of the products through the whole unrolled sequence (groups past the
-// system's own count are zero, so the sums do not depend on NT).  blk of nblk:
-// this workgroup's place in its system.
+// ahead of the products through the whole unrolled sequence.  Groups past the
+// system's own count are zero, and the order of the others (rs_first) and every
+// rounding of the term are the same for each NT, so a batch member's bits do not
+// depend on the larger members that share its launch.  (batch of 64 systems of N
+// 256-2048, 4 wavepackets: 133 ms with an order of its own per NT, 135 so.)  blk of
+// nblk: this workgroup's place in its system.
 constexpr int rs_most(int rc) { return rc == 0 ? 24 : rc == 1 ? 23 : 22; }
+constexpr int rs_max_groups(int rc) { return rc == 2 ? 30 : 32; }
+// A term takes the register groups 0 .. most - 1 in order, and LDS group most + l
+// after register group first + l, whose products cover its LDS reads.  first is
+// that of the largest NT: with fewer LDS groups the interleaved part ends earlier,
+// and a count that fits the registers has none.
+constexpr int rs_first(int rc) { return 2 * rs_most(rc) - rs_max_groups(rc); }
 // Groups of x in flight per wave: the loads of a term are bound by their
 // latency, so as many as the registers beside H hold.  Up to 8 groups of a
 // WIDE kernel this leaves room for three waves per SIMD.
@@ -235,7 +250,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
             const cplx c0 = rs_coef(a.coef + (long)(w + NW * v) * a.coef_stride);
 #pragma unroll
             for (int u = 0; u < NE; ++u)
-                if (lane + 64 * u < E) acc[v][u] = cmul(c0, ts[lane + 64 * u]);
+                if (lane + 64 * u < E) acc[v][u] = rs_cfma(c0, ts[lane + 64 * u], cplx{0.0, 0.0});
         }
 
     // flags of the rows this wave reads
@@ -304,11 +319,10 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
                     }
                 }
             };
-            // step s takes register group s, and LDS group NREG + l after register
-            // group NREG - NL + l, whose products cover its LDS reads
-            constexpr int RONLY = NREG - NL;
-            auto group = [](int st) {
-                return st < RONLY ? st : (st - RONLY) % 2 == 0 ? RONLY + (st - RONLY) / 2 : NREG + (st - RONLY) / 2;
+            constexpr int FIRST = NL > 0 ? rs_first(RC) : NT;
+            auto group = [](int st) {  // of step st
+                return st < FIRST ? st : st >= FIRST + 2 * NL ? st - NL
+                       : (st - FIRST) % 2 == 0 ? FIRST + (st - FIRST) / 2 : NREG + (st - FIRST) / 2;
             };
             xv_t xb[DEPTH][XL];
             unsigned long long t0 = 0;
@@ -340,9 +354,9 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
 #pragma unroll
             for (int st = 0; st < NT; ++st) {
                 const int g = group(st);
-                if (g < NREG && st >= RONLY && NL > 0) {
+                if (st >= FIRST && st < FIRST + 2 * NL && (st - FIRST) % 2 == 0) {
 #pragma unroll
-                    for (int rg = 0; rg < RG; ++rg) hl[rg] = hs[(((st - RONLY) / 2 * NW + w) * RG + rg) * 64 + lane];
+                    for (int rg = 0; rg < RG; ++rg) hl[rg] = hs[(((st - FIRST) / 2 * NW + w) * RG + rg) * 64 + lane];
                 }
 #pragma unroll
                 for (int p = 0; p < XL; ++p) {
@@ -406,7 +420,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
                     y.im += pp[ww * RB * PC].im;
                 }
                 const cplx xv = t1[e];
-                cplx T{alpha * y.re + beta * xv.re, alpha * y.im + beta * xv.im};
+                cplx T{fma(alpha, y.re, beta * xv.re), fma(alpha, y.im, beta * xv.im)};
                 if (k > 1) {
                     const cplx x2 = t2[e];
                     T.re -= x2.re;
@@ -423,11 +437,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
             if (k <= kq[v]) {
 #pragma unroll
                 for (int u = 0; u < NE; ++u)
-                    if (lane + 64 * u < E) {
-                        const cplx add = cmul(ck[v], tk[lane + 64 * u]);
-                        acc[v][u].re += add.re;
-                        acc[v][u].im += add.im;
-                    }
+                    if (lane + 64 * u < E) acc[v][u] = rs_cfma(ck[v], tk[lane + 64 * u], acc[v][u]);
             }
     }
     // a wave that gave up waiting marks its workgroup's result
