@@ -6,7 +6,6 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
-#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -157,6 +156,7 @@ struct dh_system {
     } graphs[2];
     int next_graph = 0;
     bool use_graph = true;
+    bool one_launch_bounds = true;  // dh_set_one_launch_bounds
     bool tuned = false;
     // 0 = FP64; 1 = mixed (FP32 MFMA term GEMM); 2 = FP32-stored H_orth with
     // FP64 products and sums
@@ -227,24 +227,17 @@ static int round_ld(int N) { return ((N + TILE - 1) / TILE) * TILE; }
 extern "C" const char* dh_last_error(void) { return dh::last_error(); }
 extern "C" int dh_version(void) { return 100; }
 
-// Contexts alive in this process.  The Lanczos recurrence is launched
-// cooperatively only while there is one: builds are where threads that drive
-// their own contexts meet first, and a traced run of two such threads, both
-// with a cooperative launch in their builds, did not come back (the kernel's own
-// waits are bounded; the cause was not found).
-static std::atomic<int> g_contexts{0};
+static CoopOwner coop_owner(const dh_context* c) { return CoopOwner{c, c->device, c->cus}; }
 
 __global__ void first_cooperative_kernel() {}
 
-// The runtime sets up its queue for cooperative launches at the first one: done
-// here, one thread at a time, and not by whichever threads come first.
-static void first_cooperative_launch(hipStream_t st) {
-    static std::mutex mu;
-    std::lock_guard<std::mutex> lk(mu);
+// The runtime sets up its queue for cooperative launches at the first one (5 ms):
+// done here and not in the first step.
+static void first_cooperative_launch(const dh_context* c) {
     void* params[] = {nullptr};
-    if (hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&first_cooperative_kernel), dim3(1), dim3(64), params,
-                                   0, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
+    if (coop_launch(coop_owner(c), reinterpret_cast<const void*>(&first_cooperative_kernel), dim3(1), dim3(64), params, 0,
+                    c->stream) != hipSuccess ||
+        hipStreamSynchronize(c->stream) != hipSuccess)
         (void)hipGetLastError();
 }
 
@@ -267,8 +260,7 @@ extern "C" int dh_init(int device, dh_context** out) {
         delete c;
         return DH_ERR_NOMEM;
     }
-    if (c->cus) first_cooperative_launch(c->stream);
-    g_contexts.fetch_add(1);
+    if (c->cus) first_cooperative_launch(c);
     *out = c;
     return DH_OK;
 }
@@ -361,7 +353,7 @@ extern "C" int dh_finalize(dh_context* c) {
     hipFree(c->d_info);
     if (c->side) hipStreamDestroy(c->side);
     hipStreamDestroy(c->stream);
-    g_contexts.fetch_sub(1);
+    coop_forget(coop_owner(c));
     delete c;
     return DH_OK;
 }
@@ -653,13 +645,13 @@ static int lanczos_count(const dh_system* s) { return std::min(s->lanczos_steps,
 
 // The Lanczos recurrence on t.Hth, its coefficients to t.lal and t.lbe: in one
 // launch where that fits (the exchange goes through t.Dinv, free by now), else,
-// and always with one_launch off, step by step.
+// and always with one_launch or the system's switch off, step by step.
 static int lanczos_into(dh_system* s, const OpsTarget& t, bool one_launch) {
     hipStream_t st = t.st;
     const int m = lanczos_count(s);
-    if (one_launch && !matvec_forced() && g_contexts.load() == 1 &&
+    if (one_launch && s->one_launch_bounds && !matvec_forced() &&
         launch_lanczos_resident(t.Hth, s->ld, s->N, m, LANCZOS_SEED, t.lal, t.lbe, t.Dinv,
-                                (long)sizeof(double) * s->ld * TILE, s->ctx->cus, st))
+                                (long)sizeof(double) * s->ld * TILE, coop_owner(s->ctx), st))
         return DH_OK;
     launch_lanczos_start(s->N, t.lv, t.lvp, LANCZOS_SEED, st);
     MatvecArgs a{};
@@ -1163,9 +1155,9 @@ struct SeriesOps {
     const int* Kq = nullptr;  // the same table on the host
     cplx* ring = nullptr;
     long ring_stride = 0;
-    // > 0: the series may run in one launch with H resident on that many compute
-    // units (series.hip), its exchange ring in `partial` (partial_cplx elements)
-    int cus = 0;
+    // coop.cus > 0: the series may run in one launch with H resident on that many
+    // compute units (series.hip), its exchange ring in `partial` (partial_cplx elements)
+    CoopOwner coop;
     long partial_cplx = 0;
 };
 
@@ -1178,7 +1170,7 @@ static bool series_resident(const dh_context* c, int prec, int ld, int R) {
 static int series_core(const SeriesOps& o, hipStream_t st) {
     const int R = o.R;
     const double c = o.c, r = o.r;
-    if (o.cus > 0) {
+    if (o.coop.cus > 0) {
         ResidentArgs ra{};
         ra.H = o.H;
         ra.ld = o.ld;
@@ -1194,7 +1186,7 @@ static int series_core(const SeriesOps& o, hipStream_t st) {
         ra.coef = o.m > 0 ? o.coefm : o.coef;
         ra.coef_stride = o.coefm_stride;
         ra.kq = o.m > 0 ? o.kq : nullptr;
-        if (launch_resident_series(ra, o.partial, o.partial_cplx * (long)sizeof(cplx), o.cus, st)) return DH_OK;
+        if (launch_resident_series(ra, o.partial, o.partial_cplx * (long)sizeof(cplx), o.coop, st)) return DH_OK;
     }
     MatvecArgs a{};
     a.M = o.H;
@@ -1314,7 +1306,7 @@ static int series_core(const SeriesOps& o, hipStream_t st) {
 static int series_launches(dh_system* s, bool one_launch = true) {
     SeriesOps o{};
     o.partial_cplx = partial_cplx_for(s->N, s->W);
-    if (one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) o.cus = s->ctx->cus;
+    if (one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) o.coop = coop_owner(s->ctx);
     o.H = s->Hth;
     o.H32 = s->H32;
     o.Hlo = s->Hlo;
@@ -1826,7 +1818,7 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     o.ring_stride = acc_n;
     o.K = Kq[m - 1];
     o.partial_cplx = partial_cplx_for(s->N, s->W);
-    if (series_resident(s->ctx, s->precision, s->ld, R)) o.cus = s->ctx->cus;
+    if (series_resident(s->ctx, s->precision, s->ld, R)) o.coop = coop_owner(s->ctx);
     if (int rc = series_core(o, st)) return rc;
     DH_HIP(hipGetLastError());
     *kmax = Kq[m - 1];
@@ -2092,6 +2084,12 @@ extern "C" int dh_set_graph(dh_system* s, int on) {
     return DH_OK;
 }
 
+extern "C" int dh_set_one_launch_bounds(dh_system* s, int on) {
+    CHECK_ARG(s, "dh_set_one_launch_bounds: null system");
+    s->one_launch_bounds = on != 0;
+    return DH_OK;
+}
+
 extern "C" int dh_get_stats(dh_system* s, double* out9) {
     CHECK_ARG(s && out9, "dh_get_stats: null argument");
     for (int i = 0; i < 9; ++i) out9[i] = s->stats[i];
@@ -2239,7 +2237,7 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
         o.K = K;
         o.c = c;
         o.r = r;
-        o.cus = one_launch && attempt == 0 ? ctx->cus : 0;
+        o.coop = one_launch && attempt == 0 ? coop_owner(ctx) : CoopOwner{};
         if (int rc = series_core(o, st)) return rc;
         launch_column_norms(N, R, w.acc, w.norms1, st);
         DH_HIP(hipGetLastError());
@@ -2699,7 +2697,8 @@ static int batch_solo_series(dh_batch* b) {
     for (int i = 0; i < b->n; ++i)
         if (b->solo[i] == 1)
             if (int rc = series_launches(b->sys[i])) return rc;
-    if (launch_resident_rounds(b->d_res, (int)b->h_res.size(), b->d_map, b->rounds, b->ctx->stream)) return DH_ERR_HIP;
+    if (launch_resident_rounds(b->d_res, (int)b->h_res.size(), b->d_map, b->rounds, coop_owner(b->ctx), b->ctx->stream))
+        return DH_ERR_HIP;
     return DH_OK;
 }
 

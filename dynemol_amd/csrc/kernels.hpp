@@ -268,9 +268,6 @@ void launch_lanczos_step(int N, cplx* v, cplx* vprev, const cplx* w, double* alp
                          hipStream_t st);
 // extreme-eigenvalue bounds of the Lanczos tridiagonal (al[0..m-1], be[1..m]),
 // on the host: bounds = [emin, emax, theta_min, theta_max, res_min, res_max]
-// the whole recurrence in one launch (lanczos.hip); false: not launched
-bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned seed, double* alpha, double* beta,
-                             void* scratch, long scratch_bytes, int cus, hipStream_t st);
 void lanczos_bounds_host(const double* al, const double* be, int m, double rel_margin, double* bounds);
 int bessel_coef_host(double x, double phase, int kmax_alloc, double tol, cplx* coef);
 void launch_bessel(double x, double phase, int kmax_alloc, double tol, cplx* coef, int* out_k,
@@ -287,6 +284,26 @@ void launch_to_bf16(const float* a, unsigned short* b, long n, hipStream_t st);
 void launch_lib_reduce(const MatvecArgs& a, const float* Phi, const float* Plo, int S, hipStream_t st);
 void launch_identity_pad(double* S, double* h, int N, int ld, hipStream_t st);
 
+
+// ---------------------------------------------------------------- cooperative launches (series.hip)
+// Whose launch it is, on which device, and how many compute units a cooperative
+// launch can fill there (0: none).
+struct CoopOwner {
+    const void* owner = nullptr;
+    int device = 0;
+    int cus = 0;
+};
+// A cooperative launch on a stream of the owner's.  Launches of different owners
+// (contexts, which threads of their own may drive) take turns: one is made only
+// when no other owner's is in flight on the device.
+hipError_t coop_launch(const CoopOwner& who, const void* f, dim3 grid, dim3 block, void** params, unsigned lds,
+                       hipStream_t st);
+// an owner that goes away (its streams have drained)
+void coop_forget(const CoopOwner& who);
+
+// the whole Lanczos recurrence in one launch (lanczos.hip); false: not launched
+bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned seed, double* alpha, double* beta,
+                             void* scratch, long scratch_bytes, const CoopOwner& who, hipStream_t st);
 
 // ---------------------------------------------------------------- resident series (series.hip)
 // A whole Chebyshev series (one launch, H resident on the chip): accumulator q
@@ -310,7 +327,7 @@ struct ResidentArgs {
 };
 bool resident_series_fits(int ld, int R, int cus);
 // false: not launched (shape, scratch or device do not allow it)
-bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, int cus, hipStream_t st);
+bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, const CoopOwner& who, hipStream_t st);
 // Batches: whether a member can run so (fills in the launcher's fields), the
 // launches that cover the members (map: workgroup -> member, its workgroup
 // there), and the launches themselves with both tables on the device.
@@ -322,7 +339,7 @@ bool resident_batch_member(ResidentArgs* a, void* scratch, long scratch_bytes, i
 bool resident_batch_rounds(const std::vector<ResidentArgs>& members, int cus, std::vector<int2>* map,
                            std::vector<ResidentRound>* rounds);
 int launch_resident_rounds(const ResidentArgs* d_members, int n, const int2* d_map,
-                           const std::vector<ResidentRound>& rounds, hipStream_t st);
+                           const std::vector<ResidentRound>& rounds, const CoopOwner& who, hipStream_t st);
 
 // Small grouped helpers for multi-system batches.
 struct NormTask {

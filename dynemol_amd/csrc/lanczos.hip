@@ -14,8 +14,8 @@
 // workgroup-wide sums: 126 us for the 48 steps at N = 514, 172 at 2078, 347 at
 // 4096 (201, 234 and 512 with one flag per workgroup and step).
 //
-// All workgroups must be on the chip at once, so the launch is cooperative, and
-// every wait is bounded (wall clock): a wave that runs out of time goes on with
+// All workgroups must be on the chip at once, so the launch is cooperative
+// (coop_launch), and every wait is bounded (wall clock): a wave that runs out of time goes on with
 // NaN, which reaches the coefficients; the caller then runs step by step.
 #include "common.hpp"
 #include "kernels.hpp"
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256) void lanczos_clear_kernel(unsigned* ring, long
 }
 
 template <int M>
-static hipError_t lanczos_go(LanczosArgs a, hipStream_t st) {
+static hipError_t lanczos_go(LanczosArgs a, const CoopOwner& who, hipStream_t st) {
     constexpr int RW = M == 1 ? 2 : M == 2 ? 4 : M <= 4 ? 8 : 16;
     const unsigned lds = M >= 6 ? 4 * M * 512 * 8 : 0;
     const void* f = reinterpret_cast<const void*>(&lanczos_resident_kernel<M>);
@@ -251,28 +251,28 @@ static hipError_t lanczos_go(LanczosArgs a, hipStream_t st) {
     hipLaunchKernelGGL(lanczos_clear_kernel, dim3((unsigned)std::min(512L, (words + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<unsigned*>(a.ring), words);
     void* params[] = {&a};
-    return hipLaunchCooperativeKernel(f, dim3(wgs), dim3(512), params, lds, st);
+    return coop_launch(who, f, dim3(wgs), dim3(512), params, lds, st);
 }
 
 // m steps into alpha[0..m-1], beta[1..m]; false (nothing launched that the caller
 // must wait for) where the operator does not fit the chip, the device has fewer
 // CUs, the scratch does not hold a vector per step, or the launch is refused
 bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned seed, double* alpha, double* beta,
-                             void* scratch, long scratch_bytes, int cus, hipStream_t st) {
+                             void* scratch, long scratch_bytes, const CoopOwner& who, hipStream_t st) {
     const int M = (ld + 511) / 512, RW = M == 1 ? 2 : M == 2 ? 4 : M <= 4 ? 8 : 16;
-    if (M > 8 || (N + RW - 1) / RW > cus) return false;
+    if (M > 8 || (N + RW - 1) / RW > who.cus) return false;
     if (8L * m * ld > scratch_bytes) return false;
     LanczosArgs a{H, ld, N, m, seed, alpha, beta, static_cast<double*>(scratch)};
     hipError_t e;
     switch (M) {
-        case 1: e = lanczos_go<1>(a, st); break;
-        case 2: e = lanczos_go<2>(a, st); break;
-        case 3: e = lanczos_go<3>(a, st); break;
-        case 4: e = lanczos_go<4>(a, st); break;
-        case 5: e = lanczos_go<5>(a, st); break;
-        case 6: e = lanczos_go<6>(a, st); break;
-        case 7: e = lanczos_go<7>(a, st); break;
-        default: e = lanczos_go<8>(a, st); break;
+        case 1: e = lanczos_go<1>(a, who, st); break;
+        case 2: e = lanczos_go<2>(a, who, st); break;
+        case 3: e = lanczos_go<3>(a, who, st); break;
+        case 4: e = lanczos_go<4>(a, who, st); break;
+        case 5: e = lanczos_go<5>(a, who, st); break;
+        case 6: e = lanczos_go<6>(a, who, st); break;
+        case 7: e = lanczos_go<7>(a, who, st); break;
+        default: e = lanczos_go<8>(a, who, st); break;
     }
     if (e != hipSuccess) (void)hipGetLastError();
     return e == hipSuccess;

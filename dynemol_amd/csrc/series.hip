@@ -19,8 +19,54 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <mutex>
 
 namespace dh {
+
+// ------------------------------------------------------------------ cooperative launches
+// One turnstile per device.  A kernel of this kind needs all its workgroups on the
+// chip at once, so two of them gain nothing from overlapping, and two that held
+// part of the chip each would wait for one another until their waits ran out.
+// The lock is held over the launch, so that no two threads are ever inside the
+// runtime's cooperative launch (nor in its first-use set-up) at the same time, and
+// over the wait for another owner's last launch to end; launches of one owner,
+// which one thread makes, are ordered by the runtime.
+namespace {
+struct Turnstile {
+    std::mutex mu;
+    hipEvent_t done = nullptr;  // after the last launch
+    const void* owner = nullptr;  // whose that was; null: none in flight
+};
+constexpr int MAX_DEVICES = 64;
+Turnstile g_turnstile[MAX_DEVICES];
+}  // namespace
+
+hipError_t coop_launch(const CoopOwner& who, const void* f, dim3 grid, dim3 block, void** params, unsigned lds,
+                       hipStream_t st) {
+    if (who.cus <= 0 || who.device < 0 || who.device >= MAX_DEVICES) return hipErrorNotSupported;
+    Turnstile& t = g_turnstile[who.device];
+    std::lock_guard<std::mutex> lk(t.mu);
+    if (!t.done)
+        if (hipError_t e = hipEventCreateWithFlags(&t.done, hipEventDisableTiming); e != hipSuccess) return e;
+    if (t.owner && t.owner != who.owner)
+        if (hipError_t e = hipEventSynchronize(t.done); e != hipSuccess) return e;
+    if (hipError_t e = hipLaunchCooperativeKernel(f, grid, block, params, lds, st); e != hipSuccess) return e;
+    t.owner = who.owner;
+    // launched: whatever becomes of the record, the caller must not launch again
+    if (hipEventRecord(t.done, st) != hipSuccess) {
+        (void)hipGetLastError();
+        if (hipStreamSynchronize(st) != hipSuccess) (void)hipGetLastError();
+        t.owner = nullptr;
+    }
+    return hipSuccess;
+}
+
+void coop_forget(const CoopOwner& who) {
+    if (who.device < 0 || who.device >= MAX_DEVICES) return;
+    Turnstile& t = g_turnstile[who.device];
+    std::lock_guard<std::mutex> lk(t.mu);
+    if (t.owner == who.owner) t.owner = nullptr;
+}
 
 // Work split: workgroup b owns RB = 4 RG consecutive rows; its NW waves split
 // the columns (the reduction index) into NW ranges of `groups` 16-column groups.
@@ -45,8 +91,8 @@ namespace dh {
 // A slot is overwritten `slots` terms later: a workgroup that writes T_{k+1}
 // has seen every flag of term k, so every wave is past reading T_{k-1}.
 //
-// All workgroups must be on the chip at once, so the launch is cooperative,
-// and every wait is bounded (wall clock): a wave that runs out of time stops
+// All workgroups must be on the chip at once, so the launch is cooperative
+// (coop_launch), and every wait is bounded (wall clock): a wave that runs out of time stops
 // waiting for good, the kernel drains, and its workgroup's accumulators are
 // written as NaN, which the caller's norm check turns into a repeat of the
 // step with one launch per term.
@@ -531,29 +577,29 @@ static long resident_slot_bytes(int ld, int R) { return (long)ld * (R <= 2 ? 32 
 static long resident_flag_bytes(int ld) { return (long)RS_COPIES * (ld / 4) * 4; }
 
 template <int RG, int NT, int RC>
-static hipError_t resident_go(const ResidentArgs& a, const ResidentPlan& p, hipStream_t st) {
+static hipError_t resident_go(const ResidentArgs& a, const ResidentPlan& p, const CoopOwner& who, hipStream_t st) {
     const void* f = reinterpret_cast<const void*>(&resident_series_kernel<8, RG, NT, RC>);
     hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, p.lds);
     if (e != hipSuccess) return e;
     ResidentArgs arg = a;
     void* params[] = {&arg};
-    return hipLaunchCooperativeKernel(f, dim3(p.wgs), dim3(512), params, (unsigned)p.lds, st);
+    return coop_launch(who, f, dim3(p.wgs), dim3(512), params, (unsigned)p.lds, st);
 }
 
 // the kernel of p.NT among LO, LO + STEP, ..., HI
 template <int RG, int RC, int LO, int HI, int STEP>
-static hipError_t resident_pick(const ResidentArgs& a, const ResidentPlan& p, hipStream_t st) {
-    if (p.NT == LO) return resident_go<RG, LO, RC>(a, p, st);
-    if constexpr (LO + STEP <= HI) return resident_pick<RG, RC, LO + STEP, HI, STEP>(a, p, st);
+static hipError_t resident_pick(const ResidentArgs& a, const ResidentPlan& p, const CoopOwner& who, hipStream_t st) {
+    if (p.NT == LO) return resident_go<RG, LO, RC>(a, p, who, st);
+    if constexpr (LO + STEP <= HI) return resident_pick<RG, RC, LO + STEP, HI, STEP>(a, p, who, st);
     return hipErrorInvalidValue;
 }
 
-static hipError_t resident_launch(const ResidentArgs& a, const ResidentPlan& p, hipStream_t st) {
+static hipError_t resident_launch(const ResidentArgs& a, const ResidentPlan& p, const CoopOwner& who, hipStream_t st) {
     const bool few = p.NT <= 8;
-    if (p.RC == 0) return few ? resident_pick<4, 0, 1, 8, 1>(a, p, st) : resident_pick<4, 0, 10, 32, 2>(a, p, st);
-    if (p.RC == 1) return few ? resident_pick<4, 1, 1, 8, 1>(a, p, st) : resident_pick<4, 1, 10, 32, 2>(a, p, st);
-    if (p.RG == 2) return few ? resident_pick<2, 2, 1, 8, 1>(a, p, st) : resident_pick<2, 2, 10, 16, 2>(a, p, st);
-    return resident_pick<4, 2, 18, 30, 2>(a, p, st);
+    if (p.RC == 0) return few ? resident_pick<4, 0, 1, 8, 1>(a, p, who, st) : resident_pick<4, 0, 10, 32, 2>(a, p, who, st);
+    if (p.RC == 1) return few ? resident_pick<4, 1, 1, 8, 1>(a, p, who, st) : resident_pick<4, 1, 10, 32, 2>(a, p, who, st);
+    if (p.RG == 2) return few ? resident_pick<2, 2, 1, 8, 1>(a, p, who, st) : resident_pick<2, 2, 10, 16, 2>(a, p, who, st);
+    return resident_pick<4, 2, 18, 30, 2>(a, p, who, st);
 }
 
 // scratch: flags, then as many ring slots as fit (at least 4)
@@ -568,12 +614,12 @@ static bool resident_scratch(ResidentArgs* a, void* scratch, long scratch_bytes)
     return true;
 }
 
-bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, int cus, hipStream_t st) {
-    const ResidentPlan p = resident_plan(a.ld, a.R, cus);
+bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, const CoopOwner& who, hipStream_t st) {
+    const ResidentPlan p = resident_plan(a.ld, a.R, who.cus);
     if (!p.ok || !resident_scratch(&a, scratch, scratch_bytes)) return false;
     a.groups = p.groups;
     hipLaunchKernelGGL(resident_clear_kernel, dim3(32), dim3(256), 0, st, a);
-    const hipError_t e = resident_launch(a, p, st);
+    const hipError_t e = resident_launch(a, p, who, st);
     if (e == hipSuccess) return true;
     (void)hipGetLastError();  // not launched: the caller runs the series term by term
     return false;
@@ -684,13 +730,13 @@ bool resident_batch_rounds(const std::vector<ResidentArgs>& members, int cus, st
 }
 
 int launch_resident_rounds(const ResidentArgs* d_members, int n, const int2* d_map,
-                           const std::vector<ResidentRound>& rounds, hipStream_t st) {
+                           const std::vector<ResidentRound>& rounds, const CoopOwner& who, hipStream_t st) {
     if (n <= 0) return 0;
     hipLaunchKernelGGL(resident_clear_grouped_kernel, dim3(n, 8), dim3(256), 0, st, d_members);
     for (const ResidentRound& r : rounds) {
         const int2* map = d_map + r.first;
         void* params[] = {&d_members, &map};
-        const hipError_t e = hipLaunchCooperativeKernel(r.f, dim3(r.wgs), dim3(r.threads), params, (unsigned)r.lds, st);
+        const hipError_t e = coop_launch(who, r.f, dim3(r.wgs), dim3(r.threads), params, (unsigned)r.lds, st);
         if (e != hipSuccess) {
             set_error("resident batch series: %s", hipGetErrorString(e));
             return -1;

@@ -37,7 +37,7 @@ SYMBOLS = [
     "dh_propagation_elhl", "dh_batch_create", "dh_batch_destroy", "dh_batch_propagate", "dh_batch_propagate_steps", "dh_set_initial_state",
     "dh_set_graph", "dh_ehrenfest_kernel", "dh_eigenpairs", "dh_set_eigenstate", "dh_batch_set_graph",
     "dh_chebyshev_work_bytes", "dh_chebyshev_apply", "dh_chebyshev_apply_noalloc", "dh_propagate_steps",
-    "dh_batch_tuning",
+    "dh_batch_tuning", "dh_set_one_launch_bounds",
 ]
 TEST_SYMBOLS = ["dh_test_gemm", "dh_test_cholesky", "dh_test_copy", "dh_test_force_matvec_variant",
                 "dh_test_matvec_timing", "dh_test_read", "dh_test_device_alloc", "dh_test_device_free",
@@ -109,6 +109,7 @@ def lib():
     L.dh_set_timing.argtypes = [_vp, ctypes.c_int]
     L.dh_set_steps_per_series.argtypes = [_vp, ctypes.c_int]
     L.dh_set_graph.argtypes = [_vp, ctypes.c_int]
+    L.dh_set_one_launch_bounds.argtypes = [_vp, ctypes.c_int]
     L.dh_matvec_tuning.argtypes = [_vp, _i]
     L.dh_set_precision.argtypes = [_vp, ctypes.c_int]
     L.dh_set_initial_state.argtypes = [_vp, ctypes.c_int, _d, _d]
@@ -369,6 +370,11 @@ class System:
     def set_graph(self, on=True):
         """Term series as one captured hipGraph per step (default) or as separate launches."""
         _check(lib().dh_set_graph(self.h, 1 if on else 0), "dh_set_graph")
+
+    def set_one_launch_bounds(self, on=True):
+        """Lanczos recurrence of the builds in one launch (default) or step by step (for contexts driven
+        from several threads at once)."""
+        _check(lib().dh_set_one_launch_bounds(self.h, 1 if on else 0), "dh_set_one_launch_bounds")
 
 
 def run_gemm(A, B, C, alpha=1.0, beta=0.0, transA=0, transB=0, kmode=0, lower_only=0):

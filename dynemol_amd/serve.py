@@ -96,8 +96,9 @@ class _Lane:
         w = padded_wp(len(req.psi_ket))
         s = hip.System(self.ctx, req.basis, n_wp=w, n_frag=req.n_frag)
         # lanes run concurrently: no stream capture, which must not overlap the
-        # other lanes' allocations and frees
+        # other lanes' allocations and frees, and bounds step by step
         s.set_graph(False)
+        s.set_one_launch_bounds(False)
         if req.mixed:
             s.set_precision(hip.DH_PREC_MIXED_CORRECTED)
         s.build(req.coords)

@@ -12,7 +12,10 @@
  * Several contexts may be driven from several host threads at once; the
  * term series' stream capture (dh_set_graph, dh_batch_set_graph; on by
  * default for N <= 2048) must then be off, since a capture must not overlap
- * another thread's device allocations and frees.
+ * another thread's device allocations and frees.  Turn the one-launch form of
+ * the spectral bounds off too (dh_set_one_launch_bounds).  Series that run in
+ * one launch (dh_set_steps_per_series) need no such care: those of different
+ * contexts on a device take turns.
  */
 #ifndef DYNEMOL_HIP_H
 #define DYNEMOL_HIP_H
@@ -218,6 +221,14 @@ int dh_set_steps_per_series(dh_system *sys, int m);
  * series that runs in one launch (dh_set_steps_per_series) uses neither.  No
  * counterpart in the reference (one cuBLAS call per term, Taylor_gpu.cpp:295-330). */
 int dh_set_graph(dh_system *sys, int on);
+/* Run the Lanczos recurrence for the spectral bounds in one launch with H_orth
+ * on the chip (on = 1, the default; up to 4096 orbitals) or step by step (on =
+ * 0).  The bounds differ in the last digits.  Off for systems of contexts that
+ * are driven from several threads at once: builds of two such threads with
+ * cooperative launches in both once did not come back under a kernel trace, for
+ * a reason that was not found.  No counterpart in the reference (its series
+ * needs no bounds). */
+int dh_set_one_launch_bounds(dh_system *sys, int on);
 /* Matvec kernel variant chosen by the autotuner for this system's shapes:
  * [Chebyshev term (2*n_wp RHS), <H> (n_wp), L phi_bra, L^-T phi, L^T ket,
  * L^-1 bra, Lanczos (1 RHS)].  No counterpart in the reference (its GEMV tile
