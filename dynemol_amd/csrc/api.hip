@@ -1159,6 +1159,7 @@ struct SeriesOps {
     // compute units (series.hip), its exchange ring in `partial` (partial_cplx elements)
     CoopOwner coop;
     long partial_cplx = 0;
+    bool* one_launch = nullptr;  // set to whether it ran in one launch
 };
 
 // whether a series of these operands runs in one launch (else one per term):
@@ -1170,6 +1171,7 @@ static bool series_resident(const dh_context* c, int prec, int ld, int R) {
 static int series_core(const SeriesOps& o, hipStream_t st) {
     const int R = o.R;
     const double c = o.c, r = o.r;
+    if (o.one_launch) *o.one_launch = false;
     if (o.coop.cus > 0) {
         ResidentArgs ra{};
         ra.H = o.H;
@@ -1186,7 +1188,10 @@ static int series_core(const SeriesOps& o, hipStream_t st) {
         ra.coef = o.m > 0 ? o.coefm : o.coef;
         ra.coef_stride = o.coefm_stride;
         ra.kq = o.m > 0 ? o.kq : nullptr;
-        if (launch_resident_series(ra, o.partial, o.partial_cplx * (long)sizeof(cplx), o.coop, st)) return DH_OK;
+        if (launch_resident_series(ra, o.partial, o.partial_cplx * (long)sizeof(cplx), o.coop, st)) {
+            if (o.one_launch) *o.one_launch = true;
+            return DH_OK;
+        }
     }
     MatvecArgs a{};
     a.M = o.H;
@@ -1303,10 +1308,13 @@ static int series_core(const SeriesOps& o, hipStream_t st) {
 }
 
 // One Chebyshev evaluation phi <- sum_k a_k T_k(Hh) phi, result in s->acc.
-static int series_launches(dh_system* s, bool one_launch = true) {
+// one_launch: whether it may run in one launch, on return whether it did.
+static int series_launches(dh_system* s, bool* one_launch) {
     SeriesOps o{};
+    const bool may = *one_launch;
+    o.one_launch = one_launch;
     o.partial_cplx = partial_cplx_for(s->N, s->W);
-    if (one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) o.coop = coop_owner(s->ctx);
+    if (may && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) o.coop = coop_owner(s->ctx);
     o.H = s->Hth;
     o.H32 = s->H32;
     o.Hlo = s->Hlo;
@@ -1337,11 +1345,12 @@ static int series_launches(dh_system* s, bool one_launch = true) {
 // The term series as one hipGraph launch: captured once per (K, bounds, buffer
 // assignment, precision, term kernel) and replayed on later steps.  The series
 // is kernels only (no memset nodes, no host synchronisation).
-static int chebyshev_series(dh_system* s, bool one_launch = true) {
+static int chebyshev_series(dh_system* s, bool* one_launch) {
     // the FP32-product modes call rocBLAS, which stays out of stream capture; a
     // series in one launch has nothing to capture
     if (!s->use_graph || fp32_products(s)) return series_launches(s, one_launch);
-    if (one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) return series_launches(s);
+    if (*one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) return series_launches(s, one_launch);
+    *one_launch = false;
     hipStream_t st = s->ctx->stream;
     const int variant = matvec_variant_for(s->N, 2 * s->W, TRI_FULL);
     for (auto& g : s->graphs)
@@ -1357,7 +1366,7 @@ static int chebyshev_series(dh_system* s, bool one_launch = true) {
         g.exec = nullptr;
     }
     DH_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    const int rc = series_launches(s, false);
+    const int rc = series_launches(s, one_launch);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(st, &graph);
     if (rc) {
@@ -1479,13 +1488,16 @@ static int propagate_checked(dh_system* s, double dt, int* n_terms, bool one_lau
     // spectrum; the mixed mode's FP32 products drift ~1e-7 per step by themselves
     // (mode 2 propagates with the exactly symmetric FP32-rounded H: FP64 drift)
     const double drift_tol = fp32_products(s) ? 1e-4 : 1e-9;
-    for (int attempt = 0; attempt < 4; ++attempt) {
+    bool may = one_launch;
+    for (int attempt = 0; attempt < 4;) {
         int rc = ensure_coefficients(s, dt);
         if (rc) return rc;
         if (s->timing) DH_HIP(hipEventRecord(s->ev0, st));
         // a repeat runs one launch per term: it also covers a series in one launch
         // that gave up waiting (NaN norms)
-        rc = chebyshev_series(s, one_launch && attempt == 0);
+        bool whole = may;
+        may = false;
+        rc = chebyshev_series(s, &whole);
         if (rc) return rc;
         if (s->timing) DH_HIP(hipEventRecord(s->ev1, st));
         std::swap(s->phi, s->acc);  // phi <- new state; acc keeps the old one
@@ -1521,11 +1533,14 @@ static int propagate_checked(dh_system* s, double dt, int* n_terms, bool one_lau
             if (n_terms) *n_terms = s->K + 1;
             return DH_OK;
         }
-        // the bounds did not enclose the spectrum: restore and widen (NaN norms
-        // after a series in one launch say nothing about the bounds)
         std::swap(s->phi, s->acc);
-        if (attempt > 0 || std::isfinite(drift)) s->widen *= 1.25;
         s->stats[3] += 1;
+        // norms that are not finite after a series in one launch say nothing about
+        // the bounds: the same again term by term.  Else the bounds did not
+        // enclose the spectrum
+        if (whole && !std::isfinite(drift)) continue;
+        s->widen *= 1.25;
+        ++attempt;
     }
     // outputs of the restored (pre-step) state, as before the call
     launch_outputs(s);
@@ -1961,7 +1976,8 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
             } else {
                 launch_column_norms(s->N, R, s->phi, d.n0 + (size_t)i * R, st);
                 if (s->timing) DH_HIP(hipEventRecord(s->evpool[2 * n_timed], st));
-                if ((rc = chebyshev_series(s))) return rc;
+                bool whole = true;
+                if ((rc = chebyshev_series(s, &whole))) return rc;
                 if (s->timing) DH_HIP(hipEventRecord(s->evpool[2 * n_timed + 1], st));
                 if (s->timing) {
                     ++n_timed;
@@ -2024,6 +2040,7 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
         } else {
             // a step left the bounds: back to the interval's start, then step by
             // step with the checked step (wider bounds where needed)
+            s->stats[3] += 1;
             DH_HIP(hipMemcpyAsync(s->phi, d.ck_phi, sizeof(cplx) * s->ld * R, hipMemcpyDeviceToDevice, st));
             DH_HIP(hipMemcpyAsync(s->out, d.ck_out, sizeof(cplx) * s->ld * 3 * W, hipMemcpyDeviceToDevice, st));
             for (int i = j; i < jend; ++i) {
@@ -2219,10 +2236,11 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
     o.coef = w.coef;
     o.prec = 0;
     o.partial_cplx = w.partial_cplx;
-    const bool one_launch = series_resident(ctx, 0, ldh, R);
+    bool may = series_resident(ctx, 0, ldh, R), whole = false;
+    o.one_launch = &whole;
     double widen = 1.0, drift = 0.0;
     double n0[8], n1[8];  // R <= 8 (check_apply_args); no host allocation on this path
-    for (int attempt = 0; attempt < 4; ++attempt) {
+    for (int attempt = 0; attempt < 4;) {
         const double c = 0.5 * (bounds[1] + bounds[0]);
         const double r = 0.5 * (bounds[1] - bounds[0]) * widen;
         launch_bessel(r * dt, c * dt, KMAX_ALLOC, BESSEL_TOL, w.coef, w.kout, st);
@@ -2237,7 +2255,8 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
         o.K = K;
         o.c = c;
         o.r = r;
-        o.coop = one_launch && attempt == 0 ? coop_owner(ctx) : CoopOwner{};
+        o.coop = may ? coop_owner(ctx) : CoopOwner{};
+        may = false;
         if (int rc = series_core(o, st)) return rc;
         launch_column_norms(N, R, w.acc, w.norms1, st);
         DH_HIP(hipGetLastError());
@@ -2255,9 +2274,12 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
             if (n_terms) *n_terms = K + 1;
             return DH_OK;
         }
-        // the bounds did not enclose the spectrum (NaN norms after a series in one
-        // launch: it gave up waiting, and runs again term by term); phi is untouched
-        if (attempt > 0 || std::isfinite(drift)) widen *= 1.25;
+        // phi is untouched.  A series in one launch whose norms are not finite may
+        // have given up waiting: the same again term by term.  Else the bounds did
+        // not enclose the spectrum
+        if (whole && !std::isfinite(drift)) continue;
+        widen *= 1.25;
+        ++attempt;
     }
     dh::set_error("dh_chebyshev_apply: Chebyshev series lost the norm (drift %g) after widening the bounds", drift);
     return DH_ERR_DIVERGED;
@@ -2696,7 +2718,7 @@ static std::vector<double> batch_graph_key(const dh_batch* b, bool multi) {
 static int batch_solo_series(dh_batch* b) {
     for (int i = 0; i < b->n; ++i)
         if (b->solo[i] == 1)
-            if (int rc = series_launches(b->sys[i])) return rc;
+            if (bool whole = false; int rc = series_launches(b->sys[i], &whole)) return rc;
     if (launch_resident_rounds(b->d_res, (int)b->h_res.size(), b->d_map, b->rounds, coop_owner(b->ctx), b->ctx->stream))
         return DH_ERR_HIP;
     return DH_OK;
@@ -3023,6 +3045,11 @@ static int batch_autotune(dh_batch* b, hipStream_t st) {
     std::lock_guard<std::mutex> lk(g_batch_family_mu);
     if (g_batch_family[slot] < 0) g_batch_family[slot] = pick;
     b->sym = g_batch_family[slot] == 1 && b->sym_ok;
+    return DH_OK;
+}
+
+extern "C" int dh_test_force_give_up(int on) {
+    coop_force_give_up(on != 0);
     return DH_OK;
 }
 
@@ -3354,7 +3381,7 @@ extern "C" int dh_batch_propagate_steps(dh_batch* b, int n_steps, double dt_ps, 
             for (int c = 0; c < R; ++c) {
                 const double n0 = nv[(size_t)i * R + c], n1 = nv[(size_t)n * R + (size_t)i * R + c];
                 const double d = n0 > 0 ? std::fabs(n1 - n0) / n0 : 0.0;
-                if (!(d < 1e-9)) ok[i] = 0;
+                if (!(d < 1e-9) || !std::isfinite(n1)) ok[i] = 0;
                 if (std::isfinite(d)) maxdrift = std::max(maxdrift, d);
             }
         // commit the last step's state for members whose norm held

@@ -300,6 +300,10 @@ hipError_t coop_launch(const CoopOwner& who, const void* f, dim3 grid, dim3 bloc
                        hipStream_t st);
 // an owner that goes away (its streams have drained)
 void coop_forget(const CoopOwner& who);
+// for tests: the waves of the launches made from now on give up waiting at once,
+// as they do when a wait has run out
+void coop_force_give_up(bool on);
+bool coop_give_up_forced();
 
 // the whole Lanczos recurrence in one launch (lanczos.hip); false: not launched
 bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned seed, double* alpha, double* beta,
@@ -310,7 +314,7 @@ bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned see
 // < m at acc + q * acc_stride takes sum_k coef[q * coef_stride + k] T_k over
 // k <= kq[q] (device table; null: k <= K for the one accumulator), Hh = (H - c)
 // / r, T_0 = phi (N x R row-major).  H: ld x ld, symmetric, rows and columns >=
-// N zero off the diagonal.  The last five fields are the launcher's.
+// N zero off the diagonal.  The last six fields are the launcher's.
 struct ResidentArgs {
     const double* H;
     int ld, N, R, m, K;
@@ -323,6 +327,7 @@ struct ResidentArgs {
     const int* kq;
     char* ring;
     int slots, slot_bytes, groups;
+    int give_up;  // coop_give_up_forced
     unsigned* flags;
 };
 bool resident_series_fits(int ld, int R, int cus);

@@ -32,6 +32,7 @@ struct LanczosArgs {
     const double* H;
     int ld, N, m;
     unsigned seed;
+    int give_up;  // coop_give_up_forced
     double *alpha, *beta;
     double* ring;  // y of step j at ring + j * ld
 };
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(512) void lanczos_resident_kernel(LanczosArgs a) {
 
     const __amdgpu_buffer_rsrc_t ring =
         __builtin_amdgcn_make_buffer_rsrc(a.ring, 0, a.m * ld * 8, 0x00020000);
-    bool dead = false;
+    bool dead = a.give_up != 0;
     double be = 0.0;
     for (int j = 0; j < a.m; ++j) {
         double s[RW];
@@ -262,7 +263,7 @@ bool launch_lanczos_resident(const double* H, int ld, int N, int m, unsigned see
     const int M = (ld + 511) / 512, RW = M == 1 ? 2 : M == 2 ? 4 : M <= 4 ? 8 : 16;
     if (M > 8 || (N + RW - 1) / RW > who.cus) return false;
     if (8L * m * ld > scratch_bytes) return false;
-    LanczosArgs a{H, ld, N, m, seed, alpha, beta, static_cast<double*>(scratch)};
+    LanczosArgs a{H, ld, N, m, seed, coop_give_up_forced(), alpha, beta, static_cast<double*>(scratch)};
     hipError_t e;
     switch (M) {
         case 1: e = lanczos_go<1>(a, who, st); break;

@@ -19,6 +19,7 @@
 #include "kernels.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 
 namespace dh {
@@ -60,6 +61,10 @@ hipError_t coop_launch(const CoopOwner& who, const void* f, dim3 grid, dim3 bloc
     }
     return hipSuccess;
 }
+
+static std::atomic<bool> g_give_up{false};
+void coop_force_give_up(bool on) { g_give_up.store(on); }
+bool coop_give_up_forced() { return g_give_up.load(); }
 
 void coop_forget(const CoopOwner& who) {
     if (who.device < 0 || who.device >= MAX_DEVICES) return;
@@ -302,7 +307,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
     // flags of the rows this wave reads
     const int f0 = k0 / RB, nf = active ? ((min(k0 + 16 * n, ld) + RB - 1) / RB - f0) * SW : 0;
     const unsigned* const myflag = a.flags + ((blk % RS_COPIES) * nblk + f0) * SW + min(lane, max(nf - 1, 0));
-    bool dead = false;
+    bool dead = a.give_up != 0;
     const double a1 = 1.0 / a.r, b1 = -a.c / a.r;
     const int K = max(a.K, 1);
     for (int k = 1; k <= K; ++k) {
@@ -526,7 +531,7 @@ __global__ __launch_bounds__(NW * 64, 2) void resident_grouped_kernel(const Resi
     a.H = m->H; a.ld = m->ld; a.N = m->N; a.R = m->R; a.m = m->m; a.K = m->K; a.c = m->c; a.r = m->r;
     a.phi = m->phi; a.acc = m->acc; a.acc_stride = m->acc_stride; a.coef = m->coef; a.coef_stride = m->coef_stride;
     a.kq = m->kq; a.ring = m->ring; a.slots = m->slots; a.slot_bytes = m->slot_bytes; a.groups = m->groups;
-    a.flags = m->flags;
+    a.give_up = m->give_up; a.flags = m->flags;
     resident_body<NW, 4, NT, RC>(a, mp[1], a.ld / 16);
 }
 
@@ -611,6 +616,7 @@ static bool resident_scratch(ResidentArgs* a, void* scratch, long scratch_bytes)
     a->ring = static_cast<char*>(scratch) + fb;
     a->slots = (int)slots;
     a->slot_bytes = (int)sb;
+    a->give_up = coop_give_up_forced();
     return true;
 }
 

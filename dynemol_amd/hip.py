@@ -41,7 +41,8 @@ SYMBOLS = [
 ]
 TEST_SYMBOLS = ["dh_test_gemm", "dh_test_cholesky", "dh_test_copy", "dh_test_force_matvec_variant",
                 "dh_test_matvec_timing", "dh_test_read", "dh_test_device_alloc", "dh_test_device_free",
-                "dh_test_memcpy", "dh_test_bessel_coefficients", "dh_test_force_batch_family"]
+                "dh_test_memcpy", "dh_test_bessel_coefficients", "dh_test_force_batch_family",
+                "dh_test_force_give_up"]
 
 # Every live context and system is released before interpreter shutdown, while
 # the HIP runtime is still up (a handle freed during finalisation aborts).
@@ -441,6 +442,10 @@ class Batch:
 
 def force_batch_family(R, family):
     _check(lib().dh_test_force_batch_family(int(R), int(family)), "dh_test_force_batch_family")
+
+
+def force_give_up(on):
+    _check(lib().dh_test_force_give_up(1 if on else 0), "dh_test_force_give_up")
 
 
 def force_matvec_variant(v):

@@ -59,6 +59,7 @@ class Request:
     admitted: float = -1.0
     finished: float = -1.0
     done_steps: int = 0
+    retries: int = 0         # steps or intervals done again (System.stats)
     lane: int = -1
     result_bra: list = None
     result_ket: list = None
@@ -150,6 +151,7 @@ class _Lane:
         for r in gone:
             n = len(r.psi_ket)
             r.result_bra, r.result_ket, r.pops, r.erg = [], [], [], []
+            r.retries = r.system.stats()["retries"]
             for i in range(n):
                 b, k = r.system.wavepacket(i)
                 _, p, e = r.system.observables(i)
@@ -325,4 +327,5 @@ def latency_stats(done):
         return {}
     wp_steps = sum(len(r.psi_ket) * r.steps for r in done)
     return {"p50_s": float(np.percentile(lat, 50)), "p99_s": float(np.percentile(lat, 99)),
-            "mean_s": float(lat.mean()), "n": int(lat.size), "wavepacket_steps": int(wp_steps)}
+            "mean_s": float(lat.mean()), "n": int(lat.size), "wavepacket_steps": int(wp_steps),
+            "retries": sum(r.retries for r in done)}

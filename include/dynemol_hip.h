@@ -189,8 +189,9 @@ int dh_get_observables(dh_system *sys, int wp, double *ao_bra, double *pops, dou
  * 250-276, 366-392); the host copies of H', A and X it needed are gone. */
 int dh_ehrenfest_kernel(dh_system *sys, int wp_el, int wp_hl, const double *X, int ldx, double *K, int ldk);
 /* Counters (9 doubles): [terms of the last recurrence (one step's, or a
- * multi-step series' in dh_propagate_steps), steps, matvec launches, divergence
- * retries, last norm drift, term-series GPU ms (HIP events, when timing is
+ * multi-step series' in dh_propagate_steps), steps, matvec launches, steps and
+ * intervals done again (bounds that did not enclose the spectrum, or a launch
+ * whose waits ran out), last norm drift, term-series GPU ms (HIP events, when timing is
  * on), term launches timed, operator rebuilds, host ms that dh_propagate_steps
  * spent launching its rebuilds beside the propagation and waiting for them]. */
 int dh_get_stats(dh_system *sys, double *out9);
