@@ -157,6 +157,7 @@ struct dh_system {
     int next_graph = 0;
     bool use_graph = true;
     bool one_launch_bounds = true;  // dh_set_one_launch_bounds
+    bool one_launch_ran = false;    // the last series ran in one launch
     bool tuned = false;
     // 0 = FP64; 1 = mixed (FP32 MFMA term GEMM); 2 = FP32-stored H_orth with
     // FP64 products and sums
@@ -1163,9 +1164,14 @@ struct SeriesOps {
 };
 
 // whether a series of these operands runs in one launch (else one per term):
-// FP64, the operator fits the chip, and no term kernel is forced
-static bool series_resident(const dh_context* c, int prec, int ld, int R) {
-    return prec == 0 && !matvec_forced() && resident_series_fits(ld, R, c->cus);
+// FP64, the operator fits the chip, `partial` holds the exchange ring, and no
+// term kernel is forced
+static bool series_resident(const dh_context* c, int prec, int ld, int R, long partial_cplx) {
+    return prec == 0 && !matvec_forced() &&
+           resident_series_fits(ld, R, c->cus, partial_cplx * (long)sizeof(cplx));
+}
+static bool series_resident(const dh_system* s) {
+    return series_resident(s->ctx, s->precision, s->ld, 2 * s->W, partial_cplx_for(s->N, s->W));
 }
 
 static int series_core(const SeriesOps& o, hipStream_t st) {
@@ -1312,9 +1318,9 @@ static int series_core(const SeriesOps& o, hipStream_t st) {
 static int series_launches(dh_system* s, bool* one_launch) {
     SeriesOps o{};
     const bool may = *one_launch;
-    o.one_launch = one_launch;
+    o.one_launch = &s->one_launch_ran;
     o.partial_cplx = partial_cplx_for(s->N, s->W);
-    if (may && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) o.coop = coop_owner(s->ctx);
+    if (may && series_resident(s)) o.coop = coop_owner(s->ctx);
     o.H = s->Hth;
     o.H32 = s->H32;
     o.Hlo = s->Hlo;
@@ -1337,7 +1343,9 @@ static int series_launches(dh_system* s, bool* one_launch) {
     o.K = s->K;
     o.c = s->coef_c;
     o.r = s->coef_r;
-    if (int rc = series_core(o, s->ctx->stream)) return rc;
+    const int rc = series_core(o, s->ctx->stream);
+    *one_launch = s->one_launch_ran;
+    if (rc) return rc;
     DH_HIP(hipGetLastError());
     return DH_OK;
 }
@@ -1349,8 +1357,8 @@ static int chebyshev_series(dh_system* s, bool* one_launch) {
     // the FP32-product modes call rocBLAS, which stays out of stream capture; a
     // series in one launch has nothing to capture
     if (!s->use_graph || fp32_products(s)) return series_launches(s, one_launch);
-    if (*one_launch && series_resident(s->ctx, s->precision, s->ld, 2 * s->W)) return series_launches(s, one_launch);
-    *one_launch = false;
+    if (*one_launch && series_resident(s)) return series_launches(s, one_launch);
+    *one_launch = s->one_launch_ran = false;
     hipStream_t st = s->ctx->stream;
     const int variant = matvec_variant_for(s->N, 2 * s->W, TRI_FULL);
     for (auto& g : s->graphs)
@@ -1833,7 +1841,8 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     o.ring_stride = acc_n;
     o.K = Kq[m - 1];
     o.partial_cplx = partial_cplx_for(s->N, s->W);
-    if (series_resident(s->ctx, s->precision, s->ld, R)) o.coop = coop_owner(s->ctx);
+    if (series_resident(s)) o.coop = coop_owner(s->ctx);
+    o.one_launch = &s->one_launch_ran;
     if (int rc = series_core(o, st)) return rc;
     DH_HIP(hipGetLastError());
     *kmax = Kq[m - 1];
@@ -2236,7 +2245,7 @@ static int chebyshev_apply_impl(dh_context* ctx, int N, const double* H, int ldh
     o.coef = w.coef;
     o.prec = 0;
     o.partial_cplx = w.partial_cplx;
-    bool may = series_resident(ctx, 0, ldh, R), whole = false;
+    bool may = series_resident(ctx, 0, ldh, R, w.partial_cplx), whole = false;
     o.one_launch = &whole;
     double widen = 1.0, drift = 0.0;
     double n0[8], n1[8];  // R <= 8 (check_apply_args); no host allocation on this path
@@ -3045,6 +3054,13 @@ static int batch_autotune(dh_batch* b, hipStream_t st) {
     std::lock_guard<std::mutex> lk(g_batch_family_mu);
     if (g_batch_family[slot] < 0) g_batch_family[slot] = pick;
     b->sym = g_batch_family[slot] == 1 && b->sym_ok;
+    return DH_OK;
+}
+
+extern "C" int dh_test_series_form(dh_system* s, int* out2) {
+    CHECK_ARG(s && out2, "dh_test_series_form: null argument");
+    out2[0] = s->one_launch_ran;
+    out2[1] = (s->graphs[0].exec != nullptr) + (s->graphs[1].exec != nullptr);
     return DH_OK;
 }
 

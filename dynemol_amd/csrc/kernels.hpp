@@ -330,7 +330,8 @@ struct ResidentArgs {
     int give_up;  // coop_give_up_forced
     unsigned* flags;
 };
-bool resident_series_fits(int ld, int R, int cus);
+// whether it can (a series whose exchange ring does not fit the scratch cannot)
+bool resident_series_fits(int ld, int R, int cus, long scratch_bytes);
 // false: not launched (shape, scratch or device do not allow it)
 bool launch_resident_series(ResidentArgs a, void* scratch, long scratch_bytes, const CoopOwner& who, hipStream_t st);
 // Batches: whether a member can run so (fills in the launcher's fields), the

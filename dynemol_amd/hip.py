@@ -42,7 +42,7 @@ SYMBOLS = [
 TEST_SYMBOLS = ["dh_test_gemm", "dh_test_cholesky", "dh_test_copy", "dh_test_force_matvec_variant",
                 "dh_test_matvec_timing", "dh_test_read", "dh_test_device_alloc", "dh_test_device_free",
                 "dh_test_memcpy", "dh_test_bessel_coefficients", "dh_test_force_batch_family",
-                "dh_test_force_give_up"]
+                "dh_test_force_give_up", "dh_test_series_form"]
 
 # Every live context and system is released before interpreter shutdown, while
 # the HIP runtime is still up (a handle freed during finalisation aborts).
@@ -110,6 +110,7 @@ def lib():
     L.dh_set_timing.argtypes = [_vp, ctypes.c_int]
     L.dh_set_steps_per_series.argtypes = [_vp, ctypes.c_int]
     L.dh_set_graph.argtypes = [_vp, ctypes.c_int]
+    L.dh_test_series_form.argtypes = [_vp, _i]
     L.dh_set_one_launch_bounds.argtypes = [_vp, ctypes.c_int]
     L.dh_matvec_tuning.argtypes = [_vp, _i]
     L.dh_set_precision.argtypes = [_vp, ctypes.c_int]
@@ -442,6 +443,13 @@ class Batch:
 
 def force_batch_family(R, family):
     _check(lib().dh_test_force_batch_family(int(R), int(family)), "dh_test_force_batch_family")
+
+
+def series_form(system):
+    """(whether the system's last series ran in one launch, captured graphs of its one-step series)"""
+    out = np.zeros(2, dtype=np.int32)
+    _check(lib().dh_test_series_form(system.h, _p(out, _i)), "dh_test_series_form")
+    return bool(out[0]), int(out[1])
 
 
 def force_give_up(on):
