@@ -374,13 +374,37 @@ static long partial_cplx_for(int N, int n_wp) {
     return n;
 }
 
+// Buffers of dh_propagate_steps that stay with the system: the outputs of several
+// steps at once (0: larger than the limit), the slices of their products (as many
+// as fit as much again, at most 8), the state an interval starts from, and room
+// for what a call keeps per step and per geometry; a call that needs more gives
+// its block back.
+constexpr size_t OUTPUTS_MAX_BYTES = 32u << 20, STEPS_ROOM_BYTES = 1u << 20;
+static size_t steps_outputs_bytes(size_t ld, size_t W) {
+    const size_t b = sizeof(cplx) * MULTI_MAX * ld * 4 * W + sizeof(double) * MULTI_MAX * 2 * W;
+    return b <= OUTPUTS_MAX_BYTES ? b : 0;
+}
+static size_t steps_slices_bytes(size_t ld, size_t W) {
+    const size_t slice = sizeof(double) * 4 * W * MULTI_MAX * ld;
+    return slice * std::min<size_t>(8, OUTPUTS_MAX_BYTES / slice);
+}
+static size_t steps_state_bytes(size_t ld, size_t W) { return sizeof(cplx) * ld * 5 * W; }
+static size_t steps_kept_bytes(size_t ld, size_t W) {
+    const size_t outputs = steps_outputs_bytes(ld, W);
+    return steps_state_bytes(ld, W) + STEPS_ROOM_BYTES + (outputs ? outputs + steps_slices_bytes(ld, W) : 0);
+}
+
 extern "C" long long dh_system_bytes(int n_orb, int n_wp) {
     const long long ld = round_ld(n_orb);
     const long long R = 2LL * n_wp;
-    long long b = 3LL * ld * ld * 8;                       // Q1, Q2, H_orth
+    // the device's memory comes in pages of 2 MiB: the large blocks in whole ones
+    auto pages = [](long long bytes) { return (bytes + (2 << 20) - 1) >> 21 << 21; };
+    auto block = [&](long long bytes) { return bytes < (2 << 20) ? bytes : pages(bytes); };
+    long long b = 3 * block(ld * ld * 8);                   // Q1, Q2, H_orth
     b += (4 * R + 3LL * n_wp + n_wp) * ld * 16;             // phi, x0, x1, acc, out, hk
-    b += (long long)partial_cplx_for(n_orb, n_wp) * 16;    // partials
+    b += block((long long)partial_cplx_for(n_orb, n_wp) * 16);  // partials
     b += 3LL * ld * 16 + (long long)KMAX_ALLOC * 24;      // Lanczos, Bessel
+    b += block((long long)steps_kept_bytes(ld, n_wp));     // dh_propagate_steps
     return b;
 }
 
@@ -920,8 +944,9 @@ static int put_column(dh_system* s, cplx* dst, long dst_stride, const double* ho
 }
 
 // Pinned host memory of n doubles for this system's results, kept until the
-// system goes.  Its users wait for the stream before they return, so no device
-// write is outstanding here.
+// system goes: a state's columns, or up to PIN_DOUBLES (read_back).  Its users
+// wait for the stream before they return, so no device write is outstanding here.
+constexpr size_t PIN_DOUBLES = 1u << 18;
 static int host_buffer(dh_system* s, size_t n) {
     if (n <= s->pin_n) return DH_OK;
     if (s->pin) hipHostFree(s->pin);
@@ -937,6 +962,32 @@ static int copy_block(double* dst, long ldd, const double* src, long lds, int ro
                       hipStream_t st) {
     DH_HIP(hipMemcpy2DAsync(dst, sizeof(double) * ldd, src, sizeof(double) * lds, sizeof(double) * rows, cols, kind,
                             st));
+    return DH_OK;
+}
+
+// Two device arrays to the host, and the host's wait for the stream: through the
+// pinned buffer in one launch, or, where they do not fit it or it cannot be had,
+// by the runtime's copies.
+static int read_back(dh_system* s, const double* a, size_t na, double* to_a, const double* b, size_t nb, double* to_b) {
+    hipStream_t st = s->ctx->stream;
+    const bool pinned = na + nb <= PIN_DOUBLES && host_buffer(s, na + nb) == DH_OK;
+    if (pinned) {
+        ExportArgs e{};
+        e.arr[0] = a;
+        e.arr[1] = b;
+        e.count[0] = (long)na;
+        e.count[1] = (long)nb;
+        e.dst = s->pin;
+        launch_export(e, st);
+        DH_HIP(hipGetLastError());
+    } else {
+        (void)hipGetLastError();
+        if (na) DH_HIP(hipMemcpyAsync(to_a, a, sizeof(double) * na, hipMemcpyDeviceToHost, st));
+        if (nb) DH_HIP(hipMemcpyAsync(to_b, b, sizeof(double) * nb, hipMemcpyDeviceToHost, st));
+    }
+    DH_HIP(hipStreamSynchronize(st));
+    if (pinned && na) std::memcpy(to_a, s->pin, sizeof(double) * na);
+    if (pinned && nb) std::memcpy(to_b, s->pin + na, sizeof(double) * nb);
     return DH_OK;
 }
 
@@ -1431,18 +1482,6 @@ static void launch_outputs(dh_system* s, double* pops, double* erg) {
 }
 static void launch_outputs(dh_system* s) { launch_outputs(s, s->pops, s->erg); }
 
-// Buffers of the outputs of several steps at once (0: larger than the limit), and
-// the slices of their products: as many as fit as much again, at most 8.
-constexpr size_t OUTPUTS_MAX_BYTES = 32u << 20;
-static size_t steps_outputs_bytes(const dh_system* s) {
-    const size_t b = sizeof(cplx) * MULTI_MAX * (size_t)s->ld * 4 * s->W + sizeof(double) * MULTI_MAX * 2 * s->W;
-    return b <= OUTPUTS_MAX_BYTES ? b : 0;
-}
-static size_t steps_slices_bytes(const dh_system* s) {
-    const size_t slice = sizeof(double) * 4 * s->W * MULTI_MAX * (size_t)s->ld;
-    return slice * std::min<size_t>(8, OUTPUTS_MAX_BYTES / slice);
-}
-
 // launch_outputs for the m states of a multi-step series (s->accm), the last one's
 // results to s->out and s->hk, in one product per operator: its columns of all
 // steps together fill matrix-core tiles, and the operator is read once.  Norms
@@ -1455,7 +1494,7 @@ static void launch_outputs_steps(dh_system* s, int m, char* buf, double* pops, d
     cplx* const hk = out + MULTI_MAX * out_n;
     double* const norms = reinterpret_cast<double*>(hk + MULTI_MAX * hk_n);
     double* const P = norms + MULTI_MAX * 2 * W;
-    const long p_doubles = (long)(steps_slices_bytes(s) / sizeof(double));
+    const long p_doubles = (long)(steps_slices_bytes(s->ld, W) / sizeof(double));
     MatvecArgs a{};
     a.ld = s->ld;
     a.N = s->N;
@@ -1849,24 +1888,33 @@ static int multi_series(dh_system* s, double dt, int m, int* kmax) {
     return DH_OK;
 }
 
-// Device buffers of one dh_propagate_steps call, in the system's kept block (a
-// block per call costs seven allocations and frees); the side stream, whose
-// launched build reads geo, has drained on every return path.
+// Device buffers of one dh_propagate_steps call, in the system's block, which is
+// kept up to steps_kept_bytes (a block per call costs seven allocations and
+// frees); the side stream, whose launched build reads geo, has drained on every
+// return path.
 struct StepsScratch {
+    dh_system* s = nullptr;
     double *geo = nullptr, *n0 = nullptr, *n1 = nullptr, *pops = nullptr, *erg = nullptr;
     cplx *ck_phi = nullptr, *ck_out = nullptr;
     char* outputs = nullptr;  // of several steps (null: step by step)
     hipStream_t side = nullptr;
     ~StepsScratch() {
         if (side) hipStreamSynchronize(side);
+        if (s && s->steps_bytes > steps_kept_bytes(s->ld, s->W)) {
+            hipStreamSynchronize(s->ctx->stream);
+            hipFree(s->steps_mem);
+            s->steps_mem = nullptr;
+            s->steps_bytes = 0;
+        }
     }
-    int take(dh_system* s, int n_steps, size_t geo_n) {
+    int take(dh_system* sys, int n_steps, size_t geo_n) {
+        s = sys;
         const size_t R = 2 * (size_t)s->W, ld = s->ld, n = n_steps;
         const size_t doubles = 2 * n * R + n * s->W * (s->n_frag + 1) + n * s->W * 2 + geo_n;
-        const size_t must = sizeof(cplx) * ld * (R + 3 * s->W) + sizeof(double) * doubles;
+        const size_t must = steps_state_bytes(ld, s->W) + sizeof(double) * doubles;
         size_t extra = 0;
-        if (n_steps > 1 && s->steps_per_series != 1 && steps_outputs_bytes(s))
-            extra = steps_outputs_bytes(s) + steps_slices_bytes(s);
+        if (n_steps > 1 && s->steps_per_series != 1 && steps_outputs_bytes(ld, s->W))
+            extra = steps_outputs_bytes(ld, s->W) + steps_slices_bytes(ld, s->W);
         if (must + extra > s->steps_bytes) {
             DH_HIP(hipStreamSynchronize(s->ctx->stream));
             if (s->steps_mem) hipFree(s->steps_mem);
@@ -1909,7 +1957,6 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
     StepsScratch d;
     const size_t geo_n = (size_t)s->n_atoms * 3;
     if ((rc = d.take(s, n_steps, geo_n * n_geo))) return rc;
-    if ((rc = host_buffer(s, (size_t)n_steps * W * std::max(4, NP + 2)))) return rc;
     if (n_geo > 0) {
         if ((rc = ensure_side(s))) return rc;
         d.side = s->ctx->side;
@@ -2014,16 +2061,9 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
                               hipMemcpyDeviceToDevice, st));
         DH_HIP(hipMemcpyAsync(s->erg, d.erg + (size_t)(jend - 1) * W * 2, sizeof(double) * W * 2,
                               hipMemcpyDeviceToDevice, st));
-        const long cnt = (long)(jend - j) * R;
-        ExportArgs e{};
-        e.arr[0] = d.n0 + (size_t)j * R;
-        e.arr[1] = d.n1 + (size_t)j * R;
-        e.count[0] = e.count[1] = cnt;
-        e.dst = s->pin;
-        launch_export(e, st);
-        DH_HIP(hipGetLastError());
-        DH_HIP(hipStreamSynchronize(st));
-        const double *h0 = s->pin, *h1 = s->pin + cnt;
+        const size_t cnt = (size_t)(jend - j) * R;
+        std::vector<double> h0(cnt), h1(cnt);
+        if ((rc = read_back(s, d.n0 + (size_t)j * R, cnt, h0.data(), d.n1 + (size_t)j * R, cnt, h1.data()))) return rc;
         float series_ms = 0.0f;
         if (s->timing)
             for (int i = 0; i < n_timed; ++i) {
@@ -2032,7 +2072,7 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
                 series_ms += ms;
             }
         double drift = 0.0;
-        for (long c = 0; c < cnt; ++c) {
+        for (size_t c = 0; c < cnt; ++c) {
             if (h0[c] > 0) drift = std::max(drift, std::fabs(h1[c] - h0[c]) / h0[c]);
             if (!std::isfinite(h1[c])) drift = INFINITY;
         }
@@ -2062,19 +2102,9 @@ extern "C" int dh_propagate_steps(dh_system* s, int n_steps, double dt_ps, int r
         }
         j = jend;
     }
-    if (pops || erg) {
-        ExportArgs e{};
-        e.arr[0] = d.pops;
-        e.arr[1] = d.erg;
-        e.count[0] = (long)n_steps * W * NP;
-        e.count[1] = (long)n_steps * W * 2;
-        e.dst = s->pin;
-        launch_export(e, st);
-        DH_HIP(hipGetLastError());
-    }
-    DH_HIP(hipStreamSynchronize(st));
-    if (pops) std::memcpy(pops, s->pin, sizeof(double) * (size_t)n_steps * W * NP);
-    if (erg) std::memcpy(erg, s->pin + (size_t)n_steps * W * NP, sizeof(double) * (size_t)n_steps * W * 2);
+    if ((rc = read_back(s, d.pops, pops ? (size_t)n_steps * W * NP : 0, pops, d.erg,
+                        erg ? (size_t)n_steps * W * 2 : 0, erg)))
+        return rc;
     if (n_terms) *n_terms = last_terms;
     return DH_OK;
 }

@@ -68,7 +68,11 @@ int dh_system_destroy(dh_system *sys);
 /* Device bytes a system of this size holds (serving admission), in FP64 and
  * with the FP32 operator copies of a precision mode (dh_set_precision);
  * dh_system_bytes_prec(n, w, 0) also counts the accumulators of the
- * multi-step series of dh_propagate_steps. */
+ * multi-step series of dh_propagate_steps.  Both count the buffers that
+ * dh_propagate_steps keeps (up to 64 MiB of step outputs and their products);
+ * not the second operator set of its rebuilds, nor what a context holds: the
+ * build workspace, and 32 MiB once matrices were copied between pitches
+ * (dh_load_operators, dh_get_matrix, dh_ehrenfest_kernel). */
 long long dh_system_bytes(int n_orb, int n_wp);
 long long dh_system_bytes_prec(int n_orb, int n_wp, int precision);
 
