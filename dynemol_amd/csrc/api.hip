@@ -997,11 +997,17 @@ static int read_back(dh_system* s, const double* a, size_t na, double* to_a, con
 // much on the host (a drop-in call with H' out at N = 1200: 27.8 -> 5.9 ms).
 static constexpr size_t MSTAGE_DOUBLES = 4u << 20;  // 32 MiB
 
-// columns per block for a host pitch, 0: a column does not fit, or the pitch
-// brings in more padding than matrix
-static int stage_columns(dh_context* c, long ld_host, int n, int* rc) {
-    if (ld_host > 2L * n || (size_t)ld_host > MSTAGE_DOUBLES) return 0;
-    if (!c->mstage) *rc = dalloc(&c->mstage, MSTAGE_DOUBLES);
+static bool g_no_transfer_buffer = false;  // dh_test_forbid_transfer_buffer
+
+// columns per block for a host pitch, 0 (one copy per column): a column does not
+// fit, the pitch brings in more padding than matrix, or the device has no memory
+// left for the buffer
+static int stage_columns(dh_context* c, long ld_host, int n) {
+    if (ld_host > 2L * n || (size_t)ld_host > MSTAGE_DOUBLES || g_no_transfer_buffer) return 0;
+    if (!c->mstage && dalloc(&c->mstage, MSTAGE_DOUBLES)) {
+        (void)hipGetLastError();
+        return 0;
+    }
     return (int)std::min<size_t>(n, MSTAGE_DOUBLES / ld_host);
 }
 
@@ -1012,9 +1018,7 @@ static int put_matrix(dh_context* c, double* dst, long ldd, const double* host, 
         DH_HIP(hipMemcpyAsync(dst, host, sizeof(double) * ((size_t)ldh * (n - 1) + n), hipMemcpyHostToDevice, st));
         return DH_OK;
     }
-    int rc = DH_OK;
-    const int cols = stage_columns(c, ldh, n, &rc);
-    if (rc) return rc;
+    const int cols = stage_columns(c, ldh, n);
     for (int j = 0; j < n; j += std::max(cols, 1)) {
         if (cols == 0) {
             DH_HIP(hipMemcpyAsync(dst + (size_t)ldd * j, host + (size_t)ldh * j, sizeof(double) * n,
@@ -1038,9 +1042,7 @@ static int get_matrix(dh_context* c, double* host, long ldh, const double* src, 
         DH_HIP(hipMemcpyAsync(host, src, sizeof(double) * (size_t)ldh * n, hipMemcpyDeviceToHost, st));
         return DH_OK;
     }
-    int rc = DH_OK;
-    const int cols = ldh == n ? stage_columns(c, ldh, n, &rc) : 0;
-    if (rc) return rc;
+    const int cols = ldh == n ? stage_columns(c, ldh, n) : 0;
     for (int j = 0; j < n; j += std::max(cols, 1)) {
         if (cols == 0) {
             DH_HIP(hipMemcpyAsync(host + (size_t)ldh * j, src + (size_t)lds * j, sizeof(double) * n,
@@ -3091,6 +3093,11 @@ extern "C" int dh_test_series_form(dh_system* s, int* out2) {
     CHECK_ARG(s && out2, "dh_test_series_form: null argument");
     out2[0] = s->one_launch_ran;
     out2[1] = (s->graphs[0].exec != nullptr) + (s->graphs[1].exec != nullptr);
+    return DH_OK;
+}
+
+extern "C" int dh_test_forbid_transfer_buffer(int on) {
+    g_no_transfer_buffer = on != 0;
     return DH_OK;
 }
 

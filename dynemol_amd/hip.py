@@ -42,7 +42,7 @@ SYMBOLS = [
 TEST_SYMBOLS = ["dh_test_gemm", "dh_test_cholesky", "dh_test_copy", "dh_test_force_matvec_variant",
                 "dh_test_matvec_timing", "dh_test_read", "dh_test_device_alloc", "dh_test_device_free",
                 "dh_test_memcpy", "dh_test_bessel_coefficients", "dh_test_force_batch_family",
-                "dh_test_force_give_up", "dh_test_series_form"]
+                "dh_test_force_give_up", "dh_test_series_form", "dh_test_forbid_transfer_buffer"]
 
 # Every live context and system is released before interpreter shutdown, while
 # the HIP runtime is still up (a handle freed during finalisation aborts).
@@ -450,6 +450,10 @@ def series_form(system):
     out = np.zeros(2, dtype=np.int32)
     _check(lib().dh_test_series_form(system.h, _p(out, _i)), "dh_test_series_form")
     return bool(out[0]), int(out[1])
+
+
+def forbid_transfer_buffer(on):
+    _check(lib().dh_test_forbid_transfer_buffer(1 if on else 0), "dh_test_forbid_transfer_buffer")
 
 
 def force_give_up(on):

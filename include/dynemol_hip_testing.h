@@ -43,6 +43,9 @@ int dh_test_bessel_coefficients(double x, double phase, double tol, int kmax, do
  * storage, 0 dense column blocks; -1: the autotuner chooses again), for the
  * batches created afterwards. */
 int dh_test_force_batch_family(int R, int family);
+/* Matrices are copied between pitches column by column, as where the device has
+ * no memory for the transfer buffer (on = 1), or through it (0). */
+int dh_test_forbid_transfer_buffer(int on);
 /* How the system's last series ran: out2[0] = 1 in one launch, 0 one launch per
  * term; out2[1] = captured graphs of its one-step series. */
 int dh_test_series_form(struct dh_system *sys, int *out2);
