@@ -340,9 +340,10 @@ def _exact(S, h, psi0, t):
 def run_many_systems(n_sys=256, steps=500, seed=3, n_wp=4, check=6):
     """Many systems in one batch: C/H/N/O clusters, N log-uniform in [256, 2048],
     4 wavepackets each (random S-normalised superpositions of 8 frontier orbitals
-    from the device eigensolver), grouped launches per Chebyshev term, 10 steps
-    per recurrence (dh_batch_propagate_steps); 11 untimed steps (the batch's
-    tuning step, then one 10-step recurrence that captures its graph) before
+    from the device eigensolver), 10 steps per recurrence
+    (dh_batch_propagate_steps: resident launches over several members each, or
+    grouped launches per Chebyshev term); 11 untimed steps (a first step, then one
+    10-step recurrence, which captures a graph where terms are grouped) before
     `steps` timed ones; sampled systems checked against the exact propagator of
     their device-built S and h (untimed)."""
     import scipy.linalg as sl
@@ -391,7 +392,9 @@ def run_many_systems(n_sys=256, steps=500, seed=3, n_wp=4, check=6):
         total = steps + 11
         out["wavepacket_steps_per_s"] = round(n_sys * n_wp * steps / el, 1)
         out["ms_per_step"] = round(1e3 * el / steps, 3)
-        out["batch_kernel"] = batch.tuning()
+        whole = sum(hip.series_form(s)[0] for s in systems)
+        out["batch_kernel"] = "one launch per series" if whole == n_sys else batch.tuning()
+        out["members_in_one_launch_series"] = whole
         out["most_terms_per_recurrence"] = kmax
         errs, perr = [], []
         for i in range(check):

@@ -107,7 +107,7 @@ struct dh_system {
     int split_max = 1;
     // Lanczos / Bessel
     cplx *lv = nullptr, *lvp = nullptr, *lw = nullptr;
-    double *lal = nullptr, *lbe = nullptr, *J = nullptr;
+    double *lal = nullptr, *lbe = nullptr;
     cplx* coef = nullptr;
     int* kout = nullptr;
     cplx* coef_h = nullptr;         // pinned staging of the coefficients
@@ -335,7 +335,7 @@ extern "C" int dh_system_destroy(dh_system* s) {
         if (p) hipHostFree(p);
     if (s->sh.done) hipEventDestroy(s->sh.done);
     void* ptrs[] = {s->basis_mem, s->coords, s->frag, s->Q1, s->Q2, s->Hth, s->phi, s->x0, s->x1, s->acc, s->out, s->stage,
-                    s->hk, s->partial, s->counters, s->lv, s->lvp, s->lw, s->lal, s->lbe, s->J, s->coef,
+                    s->hk, s->partial, s->counters, s->lv, s->lvp, s->lw, s->lal, s->lbe, s->coef,
                     s->kout, s->pops, s->erg, s->norms, s->norms0, s->norms1};
     for (void* p : ptrs)
         if (p) hipFree(p);
@@ -403,7 +403,7 @@ extern "C" long long dh_system_bytes(int n_orb, int n_wp) {
     long long b = 3 * block(ld * ld * 8);                   // Q1, Q2, H_orth
     b += (4 * R + 3LL * n_wp + n_wp) * ld * 16;             // phi, x0, x1, acc, out, hk
     b += block((long long)partial_cplx_for(n_orb, n_wp) * 16);  // partials
-    b += 3LL * ld * 16 + (long long)KMAX_ALLOC * 24;      // Lanczos, Bessel
+    b += 3LL * ld * 16 + (long long)KMAX_ALLOC * 16;      // Lanczos, Bessel
     b += block((long long)steps_kept_bytes(ld, n_wp));     // dh_propagate_steps
     return b;
 }
@@ -577,7 +577,6 @@ extern "C" int dh_system_create(dh_context* ctx, int n_atoms, const int* first_o
     SALLOC(s->lw, (size_t)ld);
     SALLOC(s->lal, LANCZOS_MAX + 2);
     SALLOC(s->lbe, LANCZOS_MAX + 2);
-    SALLOC(s->J, KMAX_ALLOC + 2);
     SALLOC(s->coef, KMAX_ALLOC + 2);
     SALLOC(s->kout, 4);
     SALLOC(s->pops, (size_t)n_wp * (n_frag + 1));
@@ -2757,6 +2756,7 @@ static std::vector<double> batch_graph_key(const dh_batch* b, bool multi) {
 // members in other precision modes run their own series after the grouped
 // terms, outside the capture (the FP32-product modes call rocBLAS)
 static int batch_solo_series(dh_batch* b) {
+    for (int i = 0; i < b->n; ++i) b->sys[i]->one_launch_ran = b->solo[i] == 2;
     for (int i = 0; i < b->n; ++i)
         if (b->solo[i] == 1)
             if (bool whole = false; int rc = series_launches(b->sys[i], &whole)) return rc;

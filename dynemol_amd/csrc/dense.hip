@@ -353,8 +353,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 }
 
 // zero the blocks above the diagonal blocks (column j: rows 0 .. 64 floor(j / 64) - 1),
-// once the factorization is done: the trailing updates run on lower tiles of
-// 128 and leave values in some of these blocks, and nothing reads them before
+// once the factorization is done: they hold the upper triangle of the matrix that
+// came in, and nothing reads or writes them before
 __global__ void zero_upper_blocks_kernel(double* A, int ld) {
     const int j = blockIdx.x;
     const int top = (j / TILE) * TILE;
