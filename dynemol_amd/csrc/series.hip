@@ -30,15 +30,16 @@ namespace dh {
 // part of the chip each would wait for one another until their waits ran out.
 // The lock is held over the launch, so that no two threads are ever inside the
 // runtime's cooperative launch (nor in its first-use set-up) at the same time, and
-// over the wait for another owner's last launch to end; launches of one owner,
-// which one thread makes, are ordered by the runtime.
+// over the wait for another owner's launches to end; launches of one owner, which
+// one thread makes, are ordered by the runtime.
 namespace {
+constexpr int MAX_DEVICES = 64, OWNER_STREAMS = 2;  // a context's stream and its side stream
 struct Turnstile {
     std::mutex mu;
-    hipEvent_t done = nullptr;  // after the last launch
-    const void* owner = nullptr;  // whose that was; null: none in flight
+    const void* owner = nullptr;  // whose launches may be in flight; null: nobody's
+    hipEvent_t done[OWNER_STREAMS] = {};     // after the last launch on each stream of the owner's
+    hipStream_t stream[OWNER_STREAMS] = {};  // null: none yet
 };
-constexpr int MAX_DEVICES = 64;
 Turnstile g_turnstile[MAX_DEVICES];
 }  // namespace
 
@@ -50,17 +51,28 @@ hipError_t coop_launch(const CoopOwner& who, const void* f, dim3 grid, dim3 bloc
     // (the event orders launches and publishes no data: with the system fence a
     // call of dh_propagate at N = 416 takes 4 us more, 156 against 152)
     constexpr unsigned flags = hipEventDisableTiming | hipEventDisableSystemFence;
-    if (!t.done)
-        if (hipError_t e = hipEventCreateWithFlags(&t.done, flags); e != hipSuccess) return e;
-    if (t.owner && t.owner != who.owner)
-        if (hipError_t e = hipEventSynchronize(t.done); e != hipSuccess) return e;
+    for (hipEvent_t& ev : t.done)
+        if (!ev)
+            if (hipError_t e = hipEventCreateWithFlags(&ev, flags); e != hipSuccess) return e;
+    int slot = 0;
+    if (t.owner == who.owner)
+        while (slot < OWNER_STREAMS && t.stream[slot] && t.stream[slot] != st) ++slot;
+    if (t.owner != who.owner || slot == OWNER_STREAMS) {  // another owner's turn ends
+        for (int i = 0; i < OWNER_STREAMS; ++i)
+            if (t.owner && t.stream[i])
+                if (hipError_t e = hipEventSynchronize(t.done[i]); e != hipSuccess) return e;
+        t.owner = nullptr;
+        for (hipStream_t& s : t.stream) s = nullptr;
+        slot = 0;
+    }
     if (hipError_t e = hipLaunchCooperativeKernel(f, grid, block, params, lds, st); e != hipSuccess) return e;
     t.owner = who.owner;
+    t.stream[slot] = st;
     // launched: whatever becomes of the record, the caller must not launch again
-    if (hipEventRecord(t.done, st) != hipSuccess) {
+    if (hipEventRecord(t.done[slot], st) != hipSuccess) {
         (void)hipGetLastError();
         if (hipStreamSynchronize(st) != hipSuccess) (void)hipGetLastError();
-        t.owner = nullptr;
+        t.stream[slot] = nullptr;
     }
     return hipSuccess;
 }
@@ -73,7 +85,9 @@ void coop_forget(const CoopOwner& who) {
     if (who.device < 0 || who.device >= MAX_DEVICES) return;
     Turnstile& t = g_turnstile[who.device];
     std::lock_guard<std::mutex> lk(t.mu);
-    if (t.owner == who.owner) t.owner = nullptr;
+    if (t.owner != who.owner) return;
+    t.owner = nullptr;
+    for (hipStream_t& s : t.stream) s = nullptr;
 }
 
 // Work split: workgroup b owns RB = 4 RG consecutive rows; its NW waves split
