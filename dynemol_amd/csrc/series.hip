@@ -494,6 +494,7 @@ __device__ __forceinline__ void resident_body(const ResidentArgs& a, const int b
                     T.re -= x2.re;
                     T.im -= x2.im;
                 }
+                if (r0 + row >= N) T = cplx{0.0, 0.0};  // whatever a caller's operator has on its padded diagonal
                 if (k < K) publish(e, T, k);
                 tk[e] = T;
             }
