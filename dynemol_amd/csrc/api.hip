@@ -1153,9 +1153,8 @@ static int ensure_coefficients(dh_system* s, double dt) {
     const double r = 0.5 * (s->emax - s->emin) * s->widen;
     if (dt == s->coef_dt && c == s->coef_c && r == s->coef_r) return DH_OK;
     hipStream_t st = s->ctx->stream;
-    // on the host (a few microseconds; the device recurrence is one thread of
-    // dependent memory accesses, about a millisecond), then one copy on the
-    // stream: the host neither launches nor waits for a kernel here
+    // on the host (a few microseconds), then one copy on the stream: the host
+    // neither launches nor waits for a kernel here
     if (!s->coef_h) {
         DH_HIP(hipHostMalloc((void**)&s->coef_h, sizeof(cplx) * (KMAX_ALLOC + 2), hipHostMallocDefault));
         DH_HIP(hipEventCreateWithFlags(&s->coef_ev, hipEventDisableTiming));

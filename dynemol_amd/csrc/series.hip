@@ -98,10 +98,11 @@ void coop_forget(const CoopOwner& who) {
 // replication: lane 16k + 4b + j takes x[16g + 4k + b][j], 16 bytes (re, im).
 // The ring keeps the vectors in this order (per group of 16 rows and pass of 4
 // columns, the 64 lanes' values), so a load is 1 KB contiguous (as fast as
-// row-major order measured, and the addresses are simpler).  A operands (H) stay in the lane's registers, up to what
-// 256 registers hold beside the products (23 groups at R = 4), and in LDS from
-// there on.  At R = 4 a group is 8 MFMAs of 16 cycles on one load; N = 4096: 32
-// groups per wave, 3.4 us of matrix-core time per term.
+// row-major order measured, and the addresses are simpler).  A operands (H) stay
+// in the lane's registers, up to what 256 registers hold beside the products (23
+// groups at R = 4), and in LDS from there on.  At R = 4 a group is 8 MFMAs of 16
+// cycles on one load; N = 4096: 32 groups per wave, 3.4 us of matrix-core time per
+// term.
 //
 // Exchange: T_k goes to slot k % slots of a ring with stores that bypass the
 // XCD's L2 (device scope); the storing wave waits for them and then raises the
@@ -118,6 +119,7 @@ void coop_forget(const CoopOwner& who) {
 // waiting for good, the kernel drains, and its workgroup's accumulators are
 // written as NaN, which the caller's norm check turns into a repeat of the
 // step with one launch per term.
+//
 // Copies of the flags, each polled by every RS_COPIES-th workgroup: with one
 // copy the 2048 waves' polls of the same few lines queue up at one memory
 // channel (a term at N = 4096, R = 4: 8.9 us with one copy, 7.6 with 8).
@@ -165,9 +167,9 @@ __device__ __forceinline__ void rs_lds_barrier() { asm volatile("s_waitcnt lgkmc
 // ahead of the products through the whole unrolled sequence.  Groups past the
 // system's own count are zero, and the order of the others (rs_first) and every
 // rounding of the term are the same for each NT, so a batch member's bits do not
-// depend on the larger members that share its launch.  (batch of 64 systems of N
-// 256-2048, 4 wavepackets: 133 ms with an order of its own per NT, 135 so.)  blk of
-// nblk: this workgroup's place in its system.
+// depend on the larger members that share its launch (64 systems of N 256-2048, 4
+// wavepackets, 40 steps: 131 to 135 ms so and with an order of its own per NT).
+// blk of nblk: this workgroup's place in its system.
 constexpr int rs_most(int rc) { return rc == 0 ? 24 : rc == 1 ? 23 : 22; }
 constexpr int rs_max_groups(int rc) { return rc == 2 ? 30 : 32; }
 // A term takes the register groups 0 .. most - 1 in order, and LDS group most + l
@@ -631,7 +633,9 @@ static hipError_t resident_launch(const ResidentArgs& a, const ResidentPlan& p, 
     return resident_pick<4, 2, 18, 30, 2>(a, p, who, st);
 }
 
-// scratch: flags, then as many ring slots as fit (at least 4)
+// scratch: flags, then as many ring slots as fit (at least 4, which the partial-sum
+// buffer of a system does not hold at N <= 256 with 4 or 8 columns, nor at N <= 512
+// with 6)
 static bool resident_scratch(ResidentArgs* a, void* scratch, long scratch_bytes) {
     const long fb = resident_flag_bytes(a->ld), sb = resident_slot_bytes(a->ld, a->R);
     const long slots = resident_slots(a->ld, a->R, scratch_bytes);

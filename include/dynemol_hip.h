@@ -108,8 +108,9 @@ int dh_set_lanczos(dh_system *sys, int steps, double rel_margin);
  * observables stay FP64; 2 = FP32-stored operator: the terms read an FP32
  * copy of H_orth (half the bytes of the HBM-bound few-wavepacket term) and
  * widen it to FP64, so products and sums are FP64 and the only error is the
- * rounding of H_orth itself; 3 = mixed with the FP64 residual correction: mode
- * 1's FP32 products plus the products of the residual H_orth - fl32(H_orth)
+ * rounding of H_orth itself (for more than 4096 orbitals: below, mode 0's series
+ * in one launch reads H_orth once and is faster); 3 = mixed with the FP64
+ * residual correction: mode 1's FP32 products plus the products of the residual H_orth - fl32(H_orth)
  * (stored in bf16, bf16 matrix-core products with FP32 accumulators of their
  * own, added to the main products in FP64), so the terms apply H_orth to 2^-32 relative instead of
  * 2^-24.  Modes 1 and 3 restore each step's FP64 norms.  No counterpart in the
@@ -154,7 +155,8 @@ int dh_propagate(dh_system *sys, double t_init, double t_max, int *n_terms);
  * (n_steps - 1) / r geometries, all copied to the device at the start).  Each
  * rebuild runs on a second stream of the context, into a second set of
  * operator buffers, while the interval before it propagates (it is launched
- * before that interval's steps, without host waits), and is swapped in at its
+ * before that interval's steps, without host waits; kernels of a build and a
+ * series that fills the chip alternate), and is swapped in at its
  * step (the system and the context then hold about 7 N^2 doubles more).  The
  * host waits once per rebuild interval, where the norms of the interval's
  * steps and the rebuild's Cholesky status are checked (a failed rebuild
@@ -207,8 +209,10 @@ int dh_set_timing(dh_system *sys, int on);
  * and term kernel): within a rebuild interval the operator is fixed and the
  * terms T_k(Hh) phi do not depend on time, so one recurrence to the last
  * step's K collects every step's state, each with its own coefficients (a
- * series of up to 8 columns and 4096 orbitals in FP64 runs in one launch with
- * the operator on the chip and keeps the accumulators there; the symmetric
+ * series of up to 8 columns and 4096 orbitals (3840 above 4 columns) in FP64
+ * runs in one launch with the operator on the chip and keeps the accumulators
+ * there, except for systems whose scratch does not hold its exchange: up to 256
+ * orbitals with 2 or 4 wavepackets, up to 512 with 3; the symmetric
  * half-storage terms add each term to the step accumulators in their epilogue;
  * the other term kernels leave the terms in a 16-slot ring that a pass adds to
  * the accumulators every 16 terms).  m = 0
@@ -243,12 +247,14 @@ int dh_matvec_tuning(dh_system *sys, int *out7);
 /*
  * Multi-system batch: n systems of possibly different N with the same number
  * of wavepackets (1, 2, 4, 8 or 16), advanced together: members of up to 4
- * wavepackets and 2048 orbitals by a few launches per series, each over as many
- * members as the chip holds with their operators in registers; the others by one
- * grouped launch per Chebyshev term (FP64 members; members in other precision
- * modes run their own term kernels in the same step).  The systems stay owned by the caller; results are read per
- * system with dh_get_wavepacket / dh_get_observables.  No counterpart in the
- * reference (one system per process, ElHl_Chebyshev.f:148-291).
+ * wavepackets and 2048 orbitals (above 256 orbitals for 2 or 4 wavepackets) by a
+ * few launches per series, each over as many members as the chip holds with their
+ * operators in registers; the others by one grouped launch per Chebyshev term
+ * (FP64 members; members in other precision modes run their own term kernels in
+ * the same step).  A member's result does not depend on the others.  The systems
+ * stay owned by the caller; results are read per system with dh_get_wavepacket /
+ * dh_get_observables.  No counterpart in the reference (one system per process,
+ * ElHl_Chebyshev.f:148-291).
  */
 typedef struct dh_batch dh_batch;
 int dh_batch_create(dh_context *ctx, int n, dh_system *const *systems, dh_batch **batch);
